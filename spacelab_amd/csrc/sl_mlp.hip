@@ -5,6 +5,15 @@
 // inference are all device kernels; every reduction has a fixed order, so a run is
 // reproducible bit for bit.
 //
+// Two forms, chosen by the layer widths (CHAIN_MAX), with the same results bit for bit:
+//   chain   k_chain takes 16 samples through all layers, the loss and the backward
+//           products in one launch (every step but the weight gradients is local to a
+//           sample), k_wgrad forms the weight and bias gradients of all layers and applies
+//           Adam.  Two launches a training step, one an inference; the batch is read from
+//           and the results written to pinned host memory by the kernels themselves.
+//   layers  one launch per product (k_gemm), for wide networks, where a 16-sample
+//           workgroup would read each layer's whole weight matrix alone.
+//
 // Output layout: y[0..2] are the class logits (stick, bounce, fragment), y[3..] are
 // regression targets.  Loss per sample: softmax cross-entropy of the logits plus the
 // mean squared error of the regression outputs; the batch loss is their mean.
@@ -12,11 +21,13 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <cstring>
 #include <new>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 namespace {
@@ -31,22 +42,8 @@ constexpr int GN = 32;         // GEMM block tile columns
 constexpr int GK = 64;         // GEMM K step staged in LDS
 constexpr int NCLS = 3;
 
-__host__ __device__ inline bf16 to_bf16(float f)
-{
-    uint32_t u;
-    std::memcpy(&u, &f, 4);
-    if ((u & 0x7f800000u) == 0x7f800000u) return (bf16)((u >> 16) | ((u & 0xffff) ? 0x40 : 0));   // inf / nan
-    u += 0x7fffu + ((u >> 16) & 1u);   // round to nearest even
-    return (bf16)(u >> 16);
-}
-
-__host__ __device__ inline float from_bf16(bf16 h)
-{
-    const uint32_t u = (uint32_t)h << 16;
-    float f;
-    std::memcpy(&f, &u, 4);
-    return f;
-}
+// Round to nearest even (the hardware's conversion).
+__device__ __forceinline__ bf16 to_bf16(float f) { return __builtin_bit_cast(bf16, (__bf16)f); }
 
 // C[M][N] = op(A)[M][K] * op(B)[K][N] (+ bias[N]) with bfloat16 operands and binary32
 // accumulation.  op(A)(m, k) = TA ? A[k * lda + m] : A[m * lda + k]; op(B)(k, n) =
@@ -145,12 +142,6 @@ __global__ __launch_bounds__(256) void k_gemm(int M, int N, int K, const bf16* A
     }
 }
 
-__global__ void k_f32_to_bf16(int n, const float* x, bf16* y)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) y[i] = to_bf16(x[i]);
-}
-
 // Rows of x (n_in wide) into a zero-padded bfloat16 matrix ld wide.
 __global__ void k_pack_input(int B, int n_in, int ld, const float* x, bf16* xb)
 {
@@ -160,14 +151,11 @@ __global__ void k_pack_input(int B, int n_in, int ld, const float* x, bf16* xb)
     xb[i] = c < n_in ? to_bf16(x[(size_t)r * n_in + c]) : (bf16)0;
 }
 
-// Loss and its gradient with respect to the outputs, one thread per sample:
-// CE(softmax(y[0..2]), cls) + mean_k (y[3+k] - t_k)^2, gradient scaled by 1 / B.
-__global__ void k_loss(int B, int n_out, int ldy, const float* y, const int* cls, const float* reg, float* dy,
-                       bf16* dyb, float* loss_s)
+// Loss of one sample and its gradient with respect to the outputs (in place over the
+// outputs z[0 .. ldy)): CE(softmax(z[0..2]), c) + mean_k (z[3+k] - reg[k])^2, gradient
+// scaled by invB.
+__device__ __forceinline__ float sample_loss(float* z, int n_out, int ldy, int c, const float* reg, float invB)
 {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= B) return;
-    const float* z = y + (size_t)b * ldy;
     float mx = z[0];
     for (int k = 1; k < NCLS; k++) mx = fmaxf(mx, z[k]);
     float se = 0.f, p[NCLS];
@@ -175,20 +163,28 @@ __global__ void k_loss(int B, int n_out, int ldy, const float* y, const int* cls
         p[k] = expf(z[k] - mx);
         se += p[k];
     }
-    const int c = cls[b];
     float loss = logf(se) + mx - z[c];
     const int nr = n_out - NCLS;
-    float* g = dy + (size_t)b * ldy;
-    const float invB = 1.0f / (float)B;
-    for (int k = 0; k < NCLS; k++) g[k] = (p[k] / se - (k == c ? 1.f : 0.f)) * invB;
+    for (int k = 0; k < NCLS; k++) z[k] = (p[k] / se - (k == c ? 1.f : 0.f)) * invB;
     for (int k = 0; k < nr; k++) {
-        const float d = z[NCLS + k] - reg[(size_t)b * nr + k];
+        const float d = z[NCLS + k] - reg[k];
         loss += d * d / (float)nr;
-        g[NCLS + k] = 2.f * d / (float)nr * invB;
+        z[NCLS + k] = 2.f * d / (float)nr * invB;
     }
-    for (int k = n_out; k < ldy; k++) g[k] = 0.f;
+    for (int k = n_out; k < ldy; k++) z[k] = 0.f;
+    return loss;
+}
+
+// One thread per sample; the gradient goes to dy (binary32) and dyb (bfloat16).
+__global__ void k_loss(int B, int n_out, int ldy, const float* y, const int* cls, const float* reg, float* dy,
+                       bf16* dyb, float* loss_s)
+{
+    const int b = blockIdx.x * blockDim.x + threadIdx.x;
+    if (b >= B) return;
+    float* g = dy + (size_t)b * ldy;
+    for (int k = 0; k < ldy; k++) g[k] = y[(size_t)b * ldy + k];
+    loss_s[b] = sample_loss(g, n_out, ldy, cls[b], reg + (size_t)b * (n_out - NCLS), 1.0f / (float)B);
     for (int k = 0; k < ldy; k++) dyb[(size_t)b * ldy + k] = to_bf16(g[k]);
-    loss_s[b] = loss;
 }
 
 // dZ = dH * (Z > 0): ReLU backward, in binary32 and bfloat16.
@@ -201,28 +197,33 @@ __global__ void k_relu_back(int n, const float* z, float* dz, bf16* dzb)
     dzb[i] = to_bf16(g);
 }
 
-// Adam (Kingma & Ba 2015) on binary32 master weights, refreshing the bfloat16 copy.
-__global__ void k_adam(int n, float* w, bf16* wb, const float* g, float* m, float* v, float lr, float b1, float b2,
-                       float eps, float c1, float c2)
+// Adam (Kingma & Ba 2015) on binary32 master weights: the step's constants, and the update
+// of one value.
+struct Adam {
+    float lr, b1, b2, eps, c1, c2;
+};
+
+__device__ __forceinline__ float adam_value(const Adam& a, float w, float g, float& m, float& v)
+{
+    const float mi = a.b1 * m + (1.f - a.b1) * g;
+    const float vi = a.b2 * v + (1.f - a.b2) * g * g;
+    m = mi;
+    v = vi;
+    return w - a.lr * (mi / a.c1) / (sqrtf(vi / a.c2) + a.eps);
+}
+
+__global__ void k_adam(int n, float* w, bf16* wb, const float* g, float* m, float* v, Adam a)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const float gi = g[i];
-    const float mi = b1 * m[i] + (1.f - b1) * gi;
-    const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-    m[i] = mi;
-    v[i] = vi;
-    const float wi = w[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+    const float wi = adam_value(a, w[i], g[i], m[i], v[i]);
     w[i] = wi;
     if (wb) wb[i] = to_bf16(wi);
 }
 
-// Softmax probabilities and predictive entropy (nats) of the class logits.
-__global__ void k_predict(int B, int ldy, const float* y, float* prob, float* ent)
+// Softmax probabilities and predictive entropy (nats) of one sample's class logits.
+__device__ __forceinline__ float sample_predict(const float* z, float* prob)
 {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= B) return;
-    const float* z = y + (size_t)b * ldy;
     float mx = z[0];
     for (int k = 1; k < NCLS; k++) mx = fmaxf(mx, z[k]);
     float p[NCLS], se = 0.f;
@@ -233,16 +234,427 @@ __global__ void k_predict(int B, int ldy, const float* y, float* prob, float* en
     float h = 0.f;
     for (int k = 0; k < NCLS; k++) {
         p[k] /= se;
-        prob[(size_t)b * NCLS + k] = p[k];
+        prob[k] = p[k];
         if (p[k] > 0.f) h -= p[k] * logf(p[k]);
     }
-    ent[b] = h;
+    return h;
+}
+
+__global__ void k_predict(int B, int ldy, const float* y, float* prob, float* ent)
+{
+    const int b = blockIdx.x * blockDim.x + threadIdx.x;
+    if (b >= B) return;
+    ent[b] = sample_predict(y + (size_t)b * ldy, prob + (size_t)b * NCLS);
+}
+
+// ---- the chain form -------------------------------------------------------------------
+
+constexpr int CHAIN_ROWS = 16;           // samples per workgroup: one MFMA tile of rows
+// Widest (padded) layer the chain form takes: two column tiles per wavefront, the ReLU masks
+// in one register, the activations in LDS.  Measured there (21-W-W-W-9, us per call, chain /
+// layers): W 512 batch 16 training 74 / 253, batch 256 78 / 340, batch 4096 169 / 1622,
+// inference 35 / 152, 36 / 180, 52 / 262; W 128 batch 256 38 / 226 and 27 / 135.
+constexpr int CHAIN_MAX = 512;
+constexpr int CHAIN_WAVES = 16;          // most wavefronts per workgroup
+constexpr int CHAIN_LD = CHAIN_MAX + 8;  // row stride of the activations in LDS: 16-byte reads of 16 rows, no conflicts
+constexpr int KF = 8;                    // weight fragments (32 of K each) a lane holds at once
+
+struct ChainArgs {
+    int B, n_in, n_out;
+    int ld[NL + 1];                 // padded widths: input, hidden layers, output
+    const float* x;                 // [B][n_in]
+    const int* cls;
+    const float* reg;               // [B][n_out - 3]
+    const bf16* Wf[NL];             // forward weights (K inputs, N outputs) as fragments
+    const bf16* Wr[NL];             // backward ones (K outputs, N inputs)
+    const float* b[NL];
+    // training: inputs and output gradients of every layer for k_wgrad, feature-major
+    // ([feature][ldb], K = sample contiguous); the gradients in binary32 too ([B][ld])
+    bf16* Ht[NL];
+    bf16* dZt[NL];
+    float* dZ[NL];
+    int ldb;
+    float* loss;                    // [B]
+    float *y, *prob, *ent;          // inference: [B][n_out], [B][3], [B]
+};
+
+// Weights for the chain are kept in the order the MFMA fragments want them: for a product
+// with K inputs and N outputs, 1 KB per (16 outputs, 32 inputs), lane l's eight values (output
+// l % 16, inputs 8 (l / 16) .. + 7 of the 32, zero past K) at 16 l bytes, the tiles of
+// 16 outputs one after another.  A wavefront's load is then 1 KB in a row; with the rows
+// of a plain [out][in] matrix it was 16 pieces of 64 bytes, and a layer of 256 x 256
+// took 4.3 us to reach a CU.  frag_at: element (k, n) of such a matrix of ks steps.
+__device__ __forceinline__ size_t frag_at(int k, int n, int ks)
+{
+    return ((size_t)(n / 16 * ks + k / 32) * 64 + k % 32 / 8 * 16 + n % 16) * 8 + k % 8;
+}
+
+__host__ __device__ inline int k_steps(int K) { return (K + 31) / 32; }
+
+// The fragments of output tile `tile`, steps s0 .. s0 + F - 1 (the last step again past the
+// end: every path sends the same number of loads, which lets the compiler wait for one
+// product's loads while the next one's stay in flight).
+template <int F>
+__device__ __forceinline__ void load_frags(bf16x8_t (&wf)[KF], const bf16* mat, int tile, int ks, int s0)
+{
+    const bf16x8_t* p = reinterpret_cast<const bf16x8_t*>(mat) + (size_t)tile * ks * 64 + threadIdx.x % 64;
+#pragma unroll
+    for (int s = 0; s < F; s++) wf[s] = p[min(s0 + s, ks - 1) * 64];
+}
+
+// One wavefront's 16 x 16 tile of (16 samples in LDS) x (weights): wf holds the first F
+// steps' fragments, loaded ahead by the caller.  The K values of a lane are those of
+// k_gemm and the steps ascend, so the sums have k_gemm's bits.
+template <int F>
+__device__ __forceinline__ float4_t chain_tile(const bf16 (*A)[CHAIN_LD], bf16x8_t (&wf)[KF], const bf16* mat,
+                                               int tile, int ks)
+{
+    const int l = threadIdx.x % 64;
+    const bf16* row = &A[l % 16][8 * (l / 16)];
+    float4_t acc = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < F; s++) {
+        if (s >= ks) break;
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8_t*>(row + 32 * s), wf[s], acc, 0, 0, 0);
+    }
+    for (int s0 = F; s0 < ks; s0 += F) {
+        load_frags<F>(wf, mat, tile, ks, s0);
+#pragma unroll
+        for (int s = 0; s < F; s++) {
+            if (s0 + s >= ks) break;
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8_t*>(row + 32 * (s0 + s)), wf[s],
+                                                          acc, 0, 0, 0);
+        }
+    }
+    return acc;
+}
+
+// Workgroup barrier for data passed through LDS only: unlike __syncthreads it leaves
+// global loads (the next layers' weights) in flight.
+__device__ __forceinline__ void lds_barrier()
+{
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// Four consecutive samples of one feature as bfloat16, at sample offset q of its row.
+__device__ __forceinline__ void store4(bf16* row, int q, const float (&v)[4])
+{
+    typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
+    *reinterpret_cast<bf16x4_t*>(row + q) = bf16x4_t{(__bf16)v[0], (__bf16)v[1], (__bf16)v[2], (__bf16)v[3]};
+}
+
+// Forward pass of 16 samples through every layer (and, TRAIN, loss and backward products
+// down to the first hidden layer's gradient), one workgroup.  Wavefront w makes the
+// column tiles w, w + nw of each layer; the activations pass from layer to layer
+// through LDS, one barrier each.  A lane that makes (sample, feature) forward makes it
+// backward too, so the ReLU masks stay in registers.
+// Bound by latency, not by throughput: 16 workgroups at batch 256, each a chain of four
+// (training: seven) products whose weights come from L2 and beyond.  So the weights of the
+// next two products are always on the way: two fragment buffers, each refilled as soon
+// as its product is done; biases, labels and targets are fetched at the start, because a
+// load waits for all those sent before it.  Measured at 21-256-256-256-9, batch 256: 20.9
+// us training (5 us of it the batch's way from host memory, 2 us a product), 15.4 us
+// inference; the products one by one took 17 us each forward, 13 and 18 us backward.
+// F0, FL: fragments held of the first product's and the first backward product's K (1 when
+// the network has at most 32 inputs or outputs, else KF).
+template <bool TRAIN, int F0, int FL>
+__global__ __launch_bounds__(CHAIN_WAVES * 64) void k_chain(ChainArgs a)
+{
+    __shared__ __attribute__((aligned(16))) bf16 act[2][CHAIN_ROWS][CHAIN_LD];
+    __shared__ float yf[CHAIN_ROWS][CHAIN_MAX + 1];
+    __shared__ float rg[TRAIN ? CHAIN_ROWS : 1][TRAIN ? CHAIN_MAX : 1];   // regression targets
+    __shared__ float bs[NL][CHAIN_MAX];                                   // biases
+    const int t = threadIdx.x, nt = blockDim.x, nw = nt / 64;
+    const int w = __builtin_amdgcn_readfirstlane(t / 64), l = t % 64;
+    const int m0 = blockIdx.x * CHAIN_ROWS;
+    const int r0 = 4 * (l / 16), cl = l % 16;     // this lane's rows r0 .. r0 + 3 and column within a tile
+    bf16x8_t wf[2][KF];
+    // Product p of the chain: 0 .. NL - 1 forward, then backward through layers NL - 1 .. 1.
+    // ask(p) sends for its first tile's fragments (a wavefront without a tile: the last one's).
+    auto ask = [&](auto pc) {
+        constexpr int p = decltype(pc)::value;
+        constexpr int k = p < NL ? p : 2 * NL - 1 - p;
+        const bf16* mat = p < NL ? a.Wf[k] : a.Wr[k];
+        const int K = p < NL ? a.ld[k] : a.ld[k + 1], N = p < NL ? a.ld[k + 1] : a.ld[k];
+        constexpr int F = p == 0 ? F0 : p == NL ? FL : KF;
+        load_frags<F>(wf[p & 1], mat, min(w, N / 16 - 1), k_steps(K), 0);
+    };
+    ask(std::integral_constant<int, 0>{});
+    ask(std::integral_constant<int, 1>{});
+    // the input rows, padded with zeros to a multiple of 32, the labels and the targets
+    int cls = 0;
+    if (TRAIN && t < CHAIN_ROWS && m0 + t < a.B) cls = a.cls[m0 + t];
+#pragma unroll 1
+    for (int r = w; r < CHAIN_ROWS; r += nw) {
+        const size_t b = m0 + r;
+        const bool in = m0 + r < a.B;
+#pragma unroll 1
+        for (int c = l; c < 32 * k_steps(a.ld[0]); c += 64)
+            act[0][r][c] = to_bf16(in && c < a.n_in ? a.x[b * a.n_in + c] : 0.f);
+        if (TRAIN && in)
+#pragma unroll 1
+            for (int c = l; c < a.n_out - NCLS; c += 64) rg[r][c] = a.reg[b * (a.n_out - NCLS) + c];
+    }
+    for (int k = 0; k < NL; k++)
+#pragma unroll 1
+        for (int c = t; c < a.ld[k + 1]; c += nt) bs[k][c] = a.b[k][c];
+    lds_barrier();
+    if (TRAIN)
+#pragma unroll 1
+        for (int e = t; e < 4 * a.ld[0]; e += nt) {
+            const int c = e / 4, q = 4 * (e % 4);
+            const unsigned lo = (unsigned)act[0][q][c] | (unsigned)act[0][q + 1][c] << 16;
+            const unsigned hi = (unsigned)act[0][q + 2][c] | (unsigned)act[0][q + 3][c] << 16;
+            *reinterpret_cast<uint2*>(a.Ht[0] + (size_t)c * a.ldb + m0 + q) = make_uint2(lo, hi);
+        }
+    unsigned mask = 0;   // 4 bits per hidden layer and tile of this wavefront: the outputs above 0
+    auto fwd = [&](auto kc) {
+        constexpr int k = decltype(kc)::value;
+        constexpr bool last = k == NL - 1;
+        constexpr int F = k == 0 ? F0 : KF;
+        const int N = a.ld[k + 1], ks = k_steps(a.ld[k]);
+        auto tile = [&](int n0, int ti) {
+            const float bias = bs[k][n0 + cl];
+            const float4_t acc = chain_tile<F>(act[k & 1], wf[k & 1], a.Wf[k], n0 / 16, ks);
+            float v[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                v[r] = acc[r] + bias;
+                if (!last && v[r] < 0.f) v[r] = 0.f;
+            }
+            if (last) {
+#pragma unroll
+                for (int r = 0; r < 4; r++) yf[r0 + r][n0 + cl] = v[r];
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    act[(k + 1) & 1][r0 + r][n0 + cl] = to_bf16(v[r]);
+                    if (TRAIN) {
+                        if (v[r] > 0.f) mask |= 1u << (8 * k + 4 * ti + r);
+                        if (m0 + r0 + r >= a.B) v[r] = 0.f;   // rows past the batch: nothing for k_wgrad
+                    }
+                }
+                if (TRAIN) store4(a.Ht[last ? 0 : k + 1] + (size_t)(n0 + cl) * a.ldb, m0 + r0, v);
+            }
+        };
+        if (16 * w < N) tile(16 * w, 0);
+        if (16 * (w + nw) < N) {   // at most two tiles: CHAIN_MAX / 16 / CHAIN_WAVES
+            load_frags<F>(wf[k & 1], a.Wf[k], w + nw, ks, 0);
+            tile(16 * (w + nw), 1);
+        }
+        if (!last && (N & 16) && w == nw - 1)
+            for (int r = 0; r < 4; r++) act[(k + 1) & 1][r0 + r][N + cl] = 0;
+        if constexpr (k + 2 < (TRAIN ? 2 * NL - 1 : NL)) ask(std::integral_constant<int, k + 2>{});
+        lds_barrier();
+    };
+    fwd(std::integral_constant<int, 0>{});
+    fwd(std::integral_constant<int, 1>{});
+    fwd(std::integral_constant<int, 2>{});
+    fwd(std::integral_constant<int, 3>{});
+    const int ldy = a.ld[NL];
+    if constexpr (!TRAIN) {
+#pragma unroll 1
+        for (int r = w; r < CHAIN_ROWS; r += nw)
+            if (m0 + r < a.B)
+#pragma unroll 1
+                for (int c = l; c < a.n_out; c += 64) a.y[(size_t)(m0 + r) * a.n_out + c] = yf[r][c];
+        if (t < CHAIN_ROWS && m0 + t < a.B) {
+            float p[NCLS];
+            a.ent[m0 + t] = sample_predict(yf[t], p);
+            for (int k = 0; k < NCLS; k++) a.prob[(size_t)(m0 + t) * NCLS + k] = p[k];
+        }
+        return;
+    }
+    // loss and output gradient (the forward products left act[0] free: NL is even)
+    if (t < CHAIN_ROWS) {
+        const int b = m0 + t;
+        if (b < a.B)
+            a.loss[b] = sample_loss(yf[t], a.n_out, ldy, cls, rg[t], 1.0f / (float)a.B);
+        else
+            for (int k = 0; k < ldy; k++) yf[t][k] = 0.f;
+    }
+    lds_barrier();
+#pragma unroll 1
+    for (int r = w; r < CHAIN_ROWS; r += nw)
+#pragma unroll 1
+        for (int c = l; c < 32 * k_steps(ldy); c += 64) {
+            const float g = c < ldy ? yf[r][c] : 0.f;
+            act[0][r][c] = to_bf16(g);
+            if (c < ldy && m0 + r < a.B) a.dZ[NL - 1][(size_t)(m0 + r) * ldy + c] = g;
+        }
+#pragma unroll 1
+    for (int e = t; e < 4 * ldy; e += nt) {
+        const int c = e / 4, q = 4 * (e % 4);
+        const float v[4] = {yf[q][c], yf[q + 1][c], yf[q + 2][c], yf[q + 3][c]};
+        store4(a.dZt[NL - 1] + (size_t)c * a.ldb, m0 + q, v);
+    }
+    lds_barrier();
+    auto bwd = [&](auto pc) {
+        constexpr int p = decltype(pc)::value;
+        constexpr int k = 2 * NL - 1 - p;             // the layer gone back through
+        constexpr int F = p == NL ? FL : KF;
+        constexpr int cur = p & 1;                    // act[0] holds the output gradient: NL is even
+        const int N = a.ld[k], ks = k_steps(a.ld[k + 1]);
+        auto tile = [&](int n0, int ti) {
+            const float4_t acc = chain_tile<F>(act[cur], wf[p & 1], a.Wr[k], n0 / 16, ks);
+            float v[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const bool in = m0 + r0 + r < a.B;
+                v[r] = in && ((mask >> (8 * (k - 1) + 4 * ti + r)) & 1u) ? acc[r] : 0.f;
+                if (in) a.dZ[k - 1][(size_t)(m0 + r0 + r) * N + n0 + cl] = v[r];
+                act[cur ^ 1][r0 + r][n0 + cl] = to_bf16(v[r]);
+            }
+            store4(a.dZt[k - 1] + (size_t)(n0 + cl) * a.ldb, m0 + r0, v);
+        };
+        if (16 * w < N) tile(16 * w, 0);
+        if (16 * (w + nw) < N) {
+            load_frags<F>(wf[p & 1], a.Wr[k], w + nw, ks, 0);
+            tile(16 * (w + nw), 1);
+        }
+        if ((N & 16) && w == nw - 1)
+            for (int r = 0; r < 4; r++) act[cur ^ 1][r0 + r][N + cl] = 0;
+        if constexpr (p + 2 < 2 * NL - 1) ask(std::integral_constant<int, p + 2>{});
+        lds_barrier();
+    };
+    bwd(std::integral_constant<int, NL>{});
+    bwd(std::integral_constant<int, NL + 1>{});
+    bwd(std::integral_constant<int, NL + 2>{});
+}
+
+// Weight and bias gradients of every layer from k_chain's feature-major buffers, then
+// Adam (STEP) or the gradients stored.  One wavefront per 16 x 16 tile of a layer's H^T dZ
+// (K = the batch, ascending: k_gemm's sums), both operands read as 16-byte fragments straight
+// from memory, KF steps in flight; after the weight tiles, one workgroup per 32 columns
+// of a layer's bias (8 row phases per column as in k_gemm).
+// Bound by latency: 560 tiles of 8 steps at batch 256.  The moments and weights a
+// tile updates are loaded beside its first operands.  Measured at 21-256-256-256-9, batch
+// 256: 5.6 us; four products of 18 us and eight Adam launches of 2.4 us before.
+struct WgradArgs {
+    int B, ldb;
+    int ld[NL + 1];
+    int tile0[NL + 1];              // first weight tile of each layer, total at the end
+    int bias0[NL + 1];              // first bias workgroup of each layer
+    int wblocks;                    // workgroups of weight tiles
+    const bf16* Ht[NL];
+    const bf16* dZt[NL];
+    const float* dZ[NL];
+    float *W[NL], *mW[NL], *vW[NL], *gW[NL];
+    bf16 *Wf[NL], *Wr[NL];
+    float *b[NL], *mb[NL], *vb[NL], *gb[NL];
+    Adam adam;
+};
+
+template <bool STEP>
+__global__ __launch_bounds__(256) void k_wgrad(WgradArgs a)
+{
+    const int tid = threadIdx.x;
+    if ((int)blockIdx.x >= a.wblocks) {
+        __shared__ float part[8][32];
+        const int q = blockIdx.x - a.wblocks;
+        int k = 0;
+        while (k + 1 < NL && q >= a.bias0[k + 1]) k++;
+        const int N = a.ld[k + 1];
+        const int cl = tid % 32, ph = tid / 32;
+        const int c = (q - a.bias0[k]) * 32 + cl;
+        float sum = 0.f;
+        if (c < N) {
+            const float* src = a.dZ[k] + c;
+#pragma unroll 8
+            for (int r = ph; r < a.B; r += 8) sum += src[(size_t)r * N];
+        }
+        part[ph][cl] = sum;
+        __syncthreads();
+        if (ph == 0 && c < N) {
+            float g = part[0][cl];
+            for (int p = 1; p < 8; p++) g += part[p][cl];
+            if (STEP)
+                a.b[k][c] = adam_value(a.adam, a.b[k][c], g, a.mb[k][c], a.vb[k][c]);
+            else
+                a.gb[k][c] = g;
+        }
+        return;
+    }
+    const int w = __builtin_amdgcn_readfirstlane(tid / 64), l = tid % 64;
+    const int tile = blockIdx.x * 4 + w;
+    if (tile >= a.tile0[NL]) return;
+    int k = 0;
+    while (k + 1 < NL && tile >= a.tile0[k + 1]) k++;
+    const int K = a.ld[k], N = a.ld[k + 1];       // the layer's input and output widths
+    const int nt = N / 16;
+    const int i0 = (tile - a.tile0[k]) / nt * 16, o0 = (tile - a.tile0[k]) % nt * 16;
+    const int out = o0 + l % 16, in0 = i0 + 4 * (l / 16);
+    float wv[4], mv[4], vv[4];
+    if (STEP) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const size_t e = (size_t)(in0 + r) * N + out;
+            wv[r] = a.W[k][e];
+            mv[r] = a.mW[k][e];
+            vv[r] = a.vW[k][e];
+        }
+    }
+    const bf16* ha = a.Ht[k] + (size_t)(i0 + l % 16) * a.ldb + 8 * (l / 16);
+    const bf16* zb = a.dZt[k] + (size_t)(o0 + l % 16) * a.ldb + 8 * (l / 16);
+    // ldb covers the batch in steps of 32; rows past it in k_chain's last 16 are zeros, and
+    // the 16 after those are not read
+    const int Bp = (a.B + CHAIN_ROWS - 1) / CHAIN_ROWS * CHAIN_ROWS;
+    float4_t acc = float4_t{0.f, 0.f, 0.f, 0.f};
+    for (int b0 = 0; b0 < Bp; b0 += 32 * KF) {
+        bf16x8_t ah[KF], bz[KF];
+#pragma unroll
+        for (int s = 0; s < KF; s++) {
+            const int q = b0 + 32 * s;
+            if (q + 8 * (l / 16) < Bp) {
+                ah[s] = *reinterpret_cast<const bf16x8_t*>(ha + q);
+                bz[s] = *reinterpret_cast<const bf16x8_t*>(zb + q);
+            } else {
+                ah[s] = bf16x8_t{};
+                bz[s] = bf16x8_t{};
+            }
+        }
+#pragma unroll
+        for (int s = 0; s < KF; s++)
+            if (b0 + 32 * s < Bp) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[s], bz[s], acc, 0, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const size_t e = (size_t)(in0 + r) * N + out;
+        if (STEP) {
+            wv[r] = adam_value(a.adam, wv[r], acc[r], mv[r], vv[r]);
+            a.W[k][e] = wv[r];
+            a.mW[k][e] = mv[r];
+            a.vW[k][e] = vv[r];
+            a.Wr[k][frag_at(out, in0 + r, k_steps(N))] = to_bf16(wv[r]);
+        } else {
+            a.gW[k][e] = acc[r];
+        }
+    }
+    if (STEP) store4(a.Wf[k] + frag_at(in0, out, k_steps(K)), 0, wv);
+}
+
+// bfloat16 copies of one layer's weights: Wb in W's layout (layer form), or Wf and Wr as
+// fragments (chain form; the parts past the layer's widths stay as they are).
+__global__ void k_weights_bf16(int K, int N, const float* W, bf16* Wb, bf16* Wf, bf16* Wr)
+{
+    const int e = blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= K * N) return;
+    const bf16 v = to_bf16(W[e]);
+    if (Wb) {
+        Wb[e] = v;
+        return;
+    }
+    Wf[frag_at(e / N, e % N, k_steps(K))] = v;
+    Wr[frag_at(e % N, e / N, k_steps(N))] = v;
 }
 
 struct Layer {
     int in, out, ldin, ldout;   // logical and padded widths
     float* W = nullptr;         // [in][out] binary32 master (padded rows/cols are zero)
-    bf16* Wb = nullptr;         // bfloat16 copy
+    bf16* Wb = nullptr;         // bfloat16 copy (layer form)
+    bf16 *Wf = nullptr, *Wr = nullptr;   // the same as fragments, forward and backward (chain form)
     float* b = nullptr;         // [out]
     float *gW = nullptr, *gb = nullptr;
     float *mW = nullptr, *vW = nullptr, *mb = nullptr, *vb = nullptr;
@@ -252,15 +664,28 @@ struct Layer {
 
 struct sl_mlp {
     int n_in = 0, width = 0, n_out = 0, max_batch = 0;
+    bool chain = false;              // the chain form (layer widths up to CHAIN_MAX)
     hipStream_t stream = nullptr;
     Layer L[NL];
-    // activations: Z (pre-activation, binary32) and H (post-activation, bfloat16) per layer
+    // One device allocation: the parameters (per layer W then b, padded), their gradients,
+    // both moments (each in the same layout, n_flat floats), the bfloat16 copies and the
+    // activations.
+    char* pool = nullptr;
+    size_t n_flat = 0;
+    float *params = nullptr, *grads = nullptr, *moments = nullptr;
+    // One pinned host allocation: a batch and its results in the chain form (the kernels
+    // read and write it), the padded parameters during exchanges.
+    char* stage = nullptr;
+    char* stage_dev = nullptr;       // its device address
+    // chain form: activations and output gradients, feature-major, and the gradients in binary32
+    bf16 *Ht[NL] = {}, *dZt[NL] = {};
+    int ldb = 0;
+    // layer form: activations Z (post-activation, binary32) and H (bfloat16) per layer
     bf16* xb = nullptr;              // packed input [max_batch][ld0]
     float* Z[NL] = {};
     bf16* Hb[NL] = {};
-    float* dZ[NL] = {};
+    float* dZ[NL] = {};              // (both forms)
     bf16* dZb[NL] = {};
-    float* dH = nullptr;             // scratch [max_batch][width]
     float *xin = nullptr, *reg = nullptr, *loss_s = nullptr, *prob = nullptr, *ent = nullptr;
     int* cls = nullptr;
     long long t = 0;                 // Adam step
@@ -277,6 +702,29 @@ int mlp_err(sl_mlp* m, int code, const char* what)
     return code;
 }
 
+// The pinned buffer's layout for a batch of B: byte offsets of its parts.
+struct Stage {
+    size_t x, cls, reg, loss, y, prob, ent, end;
+    Stage(int B, int n_in, int n_out)
+    {
+        size_t o = 0;
+        auto part = [&](size_t words) {
+            const size_t at = o;
+            o += (4 * words + 255) / 256 * 256;
+            return at;
+        };
+        const size_t b = (size_t)B;
+        x = part(b * n_in);
+        cls = part(b);
+        reg = part(b * (n_out - NCLS));
+        loss = part(b);
+        y = part(b * n_out);
+        prob = part(b * NCLS);
+        ent = part(b);
+        end = o;
+    }
+};
+
 template <bool TA, bool TB>
 void gemm(hipStream_t st, int M, int N, int K, const bf16* A, int lda, const bf16* B, int ldb, float* C, int ldc,
           bf16* Cb, int ldcb, const float* bias, bool relu, const float* csrc = nullptr, int ldcs = 0,
@@ -289,21 +737,176 @@ void gemm(hipStream_t st, int M, int N, int K, const bf16* A, int lda, const bf1
 
 void free_mlp(sl_mlp* m)
 {
-    for (auto& L : m->L) {
-        void* p[] = {L.W, L.Wb, L.b, L.gW, L.gb, L.mW, L.vW, L.mb, L.vb};
-        for (void* q : p)
-            if (q) (void)hipFree(q);
-    }
-    for (int k = 0; k < NL; k++) {
-        void* p[] = {m->Z[k], m->Hb[k], m->dZ[k], m->dZb[k]};
-        for (void* q : p)
-            if (q) (void)hipFree(q);
-    }
-    void* p[] = {m->xb, m->dH, m->xin, m->reg, m->loss_s, m->prob, m->ent, m->cls};
-    for (void* q : p)
-        if (q) (void)hipFree(q);
+    if (m->pool) (void)hipFree(m->pool);
+    if (m->stage) (void)hipHostFree(m->stage);
     if (m->stream) (void)hipStreamDestroy(m->stream);
 }
+
+// Device memory of the model: called once to measure (base NULL) and once to place.
+size_t place(sl_mlp* m, char* base)
+{
+    size_t o = 0;
+    auto part = [&](auto*& p, size_t count) {
+        using T = std::remove_reference_t<decltype(*p)>;
+        p = reinterpret_cast<T*>(base + o);
+        o += (count * sizeof(T) + 255) / 256 * 256;
+    };
+    auto flat = [&](float*& start, auto W, auto b) {
+        start = reinterpret_cast<float*>(base + o);
+        const size_t o0 = o;
+        for (Layer& L : m->L) {
+            part(L.*W, (size_t)L.ldin * L.ldout);
+            part(L.*b, L.ldout);
+        }
+        m->n_flat = (o - o0) / sizeof(float);
+    };
+    flat(m->params, &Layer::W, &Layer::b);
+    flat(m->grads, &Layer::gW, &Layer::gb);
+    float* second = nullptr;
+    flat(m->moments, &Layer::mW, &Layer::mb);
+    flat(second, &Layer::vW, &Layer::vb);
+    const size_t mb = (size_t)m->max_batch;
+    for (int k = 0; k < NL; k++) {
+        Layer& L = m->L[k];
+        const size_t na = mb * L.ldout;
+        part(m->dZ[k], na);
+        if (m->chain) {
+            part(L.Wf, (size_t)32 * k_steps(L.ldin) * L.ldout);
+            part(L.Wr, (size_t)32 * k_steps(L.ldout) * L.ldin);
+            part(m->Ht[k], (size_t)L.ldin * m->ldb);
+            part(m->dZt[k], (size_t)L.ldout * m->ldb);
+        } else {
+            part(L.Wb, (size_t)L.ldin * L.ldout);
+            part(m->Z[k], na);
+            part(m->Hb[k], na);
+            part(m->dZb[k], na);
+        }
+    }
+    if (!m->chain) {
+        part(m->xb, mb * m->L[0].ldin);
+        part(m->xin, mb * m->n_in);
+        part(m->reg, mb * (m->n_out - NCLS));
+        part(m->loss_s, mb);
+        part(m->prob, mb * NCLS);
+        part(m->ent, mb);
+        part(m->cls, mb);
+    }
+    return o;
+}
+
+// Parameters already padded in the pinned buffer: to the device, with their bfloat16 copies.
+int push_params(sl_mlp* m)
+{
+    if (hipMemcpyAsync(m->params, m->stage, sizeof(float) * m->n_flat, hipMemcpyHostToDevice, m->stream) != hipSuccess)
+        return SL_E_HIP;
+    for (Layer& L : m->L) {
+        const int nw = L.ldin * L.ldout;
+        k_weights_bf16<<<(nw + 255) / 256, 256, 0, m->stream>>>(L.ldin, L.ldout, L.W, L.Wb, L.Wf, L.Wr);
+    }
+    if (hipGetLastError() != hipSuccess ||
+        hipMemsetAsync(m->moments, 0, 2 * sizeof(float) * m->n_flat, m->stream) != hipSuccess ||
+        hipStreamSynchronize(m->stream) != hipSuccess)
+        return SL_E_HIP;
+    m->t = 0;
+    return SL_OK;
+}
+
+// A flat device block (parameters or gradients) into the caller's unpadded layout.
+int pull_flat(sl_mlp* m, const float* dev, float* out)
+{
+    if (hipMemcpyAsync(m->stage, dev, sizeof(float) * m->n_flat, hipMemcpyDeviceToHost, m->stream) != hipSuccess ||
+        hipStreamSynchronize(m->stream) != hipSuccess)
+        return SL_E_HIP;
+    const float* host = reinterpret_cast<const float*>(m->stage);
+    for (Layer& L : m->L) {
+        const float *W = host + (L.W - m->params), *b = host + (L.b - m->params);
+        for (int i = 0; i < L.in; i++, out += L.out) std::memcpy(out, W + (size_t)i * L.ldout, sizeof(float) * L.out);
+        std::memcpy(out, b, sizeof(float) * L.out);
+        out += L.out;
+    }
+    return SL_OK;
+}
+
+// ---- chain form ------------------------------------------------------------------------
+
+ChainArgs chain_args(sl_mlp* m, int B)
+{
+    ChainArgs a{};
+    const Stage s(m->max_batch, m->n_in, m->n_out);
+    auto at = [&](size_t o) { return reinterpret_cast<float*>(m->stage_dev + o); };
+    a.B = B;
+    a.n_in = m->n_in;
+    a.n_out = m->n_out;
+    a.ld[0] = m->L[0].ldin;
+    for (int k = 0; k < NL; k++) {
+        const Layer& L = m->L[k];
+        a.ld[k + 1] = L.ldout;
+        a.Wf[k] = L.Wf;
+        a.Wr[k] = L.Wr;
+        a.b[k] = L.b;
+        a.Ht[k] = m->Ht[k];
+        a.dZt[k] = m->dZt[k];
+        a.dZ[k] = m->dZ[k];
+    }
+    a.ldb = m->ldb;
+    a.x = at(s.x);
+    a.cls = reinterpret_cast<int*>(m->stage_dev + s.cls);
+    a.reg = at(s.reg);
+    a.loss = at(s.loss);
+    a.y = at(s.y);
+    a.prob = at(s.prob);
+    a.ent = at(s.ent);
+    return a;
+}
+
+template <bool TRAIN>
+void launch_chain(sl_mlp* m, int B)
+{
+    int widest = 0;   // column tiles of the widest layer: one wavefront each, up to CHAIN_WAVES
+    for (const Layer& L : m->L) widest = std::max(widest, L.ldout / 16);
+    const int threads = 64 * std::min(widest, CHAIN_WAVES), grid = (B + CHAIN_ROWS - 1) / CHAIN_ROWS;
+    const bool f0 = m->L[0].ldin > 32, fl = m->L[NL - 1].ldout > 32;
+    const ChainArgs a = chain_args(m, B);
+    if (f0)
+        fl ? k_chain<TRAIN, KF, KF><<<grid, threads, 0, m->stream>>>(a) : k_chain<TRAIN, KF, 1><<<grid, threads, 0, m->stream>>>(a);
+    else
+        fl ? k_chain<TRAIN, 1, KF><<<grid, threads, 0, m->stream>>>(a) : k_chain<TRAIN, 1, 1><<<grid, threads, 0, m->stream>>>(a);
+}
+
+template <bool STEP>
+void launch_wgrad(sl_mlp* m, int B, const Adam& adam)
+{
+    WgradArgs a{};
+    a.B = B;
+    a.ldb = m->ldb;
+    a.adam = adam;
+    a.ld[0] = m->L[0].ldin;
+    int bias = 0;
+    for (int k = 0; k < NL; k++) {
+        const Layer& L = m->L[k];
+        a.ld[k + 1] = L.ldout;
+        a.tile0[k + 1] = a.tile0[k] + (L.ldin / 16) * (L.ldout / 16);
+        bias += (L.ldout + 31) / 32;
+        a.bias0[k + 1] = bias;
+        a.Ht[k] = m->Ht[k];
+        a.dZt[k] = m->dZt[k];
+        a.dZ[k] = m->dZ[k];
+        a.W[k] = L.W;
+        a.mW[k] = L.mW;
+        a.vW[k] = L.vW;
+        a.gW[k] = L.gW;
+        a.Wf[k] = L.Wf;
+        a.Wr[k] = L.Wr;
+        a.b[k] = L.b;
+        a.mb[k] = L.mb;
+        a.vb[k] = L.vb;
+        a.gb[k] = L.gb;
+    }
+    a.wblocks = (a.tile0[NL] + 3) / 4;
+    k_wgrad<STEP><<<a.wblocks + bias, 256, 0, m->stream>>>(a);
+}
+
+// ---- layer form ------------------------------------------------------------------------
 
 // Forward pass of a batch already packed into m->xb: hidden layers keep their
 // post-activation values (binary32 in Z, whose sign is also the ReLU mask, and
@@ -348,24 +951,45 @@ int load_batch(sl_mlp* m, int B, const float* x)
     return hipGetLastError() == hipSuccess ? SL_OK : SL_E_HIP;
 }
 
-// forward + loss for a labelled batch; mean loss to *loss
-int loss_pass(sl_mlp* m, int B, const float* x, const int* cls, const float* reg, float* loss)
+// ---- both forms --------------------------------------------------------------------------
+
+// Forward, loss, backward and, with adam, the update of a labelled batch; the mean loss (of
+// the parameters before the update) to *loss.
+int train_pass(sl_mlp* m, int B, const float* x, const int* cls, const float* reg, float* loss, const Adam* adam)
 {
     for (int b = 0; b < B; b++)
         if (cls[b] < 0 || cls[b] >= NCLS) return mlp_err(m, SL_E_ARG, "class label outside 0..2");
-    if (load_batch(m, B, x)) return mlp_err(m, SL_E_HIP, "input upload failed");
     const int nr = m->n_out - NCLS;
-    if (hipMemcpyAsync(m->cls, cls, 4 * (size_t)B, hipMemcpyHostToDevice, m->stream) != hipSuccess ||
-        hipMemcpyAsync(m->reg, reg, 4 * (size_t)B * nr, hipMemcpyHostToDevice, m->stream) != hipSuccess)
-        return mlp_err(m, SL_E_HIP, "label upload failed");
-    forward(m, B);
-    const Layer& L = m->L[NL - 1];
-    k_loss<<<(B + 255) / 256, 256, 0, m->stream>>>(B, m->n_out, L.ldout, m->Z[NL - 1], m->cls, m->reg, m->dZ[NL - 1],
-                                                   m->dZb[NL - 1], m->loss_s);
-    std::vector<float> ls(B);
-    if (hipMemcpyAsync(ls.data(), m->loss_s, 4 * (size_t)B, hipMemcpyDeviceToHost, m->stream) != hipSuccess ||
-        hipStreamSynchronize(m->stream) != hipSuccess)
-        return mlp_err(m, SL_E_HIP, "loss read-back failed");
+    const Stage s(m->max_batch, m->n_in, m->n_out);
+    const float* ls = reinterpret_cast<const float*>(m->stage + s.loss);
+    if (m->chain) {
+        std::memcpy(m->stage + s.x, x, 4 * (size_t)B * m->n_in);
+        std::memcpy(m->stage + s.cls, cls, 4 * (size_t)B);
+        std::memcpy(m->stage + s.reg, reg, 4 * (size_t)B * nr);
+        launch_chain<true>(m, B);
+        adam ? launch_wgrad<true>(m, B, *adam) : launch_wgrad<false>(m, B, Adam{});
+    } else {
+        if (load_batch(m, B, x)) return mlp_err(m, SL_E_HIP, "input upload failed");
+        if (hipMemcpyAsync(m->cls, cls, 4 * (size_t)B, hipMemcpyHostToDevice, m->stream) != hipSuccess ||
+            hipMemcpyAsync(m->reg, reg, 4 * (size_t)B * nr, hipMemcpyHostToDevice, m->stream) != hipSuccess)
+            return mlp_err(m, SL_E_HIP, "label upload failed");
+        forward(m, B);
+        const Layer& L = m->L[NL - 1];
+        k_loss<<<(B + 255) / 256, 256, 0, m->stream>>>(B, m->n_out, L.ldout, m->Z[NL - 1], m->cls, m->reg,
+                                                       m->dZ[NL - 1], m->dZb[NL - 1], m->loss_s);
+        if (hipMemcpyAsync(m->stage + s.loss, m->loss_s, 4 * (size_t)B, hipMemcpyDeviceToHost, m->stream) != hipSuccess)
+            return mlp_err(m, SL_E_HIP, "loss read-back failed");
+        backward(m, B);
+        if (adam)
+            for (Layer& Lk : m->L) {
+                const int nw = Lk.ldin * Lk.ldout;
+                k_adam<<<(nw + 255) / 256, 256, 0, m->stream>>>(nw, Lk.W, Lk.Wb, Lk.gW, Lk.mW, Lk.vW, *adam);
+                k_adam<<<(Lk.ldout + 255) / 256, 256, 0, m->stream>>>(Lk.ldout, Lk.b, nullptr, Lk.gb, Lk.mb, Lk.vb,
+                                                                      *adam);
+            }
+    }
+    if (hipGetLastError() != hipSuccess || hipStreamSynchronize(m->stream) != hipSuccess)
+        return mlp_err(m, SL_E_HIP, "training pass failed");
     double sum = 0;
     for (int b = 0; b < B; b++) sum += ls[b];
     if (loss) *loss = (float)(sum / B);
@@ -397,13 +1021,35 @@ int sl_mlp_create(sl_mlp** out, int n_in, int width, int n_out, int max_batch, u
     m->width = width;
     m->n_out = n_out;
     m->max_batch = max_batch;
+    m->ldb = (max_batch + 31) / 32 * 32;
     const int dims[NL + 1] = {n_in, width, width, width, n_out};
+    m->chain = true;
+    for (int k = 0; k < NL; k++) {
+        Layer& L = m->L[k];
+        L.in = dims[k];
+        L.out = dims[k + 1];
+        L.ldin = pad16(L.in);
+        L.ldout = pad16(L.out);
+        if (L.ldin > CHAIN_MAX || L.ldout > CHAIN_MAX) m->chain = false;
+    }
     auto fail = [&](int code) {
         free_mlp(m);
         delete m;
         return code;
     };
     if (hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking) != hipSuccess) return fail(SL_E_HIP);
+    if (hipMalloc(&m->pool, place(m, nullptr)) != hipSuccess) return fail(SL_E_HIP);
+    place(m, m->pool);
+    // the fragments' parts past a layer's widths are zeros for good
+    if (m->chain)
+        for (Layer& L : m->L)
+            if (hipMemsetAsync(L.Wf, 0, 2 * (size_t)32 * k_steps(L.ldin) * L.ldout, m->stream) != hipSuccess ||
+                hipMemsetAsync(L.Wr, 0, 2 * (size_t)32 * k_steps(L.ldout) * L.ldin, m->stream) != hipSuccess)
+                return fail(SL_E_HIP);
+    const size_t stage = std::max(Stage(max_batch, n_in, n_out).end, sizeof(float) * m->n_flat);
+    if (hipHostMalloc(&m->stage, stage, 0) != hipSuccess ||
+        hipHostGetDevicePointer(reinterpret_cast<void**>(&m->stage_dev), m->stage, 0) != hipSuccess)
+        return fail(SL_E_HIP);
     // He-uniform initialisation from a SplitMix64 stream; padded entries are zero
     uint64_t s = seed;
     auto rnd = [&]() {
@@ -413,40 +1059,15 @@ int sl_mlp_create(sl_mlp** out, int n_in, int width, int n_out, int max_batch, u
         z ^= z >> 31;
         return ((z >> 11) + 0.5) * (1.0 / 9007199254740992.0);
     };
-    for (int k = 0; k < NL; k++) {
-        Layer& L = m->L[k];
-        L.in = dims[k];
-        L.out = dims[k + 1];
-        L.ldin = pad16(L.in);
-        L.ldout = pad16(L.out);
-        const size_t nw = (size_t)L.ldin * L.ldout;
-        std::vector<float> w(nw, 0.f), b(L.ldout, 0.f);
+    float* host = reinterpret_cast<float*>(m->stage);
+    std::memset(host, 0, sizeof(float) * m->n_flat);
+    for (Layer& L : m->L) {
+        float* W = host + (L.W - m->params);
         const double lim = std::sqrt(6.0 / L.in);
         for (int i = 0; i < L.in; i++)
-            for (int j = 0; j < L.out; j++) w[(size_t)i * L.ldout + j] = (float)((2 * rnd() - 1) * lim);
-        std::vector<bf16> wb(nw);
-        for (size_t q = 0; q < nw; q++) wb[q] = to_bf16(w[q]);
-        if (hipMalloc(&L.W, 4 * nw) || hipMalloc(&L.Wb, 2 * nw) || hipMalloc(&L.b, 4 * L.ldout) ||
-            hipMalloc(&L.gW, 4 * nw) || hipMalloc(&L.gb, 4 * L.ldout) || hipMalloc(&L.mW, 4 * nw) ||
-            hipMalloc(&L.vW, 4 * nw) || hipMalloc(&L.mb, 4 * L.ldout) || hipMalloc(&L.vb, 4 * L.ldout))
-            return fail(SL_E_HIP);
-        if (hipMemcpy(L.W, w.data(), 4 * nw, hipMemcpyHostToDevice) ||
-            hipMemcpy(L.Wb, wb.data(), 2 * nw, hipMemcpyHostToDevice) ||
-            hipMemcpy(L.b, b.data(), 4 * L.ldout, hipMemcpyHostToDevice) || hipMemset(L.mW, 0, 4 * nw) ||
-            hipMemset(L.vW, 0, 4 * nw) || hipMemset(L.mb, 0, 4 * L.ldout) || hipMemset(L.vb, 0, 4 * L.ldout) ||
-            hipMemset(L.gW, 0, 4 * nw) || hipMemset(L.gb, 0, 4 * L.ldout))
-            return fail(SL_E_HIP);
-        const size_t na = (size_t)max_batch * L.ldout;
-        if (hipMalloc(&m->Z[k], 4 * na) || hipMalloc(&m->Hb[k], 2 * na) || hipMalloc(&m->dZ[k], 4 * na) ||
-            hipMalloc(&m->dZb[k], 2 * na))
-            return fail(SL_E_HIP);
+            for (int j = 0; j < L.out; j++) W[(size_t)i * L.ldout + j] = (float)((2 * rnd() - 1) * lim);
     }
-    const int ld0 = m->L[0].ldin;
-    if (hipMalloc(&m->xb, 2 * (size_t)max_batch * ld0) || hipMalloc(&m->dH, 4 * (size_t)max_batch * pad16(width)) ||
-        hipMalloc(&m->xin, 4 * (size_t)max_batch * n_in) || hipMalloc(&m->reg, 4 * (size_t)max_batch * (n_out - NCLS)) ||
-        hipMalloc(&m->loss_s, 4 * (size_t)max_batch) || hipMalloc(&m->prob, 4 * (size_t)max_batch * NCLS) ||
-        hipMalloc(&m->ent, 4 * (size_t)max_batch) || hipMalloc(&m->cls, 4 * (size_t)max_batch))
-        return fail(SL_E_HIP);
+    if (push_params(m)) return fail(SL_E_HIP);
     *out = m;
     return SL_OK;
 }
@@ -463,37 +1084,22 @@ int sl_mlp_n_params(const sl_mlp* m)
 int sl_mlp_get_params(sl_mlp* m, float* w)
 {
     if (!m || !w) return SL_E_ARG;
-    for (Layer& L : m->L) {
-        std::vector<float> W((size_t)L.ldin * L.ldout), b(L.ldout);
-        if (hipMemcpy(W.data(), L.W, 4 * W.size(), hipMemcpyDeviceToHost) != hipSuccess ||
-            hipMemcpy(b.data(), L.b, 4 * b.size(), hipMemcpyDeviceToHost) != hipSuccess)
-            return mlp_err(m, SL_E_HIP, "parameter read-back failed");
-        for (int i = 0; i < L.in; i++)
-            for (int j = 0; j < L.out; j++) *w++ = W[(size_t)i * L.ldout + j];
-        for (int j = 0; j < L.out; j++) *w++ = b[j];
-    }
+    if (pull_flat(m, m->params, w)) return mlp_err(m, SL_E_HIP, "parameter read-back failed");
     return SL_OK;
 }
 
 int sl_mlp_set_params(sl_mlp* m, const float* w)
 {
     if (!m || !w) return SL_E_ARG;
+    float* host = reinterpret_cast<float*>(m->stage);
+    std::memset(host, 0, sizeof(float) * m->n_flat);
     for (Layer& L : m->L) {
-        const size_t nw = (size_t)L.ldin * L.ldout;
-        std::vector<float> W(nw, 0.f), b(L.ldout, 0.f);
-        for (int i = 0; i < L.in; i++)
-            for (int j = 0; j < L.out; j++) W[(size_t)i * L.ldout + j] = *w++;
-        for (int j = 0; j < L.out; j++) b[j] = *w++;
-        std::vector<bf16> Wb(nw);
-        for (size_t q = 0; q < nw; q++) Wb[q] = to_bf16(W[q]);
-        if (hipMemcpy(L.W, W.data(), 4 * nw, hipMemcpyHostToDevice) != hipSuccess ||
-            hipMemcpy(L.Wb, Wb.data(), 2 * nw, hipMemcpyHostToDevice) != hipSuccess ||
-            hipMemcpy(L.b, b.data(), 4 * L.ldout, hipMemcpyHostToDevice) != hipSuccess ||
-            hipMemset(L.mW, 0, 4 * nw) != hipSuccess || hipMemset(L.vW, 0, 4 * nw) != hipSuccess ||
-            hipMemset(L.mb, 0, 4 * L.ldout) != hipSuccess || hipMemset(L.vb, 0, 4 * L.ldout) != hipSuccess)
-            return mlp_err(m, SL_E_HIP, "parameter upload failed");
+        float *W = host + (L.W - m->params), *b = host + (L.b - m->params);
+        for (int i = 0; i < L.in; i++, w += L.out) std::memcpy(W + (size_t)i * L.ldout, w, sizeof(float) * L.out);
+        std::memcpy(b, w, sizeof(float) * L.out);
+        w += L.out;
     }
-    m->t = 0;
+    if (push_params(m)) return mlp_err(m, SL_E_HIP, "parameter upload failed");
     return SL_OK;
 }
 
@@ -501,6 +1107,17 @@ int sl_mlp_forward(sl_mlp* m, int B, const float* x, float* y, float* prob, floa
 {
     int rc = check_batch(m, B, x);
     if (rc) return rc;
+    if (m->chain) {
+        const Stage s(m->max_batch, m->n_in, m->n_out);
+        std::memcpy(m->stage + s.x, x, 4 * (size_t)B * m->n_in);
+        launch_chain<false>(m, B);
+        if (hipGetLastError() != hipSuccess || hipStreamSynchronize(m->stream) != hipSuccess)
+            return mlp_err(m, SL_E_HIP, "forward failed");
+        if (y) std::memcpy(y, m->stage + s.y, 4 * (size_t)B * m->n_out);
+        if (prob) std::memcpy(prob, m->stage + s.prob, 4 * (size_t)B * NCLS);
+        if (ent) std::memcpy(ent, m->stage + s.ent, 4 * (size_t)B);
+        return SL_OK;
+    }
     if (load_batch(m, B, x)) return mlp_err(m, SL_E_HIP, "input upload failed");
     forward(m, B);
     const Layer& L = m->L[NL - 1];
@@ -524,21 +1141,9 @@ int sl_mlp_gradients(sl_mlp* m, int B, const float* x, const int* cls, const flo
     int rc = check_batch(m, B, x);
     if (rc) return rc;
     if (!cls || !reg) return mlp_err(m, SL_E_ARG, "labels are NULL");
-    rc = loss_pass(m, B, x, cls, reg, loss);
+    rc = train_pass(m, B, x, cls, reg, loss, nullptr);
     if (rc) return rc;
-    backward(m, B);
-    if (hipStreamSynchronize(m->stream) != hipSuccess) return mlp_err(m, SL_E_HIP, "backward failed");
-    if (grads) {
-        for (Layer& L : m->L) {
-            std::vector<float> W((size_t)L.ldin * L.ldout), b(L.ldout);
-            if (hipMemcpy(W.data(), L.gW, 4 * W.size(), hipMemcpyDeviceToHost) != hipSuccess ||
-                hipMemcpy(b.data(), L.gb, 4 * b.size(), hipMemcpyDeviceToHost) != hipSuccess)
-                return mlp_err(m, SL_E_HIP, "gradient read-back failed");
-            for (int i = 0; i < L.in; i++)
-                for (int j = 0; j < L.out; j++) *grads++ = W[(size_t)i * L.ldout + j];
-            for (int j = 0; j < L.out; j++) *grads++ = b[j];
-        }
-    }
+    if (grads && pull_flat(m, m->grads, grads)) return mlp_err(m, SL_E_HIP, "gradient read-back failed");
     return SL_OK;
 }
 
@@ -547,20 +1152,12 @@ int sl_mlp_train_step(sl_mlp* m, int B, const float* x, const int* cls, const fl
     int rc = check_batch(m, B, x);
     if (rc) return rc;
     if (!cls || !reg || !(lr > 0)) return mlp_err(m, SL_E_ARG, "labels are NULL or lr <= 0");
-    rc = loss_pass(m, B, x, cls, reg, loss);
+    const float b1 = 0.9f, b2 = 0.999f;
+    const long long t = m->t + 1;
+    const Adam adam{lr, b1, b2, 1e-8f, 1.f - std::pow(b1, (float)t), 1.f - std::pow(b2, (float)t)};
+    rc = train_pass(m, B, x, cls, reg, loss, &adam);
     if (rc) return rc;
-    backward(m, B);
-    m->t++;
-    const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-    const float c1 = 1.f - std::pow(b1, (float)m->t), c2 = 1.f - std::pow(b2, (float)m->t);
-    for (Layer& L : m->L) {
-        const int nw = L.ldin * L.ldout;
-        k_adam<<<(nw + 255) / 256, 256, 0, m->stream>>>(nw, L.W, L.Wb, L.gW, L.mW, L.vW, lr, b1, b2, eps, c1, c2);
-        k_adam<<<(L.ldout + 255) / 256, 256, 0, m->stream>>>(L.ldout, L.b, nullptr, L.gb, L.mb, L.vb, lr, b1, b2, eps,
-                                                             c1, c2);
-    }
-    if (hipGetLastError() != hipSuccess || hipStreamSynchronize(m->stream) != hipSuccess)
-        return mlp_err(m, SL_E_HIP, "training step failed");
+    m->t = t;
     return SL_OK;
 }
 
