@@ -95,13 +95,14 @@ __global__ void k_copy_prev(State s, int n)
     s.f[QZ][b] = s.f[PZ][b];
 }
 
-// One touching pair (i, j) in the reference's contact arm (ColliderSingleCore.cpp:119-204),
-// in its orientation A = max(i, j): ball i's acc contribution to c3[0], c3[cs], c3[2 cs], its
-// aacc contribution likewise to a3, and the pair energy (write steps, i = A) to *pe.  The
+// One pair (i, j) in the reference's arithmetic, touching or not (ColliderSingleCore.cpp:
+// 119-250), in its orientation A = max(i, j): ball i's acc contribution to c3[0], c3[cs],
+// c3[2 cs], its aacc contribution likewise to a3, and the pair energy (write steps, i = A) to
+// *pe.  Returns 1 for a touching pair.  The
 // state is one array of fields, field f at base + f stride (how every caller lays it out),
 // passed as its base so that the caller has no field table to spill for the call.
-__device__ __forceinline__ void contact_pair_body(const double* base, long stride, const Phys& P, int write, int i,
-                                                  int j, double ymi, double* c3, double* a3, int cs, double* pe)
+__device__ __forceinline__ int contact_pair_body(const double* base, long stride, const Phys& P, int write, int i,
+                                                 int j, double ymi, double* c3, double* a3, int cs, double* pe)
 {
     State s;
     for (int f = 0; f < NFIELD; f++) s.f[f] = const_cast<double*>(base + f * stride);
@@ -131,12 +132,13 @@ __device__ __forceinline__ void contact_pair_body(const double* base, long strid
     a3[cs] = aa.y;
     a3[2 * cs] = aa.z;
     *pe = iA ? o.pe : 0.0;
+    return o.contact;
 }
 
-// A partner's position, radius and mass as the far-field arm reads them (48 bytes: three
-// 16-byte LDS reads).
+// A partner's position, radius, mass and Ha/6*64 R^3 (the first factors of the vdW prefactor
+// when the partner is A) as the far-field arm reads them (48 bytes: three 16-byte LDS reads).
 struct PartnerRec {
-    double x, y, z, R, m, pad;
+    double x, y, z, R, m, pref;
 };
 
 // One workgroup owns BI balls and sweeps every partner j in chunks of CJ.  NPW wavefronts
@@ -156,20 +158,21 @@ struct PartnerRec {
 // The far arm divides by dist and by m_i through correctly rounded reciprocals
 // (div_rcp): the same quotients as the reference's divisions, for five FMA-pipe
 // instructions each instead of a full division.
-__device__ __attribute__((noinline)) void contact_pair(const double* base, long stride, const Phys& P, int write,
-                                                       int i, int j, double ymi, double* c3, double* a3, int cs,
-                                                       double* pe)
+__device__ __attribute__((noinline)) int contact_pair(const double* base, long stride, const Phys& P, int write,
+                                                      int i, int j, double ymi, double* c3, double* a3, int cs,
+                                                      double* pe)
 {
-    contact_pair_body(base, stride, P, write, i, j, ymi, c3, a3, cs, pe);
+    return contact_pair_body(base, stride, P, write, i, j, ymi, c3, a3, cs, pe);
 }
 
 // CALL: the contact arm out of line (its registers weigh only on the calls) or inline.
 // WPE: the wavefronts per SIMD the register budget is held to (0: the compiler's choice).
 // UNR: how many of a thread's far-field pairs per chunk the sweep unrolls (the sums' order
 // is fixed by the contribution buffer, so it changes no bits).
-template <int BI, int NPW, int CJ, bool DED, bool CALL, int WPE, int UNR = 1>
+// WRITE: write steps (pair energies).
+template <int BI, int NPW, int CJ, bool DED, bool CALL, int WPE, int UNR, bool WRITE>
 __global__ __launch_bounds__((NPW + (DED ? 1 : 0)) * 64) __attribute__((amdgpu_waves_per_eu(WPE > 0 ? WPE : 1)))
-void k_pairs_ordered(State s, Phys P, int n, int write, double* __restrict__ pe_ball,
+void k_pairs_ordered(State s, Phys P, int n, double* __restrict__ pe_ball,
                      unsigned long long* __restrict__ contacts)
 {
     constexpr int NP = NPW * 64;            // producer threads
@@ -177,7 +180,7 @@ void k_pairs_ordered(State s, Phys P, int n, int write, double* __restrict__ pe_
     constexpr int KP = CJ / JQ;             // pairs per producer thread and chunk
     constexpr int MW = (CJ + 63) / 64;      // contact-mask words per ball and chunk
     constexpr int CS = CJ * BI + 4;         // quantity stride (staggers the consumer's banks)
-    constexpr int NQ = 7;                   // acc xyz, aacc xyz, pair energy
+    constexpr int NQ = WRITE ? 7 : 6;       // acc xyz, aacc xyz, pair energy
     static_assert(NP % BI == 0 && CJ % JQ == 0 && KP >= 1, "chunk shape");
     static_assert(NQ * BI <= 64, "one consumer lane per (ball, quantity)");
     constexpr int NT = (NPW + (DED ? 1 : 0)) * 64;   // threads of the workgroup
@@ -186,12 +189,16 @@ void k_pairs_ordered(State s, Phys P, int n, int write, double* __restrict__ pe_
     __shared__ unsigned long long cmask[2][BI][MW];
     __shared__ PartnerRec sp[2][CJ];                 // the partners of chunks k and k + 1
     __shared__ unsigned ccount;
+    __shared__ int general;                          // a ball or a parameter outside FarRange was met
     __shared__ double sgm[BI];                       // G m_i of the workgroup's balls
 
     const int t = threadIdx.x;
     const int w = __builtin_amdgcn_readfirstlane(t / 64);
     if (t < 2 * BI * MW) (&cmask[0][0][0])[t] = 0ull;
-    if (t == 0) ccount = 0;
+    if (t == 0) {
+        ccount = 0;
+        general = !FarRange::params(P);
+    }
     if (t < BI) sgm[t] = blockIdx.x * BI + t < n ? P.G * s.f[MASS][blockIdx.x * BI + t] : 0.0;
 
     // producer role
@@ -234,11 +241,18 @@ void k_pairs_ordered(State s, Phys P, int n, int write, double* __restrict__ pe_
 #pragma unroll
         for (int u = 0; u < NL; u++) {
             const int jl = t + u * NT;
-            if (jl < CJ && kc * CJ + jl < n) sp[kc & 1][jl] = nx[u];
+            if (jl < CJ && kc * CJ + jl < n) {
+                const double R = nx[u].R;
+                nx[u].pref = Hc * R * R * R;
+                sp[kc & 1][jl] = nx[u];
+                if (!FarRange::ball(R, nx[u].m)) general = 1;   // before the barrier that opens the chunk
+            }
         }
     };
     load_chunk(0);
+    __syncthreads();
     store_chunk(0);
+    if (!FarRange::ball(Ri, mi)) general = 1;
     __syncthreads();
     for (int k = 0; k <= nch; k++) {
         const int b = k & 1;
@@ -249,7 +263,7 @@ void k_pairs_ordered(State s, Phys P, int n, int write, double* __restrict__ pe_
             const int m = (n - (k - 1) * CJ) < CJ ? (n - (k - 1) * CJ) : CJ;
             if (consumer) {
                 const double* src = &cb[bb][cq * CS + cl];
-                if (cq < 3 || (cq == 6 && write)) {
+                if (cq < 3 || cq == 6) {
                     int jl = 0;
                     for (; jl + 8 <= m; jl += 8) {
                         double v[8];
@@ -279,10 +293,14 @@ void k_pairs_ordered(State s, Phys P, int n, int write, double* __restrict__ pe_
         if (w < NPW && k < nch) {
             const int j0 = k * CJ;
             const int i0 = blockIdx.x * BI;
-            unsigned pend = 0;   // pairs q of this chunk that touch: evaluated after the sweep
+            // pairs q of this chunk that touch, or whose operands are outside FarRange: evaluated
+            // by the general arm after the sweep
+            unsigned pend = 0;
+            const bool gen = general != 0;
             // One far-field pair (i, j) in the reference's orientation A = max(i, j): ball i
             // is A when IA (ColliderSingleCore.cpp:104-110, 211-227).  Writes ball i's acc
-            // contribution (and its energy on write steps), or marks the pair touching.
+            // contribution (and its energy on write steps), or marks the pair for the
+            // general arm.
             auto far_pair = [&](auto ia, int q) {
                 constexpr bool IA = decltype(ia)::value;
                 const int jl = jq + JQ * q;
@@ -294,9 +312,11 @@ void k_pairs_ordered(State s, Phys P, int n, int write, double* __restrict__ pe_
                     const double Rj = pr.R, mj = pr.m;
                     const double S = IA ? Ri + Rj : Rj + Ri;
                     const D3 r = IA ? pj - pi : pi - pj;               // x_B - x_A
-                    const double dist = norm(r);
+                    const double d2 = dot(r, r);
+                    double dist, yd;                                   // norm(r) and its reciprocal
+                    sqrt_rcp(d2, dist, yd);
                     const double overlap = S - dist;
-                    if (overlap > 0) {
+                    if (overlap > 0 || gen || !FarRange::distance2(d2)) {
                         pend |= 1u << q;
                     } else {
                         double h = ::fabs(overlap);
@@ -308,9 +328,8 @@ void k_pairs_ordered(State s, Phys P, int n, int write, double* __restrict__ pe_
                         const double twoRbh = IA ? (2 * Rj) * h : two_Ri * h;
                         const double sv = h2 + twoRah + twoRbh;
                         const double tv = sv + (IA ? four_Ri * Rj : (4 * Rj) * Ri);
-                        const double quot = (IA ? h + Ri + Rj : h + Rj + Ri) / (sv * sv * tv * tv);
-                        const double fv = IA ? prefA * Rj * Rj * Rj * quot : Hc * Rj * Rj * Rj * Ri * Ri * Ri * quot;
-                        const double yd = 1.0 / dist;
+                        const double quot = div_plain(IA ? h + Ri + Rj : h + Rj + Ri, sv * sv * tv * tv);
+                        const double fv = IA ? prefA * Rj * Rj * Rj * quot : pr.pref * Ri * Ri * Ri * quot;
                         const D3 rh = d3(div_rcp(r.x, dist, yd), div_rcp(r.y, dist, yd), div_rcp(r.z, dist, yd));
                         D3 F = rh * fv;
                         if (P.far_gravity) {
@@ -321,7 +340,7 @@ void k_pairs_ordered(State s, Phys P, int n, int write, double* __restrict__ pe_
                             double gmi = Gmi;
                             if constexpr (WPE > 0)
                                 gmi = __hip_atomic_load(&sgm[il], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                            F = F + rh * ((IA ? gmi * mj : P.G * mj * mi) / (dist * dist));
+                            F = F + rh * div_sq(IA ? gmi * mj : P.G * mj * mi, dist * dist, yd);
                         }
                         // acc[A] += F/m[A]  or  acc[B] -= F/m[B]   (:187-188, 249-250)
                         c0 = div_rcp(F.x, mi, ymi);
@@ -331,7 +350,7 @@ void k_pairs_ordered(State s, Phys P, int n, int write, double* __restrict__ pe_
                             c0 = -c0;
                             c1 = -c1;
                             c2 = -c2;
-                        } else if (write) {                            // :228-240
+                        } else if (WRITE) {                            // :228-240
                             u = vdw_energy(P.Ha, Ri, Rj, S, h);
                             if (P.far_gravity) u = u + -P.G * mi * mj / dist;
                         }
@@ -341,7 +360,7 @@ void k_pairs_ordered(State s, Phys P, int n, int write, double* __restrict__ pe_
                 cb[b][0 * CS + o_] = c0;
                 cb[b][1 * CS + o_] = c1;
                 cb[b][2 * CS + o_] = c2;
-                if (write) cb[b][6 * CS + o_] = u;
+                if (WRITE) cb[b][6 * CS + o_] = u;
             };
             if (j0 + CJ <= i0) {
                 // every partner of the chunk precedes every ball of the block: i is A
@@ -368,15 +387,16 @@ void k_pairs_ordered(State s, Phys P, int n, int write, double* __restrict__ pe_
                 const int jl = jq + JQ * q;
                 const int o_ = jl * BI + il;
                 double pc = 0;
+                int touch;
                 if constexpr (CALL)
-                    contact_pair(s.f[0], s.f[1] - s.f[0], P, write, i, j0 + jl, ymi, &cb[b][o_], &cb[b][3 * CS + o_],
-                                 CS, &pc);
+                    touch = contact_pair(s.f[0], s.f[1] - s.f[0], P, WRITE, i, j0 + jl, ymi, &cb[b][o_],
+                                         &cb[b][3 * CS + o_], CS, &pc);
                 else
-                    contact_pair_body(s.f[0], s.f[1] - s.f[0], P, write, i, j0 + jl, ymi, &cb[b][o_],
-                                      &cb[b][3 * CS + o_], CS, &pc);
-                if (write) cb[b][6 * CS + o_] = pc;
+                    touch = contact_pair_body(s.f[0], s.f[1] - s.f[0], P, WRITE, i, j0 + jl, ymi, &cb[b][o_],
+                                              &cb[b][3 * CS + o_], CS, &pc);
+                if (WRITE) cb[b][6 * CS + o_] = pc;
                 atomicOr(&cmask[b][il][jl >> 6], 1ull << (jl & 63));
-                if (i > j0 + jl) cnt++;
+                if (touch && i > j0 + jl) cnt++;
             }
         }
         // chunk k + 1's partners into the buffer chunk k - 1 used (all reads of it ended
@@ -392,7 +412,7 @@ void k_pairs_ordered(State s, Phys P, int n, int write, double* __restrict__ pe_
                 s.f[AX + cq][ib] = run;
             else if (cq < 6)
                 s.f[BX + cq - 3][ib] = run;
-            else if (write)
+            else if (WRITE)
                 pe_ball[ib] = run;
         }
     }
@@ -402,7 +422,7 @@ void k_pairs_ordered(State s, Phys P, int n, int write, double* __restrict__ pe_
     // contacts[0]: the running total; contacts[1]: this write step's touching pairs
     if (t == 0 && ccount) {
         atomicAdd(contacts, (unsigned long long)ccount);
-        if (write) atomicAdd(contacts + 1, (unsigned long long)ccount);
+        if (WRITE) atomicAdd(contacts + 1, (unsigned long long)ccount);
     }
 }
 
@@ -555,17 +575,26 @@ hipError_t launch_pairs_ordered(const State& s, const Phys& P, int n, int write,
     // wavefront, contact arm out of line, wavefronts per SIMD the registers are held to,
     // unroll of the far-field loop (case 5: both of a thread's pairs per chunk, 1% faster at
     // 5,000 balls than one at a time)
+#define SL_ORD(BI, NPW, CJ, DED, CALL, WPE, UNR)                                                                \
+    do {                                                                                                         \
+        constexpr int T = 64 * (NPW + (DED ? 1 : 0));                                                            \
+        if (write)                                                                                               \
+            k_pairs_ordered<BI, NPW, CJ, DED, CALL, WPE, UNR, true><<<nb, T, 0, st>>>(s, P, n, pe_ball, contacts);  \
+        else                                                                                                     \
+            k_pairs_ordered<BI, NPW, CJ, DED, CALL, WPE, UNR, false><<<nb, T, 0, st>>>(s, P, n, pe_ball, contacts); \
+    } while (0)
     switch (shape) {
-    case 0: k_pairs_ordered<2, 3, 192, true, false, 3><<<nb, 256, 0, st>>>(s, P, n, write, pe_ball, contacts); break;
-    case 1: k_pairs_ordered<4, 3, 48, true, false, 3><<<nb, 256, 0, st>>>(s, P, n, write, pe_ball, contacts); break;
-    case 2: k_pairs_ordered<4, 4, 64, false, false, 3><<<nb, 256, 0, st>>>(s, P, n, write, pe_ball, contacts); break;
-    case 3: k_pairs_ordered<8, 4, 32, false, false, 3><<<nb, 256, 0, st>>>(s, P, n, write, pe_ball, contacts); break;
-    case 4: k_pairs_ordered<2, 2, 128, false, false, 0><<<nb, 128, 0, st>>>(s, P, n, write, pe_ball, contacts); break;
-    case 5: k_pairs_ordered<4, 3, 96, true, false, 3, 2><<<nb, 256, 0, st>>>(s, P, n, write, pe_ball, contacts); break;
-    case 6: k_pairs_ordered<2, 2, 128, false, true, 0><<<nb, 128, 0, st>>>(s, P, n, write, pe_ball, contacts); break;
-    case 7: k_pairs_ordered<2, 4, 128, false, false, 3><<<nb, 256, 0, st>>>(s, P, n, write, pe_ball, contacts); break;
-    default: k_pairs_ordered<2, 4, 128, false, false, 0><<<nb, 256, 0, st>>>(s, P, n, write, pe_ball, contacts); break;
+    case 0: SL_ORD(2, 3, 192, true, false, 3, 1); break;
+    case 1: SL_ORD(4, 3, 48, true, false, 3, 1); break;
+    case 2: SL_ORD(4, 4, 64, false, false, 3, 1); break;
+    case 3: SL_ORD(8, 4, 32, false, false, 3, 1); break;
+    case 4: SL_ORD(2, 2, 128, false, false, 0, 1); break;
+    case 5: SL_ORD(4, 3, 96, true, false, 3, 2); break;
+    case 6: SL_ORD(2, 2, 128, false, true, 0, 1); break;
+    case 7: SL_ORD(2, 4, 128, false, false, 3, 1); break;
+    default: SL_ORD(2, 4, 128, false, false, 0, 1); break;
     }
+#undef SL_ORD
     return hipGetLastError();
 }
 

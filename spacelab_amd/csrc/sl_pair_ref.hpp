@@ -73,6 +73,64 @@ __device__ __forceinline__ double div_rcp(double a, double b, double y)
     return __builtin_fma(__builtin_fma(-q1, b, a), y, q1);
 }
 
+// ---- square root and division without the special cases ---------------------------------
+// For operands whose exponents (and their results') stay far inside binary64's range the
+// compiler's square root and division spend a third of their instructions on scaling and
+// special values.  These are the same iterations without those, for the far-field arm, which
+// sends pairs outside FarRange to the general arm: bit for bit sqrt(x) and n / d.
+
+// s = RN(sqrt(x)) by Goldschmidt's iteration from the hardware estimate (24 bits), two
+// corrections by the FMA-exact residual x - s^2; y = RN(1/s) from the iteration's other half,
+// h = 1/(2 sqrt x) to 46 bits, by two Newton steps (the first leaves y within an ulp, the
+// residual 1 - s y of the second is exact; only a significand of all ones can come out one
+// ulp off, where div_rcp's quotient is still right).
+__device__ __forceinline__ void sqrt_rcp(double x, double& s, double& y)
+{
+    const double y0 = __builtin_amdgcn_rsq(x);
+    const double g0 = x * y0, h0 = 0.5 * y0;
+    const double r0 = __builtin_fma(-h0, g0, 0.5);
+    const double g1 = __builtin_fma(g0, r0, g0), h1 = __builtin_fma(h0, r0, h0);
+    const double g2 = __builtin_fma(__builtin_fma(-g1, g1, x), h1, g1);
+    s = __builtin_fma(__builtin_fma(-g2, g2, x), h1, g2);
+    const double y1 = h1 + h1;
+    const double y2 = __builtin_fma(__builtin_fma(-s, y1, 1.0), y1, y1);
+    y = __builtin_fma(__builtin_fma(-s, y2, 1.0), y2, y2);
+}
+
+// RN(n / d): two Newton steps on the hardware reciprocal, one residual correction (the
+// sequence of the compiler's division).
+__device__ __forceinline__ double div_plain(double n, double d)
+{
+    double y = __builtin_amdgcn_rcp(d);
+    y = __builtin_fma(y, __builtin_fma(-d, y, 1.0), y);
+    y = __builtin_fma(y, __builtin_fma(-d, y, 1.0), y);
+    const double q = n * y;
+    return __builtin_fma(__builtin_fma(-d, q, n), y, q);
+}
+
+// n / s^2 for the distance s and y = RN(1/s): 1/s^2 from y^2 (2 ulps) by one Newton step,
+// which leaves it within 2^-48 of half an ulp of 1/s^2; div_rcp's quotient needs no more.
+__device__ __forceinline__ double div_sq(double n, double s2, double y)
+{
+    const double z = y * y;
+    return div_rcp(n, s2, __builtin_fma(__builtin_fma(-s2, z, 1.0), z, z));
+}
+
+// The range of the above: d^2 in [2^-200, 2^200) (checked pair by pair), radii and h_min in
+// [2^-100, 2^100), masses in [2^-300, 2^300), G 0 or in [2^-100, 2^100).  Then s t of the far
+// arm's denominator lies in 2^-400 .. 2^410, its square and every quotient and residual
+// inside 2^+-910.
+struct FarRange {
+    __device__ static bool within(double x, int lo, int hi)   // 2^lo <= x < 2^hi
+    {
+        const unsigned e = (unsigned)(__double_as_longlong(x) >> 52);   // sign and exponent
+        return e - (unsigned)(1023 + lo) < (unsigned)(hi - lo);
+    }
+    __device__ static bool ball(double R, double m) { return within(R, -100, 100) && within(m, -300, 300); }
+    __device__ static bool params(const Phys& P) { return within(P.h_min, -100, 100) && (P.G == 0 || within(P.G, -100, 100)); }
+    __device__ static bool distance2(double d2) { return within(d2, -200, 200); }
+};
+
 struct PairIn {
     D3 pA, pB;    // positions (after this step's drift)
     double RA, RB, mA, mB;
