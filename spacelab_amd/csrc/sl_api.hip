@@ -242,10 +242,11 @@ void clear_ord_graphs(sl_ctx* c)
 
 constexpr int ORD_GRAPH_MAX_STEPS = 128;
 
-// len ordered steps without energies, as one replay of a graph captured on first use:
-// drift, then per step the pair pass and the closing kick, each kick but the last fused
-// with the next step's drift (the same operations as the direct launches, so the same
-// bits, with one launch fewer per step).
+// len ordered steps without energies, as one replay of a graph captured on first use: the
+// drift, then one launch per step (pair pass, closing kick, next step's drift), between the
+// context's arrays and the fast engine's first set, which this order leaves idle (its owner
+// reloads it before its next step).  An even number of steps ends in the context's arrays.
+// One sphere, or a single step, takes the direct launches' kernels.
 int ordered_run(sl_ctx* c, int len)
 {
     hipGraphExec_t ex = nullptr;
@@ -257,10 +258,17 @@ int ordered_run(sl_ctx* c, int len)
         if (hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal) != hipSuccess)
             return set_err(c, SL_E_HIP, "ordered step capture");
         bool ok = launch_drift(c->st, c->n, c->p.dt, c->stream) == hipSuccess;
-        for (int k = 0; k < len && ok; k++)
-            ok = launch_pairs_ordered(c->st, P, c->n, 0, c->pe_part, c->cnt, c->stream, c->ord_shape) == hipSuccess &&
-                 (k + 1 < len ? launch_kick_drift(c->st, c->n, c->p.dt, c->nonfinite, c->stream)
-                              : launch_kick(c->st, c->n, c->p.dt, 0, 1, c->e_part, c->nonfinite, c->stream)) == hipSuccess;
+        if (c->n > 1 && len % 2 == 0) {
+            double* set[2] = {c->base, c->fb.eng[0].f[0]};
+            for (int k = 0; k < len && ok; k++)
+                ok = launch_step_ordered(c->base, set[k & 1], set[1 - (k & 1)], c->n_pad, P, c->n, k + 1 < len, c->cnt,
+                                         c->nonfinite, c->stream, c->ord_shape) == hipSuccess;
+        } else {
+            for (int k = 0; k < len && ok; k++)
+                ok = (k == 0 || launch_drift(c->st, c->n, c->p.dt, c->stream) == hipSuccess) &&
+                     launch_pairs_ordered(c->st, P, c->n, 0, c->pe_part, c->cnt, c->stream, c->ord_shape) == hipSuccess &&
+                     launch_kick(c->st, c->n, c->p.dt, 0, 1, c->e_part, c->nonfinite, c->stream) == hipSuccess;
+        }
         hipGraph_t g = nullptr;
         const hipError_t e = hipStreamEndCapture(c->stream, &g);
         if (!ok || e != hipSuccess || !g) {
@@ -306,7 +314,8 @@ int tune_ordered(sl_ctx* c)
         c->ord_shape = c->forced_ord_shape - 1;
         return SL_OK;
     }
-    const std::string key = "ordered:n" + std::to_string(c->n) + ":grav" + std::to_string(c->p.far_gravity);
+    // ("ordered:" entries of older caches number other shapes)
+    const std::string key = "ring:n" + std::to_string(c->n) + ":grav" + std::to_string(c->p.far_gravity);
     if (const int cached = tune_cache_get(key); cached >= 1 && cached <= ordered_shapes()) {
         c->ord_shape = cached - 1;
         return SL_OK;
@@ -626,6 +635,7 @@ int sl_step(sl_ctx* c, int n_steps, int write_every, sl_energy* e_out, int e_cap
                 if (write_every > 0 && s % write_every == 0) break;
                 len++;
             }
+            if (len > 1 && c->n > 1) len -= len % 2;
             if (len > 0) {
                 const int rc = ordered_run(c, len);
                 if (rc) return rc;

@@ -23,9 +23,11 @@ hipError_t launch_pairs_ordered(const State& s, const Phys& P, int n, int write,
 int kick_blocks(int n);
 hipError_t launch_kick(const State& s, int n, double dt, int write, int kick, double* e_part,
                        int* nonfinite, hipStream_t st);
-// A step's closing kick (no energies) and the next step's drift in one launch: the same
-// operations as launch_kick then launch_drift, so the same bits.
-hipError_t launch_kick_drift(const State& s, int n, double dt, int* nonfinite, hipStream_t st);
+// Pair pass, closing kick (no energies) and, with drift, the next step's drift in one launch, of
+// n >= 2 balls: the dynamic fields (field f at cur + f stride) after it go to nxt; radii,
+// masses and moments of inertia are read at konst + f stride.
+hipError_t launch_step_ordered(const double* konst, double* cur, double* nxt, long stride, const Phys& P, int n, int drift,
+                               unsigned long long* contacts, int* nonfinite, hipStream_t st, int shape);
 
 // ---- small utilities: sl_util.hip
 hipError_t launch_zero_u64(unsigned long long* p, int n, hipStream_t st);

@@ -5,8 +5,8 @@
 // ColliderSingleCore.cpp:100-103).  Floating-point addition is not associative,
 // so the GPU reproduces that order with one sequential accumulator per (ball,
 // component), while the expensive part -- evaluating the pair -- runs on every
-// producer lane of the workgroup (k_pairs_ordered below: BI balls per workgroup,
-// partners in chunks, evaluation and summation of consecutive chunks overlapped).
+// lane (k_pairs_ordered below: a ring of wavefronts per group of balls, each evaluating
+// a batch of partners and adding it when the sums reach it).
 // Far pairs contribute +0.0 to aacc and j == i contributes +0.0 to both; an
 // accumulator that starts at +0.0 under round-to-nearest never becomes -0.0,
 // so these additions leave it bit-for-bit unchanged and are skipped.
@@ -41,6 +41,8 @@ struct GlobalContact {
         return norm(qb - qa);
     }
 };
+
+__device__ __forceinline__ D3 load3(const State& s, int f, int b) { return d3(s.f[f][b], s.f[f + 1][b], s.f[f + 2][b]); }
 
 template <int N>
 __device__ __forceinline__ double block_sum(double v, double* red)
@@ -97,15 +99,11 @@ __global__ void k_copy_prev(State s, int n)
 
 // One pair (i, j) in the reference's arithmetic, touching or not (ColliderSingleCore.cpp:
 // 119-250), in its orientation A = max(i, j): ball i's acc contribution to c3[0], c3[cs],
-// c3[2 cs], its aacc contribution likewise to a3, and the pair energy (write steps, i = A) to
-// *pe.  Returns 1 for a touching pair.  The
-// state is one array of fields, field f at base + f stride (how every caller lays it out),
-// passed as its base so that the caller has no field table to spill for the call.
-__device__ __forceinline__ int contact_pair_body(const double* base, long stride, const Phys& P, int write, int i,
-                                                 int j, double ymi, double* c3, double* a3, int cs, double* pe)
+// c3[2 cs], its aacc contribution to a3[0], a3[as], a3[2 as], and the pair energy (write
+// steps, i = A) to *pe.  Returns 1 for a touching pair.
+__device__ __forceinline__ int general_pair(const State& s, const Phys& P, int write, int i, int j, double ymi, double* c3,
+                                            int cs, double* a3, int as, double* pe)
 {
-    State s;
-    for (int f = 0; f < NFIELD; f++) s.f[f] = const_cast<double*>(base + f * stride);
     const bool iA = i > j;
     const D3 pi = d3(s.f[PX][i], s.f[PY][i], s.f[PZ][i]);
     const D3 pj = d3(s.f[PX][j], s.f[PY][j], s.f[PZ][j]);
@@ -129,8 +127,8 @@ __device__ __forceinline__ int contact_pair_body(const double* base, long stride
     c3[cs] = a.y;
     c3[2 * cs] = a.z;
     a3[0] = aa.x;
-    a3[cs] = aa.y;
-    a3[2 * cs] = aa.z;
+    a3[as] = aa.y;
+    a3[2 * as] = aa.z;
     *pe = iA ? o.pe : 0.0;
     return o.contact;
 }
@@ -141,72 +139,103 @@ struct PartnerRec {
     double x, y, z, R, m, pref;
 };
 
-// One workgroup owns BI balls and sweeps every partner j in chunks of CJ.  NPW wavefronts
-// evaluate pairs (producers); the running sums are kept by consumer lanes, one per (ball,
-// quantity): acc x, y, z, aacc x, y, z and, on write steps, the pair energy of the ball as
-// A.  With DED the consumer lanes are a wavefront of their own; otherwise they are the first
-// 7 BI lanes of wavefront 0, which then also produces.
-//   produce (chunk k): thread (il, jq) evaluates the pairs (i0 + il, j0 + jq + JQ q) in the
-//     reference orientation and writes ball i's signed acc contribution (for a touching
-//     pair also its aacc contribution and a bit of the chunk's contact mask; on write
-//     steps the pair energy when i is A) to LDS buffer k mod 2;
-//   consume (chunk k - 1, at the same time): each consumer lane adds its ball's CJ
-//     contributions of its quantity in ascending j (aacc: only at the masked positions).
-// One barrier per chunk separates the two buffers' roles.  Every sum has the same order
-// whatever BI, NPW, CJ and DED are, so all launch shapes give the same bits (the energies
-// included: per-ball sums, added over the balls in ascending order by the caller).
-// The far arm divides by dist and by m_i through correctly rounded reciprocals
-// (div_rcp): the same quotients as the reference's divisions, for five FMA-pipe
-// instructions each instead of a full division.
-__device__ __attribute__((noinline)) int contact_pair(const double* base, long stride, const Phys& P, int write,
-                                                      int i, int j, double ymi, double* c3, double* a3, int cs,
-                                                      double* pe)
-{
-    return contact_pair_body(base, stride, P, write, i, j, ymi, c3, a3, cs, pe);
-}
+// The pair pass as a ring of wavefronts.  A workgroup owns NB balls and its W wavefronts take
+// the partners in batches of BP = CH * 64/NB, batch m by wavefront m mod W:
+//   evaluate  lane (ball l % NB, slot l / NB) evaluates CH pairs of its ball, one per step q,
+//             by the far-field arm in the reference orientation and writes the ball's signed
+//             acc contribution to the wavefront's own LDS buffer.  Lanes whose pair touches
+//             are noted by step; what the far arm wrote for them is replaced before it is
+//             added.
+//   add       when the running sums have passed through every earlier batch (turn == m), one
+//             lane per (ball, component) adds its BP contributions in ascending j and hands
+//             the sums on.  aacc gets only the touching pairs' contributions: the others are
+//             +0.0, a no-op on a sum that starts at +0.0.
+// Only the adding is serial (about 20 cycles a partner), and only the wavefront whose turn
+// it is takes part in it: the others go on evaluating, with no barrier anywhere.  Every
+// sum has the same order whatever the shape, so all launch shapes give the same bits (the
+// energies included: per-ball sums, added over the balls in ascending order by the caller).
+// Every wavefront of a workgroup is resident, and the owner of the batch whose turn it is
+// waits for nothing but the contact table's maker, which waits for nothing: every wait ends.
+// LDS instructions of a wavefront take effect in their order, which is all the handing on
+// needs: sums, then turn; turn, then sums.
+//
+// Touching pairs.  The contact arm is five times the far arm's instructions, for one or two
+// lanes of a wavefront.  With SCAN the workgroup first tests its balls against every partner
+// (16 instructions a step), and one wavefront evaluates the touching pairs found, up to
+// 64, side by side while the others start on their batches; a pair met in the sweep is then
+// copied from that table.  Pairs that did not fit in it, and all touching pairs without SCAN,
+// are evaluated where they are met, those of the first AD steps before the turn.  The scan
+// pays up to about 2,500 balls (4 balls, 4 wavefronts, us per step with / without: 2,000 balls
+// 43.7 / 45.4, 3,000 77 / 73.5, 5,000 175 / 161): its cost grows with the partners, what it
+// saves only with the contacts.
+//
+// Bound by the binary64 pipe: 131 VALU instructions a step of 64 evaluations (105 of them the
+// reference's arithmetic), 150-170 with the staging, the adding and the contacts; at 15,039
+// balls that is 75% of the time, at 5,000 57% (1,250 workgroups, 3 to a CU).  Small systems are
+// bound by the chain of adds (6.5 cycles each and about 400 a batch) and by the first
+// contacts' 5,000 cycles.  Measured per step, before (chunks of partners, a barrier each,
+// sums by a wavefront of its own, the kick in a launch of its own) and now: 129 balls 16.5 ->
+// 9 us, 1,000 29 -> 19, 2,200 87 -> 57, 5,000 259 -> 161, 15,039 1,750 -> 1,095.
+//
+// With a second set of arrays (os.nxt) the owner of the last batch also kicks its balls and,
+// with os.drift, drifts them into the next step (the operations of k_kick and k_drift): one
+// launch a step instead of two.  The other workgroups may still be reading this step's positions and
+// velocities, hence the second set.
+struct OrdState {
+    double* cur;           // dynamic fields, field f at cur + f stride
+    const double* konst;   // radii, masses, moments of inertia, likewise (RAD ..)
+    double* nxt;           // where the state after the step goes, or NULL: only acc and aacc, in place
+    long stride;
+    int drift;
+    int* nonfinite;
+};
 
-// CALL: the contact arm out of line (its registers weigh only on the calls) or inline.
-// WPE: the wavefronts per SIMD the register budget is held to (0: the compiler's choice).
-// UNR: how many of a thread's far-field pairs per chunk the sweep unrolls (the sums' order
-// is fixed by the contribution buffer, so it changes no bits).
-// WRITE: write steps (pair energies).
-template <int BI, int NPW, int CJ, bool DED, bool CALL, int WPE, int UNR, bool WRITE>
-__global__ __launch_bounds__((NPW + (DED ? 1 : 0)) * 64) __attribute__((amdgpu_waves_per_eu(WPE > 0 ? WPE : 1)))
-void k_pairs_ordered(State s, Phys P, int n, double* __restrict__ pe_ball,
+template <int NB, int CH, int W, int AD, int WPE, int UNR, bool SCAN, bool WRITE>
+__global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(WPE)))
+void k_pairs_ordered(OrdState os, Phys P, int n, double* __restrict__ pe_ball,
                      unsigned long long* __restrict__ contacts)
 {
-    constexpr int NP = NPW * 64;            // producer threads
-    constexpr int JQ = NP / BI;             // producer threads per ball
-    constexpr int KP = CJ / JQ;             // pairs per producer thread and chunk
-    constexpr int MW = (CJ + 63) / 64;      // contact-mask words per ball and chunk
-    constexpr int CS = CJ * BI + 4;         // quantity stride (staggers the consumer's banks)
-    constexpr int NQ = WRITE ? 7 : 6;       // acc xyz, aacc xyz, pair energy
-    static_assert(NP % BI == 0 && CJ % JQ == 0 && KP >= 1, "chunk shape");
-    static_assert(NQ * BI <= 64, "one consumer lane per (ball, quantity)");
-    constexpr int NT = (NPW + (DED ? 1 : 0)) * 64;   // threads of the workgroup
-    constexpr int NL = (CJ + NT - 1) / NT;           // partner records each thread stages per chunk
-    __shared__ double cb[2][NQ * CS];
-    __shared__ unsigned long long cmask[2][BI][MW];
-    __shared__ PartnerRec sp[2][CJ];                 // the partners of chunks k and k + 1
+    State s;
+    for (int f = 0; f < NFIELD; f++) s.f[f] = (f < RAD ? os.cur : const_cast<double*>(os.konst)) + f * os.stride;
+    constexpr int JS = 64 / NB;             // partners a wavefront evaluates at once
+    constexpr int BP = CH * JS;             // partners per batch
+    constexpr int NQ = WRITE ? 4 : 3;       // acc xyz, pair energy
+    // A ball's contributions lie in a row, so that an adding lane reads two at once.  Row and
+    // component strides: the 32 lanes of half a wavefront's store (32/NB slots of NB balls) and
+    // the adding lanes' 16-byte reads each cover every LDS bank once.
+    constexpr int RS = (BP + 31) / 32 * 32 + 32 / NB, CS = NB * RS + 2;
+    constexpr int AH = BP < 16 ? BP : 16;   // contributions a lane adds from registers at once
+    static_assert(64 % NB == 0 && BP <= 64 && NQ * NB <= 64 && BP % AH == 0 && CH <= 32, "batch shape");
+    __shared__ __attribute__((aligned(16))) double cb[W][NQ][CS];   // acc contributions (and energies)
+    __shared__ double ab[W][AD][3][64];     // aacc contributions of AD steps' touching pairs, by lane
+    __shared__ PartnerRec sp[W][BP];
+    __shared__ double run[7][NB];           // the sums: acc xyz, aacc xyz, energy
+    __shared__ double own[3][3][NB];        // half-step velocities and spins, positions: for the kick and the drift
+    __shared__ int turn, ready, found;
     __shared__ unsigned ccount;
-    __shared__ int general;                          // a ball or a parameter outside FarRange was met
-    __shared__ double sgm[BI];                       // G m_i of the workgroup's balls
+    __shared__ unsigned tkey[SCAN ? 64 : 1];        // contact table: ball << 24 | partner ...
+    __shared__ double tres[SCAN ? 64 : 1][7];       // ... acc xyz, aacc xyz, energy
 
     const int t = threadIdx.x;
-    const int w = __builtin_amdgcn_readfirstlane(t / 64);
-    if (t < 2 * BI * MW) (&cmask[0][0][0])[t] = 0ull;
-    if (t == 0) {
-        ccount = 0;
-        general = !FarRange::params(P);
+    const int w = __builtin_amdgcn_readfirstlane(t / 64), l = t % 64;
+    for (int e = t; e < 7 * NB; e += 64 * W) (&run[0][0])[e] = 0.0;
+    if (!WRITE && os.nxt && t < 3 * NB && (int)blockIdx.x * NB + t % NB < n) {
+        const long e = t / NB * os.stride + blockIdx.x * NB + t % NB;
+        (&own[0][0][0])[t] = os.cur[HX * os.stride + e];
+        (&own[1][0][0])[t] = os.cur[GX * os.stride + e];
+        (&own[2][0][0])[t] = os.cur[PX * os.stride + e];
     }
-    if (t < BI) sgm[t] = blockIdx.x * BI + t < n ? P.G * s.f[MASS][blockIdx.x * BI + t] : 0.0;
+    if (t == 0) {
+        turn = 0;
+        ready = 0;
+        found = 0;
+        ccount = 0;
+    }
 
-    // producer role
-    const int il = t % BI;
-    const int jq = (t / BI) % JQ;
-    const int i = blockIdx.x * BI + il;
-    const bool iv = w < NPW && i < n;
-    const int ic = i < n ? i : 0;
+    const int il = l % NB, jq = l / NB;
+    const int i0 = blockIdx.x * NB, i = i0 + il;
+    const bool iv = i < n;
+    const int ic = iv ? i : 0;
     const D3 pi = d3(s.f[PX][ic], s.f[PY][ic], s.f[PZ][ic]);
     const double Ri = s.f[RAD][ic], mi = s.f[MASS][ic];
     const double ymi = 1.0 / mi;             // divisions by m_i through div_rcp
@@ -215,207 +244,342 @@ void k_pairs_ordered(State s, Phys P, int n, double* __restrict__ pe_ball,
     const double Hc = P.Ha / 6 * 64;
     const double prefA = Hc * Ri * Ri * Ri;
     const double Gmi = P.G * mi;
+    const bool gen_i = !FarRange::params(P) || !FarRange::ball(Ri, mi);
     unsigned cnt = 0;
 
-    // consumer role: lane c of the consumer wavefront, (ball c % BI, quantity c / BI)
-    constexpr int CW = DED ? NPW : 0;       // the consumer wavefront
-    const int c = t - CW * 64;
-    const int cl = c % BI, cq = c / BI;
-    const bool consumer = w == CW && c < NQ * BI;
-    double run = 0.0;
+    const int nm = (n + BP - 1) / BP;        // batches
+    PartnerRec nx;                           // this lane's partner of the wavefront's next batch
+    auto load_batch = [&](int m) {
+        const int j = m * BP + l;
+        if (l < BP && j < n)
+            nx = PartnerRec{s.f[PX][j], s.f[PY][j], s.f[PZ][j], s.f[RAD][j], s.f[MASS][j], 0.0};
+    };
+    load_batch(w);
+    __syncthreads();
+    // Pair (ball bi, partner j) in full, by the touching arm where it holds: acc and aacc
+    // contributions to c3[0], c3[cs], .. and a3[0], a3[as], ..; returns 1 if it touches.
+    auto contact = [&](int bi, int j, const D3& pb, double Rb, double mb, double ymb, double* c3, int cs, double* a3,
+                       int as, double* pe) -> int {
+        const bool iA = bi > j;
+        const D3 pj = d3(s.f[PX][j], s.f[PY][j], s.f[PZ][j]);
+        const double Rj = s.f[RAD][j], mj = s.f[MASS][j];
+        const D3 d = pj - pb;
+        // (a scanned pair may not touch, nor one met beside a ball out of range)
+        bool ok = FarRange::params(P) && FarRange::ball(Rb, mb) && FarRange::ball(Rj, mj) &&
+                  FarRange::distance2(dot(d, d)) && (Rb + Rj) - norm(d) > 0;
+        if (ok) {
+            const int A = iA ? bi : j, B = iA ? j : bi;
+            const TouchState ts{load3(s, VX, A), load3(s, VX, B), load3(s, WX, A), load3(s, WX, B),
+                                load3(s, QX, B) - load3(s, QX, A)};
+            const double Ib = s.f[MOI][bi];
+            const PairIn in{iA ? pb : pj, iA ? pj : pb, iA ? Rb : Rj, iA ? Rj : Rb, iA ? mb : mj, iA ? mj : mb};
+            PairOut o;
+            ok = touch_pair_ref(P, WRITE && iA, in, ts, o);
+            // acc[A] += F/m[A] or acc[B] -= F/m[B]; aacc[A] += tA/moi[A], aacc[B] += tB/moi[B]
+            const D3 a = d3(div_rcp(o.F.x, mb, ymb), div_rcp(o.F.y, mb, ymb), div_rcp(o.F.z, mb, ymb));
+            const D3 aa = (iA ? o.tA : o.tB) / Ib;
+            c3[0] = iA ? a.x : -a.x;
+            c3[cs] = iA ? a.y : -a.y;
+            c3[2 * cs] = iA ? a.z : -a.z;
+            a3[0] = aa.x;
+            a3[as] = aa.y;
+            a3[2 * as] = aa.z;
+            *pe = o.pe;
+        }
+        if (ok) return 1;
+        return general_pair(s, P, WRITE, bi, j, ymb, c3, cs, a3, as, pe);
+    };
 
-    // Partner records are staged in LDS a chunk ahead: the loads of chunk k + 1 are issued
-    // before chunk k is evaluated and stored after it, so their latency is hidden.
-    const int nch = (n + CJ - 1) / CJ;
-    PartnerRec nx[NL];
-    auto load_chunk = [&](int kc) {
+    unsigned mykey = ~0u;     // SCAN: the table's keys, one per lane, once read
+    if constexpr (SCAN) {
+        // every wavefront scans every W-th group of JS partners; a superset of the touching
+        // pairs (d^2 against S^2, a little enlarged)
+        constexpr int SU = 4;   // groups whose loads are in flight together
+        for (int j1 = w * JS + jq; j1 - jq < n; j1 += SU * W * JS) {
+            D3 pj[SU];
+            double Rj[SU];
 #pragma unroll
-        for (int u = 0; u < NL; u++) {
-            const int jl = t + u * NT;
-            const int j = kc * CJ + jl;
-            if (jl < CJ && j < n)
-                nx[u] = PartnerRec{s.f[PX][j], s.f[PY][j], s.f[PZ][j], s.f[RAD][j], s.f[MASS][j], 0.0};
-        }
-    };
-    auto store_chunk = [&](int kc) {
-#pragma unroll
-        for (int u = 0; u < NL; u++) {
-            const int jl = t + u * NT;
-            if (jl < CJ && kc * CJ + jl < n) {
-                const double R = nx[u].R;
-                nx[u].pref = Hc * R * R * R;
-                sp[kc & 1][jl] = nx[u];
-                if (!FarRange::ball(R, nx[u].m)) general = 1;   // before the barrier that opens the chunk
+            for (int u = 0; u < SU; u++) {
+                const int j = min(j1 + u * W * JS, n - 1);
+                pj[u] = d3(s.f[PX][j], s.f[PY][j], s.f[PZ][j]);
+                Rj[u] = s.f[RAD][j];
             }
-        }
-    };
-    load_chunk(0);
-    __syncthreads();
-    store_chunk(0);
-    if (!FarRange::ball(Ri, mi)) general = 1;
-    __syncthreads();
-    for (int k = 0; k <= nch; k++) {
-        const int b = k & 1;
-        if (k + 1 < nch) load_chunk(k + 1);
-        if (w == CW && k > 0) {
-            // sums of chunk k - 1
-            const int bb = b ^ 1;
-            const int m = (n - (k - 1) * CJ) < CJ ? (n - (k - 1) * CJ) : CJ;
-            if (consumer) {
-                const double* src = &cb[bb][cq * CS + cl];
-                if (cq < 3 || cq == 6) {
-                    int jl = 0;
-                    for (; jl + 8 <= m; jl += 8) {
-                        double v[8];
 #pragma unroll
-                        for (int u = 0; u < 8; u++) v[u] = src[(jl + u) * BI];
-#pragma unroll
-                        for (int u = 0; u < 8; u++) run = run + v[u];
-                    }
-                    for (; jl < m; jl++) run = run + src[jl * BI];
-                } else if (cq < 6) {
-                    // aacc: only touching pairs contribute (the others add +0.0, a no-op on
-                    // a sum that starts at +0.0), in ascending j
-                    for (int wd = 0; wd < MW; wd++) {
-                        unsigned long long mk = cmask[bb][cl][wd];
-                        while (mk) {
-                            const int bit = __ffsll((long long)mk) - 1;
-                            mk &= mk - 1;
-                            run = run + src[(wd * 64 + bit) * BI];
-                        }
-                    }
+            for (int u = 0; u < SU; u++) {
+                const int j = j1 + u * W * JS;
+                const D3 d = pj[u] - pi;
+                const double S = Ri + Rj[u];
+                if (dot(d, d) < S * S * (1 + 1e-12) && iv && j < n && j != i) {
+                    const int e = atomicAdd(&found, 1);
+                    if (e < 64) tkey[e] = (unsigned)il << 24 | (unsigned)j;
                 }
             }
-            // every lane of this wavefront has read the masks: clear them for chunk k + 1
-            __builtin_amdgcn_wave_barrier();
-            if (c >= 0 && c < BI * MW) (&cmask[bb][0][0])[c] = 0ull;
         }
-        if (w < NPW && k < nch) {
-            const int j0 = k * CJ;
-            const int i0 = blockIdx.x * BI;
-            // pairs q of this chunk that touch, or whose operands are outside FarRange: evaluated
-            // by the general arm after the sweep
-            unsigned pend = 0;
-            const bool gen = general != 0;
-            // One far-field pair (i, j) in the reference's orientation A = max(i, j): ball i
-            // is A when IA (ColliderSingleCore.cpp:104-110, 211-227).  Writes ball i's acc
-            // contribution (and its energy on write steps), or marks the pair for the
-            // general arm.
-            auto far_pair = [&](auto ia, int q) {
-                constexpr bool IA = decltype(ia)::value;
-                const int jl = jq + JQ * q;
-                const int j = j0 + jl;
-                double c0 = 0, c1 = 0, c2 = 0, u = 0;
-                if (iv && j < n && j != i) {
-                    const PartnerRec& pr = sp[b][jl];
-                    const D3 pj = d3(pr.x, pr.y, pr.z);
-                    const double Rj = pr.R, mj = pr.m;
-                    const double S = IA ? Ri + Rj : Rj + Ri;
-                    const D3 r = IA ? pj - pi : pi - pj;               // x_B - x_A
-                    const double d2 = dot(r, r);
-                    double dist, yd;                                   // norm(r) and its reciprocal
-                    sqrt_rcp(d2, dist, yd);
-                    const double overlap = S - dist;
-                    if (overlap > 0 || gen || !FarRange::distance2(d2)) {
-                        pend |= 1u << q;
-                    } else {
-                        double h = ::fabs(overlap);
-                        if (h < P.h_min) h = P.h_min;
-                        const double h2 = h * h;
-                        // vdw_factor with Ra = R_A, Rb = R_B: 2 Ra h, 2 Rb h, 4 Ra Rb and
-                        // Ha/6*64 Ra Ra Ra Rb Rb Rb in the reference's product order
-                        const double twoRah = IA ? two_Ri * h : (2 * Rj) * h;
-                        const double twoRbh = IA ? (2 * Rj) * h : two_Ri * h;
-                        const double sv = h2 + twoRah + twoRbh;
-                        const double tv = sv + (IA ? four_Ri * Rj : (4 * Rj) * Ri);
-                        const double quot = div_plain(IA ? h + Ri + Rj : h + Rj + Ri, sv * sv * tv * tv);
-                        const double fv = IA ? prefA * Rj * Rj * Rj * quot : pr.pref * Ri * Ri * Ri * quot;
-                        const D3 rh = d3(div_rcp(r.x, dist, yd), div_rcp(r.y, dist, yd), div_rcp(r.z, dist, yd));
-                        D3 F = rh * fv;
-                        if (P.far_gravity) {
-                            // Under a register cap G m_i is read from LDS at each use (an atomic
-                            // load, which the compiler keeps in the loop): held in a register it
-                            // is spilled, and the spill's reload waits for every load in flight,
-                            // the next chunk's partners included.
-                            double gmi = Gmi;
-                            if constexpr (WPE > 0)
-                                gmi = __hip_atomic_load(&sgm[il], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                            F = F + rh * div_sq(IA ? gmi * mj : P.G * mj * mi, dist * dist, yd);
-                        }
-                        // acc[A] += F/m[A]  or  acc[B] -= F/m[B]   (:187-188, 249-250)
-                        c0 = div_rcp(F.x, mi, ymi);
-                        c1 = div_rcp(F.y, mi, ymi);
-                        c2 = div_rcp(F.z, mi, ymi);
-                        if (!IA) {
-                            c0 = -c0;
-                            c1 = -c1;
-                            c2 = -c2;
-                        } else if (WRITE) {                            // :228-240
-                            u = vdw_energy(P.Ha, Ri, Rj, S, h);
-                            if (P.far_gravity) u = u + -P.G * mi * mj / dist;
-                        }
-                    }
-                }
-                const int o_ = jl * BI + il;
-                cb[b][0 * CS + o_] = c0;
-                cb[b][1 * CS + o_] = c1;
-                cb[b][2 * CS + o_] = c2;
-                if (WRITE) cb[b][6 * CS + o_] = u;
-            };
-            if (j0 + CJ <= i0) {
-                // every partner of the chunk precedes every ball of the block: i is A
-#pragma unroll UNR
-                for (int q = 0; q < KP; q++) far_pair(std::true_type{}, q);
-            } else if (j0 >= i0 + BI) {
-                // every partner follows: i is B
-#pragma unroll UNR
-                for (int q = 0; q < KP; q++) far_pair(std::false_type{}, q);
-            } else {
-#pragma unroll 1
-                for (int q = 0; q < KP; q++) {
-                    if (i > j0 + jq + JQ * q)
-                        far_pair(std::true_type{}, q);
-                    else
-                        far_pair(std::false_type{}, q);
-                }
-            }
-            // touching pairs: the reference's contact arm in full (:119-204), out of line so
-            // that its registers do not weigh on the far-field sweep
-            while (pend) {
-                const int q = __ffs(pend) - 1;
-                pend &= pend - 1;
-                const int jl = jq + JQ * q;
-                const int o_ = jl * BI + il;
-                double pc = 0;
-                int touch;
-                if constexpr (CALL)
-                    touch = contact_pair(s.f[0], s.f[1] - s.f[0], P, WRITE, i, j0 + jl, ymi, &cb[b][o_],
-                                         &cb[b][3 * CS + o_], CS, &pc);
-                else
-                    touch = contact_pair_body(s.f[0], s.f[1] - s.f[0], P, WRITE, i, j0 + jl, ymi, &cb[b][o_],
-                                              &cb[b][3 * CS + o_], CS, &pc);
-                if (WRITE) cb[b][6 * CS + o_] = pc;
-                atomicOr(&cmask[b][il][jl >> 6], 1ull << (jl & 63));
-                if (touch && i > j0 + jl) cnt++;
-            }
-        }
-        // chunk k + 1's partners into the buffer chunk k - 1 used (all reads of it ended
-        // before the previous barrier)
-        if (k + 1 < nch) store_chunk(k + 1);
         __syncthreads();
-    }
-
-    if (consumer) {
-        const int ib = blockIdx.x * BI + cl;
-        if (ib < n) {
-            if (cq < 3)
-                s.f[AX + cq][ib] = run;
-            else if (cq < 6)
-                s.f[BX + cq - 3][ib] = run;
-            else if (WRITE)
-                pe_ball[ib] = run;
+        const int nt = min(found, 64);
+        if (w == W - 1) {
+            __builtin_amdgcn_s_setprio(3);
+            if (l < nt) {
+                const unsigned key = tkey[l];
+                const int bi = i0 + (int)(key >> 24), j = (int)(key & 0xffffffu);
+                const D3 pb = d3(s.f[PX][bi], s.f[PY][bi], s.f[PZ][bi]);
+                const double mb = s.f[MASS][bi];
+                double pe = 0;
+                const int touch = contact(bi, j, pb, s.f[RAD][bi], mb, 1.0 / mb, &tres[l][0], 1, &tres[l][3], 1, &pe);
+                if (WRITE) tres[l][6] = pe;
+                if (!touch) tkey[l] = ~0u;
+            }
+            __builtin_amdgcn_s_setprio(0);
+            asm volatile("" ::: "memory");
+            if (l == 0) __hip_atomic_store(&ready, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         }
     }
+    bool have_table = false;
+
+#pragma unroll 1
+    for (int m = w; m < nm; m += W) {
+        const int j0 = m * BP;
+        // the batch's partners to LDS, the next batch's on their way
+        bool bad = false;
+        if (l < BP && j0 + l < n) {
+            bad = !FarRange::ball(nx.R, nx.m);
+            nx.pref = Hc * nx.R * nx.R * nx.R;
+            sp[w][l] = nx;
+        }
+        const bool gen = gen_i || __any(bad);
+        if (m + W < nm) load_batch(m + W);
+        asm volatile("" ::: "memory");
+
+        // steps whose pair touches or has operands outside FarRange: replaced after the sweep
+        unsigned pend = 0;
+        // One far-field pair (i, j) in the reference's orientation A = max(i, j): ball i
+        // is A when IA (ColliderSingleCore.cpp:104-110, 211-227).  Writes ball i's acc
+        // contribution (and its energy on write steps).
+        auto far_pair = [&](auto ia, auto checked, int q) {
+            constexpr bool IA = decltype(ia)::value;
+            constexpr bool CHK = decltype(checked)::value;
+            const int jl = jq + JS * q;
+            const int j = j0 + jl;
+            const bool pair = !CHK || (iv && j < n && j != i);
+            const PartnerRec& pr = sp[w][jl];
+            const D3 pj = d3(pr.x, pr.y, pr.z);
+            const double Rj = pr.R, mj = pr.m;
+            const double S = IA ? Ri + Rj : Rj + Ri;
+            const D3 r = IA ? pj - pi : pi - pj;               // x_B - x_A
+            const double d2 = dot(r, r);
+            double dist, yd;                                   // norm(r) and its reciprocal
+            sqrt_rcp(d2, dist, yd);
+            const double overlap = S - dist;
+            if (pair && (overlap > 0 || gen || !FarRange::distance2(d2))) pend |= 1u << q;
+            double h = ::fabs(overlap);
+            if (h < P.h_min) h = P.h_min;
+            const double h2 = h * h;
+            // vdw_factor with Ra = R_A, Rb = R_B: 2 Ra h, 2 Rb h, 4 Ra Rb and
+            // Ha/6*64 Ra Ra Ra Rb Rb Rb in the reference's product order
+            const double twoRah = IA ? two_Ri * h : (2 * Rj) * h;
+            const double twoRbh = IA ? (2 * Rj) * h : two_Ri * h;
+            const double sv = h2 + twoRah + twoRbh;
+            const double tv = sv + (IA ? four_Ri * Rj : (4 * Rj) * Ri);
+            const double quot = div_plain(IA ? h + Ri + Rj : h + Rj + Ri, sv * sv * tv * tv);
+            const double fv = IA ? prefA * Rj * Rj * Rj * quot : pr.pref * Ri * Ri * Ri * quot;
+            const D3 rh = d3(div_rcp(r.x, dist, yd), div_rcp(r.y, dist, yd), div_rcp(r.z, dist, yd));
+            D3 F = rh * fv;
+            if (P.far_gravity) F = F + rh * div_sq(IA ? Gmi * mj : P.G * mj * mi, dist * dist, yd);
+            // acc[A] += F/m[A]  or  acc[B] -= F/m[B]   (:187-188, 249-250)
+            double c0 = div_rcp(F.x, mi, ymi), c1 = div_rcp(F.y, mi, ymi), c2 = div_rcp(F.z, mi, ymi);
+            double u = 0;
+            if (WRITE && IA) {                                 // :228-240
+                u = vdw_energy(P.Ha, Ri, Rj, S, h);
+                if (P.far_gravity) u = u + -P.G * mi * mj / dist;
+            }
+            if (CHK && !pair) c0 = c1 = c2 = u = 0;            // no partner, or the ball itself
+            const int o_ = il * RS + jl;
+            cb[w][0][o_] = IA ? c0 : -c0;
+            cb[w][1][o_] = IA ? c1 : -c1;
+            cb[w][2][o_] = IA ? c2 : -c2;
+            if (WRITE) cb[w][NQ - 1][o_] = u;
+        };
+        if (j0 + BP <= i0 && i0 + NB <= n) {
+            // every partner of the batch precedes every ball of the workgroup: i is A
+#pragma unroll UNR
+            for (int q = 0; q < CH; q++) far_pair(std::true_type{}, std::false_type{}, q);
+        } else if (j0 >= i0 + NB && j0 + BP <= n) {
+            // every partner follows: i is B
+#pragma unroll UNR
+            for (int q = 0; q < CH; q++) far_pair(std::false_type{}, std::false_type{}, q);
+        } else {
+#pragma unroll 1
+            for (int q = 0; q < CH; q++) {
+                if (i > j0 + jq + JS * q)
+                    far_pair(std::true_type{}, std::true_type{}, q);
+                else
+                    far_pair(std::false_type{}, std::true_type{}, q);
+            }
+        }
+        asm volatile("" ::: "memory");
+
+        __builtin_amdgcn_s_setprio(3);
+        // the lanes of step q with a touching pair, and their contributions into cb and ab
+        auto touching = [&](int q, int d) -> unsigned long long {
+            bool mine = (pend >> q) & 1u;
+            unsigned long long lanes = __ballot(mine);
+            unsigned long long out = 0;
+            if constexpr (SCAN) {
+                if (!have_table) {
+                    while (!__builtin_amdgcn_readfirstlane(__hip_atomic_load(&ready, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP))) {
+                    }
+                    asm volatile("" ::: "memory");
+                    if (l < min(found, 64)) mykey = tkey[l];
+                    have_table = true;
+                }
+                for (unsigned long long z = lanes; z; z &= z - 1) {
+                    const int ln = __ffsll((long long)z) - 1;
+                    const unsigned key = (unsigned)(ln % NB) << 24 | (unsigned)(j0 + JS * q + ln / NB);
+                    const unsigned long long hit = __ballot(mykey == key);
+                    if (!hit) continue;
+                    const int e = __ffsll((long long)hit) - 1;
+                    const int o_ = ln % NB * RS + JS * q + ln / NB;
+                    if (l < 3) cb[w][l][o_] = tres[e][l];
+                    else if (l < 6) ab[w][d][l - 3][ln] = tres[e][l];
+                    else if (WRITE && l == 6) cb[w][NQ - 1][o_] = tres[e][6];
+                    out |= 1ull << ln;
+                    if (l == ln) mine = false;
+                }
+                if (((out >> l) & 1ull) && i > j0 + JS * q + jq) cnt++;
+            }
+            if (mine) {
+                const int j = j0 + JS * q + jq;
+                const int o_ = il * RS + JS * q + jq;
+                double pe = 0;
+                const int touch = contact(i, j, pi, Ri, mi, ymi, &cb[w][0][o_], CS, &ab[w][d][0][l], 64, &pe);
+                if (WRITE) cb[w][NQ - 1][o_] = pe;
+                if (touch && i > j) cnt++;
+            }
+            asm volatile("" ::: "memory");
+            return out | __ballot(mine);
+        };
+        const bool adds = l < NQ * NB;
+        const int comp = adds ? jq : 0;
+        double* const pr = &run[comp < 3 ? comp : 6][il];
+        double r;
+        auto wait_turn = [&]() {
+            for (;;) {
+                const int now = __hip_atomic_load(&turn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                asm volatile("" ::: "memory");
+                r = __hip_atomic_load(pr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);   // read after turn
+                if (__builtin_amdgcn_readfirstlane(now) == m) break;
+            }
+            asm volatile("" ::: "memory");
+        };
+        // aacc: the touching lanes of a step in ascending order (their slots ascend with j)
+        auto add_aacc = [&](unsigned long long lanes, int d) {
+            if (comp < 3 && adds) {
+                double ra = run[3 + comp][il];
+                for (unsigned long long z = lanes; z; z &= z - 1) {
+                    const int ln = __ffsll((long long)z) - 1;
+                    const double c = ab[w][d][comp][ln];
+                    if (ln % NB == il) ra = ra + c;
+                }
+                run[3 + comp][il] = ra;
+            }
+            asm volatile("" ::: "memory");
+        };
+        unsigned long long lanes[AD];       // touching lanes of up to AD steps, evaluated before the turn
+        unsigned steps = 0;                 // steps with touching lanes, those not yet evaluated
+        bool any = false;
+        if (__any(pend != 0)) {
+            unsigned o = pend;
+            for (int k = 1; k < 64; k <<= 1) o |= __shfl_xor(o, k, 64);
+            steps = __builtin_amdgcn_readfirstlane(o);
+            any = true;
+        }
+#pragma unroll
+        for (int d = 0; d < AD; d++) {
+            lanes[d] = 0;
+            if (steps) {
+                lanes[d] = touching(__ffs(steps) - 1, d);
+                steps &= steps - 1;
+            }
+        }
+        // ab holds AD steps' pairs: with more steps the sums' turn has to come first
+        if (steps) {
+            wait_turn();
+#pragma unroll
+            for (int d = 0; d < AD; d++) add_aacc(lanes[d], d);
+            any = false;
+            for (; steps; steps &= steps - 1) add_aacc(touching(__ffs(steps) - 1, 0), 0);
+        }
+        // add: lane (ball l % NB, component l / NB)
+        if (adds) {
+            typedef double double2_t __attribute__((ext_vector_type(2)));
+            const double2_t* src = reinterpret_cast<const double2_t*>(&cb[w][comp][il * RS]);
+            double2_t v[AH / 2];
+#pragma unroll
+            for (int q = 0; q < AH / 2; q++) v[q] = src[q];
+            wait_turn();
+#pragma unroll
+            for (int q0 = 0; q0 < BP; q0 += AH) {
+                double2_t u[AH / 2];
+                if (q0 + AH < BP) {
+#pragma unroll
+                    for (int q = 0; q < AH / 2; q++) u[q] = src[(q0 + AH) / 2 + q];
+                }
+#pragma unroll
+                for (int q = 0; q < AH / 2; q++) r = (r + v[q].x) + v[q].y;
+                if (q0 + AH < BP) {
+#pragma unroll
+                    for (int q = 0; q < AH / 2; q++) v[q] = u[q];
+                }
+            }
+            *pr = r;
+        }
+        if (any) {
+#pragma unroll
+            for (int d = 0; d < AD; d++)
+                if (lanes[d]) add_aacc(lanes[d], d);
+        }
+        asm volatile("" ::: "memory");
+        if (l == 0) __hip_atomic_store(&turn, m + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (m == nm - 1 && adds && iv) {
+            if (comp == 3) {
+                pe_ball[i] = r;
+            } else {
+                const double al = run[3 + comp][il];
+                const long c0 = comp * os.stride + i;
+                auto at = [&](double* base, int f) -> double& { return base[f * os.stride + c0]; };
+                if (WRITE || !os.nxt) {
+                    at(os.cur, AX) = r;
+                    at(os.cur, BX) = al;
+                } else {
+                    // closing kick (ColliderSingleCore.cpp:263-287)
+                    const double dt = P.dt;
+                    const double h0 = own[0][comp][il], g0 = own[1][comp][il], p0 = own[2][comp][il];
+                    const double v = h0 + .5 * r * dt;
+                    const double wv = g0 + .5 * al * dt;
+                    if (!(isfinite(v) && isfinite(wv) && isfinite(p0))) atomicOr(os.nonfinite, 1);
+                    at(os.nxt, VX) = v;
+                    at(os.nxt, WX) = wv;
+                    at(os.nxt, AX) = r;
+                    at(os.nxt, BX) = al;
+                    if (os.drift) {   // of the next step (:82-97)
+                        const double hx = v + .5 * r * dt;
+                        at(os.nxt, HX) = hx;
+                        at(os.nxt, GX) = wv + .5 * al * dt;
+                        at(os.nxt, QX) = p0;
+                        at(os.nxt, PX) = p0 + hx * dt;
+                    } else {
+                        at(os.nxt, HX) = h0;
+                        at(os.nxt, GX) = g0;
+                        at(os.nxt, QX) = at(os.cur, QX);
+                        at(os.nxt, PX) = p0;
+                    }
+                }
+            }
+        }
+        __builtin_amdgcn_s_setprio(0);
+        asm volatile("" ::: "memory");
+    }
+
     // contact count (integer, order-independent)
     if (cnt) atomicAdd(&ccount, cnt);
     __syncthreads();
@@ -476,51 +640,6 @@ __global__ __launch_bounds__(256) void k_kick(State s, int n, double dt, int wri
     }
 }
 
-// The closing kick of a step without energies (k_kick with kick = 1, write = 0) and the
-// next step's drift (k_drift) in one pass over the balls: the velocities the kick writes
-// are the ones the drift reads, and the accelerations are the same pair pass's, so every
-// value is computed by the same operations as in the two launches.
-__global__ void k_kick_drift(State s, int n, double dt, int* __restrict__ nonfinite)
-{
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= n) return;
-    const double ax = s.f[AX][b], ay = s.f[AY][b], az = s.f[AZ][b];
-    const double bx = s.f[BX][b], by = s.f[BY][b], bz = s.f[BZ][b];
-    // kick (ColliderSingleCore.cpp:263-287)
-    const double vx = s.f[HX][b] + .5 * ax * dt;
-    const double vy = s.f[HY][b] + .5 * ay * dt;
-    const double vz = s.f[HZ][b] + .5 * az * dt;
-    const double wx = s.f[GX][b] + .5 * bx * dt;
-    const double wy = s.f[GY][b] + .5 * by * dt;
-    const double wz = s.f[GZ][b] + .5 * bz * dt;
-    s.f[VX][b] = vx;
-    s.f[VY][b] = vy;
-    s.f[VZ][b] = vz;
-    s.f[WX][b] = wx;
-    s.f[WY][b] = wy;
-    s.f[WZ][b] = wz;
-    const double px = s.f[PX][b], py = s.f[PY][b], pz = s.f[PZ][b];
-    if (!(isfinite(vx) && isfinite(vy) && isfinite(vz) && isfinite(wx) && isfinite(wy) &&
-          isfinite(wz) && isfinite(px) && isfinite(py) && isfinite(pz)))
-        atomicOr(nonfinite, 1);
-    // drift of the next step (ColliderSingleCore.cpp:82-97)
-    s.f[QX][b] = px;
-    s.f[QY][b] = py;
-    s.f[QZ][b] = pz;
-    const double hx = vx + .5 * ax * dt;
-    const double hy = vy + .5 * ay * dt;
-    const double hz = vz + .5 * az * dt;
-    s.f[HX][b] = hx;
-    s.f[HY][b] = hy;
-    s.f[HZ][b] = hz;
-    s.f[GX][b] = wx + .5 * bx * dt;
-    s.f[GY][b] = wy + .5 * by * dt;
-    s.f[GZ][b] = wz + .5 * bz * dt;
-    s.f[PX][b] = px + hx * dt;
-    s.f[PY][b] = py + hy * dt;
-    s.f[PZ][b] = pz + hz * dt;
-}
-
 // ---- launchers --------------------------------------------------------------
 
 hipError_t launch_drift(const State& s, int n, double dt, hipStream_t st)
@@ -537,75 +656,84 @@ hipError_t launch_copy_prev(const State& s, int n, hipStream_t st)
     return hipGetLastError();
 }
 
-// Launch shapes of the ordered pair pass: {balls per workgroup, producer wavefronts, partners
-// per chunk, consumer wavefront of its own}.  All give the same results bit for bit.
+// Launch shapes of the ordered pair pass: balls per workgroup, pairs per lane and batch,
+// wavefronts, steps of touching pairs kept, wavefronts per SIMD the registers are held to, pairs unrolled.  All give
+// the same results bit for bit.
+#define SL_ORD_SHAPES(X) \
+    X(0, 2, 2, 8, 2, 2, 2, true) \
+    X(1, 4, 4, 8, 2, 2, 2, true) \
+    X(2, 4, 4, 4, 1, 3, 2, true) \
+    X(3, 4, 4, 4, 1, 3, 2, false) \
+    X(4, 8, 4, 4, 1, 3, 2, false) \
+    X(5, 2, 2, 4, 1, 3, 2, true) \
+    X(6, 4, 2, 8, 2, 2, 2, true) \
+    X(7, 2, 1, 8, 1, 2, 1, true) \
+    X(8, 2, 1, 4, 1, 2, 1, true)
+
 namespace {
-struct OrdShape {
-    int bi, npw, cj, ded;
-};
-constexpr OrdShape ORD_SHAPES[] = {
-    {2, 3, 192, 1}, {4, 3, 48, 1}, {4, 4, 64, 0}, {8, 4, 32, 0}, {2, 2, 128, 0},
-    {4, 3, 96, 1},  {2, 2, 128, 0}, {2, 4, 128, 0}, {2, 4, 128, 0},
-};
-constexpr int N_ORD_SHAPES = (int)(sizeof(ORD_SHAPES) / sizeof(ORD_SHAPES[0]));
+#define SL_X(id, NB, CH, W, AD, WPE, UNR, SCAN) NB,
+constexpr int ORD_BALLS[] = {SL_ORD_SHAPES(SL_X)};
+#undef SL_X
+constexpr int N_ORD_SHAPES = (int)(sizeof(ORD_BALLS) / sizeof(ORD_BALLS[0]));
 }  // namespace
 
 int ordered_shapes() { return N_ORD_SHAPES; }
 
-// The shape used when none is chosen (the allocation-free entry point, and until the
-// tuner has run), from timings on MI355X, both with a consumer wavefront of their own and
-// registers held to 3 wavefronts per SIMD: up to about 1500 balls 2 balls per workgroup and
-// chunks of 192 partners; above, 4 balls and chunks of 96 (the fastest shape from 2,200 to
-// 65,536 balls).
-int ordered_default_shape(int n) { return n < 1500 ? 0 : 5; }
+// The shape used when none is chosen (the allocation-free entry point, and until the tuner has
+// run).  Shapes 0 and 1 put 8 wavefronts on a CU, one workgroup of 2 or 4 balls: they are the
+// fastest while every workgroup has a CU of its own (512 and 1,024 balls on 256 CUs: 450
+// balls 11.8 and 14.8 us per step, 600 19.2 and 16.8, 1,000 26 and 18.9, 1,200 41 and 33.6).
+// Then 4 wavefronts and three workgroups a CU, with the scan up to 2,500 balls; from about
+// 20,000 on 8 balls a workgroup (fewer adds per pair: 15,039 balls 1,099 and 1,132 us with 4
+// and 8, 40,000 7,485 and 7,266).
+int ordered_default_shape(int n)
+{
+    return n <= 512 ? 0 : n <= 1024 ? 1 : n <= 2500 ? 2 : n <= 20000 ? 3 : 4;
+}
 
 int ordered_blocks(int n, int shape)
 {
-    const int bi = ORD_SHAPES[(shape >= 0 && shape < N_ORD_SHAPES) ? shape : 0].bi;
-    return (n + bi - 1) / bi;
+    const int nb = ORD_BALLS[(shape >= 0 && shape < N_ORD_SHAPES) ? shape : 0];
+    return (n + nb - 1) / nb;
 }
+
+namespace {
+hipError_t launch_ordered(const OrdState& os, const Phys& P, int n, int write, double* pe_ball,
+                          unsigned long long* contacts, hipStream_t st, int shape)
+{
+    if (shape < 0 || shape >= N_ORD_SHAPES) shape = 0;
+    const int nb = ordered_blocks(n, shape);
+#define SL_X(id, NB, CH, W, AD, WPE, UNR, SCAN)                                                                     \
+    case id:                                                                                                    \
+        if (write)                                                                                              \
+            k_pairs_ordered<NB, CH, W, AD, WPE, UNR, SCAN, true><<<nb, 64 * W, 0, st>>>(os, P, n, pe_ball, contacts);  \
+        else                                                                                                    \
+            k_pairs_ordered<NB, CH, W, AD, WPE, UNR, SCAN, false><<<nb, 64 * W, 0, st>>>(os, P, n, pe_ball, contacts); \
+        break;
+    switch (shape) {
+        SL_ORD_SHAPES(SL_X)
+    }
+#undef SL_X
+    return hipGetLastError();
+}
+}  // namespace
 
 hipError_t launch_pairs_ordered(const State& s, const Phys& P, int n, int write, double* pe_ball,
                                 unsigned long long* contacts, hipStream_t st, int shape)
 {
     if (n <= 1) return hipSuccess;
-    if (shape < 0 || shape >= N_ORD_SHAPES) shape = 0;
-    const int nb = ordered_blocks(n, shape);
-    // template arguments: balls, producer wavefronts, partners per chunk, dedicated consumer
-    // wavefront, contact arm out of line, wavefronts per SIMD the registers are held to,
-    // unroll of the far-field loop (case 5: both of a thread's pairs per chunk, 1% faster at
-    // 5,000 balls than one at a time)
-#define SL_ORD(BI, NPW, CJ, DED, CALL, WPE, UNR)                                                                \
-    do {                                                                                                         \
-        constexpr int T = 64 * (NPW + (DED ? 1 : 0));                                                            \
-        if (write)                                                                                               \
-            k_pairs_ordered<BI, NPW, CJ, DED, CALL, WPE, UNR, true><<<nb, T, 0, st>>>(s, P, n, pe_ball, contacts);  \
-        else                                                                                                     \
-            k_pairs_ordered<BI, NPW, CJ, DED, CALL, WPE, UNR, false><<<nb, T, 0, st>>>(s, P, n, pe_ball, contacts); \
-    } while (0)
-    switch (shape) {
-    case 0: SL_ORD(2, 3, 192, true, false, 3, 1); break;
-    case 1: SL_ORD(4, 3, 48, true, false, 3, 1); break;
-    case 2: SL_ORD(4, 4, 64, false, false, 3, 1); break;
-    case 3: SL_ORD(8, 4, 32, false, false, 3, 1); break;
-    case 4: SL_ORD(2, 2, 128, false, false, 0, 1); break;
-    case 5: SL_ORD(4, 3, 96, true, false, 3, 2); break;
-    case 6: SL_ORD(2, 2, 128, false, true, 0, 1); break;
-    case 7: SL_ORD(2, 4, 128, false, false, 3, 1); break;
-    default: SL_ORD(2, 4, 128, false, false, 0, 1); break;
-    }
-#undef SL_ORD
-    return hipGetLastError();
+    const OrdState os{s.f[0], s.f[0], nullptr, (long)(s.f[1] - s.f[0]), 0, nullptr};
+    return launch_ordered(os, P, n, write, pe_ball, contacts, st, shape);
+}
+
+hipError_t launch_step_ordered(const double* konst, double* cur, double* nxt, long stride, const Phys& P, int n, int drift,
+                               unsigned long long* contacts, int* nonfinite, hipStream_t st, int shape)
+{
+    const OrdState os{cur, konst, nxt, stride, drift, nonfinite};
+    return launch_ordered(os, P, n, 0, nullptr, contacts, st, shape);
 }
 
 int kick_blocks(int n) { return (n + 255) / 256; }
-
-hipError_t launch_kick_drift(const State& s, int n, double dt, int* nonfinite, hipStream_t st)
-{
-    if (n <= 0) return hipSuccess;
-    k_kick_drift<<<kick_blocks(n), 256, 0, st>>>(s, n, dt, nonfinite);
-    return hipGetLastError();
-}
 
 hipError_t launch_kick(const State& s, int n, double dt, int write, int kick, double* e_part,
                        int* nonfinite, hipStream_t st)
