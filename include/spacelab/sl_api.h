@@ -115,6 +115,9 @@ int sl_download(sl_ctx* ctx, double* pos3, double* vel3, double* w3, double* acc
                 double* aacc3);
 /* Half-step velocities of the last step (velh, wh in the reference). */
 int sl_download_half(sl_ctx* ctx, double* velh3, double* wh3);
+/* Both in one read.  Any of the arrays may be NULL. */
+int sl_download_state(sl_ctx* ctx, double* pos3, double* vel3, double* w3, double* acc3, double* aacc3,
+                      double* velh3, double* wh3);
 
 int sl_synchronize(sl_ctx* ctx);
 long long sl_step_count(const sl_ctx* ctx);

@@ -113,6 +113,16 @@ class Energy:
         return Energy(e.PE, e.KE, np.array(e.p[:]), np.array(e.L[:]), bool(e.nonfinite),
                       int(e.contacts))
 
+    @staticmethod
+    def _from_buffer(buf, n: int) -> list["Energy"]:
+        """The first n of a ctypes array of _Energy; p and L are rows of arrays of this call."""
+        a = np.frombuffer(buf, dtype=_ENERGY, count=n)
+        return [Energy(pe, ke, p, L, bool(bad), contacts) for pe, ke, p, L, bad, contacts in
+                zip(a["PE"].tolist(), a["KE"].tolist(), a["p"].copy(), a["L"].copy(),
+                    a["nonfinite"].tolist(), a["contacts"].tolist())]
+
+
+_ENERGY = np.dtype(_Energy)
 
 _lib = None
 
@@ -137,6 +147,7 @@ def lib():
     L.sl_step.argtypes = [vp, C.c_int, C.c_int, C.POINTER(_Energy), C.c_int]
     L.sl_download.argtypes = [vp] + [dp] * 5
     L.sl_download_half.argtypes = [vp, dp, dp]
+    L.sl_download_state.argtypes = [vp] + [dp] * 7
     L.sl_synchronize.argtypes = [vp]
     L.sl_step_count.argtypes = [vp]
     L.sl_step_count.restype = C.c_longlong
@@ -516,7 +527,7 @@ class Collider:
         buf = (_Energy * max(cap, 1))()
         nw = self._check(lib().sl_step(self._ctx, int(n_steps), int(write_every), buf, max(cap, 1)),
                          "sl_step")
-        return [Energy._from(buf[k]) for k in range(min(nw, cap))]
+        return Energy._from_buffer(buf, min(nw, cap))
 
     def sim_one_step(self, write_step: bool) -> Energy | None:
         """One step (ColliderSingleCore.cpp:78-288); energies when write_step."""
@@ -541,9 +552,8 @@ class Collider:
         pos = np.empty((n, 3)); vel = np.empty((n, 3)); w = np.empty((n, 3))
         acc = np.empty((n, 3)); aacc = np.empty((n, 3))
         velh = np.empty((n, 3)); wh = np.empty((n, 3))
-        self._check(lib().sl_download(self._ctx, _dp(pos), _dp(vel), _dp(w), _dp(acc), _dp(aacc)),
-                    "sl_download")
-        self._check(lib().sl_download_half(self._ctx, _dp(velh), _dp(wh)), "sl_download_half")
+        self._check(lib().sl_download_state(self._ctx, _dp(pos), _dp(vel), _dp(w), _dp(acc), _dp(aacc),
+                                            _dp(velh), _dp(wh)), "sl_download_state")
         R, m, moi = self._static
         return BallGroup(pos, vel, w, R.copy(), m.copy(), moi.copy(), acc, aacc, velh, wh)
 
@@ -645,7 +655,7 @@ class Batch:
     def init_conditions(self) -> list[Energy]:
         buf = (_Energy * self.n_sys)()
         self._check(lib().sl_batch_init_forces(self._b, buf), "sl_batch_init_forces")
-        return [Energy._from(buf[s]) for s in range(self.n_sys)]
+        return Energy._from_buffer(buf, self.n_sys)
 
     def step(self, n_steps: int, write_every: int = 0) -> list[list[Energy]]:
         if write_every > 0:
@@ -657,7 +667,8 @@ class Batch:
         buf = (_Energy * max(cap * ns, 1))()
         nw = self._check(lib().sl_batch_step(self._b, int(n_steps), int(write_every), buf,
                                              max(cap, 1) if cap else 0), "sl_batch_step")
-        return [[Energy._from(buf[k * ns + s]) for s in range(ns)] for k in range(min(nw, cap))]
+        out = Energy._from_buffer(buf, min(nw, cap) * ns)
+        return [out[k * ns:(k + 1) * ns] for k in range(min(nw, cap))]
 
     @property
     def step_count(self) -> int:
@@ -669,13 +680,13 @@ class Batch:
         acc = np.empty((n, 3)); aacc = np.empty((n, 3))
         self._check(lib().sl_batch_download(self._b, _dp(pos), _dp(vel), _dp(w), _dp(acc),
                                             _dp(aacc)), "sl_batch_download")
-        R, m, moi = self._static
+        # each group's arrays are its parts of this call's arrays
+        R, m, moi = (a.copy() for a in self._static)
         out, o = [], 0
         for k in self.sizes:
-            sl_ = slice(o, o + k)
-            out.append(BallGroup(pos[sl_].copy(), vel[sl_].copy(), w[sl_].copy(), R[sl_].copy(),
-                                 m[sl_].copy(), moi[sl_].copy(), acc[sl_].copy(), aacc[sl_].copy()))
-            o += k
+            e = o + k
+            out.append(BallGroup(pos[o:e], vel[o:e], w[o:e], R[o:e], m[o:e], moi[o:e], acc[o:e], aacc[o:e]))
+            o = e
         return out
 
     def set_option(self, name: str, value: int):

@@ -28,17 +28,18 @@ struct sl_ctx {
     sl_params p{};
     double* base = nullptr;     // NFIELD * n_pad doubles
     State st{};
-    double* pe_part = nullptr;  // per-ball pair energies (write steps)
-    double* e_part = nullptr;   // per-block KE/p/L partials
-    unsigned long long* cnt = nullptr;  // [0] contacts total, [1] contacts this write step, [2..3] tuner trials
+    // what a write step reads back, one after another in one allocation (and its pinned copy):
+    // contact counters ([0] total, [1] this write step, [2..3] tuner trials), the non-finite
+    // flag, per-block KE/p/L partials, per-ball pair energies
+    unsigned long long* cnt = nullptr;
+    int* nonfinite = nullptr;
+    double* e_part = nullptr;
+    double* pe_part = nullptr;
     int ord_shape = -1;         // launch shape of the ordered pair pass (-1: not chosen yet)
     int forced_ord_shape = 0;   // 1 + shape forces it
     std::map<int, hipGraphExec_t> ord_graphs;   // captured runs of ordered non-write steps, by length
-    int* nonfinite = nullptr;
-    double* h_pe = nullptr;     // pinned
-    double* h_e = nullptr;      // pinned
-    unsigned long long* h_cnt = nullptr;
-    int* h_nonfinite = nullptr;
+    char* h_back = nullptr;     // pinned
+    HostStage stage{};
     FastBuffers fb{};
     long long step = 0;
     bool uploaded = false;
@@ -166,14 +167,9 @@ int flush_profile(sl_ctx* c)
 int free_ctx_buffers(sl_ctx* c)
 {
     if (c->base) hipFree(c->base);
-    if (c->pe_part) hipFree(c->pe_part);
-    if (c->e_part) hipFree(c->e_part);
     if (c->cnt) hipFree(c->cnt);
-    if (c->nonfinite) hipFree(c->nonfinite);
-    if (c->h_pe) hipHostFree(c->h_pe);
-    if (c->h_e) hipHostFree(c->h_e);
-    if (c->h_cnt) hipHostFree(c->h_cnt);
-    if (c->h_nonfinite) hipHostFree(c->h_nonfinite);
+    if (c->h_back) hipHostFree(c->h_back);
+    stage_free(c->stage);
     fast_free(c->fb);
     c->base = nullptr;
     return SL_OK;
@@ -203,26 +199,26 @@ void hook_after(void* u, int kind)
 // Read back and sum the partials of a write step (fixed order: deterministic).
 int read_energy(sl_ctx* c, int n_pe_blocks, int n_e_blocks, sl_energy* out, bool has_pe)
 {
-    if (has_pe && n_pe_blocks > 0)
-        HIPCHK(c, hipMemcpyAsync(c->h_pe, c->pe_part, sizeof(double) * n_pe_blocks, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipMemcpyAsync(c->h_e, c->e_part, sizeof(double) * 7 * n_e_blocks, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipMemcpyAsync(c->h_cnt, c->cnt, sizeof(unsigned long long) * 2, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipMemcpyAsync(c->h_nonfinite, c->nonfinite, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    const size_t e_off = (char*)c->e_part - (char*)c->cnt, pe_off = (char*)c->pe_part - (char*)c->cnt;
+    const size_t bytes = pe_off + sizeof(double) * (has_pe ? n_pe_blocks : 0);
+    HIPCHK(c, hipMemcpyAsync(c->h_back, c->cnt, bytes, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
+    const double* h_e = reinterpret_cast<const double*>(c->h_back + e_off);
+    const double* h_pe = reinterpret_cast<const double*>(c->h_back + pe_off);
     sl_energy e{};
     if (has_pe)
-        for (int b = 0; b < n_pe_blocks; b++) e.PE += c->h_pe[b];
+        for (int b = 0; b < n_pe_blocks; b++) e.PE += h_pe[b];
     for (int b = 0; b < n_e_blocks; b++) {
-        e.KE += c->h_e[7 * b + 0];
-        e.p[0] += c->h_e[7 * b + 1];
-        e.p[1] += c->h_e[7 * b + 2];
-        e.p[2] += c->h_e[7 * b + 3];
-        e.L[0] += c->h_e[7 * b + 4];
-        e.L[1] += c->h_e[7 * b + 5];
-        e.L[2] += c->h_e[7 * b + 6];
+        e.KE += h_e[7 * b + 0];
+        e.p[0] += h_e[7 * b + 1];
+        e.p[1] += h_e[7 * b + 2];
+        e.p[2] += h_e[7 * b + 3];
+        e.L[0] += h_e[7 * b + 4];
+        e.L[1] += h_e[7 * b + 5];
+        e.L[2] += h_e[7 * b + 6];
     }
-    e.contacts = (long long)c->h_cnt[1];
-    e.nonfinite = *c->h_nonfinite;
+    e.contacts = (long long)reinterpret_cast<const unsigned long long*>(c->h_back)[1];
+    e.nonfinite = *reinterpret_cast<const int*>(c->h_back + 4 * sizeof(unsigned long long));
     if (out) *out = e;
     return SL_OK;
 }
@@ -421,21 +417,18 @@ int sl_create(sl_ctx** out, int n_max, const sl_params* p)
     };
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) return fail(SL_E_HIP);
     if (hipMalloc(&c->base, sizeof(double) * (size_t)NFIELD * c->n_pad) != hipSuccess) return fail(SL_E_HIP);
-    const int max_blocks = n_max + 8;   // per-ball pair energies
-    const int e_blocks = kick_blocks(n_max) + 8;
-    if (hipMalloc(&c->pe_part, sizeof(double) * max_blocks) != hipSuccess) return fail(SL_E_HIP);
-    if (hipMalloc(&c->e_part, sizeof(double) * 7 * e_blocks) != hipSuccess) return fail(SL_E_HIP);
-    if (hipMalloc(&c->cnt, sizeof(unsigned long long) * 4) != hipSuccess) return fail(SL_E_HIP);
-    if (hipMalloc(&c->nonfinite, sizeof(int)) != hipSuccess) return fail(SL_E_HIP);
-    if (hipHostMalloc(&c->h_pe, sizeof(double) * max_blocks, 0) != hipSuccess) return fail(SL_E_HIP);
-    if (hipHostMalloc(&c->h_e, sizeof(double) * 7 * e_blocks, 0) != hipSuccess) return fail(SL_E_HIP);
-    if (hipHostMalloc(&c->h_cnt, sizeof(unsigned long long) * 2, 0) != hipSuccess) return fail(SL_E_HIP);
-    if (hipHostMalloc(&c->h_nonfinite, sizeof(int), 0) != hipSuccess) return fail(SL_E_HIP);
+    const size_t e_off = 64, pe_off = e_off + sizeof(double) * 7 * kick_blocks(n_max);
+    const size_t back = pe_off + sizeof(double) * n_max;
+    if (hipMalloc(&c->cnt, back) != hipSuccess) return fail(SL_E_HIP);
+    c->nonfinite = reinterpret_cast<int*>(c->cnt + 4);
+    c->e_part = reinterpret_cast<double*>((char*)c->cnt + e_off);
+    c->pe_part = reinterpret_cast<double*>((char*)c->cnt + pe_off);
+    if (hipHostMalloc(&c->h_back, back, 0) != hipSuccess) return fail(SL_E_HIP);
+    if (stage_alloc(c->stage, stage_size(n_max)) != SL_OK) return fail(SL_E_HIP);
     if (fast_alloc(c->fb, c->n_pad, 1) != 0) return fail(SL_E_HIP);
     for (int f = 0; f < NFIELD; f++) c->st.f[f] = c->base + (size_t)f * c->n_pad;
     if (hipMemsetAsync(c->base, 0, sizeof(double) * (size_t)NFIELD * c->n_pad, c->stream) != hipSuccess ||
-        hipMemsetAsync(c->cnt, 0, sizeof(unsigned long long) * 4, c->stream) != hipSuccess ||
-        hipMemsetAsync(c->nonfinite, 0, sizeof(int), c->stream) != hipSuccess ||
+        hipMemsetAsync(c->cnt, 0, e_off, c->stream) != hipSuccess ||
         hipStreamSynchronize(c->stream) != hipSuccess)
         return fail(SL_E_HIP);
     *out = c;
@@ -669,48 +662,31 @@ int sl_step(sl_ctx* c, int n_steps, int write_every, sl_energy* e_out, int e_cap
     return nw;
 }
 
-int sl_download(sl_ctx* c, double* pos3, double* vel3, double* w3, double* acc3, double* aacc3)
+int sl_download_state(sl_ctx* c, double* pos3, double* vel3, double* w3, double* acc3, double* aacc3, double* velh3,
+                      double* wh3)
 {
     if (!c) return SL_E_ARG;
     if (!c->uploaded) return set_err(c, SL_E_STATE, "download before upload");
-    const int rc = fast_sync_to(c->fb, c->st, c->stream, &c->err);
-    if (rc) return rc;
-    const size_t np = (size_t)c->n_pad;
-    std::vector<double> h((size_t)NFIELD * np);
-    HIPCHK(c, hipMemcpyAsync(h.data(), c->base, sizeof(double) * h.size(), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    auto get3 = [&](int f0, double* a) {
-        if (!a) return;
-        for (int i = 0; i < c->n; i++) {
-            a[3 * i + 0] = h[(size_t)(f0 + 0) * np + i];
-            a[3 * i + 1] = h[(size_t)(f0 + 1) * np + i];
-            a[3 * i + 2] = h[(size_t)(f0 + 2) * np + i];
+    const int fields[MAX_READ] = {PX, VX, WX, AX, BX, HX, GX};
+    double* const outs[MAX_READ] = {pos3, vel3, w3, acc3, aacc3, velh3, wh3};
+    int field[MAX_READ], nv = 0;
+    double* out[MAX_READ];
+    for (int v = 0; v < MAX_READ; v++)
+        if (outs[v]) {
+            field[nv] = fields[v];
+            out[nv++] = outs[v];
         }
-    };
-    get3(PX, pos3);
-    get3(VX, vel3);
-    get3(WX, w3);
-    get3(AX, acc3);
-    get3(BX, aacc3);
-    return SL_OK;
+    return fast_read(c->fb, c->st, c->stage, field, out, nv, c->stream, &c->err);
+}
+
+int sl_download(sl_ctx* c, double* pos3, double* vel3, double* w3, double* acc3, double* aacc3)
+{
+    return sl_download_state(c, pos3, vel3, w3, acc3, aacc3, nullptr, nullptr);
 }
 
 int sl_download_half(sl_ctx* c, double* velh3, double* wh3)
 {
-    if (!c) return SL_E_ARG;
-    if (!c->uploaded) return set_err(c, SL_E_STATE, "download before upload");
-    const int rc = fast_sync_to(c->fb, c->st, c->stream, &c->err);
-    if (rc) return rc;
-    const size_t np = (size_t)c->n_pad;
-    std::vector<double> h(6 * np);
-    HIPCHK(c, hipMemcpyAsync(h.data(), c->st.f[HX], sizeof(double) * 6 * np, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    for (int i = 0; i < c->n; i++)
-        for (int k = 0; k < 3; k++) {
-            if (velh3) velh3[3 * i + k] = h[(size_t)k * np + i];
-            if (wh3) wh3[3 * i + k] = h[(size_t)(3 + k) * np + i];
-        }
-    return SL_OK;
+    return sl_download_state(c, nullptr, nullptr, nullptr, nullptr, nullptr, velh3, wh3);
 }
 
 int sl_synchronize(sl_ctx* c)
@@ -755,10 +731,10 @@ int sl_profile_read(sl_ctx* c, sl_profile* out)
     if (!c || !out) return SL_E_ARG;
     int rc = flush_profile(c);
     if (rc) return rc;
-    HIPCHK(c, hipMemcpyAsync(c->h_cnt, c->cnt, sizeof(unsigned long long) * 2, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, hipMemcpyAsync(c->h_back, c->cnt, sizeof(unsigned long long) * 2, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     *out = c->acc_prof;
-    out->contacts = (long long)c->h_cnt[0];
+    out->contacts = (long long)*reinterpret_cast<const unsigned long long*>(c->h_back);
     long long fc = 0, fn = 0;
     if (fast_read_counters(c->fb, c->stream, &fc, &fn) != 0) return set_err(c, SL_E_HIP, "reading counters failed");
     out->contacts += fc;

@@ -25,6 +25,7 @@ struct sl_batch {
     double* base = nullptr;   // NFIELD * n_pad doubles
     State st{};
     FastBuffers fb{};
+    HostStage stage{};
     FastLayout lay;
     std::vector<Phys> P;
     std::vector<int> n_sys_balls;
@@ -53,6 +54,7 @@ bool positive(double x) { return x > 0 && std::isfinite(x); }
 void release(sl_batch* b)
 {
     fast_free(b->fb);
+    stage_free(b->stage);
     if (b->base) (void)hipFree(b->base);
     b->base = nullptr;
     if (b->stream) (void)hipStreamDestroy(b->stream);
@@ -123,6 +125,7 @@ int sl_batch_create(sl_batch** out, int max_systems, int max_balls, const sl_par
     if (hipMemset(b->base, 0, sizeof(double) * (size_t)NFIELD * b->n_pad) != hipSuccess) return fail(SL_E_HIP);
     for (int f = 0; f < NFIELD; f++) b->st.f[f] = b->base + (size_t)f * b->n_pad;
     if (fast_alloc(b->fb, b->n_pad, max_systems) != 0) return fail(SL_E_HIP);
+    if (stage_alloc(b->stage, stage_size(b->n_pad)) != SL_OK) return fail(SL_E_HIP);
     *out = b;
     return SL_OK;
 }
@@ -226,27 +229,16 @@ int sl_batch_download(sl_batch* b, double* pos3, double* vel3, double* w3, doubl
 {
     if (!b) return SL_E_ARG;
     if (!b->uploaded) return berr(b, SL_E_STATE, "download before upload");
-    const int rc = fast_sync_to(b->fb, b->st, b->stream, &b->err);
-    if (rc) return rc;
-    const size_t np = (size_t)b->n_pad;
-    const int nf = BZ + 1;   // positions through angular accelerations
-    std::vector<double> h((size_t)nf * np);
-    if (hipMemcpyAsync(h.data(), b->base, sizeof(double) * h.size(), hipMemcpyDeviceToHost, b->stream) != hipSuccess ||
-        hipStreamSynchronize(b->stream) != hipSuccess)
-        return berr(b, SL_E_HIP, "state download failed");
-    int dst = 0;
-    for (int s = 0; s < b->lay.n_sys; s++)
-        for (int k = 0; k < b->lay.n[s]; k++, dst++) {
-            const size_t d = (size_t)b->lay.off[s] + k;
-            for (int x = 0; x < 3; x++) {
-                if (pos3) pos3[3 * dst + x] = h[(size_t)(PX + x) * np + d];
-                if (vel3) vel3[3 * dst + x] = h[(size_t)(VX + x) * np + d];
-                if (w3) w3[3 * dst + x] = h[(size_t)(WX + x) * np + d];
-                if (acc3) acc3[3 * dst + x] = h[(size_t)(AX + x) * np + d];
-                if (aacc3) aacc3[3 * dst + x] = h[(size_t)(BX + x) * np + d];
-            }
+    const int fields[5] = {PX, VX, WX, AX, BX};
+    double* const outs[5] = {pos3, vel3, w3, acc3, aacc3};
+    int field[5], nv = 0;
+    double* out[5];
+    for (int v = 0; v < 5; v++)
+        if (outs[v]) {
+            field[nv] = fields[v];
+            out[nv++] = outs[v];
         }
-    return SL_OK;
+    return fast_read(b->fb, b->st, b->stage, field, out, nv, b->stream, &b->err);
 }
 
 int sl_batch_set_option(sl_batch* b, int option, int value)

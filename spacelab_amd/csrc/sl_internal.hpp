@@ -49,7 +49,8 @@ struct FastAux {
 // slots up to the next system are padding.  A single simulation is one system.
 struct FastLayout {
     int n_sys = 0;
-    std::vector<int> n, off, nb;   // balls, first ball, 64-ball blocks per system
+    std::vector<int> n, off, nb;   // balls, first slot, 64-ball blocks per system
+    std::vector<int> first;        // balls of the systems before
     int n_used = 0;                // ball slots in use (padded)
     int nb_max = 0;                // largest block count of one system
 };
@@ -79,6 +80,7 @@ struct FastBuffers {
     State eng[2] = {};
     int cur = 0;                  // engine set holding the current state
     int* perm = nullptr;          // device, n_pad
+    int* slot_of = nullptr;       // its inverse: canonical slot -> engine slot
     bool canon_valid = true;      // the canonical set holds the current state
     bool eng_valid = false;       // the engine sets hold the current state
     bool drifted = false;         // the next step's drift was already applied
@@ -92,6 +94,7 @@ struct FastBuffers {
     int* sys_off = nullptr;
     int* sys_n = nullptr;
     int* sys_nb = nullptr;
+    int* sys_first = nullptr;     // balls of the systems before
     Phys* sysP = nullptr;
     int4* tiles = nullptr;        // {I, J, system, first block of system}, I >= J
     int n_tiles = 0, cap_tiles = 0;
@@ -127,6 +130,31 @@ struct FastBuffers {
 };
 
 constexpr int FAST_E_STRIDE = 10;   // doubles per energy block
+
+// ---- state read-back: sl_io.hip
+constexpr int MAX_READ = 7;         // vectors one read can ask for
+struct HostStage {                  // pinned host memory the packing kernel writes
+    char *h = nullptr, *d = nullptr;   // host and device address
+    size_t bytes = 0;
+    hipEvent_t ev[2] = {};
+};
+int stage_alloc(HostStage& hs, size_t bytes);
+void stage_free(HostStage& hs);
+// Staging for n_max balls: all of them twice, at least one block and at most 2 MB (what the
+// host's cache holds while a piece is copied out of it).
+inline size_t stage_size(long long n_max)
+{
+    const long long want = 2LL * MAX_READ * 24 * ((n_max + FAST_TILE - 1) / FAST_TILE) * FAST_TILE;
+    return (size_t)(want < (2 << 20) ? want : (2 << 20));
+}
+// nv vectors (fields field[v] .. + 2) of the state s, whose slot for the caller's slot c is
+// slot_of[c] (NULL: c), to out[v] (x, y, z per ball, systems one after another).  Waits for
+// the stream's work.  fb: the device's layout tables (more than one system).
+int read_state(HostStage& hs, const State& s, const int* slot_of, const FastLayout& lay, const FastBuffers* fb,
+               const int* field, double* const* out, int nv, hipStream_t st);
+// The engine's (or, when it is the one up to date, the canonical) state read like that.
+int fast_read(FastBuffers& fb, State& canon, HostStage& hs, const int* field, double* const* out, int nv, hipStream_t st,
+              std::string* err);
 
 int fast_alloc(FastBuffers& fb, int n_pad, int max_sys);
 void fast_free(FastBuffers& fb);

@@ -540,6 +540,7 @@ FastLayout fast_layout(int n_sys, const int* n_per_sys)
     for (int s = 0; s < n_sys; s++) {
         const int n = n_per_sys[s];
         const int nb = (n + TB - 1) / TB;
+        L.first.push_back(s ? L.first[s - 1] + L.n[s - 1] : 0);
         L.n.push_back(n);
         L.off.push_back(off);
         L.nb.push_back(nb);
@@ -562,7 +563,8 @@ int fast_alloc(FastBuffers& fb, int n_pad, int max_sys)
     fb.max_sys = max_sys;
     const int nblocks = (n_pad + TB - 1) / TB;
     if (hipMalloc(&fb.eng_base, sizeof(double) * 2 * (size_t)NFIELD * n_pad) != hipSuccess) return -1;
-    if (hipMalloc(&fb.perm, sizeof(int) * n_pad) != hipSuccess) return -1;
+    if (hipMalloc(&fb.perm, sizeof(int) * 2 * n_pad) != hipSuccess) return -1;
+    fb.slot_of = fb.perm + n_pad;
     if (hipMalloc(&fb.aux.q, sizeof(double) * n_pad) != hipSuccess) return -1;
     if (hipMalloc(&fb.aux.g, sizeof(double) * n_pad) != hipSuccess) return -1;
     if (hipMalloc(&fb.aux.q32, sizeof(float) * n_pad) != hipSuccess) return -1;
@@ -575,7 +577,8 @@ int fast_alloc(FastBuffers& fb, int n_pad, int max_sys)
     if (hipMalloc(&fb.blk_sys, sizeof(int) * nblocks) != hipSuccess) return -1;
     if (hipMalloc(&fb.sys_off, sizeof(int) * max_sys) != hipSuccess) return -1;
     if (hipMalloc(&fb.sys_n, sizeof(int) * max_sys) != hipSuccess) return -1;
-    if (hipMalloc(&fb.sys_nb, sizeof(int) * max_sys) != hipSuccess) return -1;
+    if (hipMalloc(&fb.sys_nb, sizeof(int) * 2 * max_sys) != hipSuccess) return -1;
+    fb.sys_first = fb.sys_nb + max_sys;
     if (hipMalloc(&fb.sysP, sizeof(Phys) * max_sys) != hipSuccess) return -1;
     if (hipMalloc(&fb.flags, sizeof(int) * 4) != hipSuccess) return -1;
     const int eblocks = (n_pad + BPB - 1) / BPB;
@@ -726,6 +729,7 @@ int fast_configure(FastBuffers& fb, State& canon, const FastLayout& lay, const P
             hipMemcpyAsync(fb.sys_off, lay.off.data(), sizeof(int) * lay.n_sys, hipMemcpyHostToDevice, st) != hipSuccess ||
             hipMemcpyAsync(fb.sys_n, lay.n.data(), sizeof(int) * lay.n_sys, hipMemcpyHostToDevice, st) != hipSuccess ||
             hipMemcpyAsync(fb.sys_nb, lay.nb.data(), sizeof(int) * lay.n_sys, hipMemcpyHostToDevice, st) != hipSuccess ||
+            hipMemcpyAsync(fb.sys_first, lay.first.data(), sizeof(int) * lay.n_sys, hipMemcpyHostToDevice, st) != hipSuccess ||
             hipStreamSynchronize(st) != hipSuccess)
             return err_hip(err, "layout tables");
         fb.n_tiles = nt;
@@ -742,8 +746,10 @@ int fast_configure(FastBuffers& fb, State& canon, const FastLayout& lay, const P
         hipMemcpyAsync(z.data(), canon.f[PZ], sizeof(double) * nu, hipMemcpyDeviceToHost, st) != hipSuccess ||
         hipStreamSynchronize(st) != hipSuccess)
         return err_hip(err, "read positions");
-    const std::vector<int> perm = morton_perm(lay, x, y, z, fb.n_pad);
-    if (hipMemcpyAsync(fb.perm, perm.data(), sizeof(int) * fb.n_pad, hipMemcpyHostToDevice, st) != hipSuccess ||
+    std::vector<int> perm = morton_perm(lay, x, y, z, fb.n_pad);
+    perm.resize(2 * (size_t)fb.n_pad);
+    for (int k = 0; k < fb.n_pad; k++) perm[(size_t)fb.n_pad + perm[k]] = k;
+    if (hipMemcpyAsync(fb.perm, perm.data(), sizeof(int) * perm.size(), hipMemcpyHostToDevice, st) != hipSuccess ||
         hipStreamSynchronize(st) != hipSuccess)
         return err_hip(err, "permutation");
     k_gather<<<(nu + 255) / 256, 256, 0, st>>>(fb.eng[0], canon, fb.perm, nu, RAD, NFIELD);
@@ -762,6 +768,15 @@ int fast_sync_to(FastBuffers& fb, State& canon, hipStream_t st, std::string* err
     k_scatter<<<(fb.lay.n_used + 255) / 256, 256, 0, st>>>(canon, fb.eng[fb.cur], fb.perm, fb.lay.n_used, PX, RAD);
     if (hipGetLastError() != hipSuccess || hipStreamSynchronize(st) != hipSuccess) return err_hip(err, "copy state");
     fb.canon_valid = true;
+    return 0;
+}
+
+int fast_read(FastBuffers& fb, State& canon, HostStage& hs, const int* field, double* const* out, int nv, hipStream_t st,
+              std::string* err)
+{
+    const bool here = fb.canon_valid;
+    if (read_state(hs, here ? canon : fb.eng[fb.cur], here ? nullptr : fb.slot_of, fb.lay, &fb, field, out, nv, st) != SL_OK)
+        return err_hip(err, "state read-back");
     return 0;
 }
 
