@@ -117,7 +117,10 @@ struct TileArgs {
     double Kf;              // mixed: force = Kf * (scaled binary32 factor) * (r / L0)
     double* part;           // [slot][xyz][n_pad]; the mixed mode stores binary32 sums, Kf left out,
                             // in the first half of the same buffer ([slot][xyz][n_pad] floats)
-    unsigned long long* nbm;   // [slot][n_pad]: near-partner masks
+    unsigned long long* nbm;   // [slot][n_pad]: near-partner masks; with near, only where it is set
+    unsigned char* near;    // per 64-ball block and slot (near_stride apart): the slot's masks have a bit
+                            // set (NULL: every mask is written)
+    int near_stride;
     double* pe_tile;        // per tile: far-field pair energy (write steps)
     int* queue;             // k_tiles_q: next group per segment, workgroups done (all 0 between launches)
 };
@@ -135,10 +138,54 @@ __device__ __forceinline__ unsigned long long wave_or(unsigned long long v)
     return v;
 }
 
+// Sums over lanes 0 .. l (DPP row shifts, then the rows' totals).
+__device__ __forceinline__ int wave_iscan(int v)
+{
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);   // row_shr:1, 2, 4, 8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // row_bcast:15 to rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // row_bcast:31 to rows 2 and 3
+    return v;
+}
+
 __device__ __forceinline__ int wave_isum(int v)
 {
     for (int m = 1; m < TB; m <<= 1) v += __shfl_xor(v, m, TB);
     return v;
+}
+
+// Smallest and largest value of the valid lanes (every lane gets the result; +inf and -inf
+// without any).  Quads, rows of 16 by DPP mirrors, then the four rows.
+__device__ __forceinline__ void wave_minmax(double v, bool valid, double& lo, double& hi)
+{
+    const double inf = __builtin_huge_val();
+    lo = valid ? v : inf;
+    hi = valid ? v : -inf;
+    auto mv = [](double d, auto ctrl) {
+        const long long b = __double_as_longlong(d);
+        const int l = __builtin_amdgcn_mov_dpp((int)b, decltype(ctrl)::value, 0xf, 0xf, false);
+        const int h = __builtin_amdgcn_mov_dpp((int)(b >> 32), decltype(ctrl)::value, 0xf, 0xf, false);
+        return __longlong_as_double((long long)(((unsigned long long)(unsigned)h << 32) | (unsigned)l));
+    };
+    auto step = [&](auto ctrl) {
+        lo = fmin(lo, mv(lo, ctrl));
+        hi = fmax(hi, mv(hi, ctrl));
+    };
+    step(std::integral_constant<int, 0xB1>{});    // quad_perm 1,0,3,2
+    step(std::integral_constant<int, 0x4E>{});    // quad_perm 2,3,0,1
+    step(std::integral_constant<int, 0x141>{});   // row_half_mirror
+    step(std::integral_constant<int, 0x140>{});   // row_mirror
+    auto lane = [](double d, int k) {
+        const long long b = __double_as_longlong(d);
+        const int l = __builtin_amdgcn_readlane((int)b, k), h = __builtin_amdgcn_readlane((int)(b >> 32), k);
+        return __longlong_as_double((long long)(((unsigned long long)(unsigned)h << 32) | (unsigned)l));
+    };
+    const double l0 = fmin(lane(lo, 0), lane(lo, 16)), l1 = fmin(lane(lo, 32), lane(lo, 48));
+    const double h0 = fmax(lane(hi, 0), lane(hi, 16)), h1 = fmax(lane(hi, 32), lane(hi, 48));
+    lo = fmin(l0, l1);
+    hi = fmax(h0, h1);
 }
 
 // Bounding box of the valid balls held one per lane (every lane gets the result):
@@ -146,21 +193,13 @@ __device__ __forceinline__ int wave_isum(int v)
 __device__ __forceinline__ void wave_aabb(double x, double y, double z, double R, bool valid, double4& lo,
                                           double4& hi)
 {
-    const double inf = __builtin_huge_val();
-    double lx = valid ? x : inf, ly = valid ? y : inf, lz = valid ? z : inf;
-    double hx = valid ? x : -inf, hy = valid ? y : -inf, hz = valid ? z : -inf;
-    double rm = valid ? R : 0.0;
-    for (int m = 1; m < TB; m <<= 1) {
-        lx = fmin(lx, __shfl_xor(lx, m, TB));
-        ly = fmin(ly, __shfl_xor(ly, m, TB));
-        lz = fmin(lz, __shfl_xor(lz, m, TB));
-        hx = fmax(hx, __shfl_xor(hx, m, TB));
-        hy = fmax(hy, __shfl_xor(hy, m, TB));
-        hz = fmax(hz, __shfl_xor(hz, m, TB));
-        rm = fmax(rm, __shfl_xor(rm, m, TB));
-    }
-    lo = make_double4(lx, ly, lz, rm);
-    hi = make_double4(hx, hy, hz, 0.0);
+    double none, rm;
+    wave_minmax(x, valid, lo.x, hi.x);
+    wave_minmax(y, valid, lo.y, hi.y);
+    wave_minmax(z, valid, lo.z, hi.z);
+    wave_minmax(R, valid, none, rm);
+    lo.w = fmax(rm, 0.0);
+    hi.w = 0;
 }
 
 // A tile is far when the gap between its two blocks' bounding boxes exceeds the two
@@ -623,7 +662,9 @@ __device__ __forceinline__ void tile_pass(const TileArgs& a, int tbase)
         part[(si * 3 + 0) * np + i] = v[0] + v[3];
         part[(si * 3 + 1) * np + i] = v[1] + v[4];
         part[(si * 3 + 2) * np + i] = v[2] + v[5];
-        a.nbm[si * np + i] = mi | mj;
+        const bool near = !a.near || __any((mi | mj) != 0);
+        if (near) a.nbm[si * np + i] = mi | mj;
+        if (a.near && l == 0) a.near[(size_t)I * a.near_stride + si] = near;
     } else {
         part[(si * 3 + 0) * np + i] = v[0];
         part[(si * 3 + 1) * np + i] = v[1];
@@ -631,8 +672,15 @@ __device__ __forceinline__ void tile_pass(const TileArgs& a, int tbase)
         part[(sj_ * 3 + 0) * np + j0] = v[3];
         part[(sj_ * 3 + 1) * np + j0] = v[4];
         part[(sj_ * 3 + 2) * np + j0] = v[5];
-        a.nbm[si * np + i] = mi;
-        a.nbm[sj_ * np + j0] = mj;
+        const bool near = !a.near || __any(mi != 0);   // a pair sets a bit on both sides
+        if (near) {
+            a.nbm[si * np + i] = mi;
+            a.nbm[sj_ * np + j0] = mj;
+        }
+        if (a.near && l == 0) {
+            a.near[(size_t)I * a.near_stride + si] = near;
+            a.near[(size_t)J * a.near_stride + sj_] = near;
+        }
     }
     if (WRITE && l == 0) {
         double pt = pe_w[w0];
@@ -685,72 +733,85 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WRITE ? 1 : 
     }
 }
 
-__device__ __forceinline__ D3 load3(const State& c, int f, int b)
+// A near pair's dynamic state for pair_ref.
+struct NearState {
+    const TouchState& ts;
+    __device__ D3 vA() const { return ts.vA; }
+    __device__ D3 vB() const { return ts.vB; }
+    __device__ D3 wA() const { return ts.wA; }
+    __device__ D3 wB() const { return ts.wB; }
+    __device__ double old_dist() const { return norm(ts.q); }
+};
+
+// The engine's state: dynamic field f of ball b at cur[f np + b], the fields both sets
+// share (radius, mass, moment of inertia) at konst.
+struct EngineState {
+    const double* cur;
+    const double* konst;
+    size_t np;
+    __device__ double at(int f, int b) const { return cur[f * np + b]; }
+    __device__ D3 at3(int f, int b) const { return d3(at(f, b), at(f + 1, b), at(f + 2, b)); }
+    __device__ double c(int f, int b) const { return konst[f * np + b]; }
+};
+
+// The near pair of ball b and partner p in the reference's orientation: A is the ball with the
+// larger index in the caller's numbering (the friction terms are not symmetric in A and B).
+// Everything is loaded at once, before the orientation and whether the pair touches are known
+// (in an aggregate nearly every near pair touches): one trip to memory where there were three.
+struct NearPair {
+    PairIn in;
+    TouchState ts;
+    bool is_a;    // b is A
+};
+__device__ __forceinline__ NearPair near_load(const EngineState& c, const int* perm, int b, int p)
 {
-    return d3(c.f[f][b], c.f[f + 1][b], c.f[f + 2][b]);
+    const int cb = perm[b], cp = perm[p];
+    const D3 xb = c.at3(PX, b), xp = c.at3(PX, p), vb = c.at3(VX, b), vp = c.at3(VX, p);
+    const D3 wb = c.at3(WX, b), wp = c.at3(WX, p), qb = c.at3(QX, b), qp = c.at3(QX, p);
+    const double Rb = c.c(RAD, b), Rp = c.c(RAD, p), mb = c.c(MASS, b), mp = c.c(MASS, p);
+    const bool is_a = cb > cp;
+    auto sel = [is_a](D3 x, D3 y) { return d3(is_a ? x.x : y.x, is_a ? x.y : y.y, is_a ? x.z : y.z); };
+    return NearPair{{sel(xb, xp), sel(xp, xb), is_a ? Rb : Rp, is_a ? Rp : Rb, is_a ? mb : mp, is_a ? mp : mb},
+                    {sel(vb, vp), sel(vp, vb), sel(wb, wp), sel(wp, wb), sel(qp, qb) - sel(qb, qp)},
+                    is_a};
 }
 
-// Result of one (ball, partner) near evaluation, for the ball: force, torque, and the
-// pair's energy and touching flag when the ball is A (counted once per pair).
-struct NearRes {
-    double f[6];
-    double pe;
-    int contact, is_a;
-};
-
-// Velocities, spins and previous positions of a pair's two balls, read only when
-// the pair touches.
-struct NearStateG {
-    const State& s;
-    int A, B;
-    __device__ D3 vA() const { return d3(s.f[VX][A], s.f[VY][A], s.f[VZ][A]); }
-    __device__ D3 vB() const { return d3(s.f[VX][B], s.f[VY][B], s.f[VZ][B]); }
-    __device__ D3 wA() const { return d3(s.f[WX][A], s.f[WY][A], s.f[WZ][A]); }
-    __device__ D3 wB() const { return d3(s.f[WX][B], s.f[WY][B], s.f[WZ][B]); }
-    __device__ double old_dist() const
-    {
-        return norm(d3(s.f[QX][B], s.f[QY][B], s.f[QZ][B]) - d3(s.f[QX][A], s.f[QY][A], s.f[QZ][A]));
-    }
-};
-
-// Evaluate the near pair of ball b and partner p with the reference arithmetic in the
-// reference orientation: A is the ball with the larger index in the caller's
-// numbering (the friction terms are not symmetric in A and B).
+// Its evaluation in the reference's arithmetic: force and torque on b to f[0 .. 5], fs apart;
+// the pair's energy when b is A to pe; returns bit 0: touching and b is A, bit 1: b is A.
 template <bool WRITE>
-__device__ __forceinline__ void eval_entry(const State& c, const int* perm, const Phys& P, int b, int p, NearRes& r)
+__device__ __forceinline__ int near_eval(const NearPair& z, const Phys& P, double* f, int fs, double& pe)
 {
-    const bool is_a = perm[b] > perm[p];
-    const int A = is_a ? b : p, B = is_a ? p : b;
-    PairIn in;
-    in.pA = load3(c, PX, A);
-    in.pB = load3(c, PX, B);
-    in.RA = c.f[RAD][A];
-    in.RB = c.f[RAD][B];
-    in.mA = c.f[MASS][A];
-    in.mB = c.f[MASS][B];
-    NearStateG ns{c, A, B};
-    PairOut po;
-    pair_ref(P, WRITE, in, ns, po);
-    const D3 F = is_a ? po.F : -po.F;
-    const D3 T = is_a ? po.tA : po.tB;
-    r.f[0] = F.x; r.f[1] = F.y; r.f[2] = F.z;
-    r.f[3] = T.x; r.f[4] = T.y; r.f[5] = T.z;
-    r.pe = is_a ? po.pe : 0.0;
-    r.contact = is_a ? po.contact : 0;
-    r.is_a = is_a;
+    const PairIn& in = z.in;
+    const D3 r = in.pB - in.pA;
+    const double d2 = dot(r, r);
+    PairOut o;
+    bool done = FarRange::params(P) && FarRange::ball(in.RA, in.mA) && FarRange::ball(in.RB, in.mB) && FarRange::distance2(d2);
+    if (done) {
+        double dist, y;
+        sqrt_rcp(d2, dist, y);
+        done = (in.RA + in.RB) - dist > 0 && touch_pair_ref(P, WRITE, in, z.ts, o);
+    }
+    if (!done) pair_ref(P, WRITE, in, NearState{z.ts}, o);
+    const D3 F = z.is_a ? o.F : -o.F;
+    const D3 T = z.is_a ? o.tA : o.tB;
+    f[0] = F.x; f[fs] = F.y; f[2 * fs] = F.z;
+    f[3 * fs] = T.x; f[4 * fs] = T.y; f[5 * fs] = T.z;
+    pe = z.is_a ? o.pe : 0.0;
+    return z.is_a ? o.contact | 2 : 0;
 }
 
 struct BallArgs {
-    State cur, nxt;
+    const double* cur;  // state sets, as in EngineState
+    double* nxt;
+    const double* konst;
     const Phys* sysP;
-    const int* blk_sys;
-    const int* sys_off;
-    const int* sys_n;
-    const int* sys_nb;
-    int n_used, n_pad;
+    const int4* blk_info;   // per 64-ball block: {first slot, balls, blocks of its system, system}
+    int n_pad;
     const double* part;     // [slot][xyz][n_pad]; mixed: binary32, to be scaled by Kf
     double Kf;
-    const unsigned long long* nbm;
+    const unsigned long long* nbm;   // near-partner masks; NEARF: of the slots that near marks
+    const unsigned char* near;
+    int near_stride;
     const int* perm;    // engine slot -> the caller's ball index (fixes near-pair orientation)
     int kick, drift_next;
     double4* bnd;       // per 64-ball block: bounding box of the drifted positions (lo, hi)
@@ -761,23 +822,21 @@ struct BallArgs {
     int* flags;         // [1]: a non-finite state appeared
 };
 
-// Block-local binary32 position of ball l of a block whose bounding box is (lo, hi); padding
-// lanes get far, distinct, finite places (their weights are 0, so they add nothing).
-__device__ __forceinline__ float4 local_pos(double x, double y, double z, double R, bool valid, double4 lo,
-                                            double4 hi, double L0inv, int l)
+// One coordinate of a ball's block-local binary32 position, in a block whose bounding box is
+// [lo, hi] there; padding lanes get far, distinct, finite places (their weights are 0, so they
+// add nothing).
+__device__ __forceinline__ float local_coord(double x, bool valid, double lo, double hi, double L0inv, int l)
 {
-    if (!valid) return make_float4(1e6f + 2048.f * (float)l, 1e6f, 1e6f, 0.f);
-    const double3 c = block_ref(lo, hi);
-    return make_float4((float)((x - c.x) * L0inv), (float)((y - c.y) * L0inv), (float)((z - c.z) * L0inv),
-                       (float)(R * L0inv));
+    return valid ? (float)((x - 0.5 * (lo + hi)) * L0inv) : 1e6f + 2048.f * (float)l;
 }
 
 constexpr int BPB = TB;              // balls per k_ball block
 constexpr int KB_C = 8;              // slot classes K = c, c + KB_C, ...: they fix the order of every sum
-constexpr int SLOTS_IN_FLIGHT = 10;  // slots per lane loaded together: 40 loads, one batch for systems of up to 80 blocks
+constexpr int SLOTS_IN_FLIGHT = 10;  // slots per lane loaded together: 40 loads
+constexpr int KB_BATCH = SLOTS_IN_FLIGHT * KB_C;   // one batch for systems of up to 80 blocks
 // k_ball workgroups have 8 wavefronts (one slot class each: the fewest dependent loads
-// per wavefront, for a lone system of few blocks) or 4 (two classes each, 161 VGPRs and
-// 48 KB of LDS: three workgroups share a CU, for launches of more blocks than CUs).
+// per wavefront, for a lone system of few blocks) or 4 (two classes each, at most 170 VGPRs
+// and 53 KB of LDS: three workgroups share a CU, for launches of more blocks than CUs).
 // The results are the same bit for bit.
 constexpr int kb_threads(int nwv) { return nwv * TB; }
 
@@ -790,156 +849,229 @@ constexpr int kb_threads(int nwv) { return nwv * TB; }
 //    and added with Kahan compensation), counts
 //    the near-partner bits and keeps the first MC nonzero partner masks of each ball
 //    in LDS (more than that: they are read again).
-// 2. The block's near entries are numbered ball by ball (then by class, slot and bit),
-//    and all threads evaluate them, one round of NWV * 64 at a time, with the reference
-//    arithmetic and orientation.  Lane l of wavefront 0 adds its ball's results in
-//    entry order.  Each near pair is so evaluated once from each of its balls,
-//    identically, and no sum needs an atomic.
-// 3. Wavefront 0 combines the KB_C class sums in a fixed order and finishes the step
-//    for the 64 balls (coalesced stores).
-template <bool COMP, bool WRITE, int NWV>
+// 2. The block's near entries are numbered ball by ball (then by class, slot and bit; every
+//    wavefront makes the same scan of the counts), and all threads evaluate them, one round
+//    of NWV * 64 at a time, with the reference arithmetic and orientation.  Each near pair is
+//    so evaluated once from each of its balls, identically, and no sum needs an atomic.
+// 3. The step is finished component by component: wavefront q adds component q (force, then
+//    torque) of its balls' near results in entry order and of the class sums in a fixed order
+//    and carries that axis through kick, drift and bounding box; component 6 is the pair
+//    counts.  (Wavefront 0 alone took 5,200 cycles for what is now about 2,000.)
+//
+// Bound by latency: a chain of four trips to memory (the block's table, the partials, the near
+// pairs' state, each a kernel's worth of L2 misses) and of the touching pair's arithmetic,
+// with one workgroup on a CU.  Finishing by component, both balls' state loaded at once, the
+// pair's short divisions (touch_pair_ref), scans by DPP and the sums' loads kept in flight
+// behind the pairs took it from 12.6 to 9.4 us at 1,000 spheres, from 13.2 to 11.2 at 5,000
+// (mixed 12.6 to 10.8), from 40 to 32 for 512 systems of 33 to 550 and from 56 to 49 for 96 of
+// 200 to 4,500.
+//
+// NEARF, for systems of more than KB_BATCH slots: the masks of slots without near pairs, nine
+// in ten of a large system's, are neither written nor read (200 of 800 bytes a ball and slot
+// at 40,000 spheres: 201 -> 170 us).  Smaller systems load one batch of masks unseen: finding
+// out which first cost 0.4 us of 11 at 79 slots and 5 of 49 in the four-wavefront shape.
+template <bool COMP, bool WRITE, int NWV, bool NEARF>
 __global__ __launch_bounds__(kb_threads(NWV)) void k_ball(BallArgs a)
 {
-    static_assert(NWV == 8 || NWV == 4, "8 or 4 wavefronts");
+    static_assert(NWV == 8 || (NWV == 4 && !NEARF), "8 or 4 wavefronts; NEARF: one class each");
     constexpr int KB_W = NWV;                 // wavefronts
     constexpr int KB_T = kb_threads(NWV);     // threads, and near entries per round
     constexpr int KB_MC = NWV == 8 ? 4 : 2;   // partner masks kept per (class, ball)
+    constexpr int NQ = 7;                     // components: force, torque, pair counts
+    constexpr int QW = 8 / NWV;               // of these a wavefront has w, w + NWV
+    // One class a wavefront: its sums' loads stay in flight behind the near pairs' evaluation
+    constexpr bool SUMS_LATE = NWV == KB_C;
     __shared__ double sf[KB_C][3][TB];       // far-field force sums per class
     __shared__ int s_cnt[KB_C][TB];          // near entries per (class, ball)
-    __shared__ int s_off[KB_C][TB];          // first entry of (class, ball)
     __shared__ int s_nm[KB_C][TB];           // slots of (class, ball) with near partners
-    __shared__ int s_total;
     __shared__ int ent[KB_T];                // entries of the current round
-    __shared__ NearRes res[KB_T];
+    __shared__ double res[6][KB_T];          // their forces and torques
+    __shared__ double res_pe[WRITE ? KB_T : 1];
+    __shared__ unsigned char res_fl[KB_T];
     __shared__ unsigned long long s_mk[KB_C][KB_MC][TB];   // nonzero partner masks ...
     __shared__ int s_mks[KB_C][KB_MC][TB];                  // ... and their slots
+    __shared__ double fin[WRITE ? 9 : 1][TB];               // v, w, position (write steps)
     // the wavefront index is uniform: in a scalar register, the slot indices derived from
     // it are too
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / TB), l = threadIdx.x % TB;
     const int i = blockIdx.x * TB + l;
-    const int sys = a.blk_sys[blockIdx.x];
-    const int off = a.sys_off[sys];
-    const bool valid = (i - off) < a.sys_n[sys];
+    // NEARF: slots of a class that have near pairs, a byte each: 60 of them (six batches of
+    // SLOTS_IN_FLIGHT) a load, the first while the block's table is on its way
+    auto near_bytes = [&](int K0) {
+        const int K = K0 + KB_C * l;
+        return NEARF && l < 60 && K < a.near_stride ? (int)a.near[(size_t)blockIdx.x * a.near_stride + K] : 0;
+    };
+    const int near0 = near_bytes(w);
+    const int4 bi = a.blk_info[blockIdx.x];
+    const int off = bi.x, nb = bi.z;
+    const bool valid = i - off < bi.y;
     const int ic = valid ? i : off;
-    const int nblk = valid ? a.sys_nb[sys] : 0;
-    const Phys& P = a.sysP[sys];
-    const State& c = a.cur;
+    const Phys P = a.sysP[bi.w];
     const size_t np = (size_t)a.n_pad;
+    const EngineState c{a.cur, a.konst, np};
     // far-field partials: binary32 in the mixed mode (the force is Kf times the stored sum)
     using PT = std::conditional_t<COMP, float, double>;
     const double Kf = a.Kf;
 
-    // wavefront 0 finishes the step: its own-state loads (and the block's running pair
-    // counters) go out first
+    // what this wavefront's components need of the balls' own state goes out first
+    double x0[QW], h0[QW], inr[QW], Rb = 0;
     unsigned long long ctr0 = 0, ctr1 = 0;
-    if (w == 0 && l == 0) {
-        ctr0 = a.blk_ctr[2 * blockIdx.x];
-        ctr1 = a.blk_ctr[2 * blockIdx.x + 1];
-    }
-    D3 p0 = d3(0, 0, 0), h0 = p0, g0 = p0;
-    double mi = 1, Ii = 1, Rb = 0;
-    if (w == 0 && valid) {
-        p0 = load3(c, PX, i);
-        h0 = load3(c, HX, i);
-        g0 = load3(c, GX, i);
-        mi = c.f[MASS][i];
-        Ii = c.f[MOI][i];
-        Rb = c.f[RAD][i];
+#pragma unroll
+    for (int u = 0; u < QW; u++) {
+        const int q = w + u * NWV;
+        x0[u] = h0[u] = 0;
+        inr[u] = 1;
+        if (q < 3) {
+            x0[u] = c.at(PX + q, ic);
+            h0[u] = c.at(HX + q, ic);
+            inr[u] = c.c(MASS, ic);
+        } else if (q < 6) {
+            h0[u] = c.at(GX + q - 3, ic);
+            inr[u] = c.c(MOI, ic);
+            if (q == 3) Rb = c.c(RAD, ic);
+        } else if (q == 6 && l == 0) {
+            ctr0 = a.blk_ctr[2 * blockIdx.x];
+            ctr1 = a.blk_ctr[2 * blockIdx.x + 1];
+        }
     }
 
+    // slots K0, K0 + KB_C, ... of a class: SLOTS_IN_FLIGHT loaded together (4 for small systems)
+    const bool wide = nb > 4 * KB_C;
+    auto slot = [&](int K0, int u) { return K0 + u * KB_C < nb ? K0 + u * KB_C : nb - 1; };
+    auto each_slot = [&](auto f) {
+#pragma unroll
+        for (int u = 0; u < 4; u++) f(u);
+        if (wide) {
+#pragma unroll
+            for (int u = 4; u < SLOTS_IN_FLIGHT; u++) f(u);
+        }
+    };
+    // masks of the batch at K0 (NEARF: bit u of near, its slot u has any)
+    auto load_masks = [&](int K0, unsigned long long near, unsigned long long* mk) {
+        each_slot([&](int u) {
+            if constexpr (NEARF) {
+                mk[u] = 0;
+                if ((near >> u) & 1) mk[u] = a.nbm[(size_t)(K0 + u * KB_C) * np + ic];
+            } else {
+                mk[u] = a.nbm[(size_t)slot(K0, u) * np + ic];
+            }
+        });
+    };
+    auto near_slots = [&](int K0, int byte) { return __ballot(byte != 0 && K0 + KB_C * l < nb); };
+    auto load_sums = [&](int K0, PT (*q)[3]) {
+        each_slot([&](int u) {
+            const PT* pp = reinterpret_cast<const PT*>(a.part) + (size_t)slot(K0, u) * 3 * np + ic;
+            q[u][0] = pp[0];
+            q[u][1] = pp[np];
+            q[u][2] = pp[2 * np];
+        });
+    };
+    struct Near {
+        int cn, nm;   // near entries of this (class, ball), slots that have any
+    };
+    auto count = [&](int cl, int K0, const unsigned long long* mk, Near& t) {
+        each_slot([&](int u) {
+            const unsigned long long m = valid && K0 + u * KB_C < nb ? mk[u] : 0ull;
+            t.cn += __popcll(m);
+            if (m) {
+                if (t.nm < KB_MC) {
+                    s_mk[cl][t.nm][l] = m;
+                    s_mks[cl][t.nm][l] = K0 + u * KB_C;
+                }
+                t.nm++;
+            }
+        });
+    };
+    struct Sum {
+        double f[3], c[3];
+    };
+    auto add = [&](int K0, PT (*q)[3], Sum& t) {
+        each_slot([&](int u) {
+            if (K0 + u * KB_C >= nb) return;
+#pragma unroll
+            for (int x = 0; x < 3; x++) {
+                if (COMP) {
+                    const double y = Kf * (double)q[u][x] - t.c[x], z = t.f[x] + y;
+                    t.c[x] = (z - t.f[x]) - y;
+                    t.f[x] = z;
+                } else {
+                    t.f[x] = t.f[x] + q[u][x];
+                }
+            }
+        });
+    };
+    PT q0[SLOTS_IN_FLIGHT][3];
+    auto class_sums = [&](int cl) {   // q0: the class's first slots, loaded
+        Sum t{};
+        add(cl, q0, t);
+        for (int K0 = cl + KB_BATCH; K0 < nb; K0 += KB_BATCH) {
+            load_sums(K0, q0);
+            add(K0, q0, t);
+        }
+#pragma unroll
+        for (int x = 0; x < 3; x++) sf[cl][x][l] = t.f[x] - t.c[x];
+    };
 #pragma unroll 1
     for (int cl = w; cl < KB_C; cl += KB_W) {
-        double fx = 0, fy = 0, fz = 0, cx = 0, cy = 0, cz = 0;
-        int cn = 0;                    // near entries of this (class, ball)
-        int nm = 0;                    // slots of this (class, ball) with near partners
-        for (int K0 = cl; K0 < nblk; K0 += SLOTS_IN_FLIGHT * KB_C) {
-            PT q[SLOTS_IN_FLIGHT][3];
-            unsigned long long mk[SLOTS_IN_FLIGHT];
-#pragma unroll
-            for (int u = 0; u < SLOTS_IN_FLIGHT; u++) {
-                const int K = K0 + u * KB_C;
-                const int Kc = K < nblk ? K : 0;
-                const PT* pp = reinterpret_cast<const PT*>(a.part) + (size_t)Kc * 3 * np + ic;
-                q[u][0] = pp[0];
-                q[u][1] = pp[np];
-                q[u][2] = pp[2 * np];
-                mk[u] = K < nblk ? a.nbm[(size_t)Kc * np + ic] : 0ull;
-            }
-#pragma unroll
-            for (int u = 0; u < SLOTS_IN_FLIGHT; u++) {
-                if (K0 + u * KB_C >= nblk) break;
-                cn += __popcll(mk[u]);
-                if (mk[u]) {
-                    if (nm < KB_MC) {
-                        s_mk[cl][nm][l] = mk[u];
-                        s_mks[cl][nm][l] = K0 + u * KB_C;
-                    }
-                    nm++;
-                }
-                if (COMP) {
-                    double y, t;
-                    y = Kf * (double)q[u][0] - cx; t = fx + y; cx = (t - fx) - y; fx = t;
-                    y = Kf * (double)q[u][1] - cy; t = fy + y; cy = (t - fy) - y; fy = t;
-                    y = Kf * (double)q[u][2] - cz; t = fz + y; cz = (t - fz) - y; fz = t;
-                } else {
-                    fx = fx + q[u][0];
-                    fy = fy + q[u][1];
-                    fz = fz + q[u][2];
-                }
-            }
+        unsigned long long mk[SLOTS_IN_FLIGHT];
+        Near t{};
+        unsigned long long near = 0;
+        if constexpr (NEARF) near = near_slots(cl, near0);
+        load_masks(cl, near, mk);
+        load_sums(cl, q0);
+        count(cl, cl, mk, t);
+        int batch = 1;
+        for (int K0 = cl + KB_BATCH; K0 < nb; K0 += KB_BATCH, batch++) {
+            if constexpr (NEARF) near = batch % 6 ? near >> SLOTS_IN_FLIGHT : near_slots(K0, near_bytes(K0));
+            load_masks(K0, near, mk);
+            count(cl, K0, mk, t);
         }
-        sf[cl][0][l] = fx - cx;
-        sf[cl][1][l] = fy - cy;
-        sf[cl][2][l] = fz - cz;
-        s_cnt[cl][l] = cn;
-        s_nm[cl][l] = nm;
+        s_cnt[cl][l] = t.cn;
+        s_nm[cl][l] = t.nm;
+        if constexpr (!SUMS_LATE) class_sums(cl);
     }
     __syncthreads();
 
     // number the block's near entries: ball-major, then class, slot and bit
-    if (w == 0) {
-        int tot = 0;
-        for (int q = 0; q < KB_C; q++) tot += s_cnt[q][l];
-        int incl = tot;
-        for (int m = 1; m < TB; m <<= 1) {
-            const int y = __shfl_up(incl, m, TB);
-            if (l >= m) incl += y;
-        }
-        int o = incl - tot;
-        for (int q = 0; q < KB_C; q++) {
-            s_off[q][l] = o;
-            o += s_cnt[q][l];
-        }
-        if (l == TB - 1) s_total = incl;
+    int cnt[KB_C], tot = 0;
+#pragma unroll
+    for (int q = 0; q < KB_C; q++) {
+        cnt[q] = s_cnt[q][l];
+        tot += cnt[q];
     }
-    __syncthreads();
-    const int total = s_total;
+    const int incl = wave_iscan(tot);
+    const int total = __builtin_amdgcn_readlane(incl, TB - 1);
+    const int b0 = incl - tot, b1 = incl;   // ball l's entries are [b0, b1)
 
-    double n[6] = {0, 0, 0, 0, 0, 0};
-    double npe = 0;
+    double n[QW] = {}, npe = 0;
     int ncon = 0, npair = 0;
-    for (int r0 = 0; r0 < total; r0 += KB_T) {
+    for (int r0 = 0;; r0 += KB_T) {
         const int r1 = r0 + KB_T;
         // write this round's entries of (class cl, ball l) for the classes of wavefront w
 #pragma unroll 1
         for (int cl = w; cl < KB_C; cl += KB_W) {
-            const int cn = s_cnt[cl][l], nm = s_nm[cl][l];
-            const int my0 = s_off[cl][l];   // (class, ball) entries are [my0, my0 + cn)
-            if (cn && my0 < r1 && my0 + cn > r0) {
-                int k = my0;
-                auto put = [&](int K, unsigned long long m) {
-                    while (m && k < r1) {
-                        const int bit = __ffsll((long long)m) - 1;
-                        m &= m - 1;
-                        if (k >= r0) ent[k - r0] = l | (bit << 6) | (K << 12);
-                        k++;
-                    }
+            int k = b0, cn = 0;         // (class, ball) entries are [k, k + cn)
+#pragma unroll
+            for (int q = 0; q < KB_C; q++) {
+                if (q < cl) k += cnt[q];
+                if (q == cl) cn = cnt[q];
+            }
+            if (!(cn && k < r1 && k + cn > r0)) continue;
+            const int nm = s_nm[cl][l];
+            auto put = [&](int K, unsigned long long m) {
+                const int e = l | (K << 12);
+                auto half = [&](unsigned h, int at) {
+                    for (; h; h &= h - 1, k++)
+                        if (k >= r0 && k < r1) ent[k - r0] = e | ((at + __builtin_ctz(h)) << 6);
                 };
-                if (nm <= KB_MC) {
-                    for (int q = 0; q < nm && k < r1; q++) put(s_mks[cl][q][l], s_mk[cl][q][l]);
-                } else {
-                    for (int K = cl; K < nblk && k < r1; K += KB_C) put(K, a.nbm[(size_t)K * np + ic]);
-                }
+                half((unsigned)m, 0);
+                half((unsigned)(m >> 32), 32);
+            };
+            if (nm <= KB_MC) {
+                for (int q = 0; q < nm && k < r1; q++) put(s_mks[cl][q][l], s_mk[cl][q][l]);
+            } else {
+                for (int K = cl; K < nb && k < r1; K += KB_C)
+                    if (!NEARF || a.near[(size_t)blockIdx.x * a.near_stride + K]) put(K, a.nbm[(size_t)K * np + ic]);
             }
         }
         __syncthreads();
@@ -947,126 +1079,140 @@ __global__ __launch_bounds__(kb_threads(NWV)) void k_ball(BallArgs a)
         if (r0 + t < total) {
             const int e = ent[t];
             const int el = e & (TB - 1), bit = (e >> 6) & (TB - 1), K = e >> 12;
-            NearRes rr;
-            eval_entry<WRITE>(c, a.perm, P, blockIdx.x * TB + el, off + K * TB + bit, rr);
-            res[t] = rr;
+            const NearPair z = near_load(c, a.perm, blockIdx.x * TB + el, off + K * TB + bit);
+            double pe;
+            res_fl[t] = (unsigned char)near_eval<WRITE>(z, P, &res[0][t], KB_T, pe);
+            if (WRITE) res_pe[t] = pe;
         }
         __syncthreads();
-        if (w == 0) {
-            // ball l's entries in this round, in order
-            int tot = 0;
-            for (int q = 0; q < KB_C; q++) tot += s_cnt[q][l];
-            const int b0 = s_off[0][l], b1 = b0 + tot;
-            const int k0 = b0 > r0 ? b0 : r0, k1 = b1 < r1 ? b1 : r1;
-            for (int k = k0; k < k1; k++) {
-                const NearRes& rr = res[k - r0];
-                for (int q = 0; q < 6; q++) n[q] = n[q] + rr.f[q];
-                npe = npe + rr.pe;
-                ncon += rr.contact;
-                npair += rr.is_a;
+        // ball l's entries in this round, in order
+        const int k0 = (b0 > r0 ? b0 : r0) - r0, k1 = (b1 < r1 ? b1 : r1) - r0;
+#pragma unroll
+        for (int u = 0; u < QW; u++) {
+            const int q = w + u * NWV;
+            if (q < 6) {
+                for (int k = k0; k < k1; k++) n[u] = n[u] + res[q][k];
+            } else if (q == 6) {
+                for (int k = k0; k < k1; k++) {
+                    const int fl = res_fl[k];
+                    ncon += fl & 1;
+                    npair += fl >> 1;
+                    if (WRITE) npe = npe + res_pe[k];
+                }
             }
         }
-        __syncthreads();
+        if (r1 >= total) break;
+        __syncthreads();   // the next round writes ent and res
     }
-    if (w != 0) return;
 
-    // wavefront 0: combine in a fixed order and finish the step of ball l
-    double F[3], T[3];
-    for (int k = 0; k < 3; k++) {
-        double s = sf[0][k][l], cmp = 0;
-        for (int q = 1; q < KB_C; q++) {
-            if (COMP) {
-                const double y = sf[q][k][l] - cmp, t = s + y;
-                cmp = (t - s) - y;
-                s = t;
-            } else {
-                s = s + sf[q][k][l];
+    if constexpr (SUMS_LATE) class_sums(w);
+    __syncthreads();
+
+    const double dt = P.dt;
+#pragma unroll
+    for (int u = 0; u < QW; u++) {
+        const int q = w + u * NWV;
+        if (q >= 6) {
+            if (q == 6) {
+                // the block's near-pair energy and pair counts (each pair counted by its ball A)
+                const double bpe = WRITE ? wave_sum(npe) : 0.0;
+                const int bcc = wave_isum(ncon), bcn = wave_isum(npair);
+                if (l == 0) {
+                    a.blk_ctr[2 * blockIdx.x] = ctr0 + (unsigned long long)bcc;
+                    a.blk_ctr[2 * blockIdx.x + 1] = ctr1 + (unsigned long long)bcn;
+                    if (WRITE) {
+                        a.e_blk[blockIdx.x * FAST_E_STRIDE] = bpe;
+                        a.e_blk[blockIdx.x * FAST_E_STRIDE + 8] = (double)bcc;
+                    }
+                }
             }
+            continue;
         }
-        F[k] = (s - cmp) + n[k];
-        T[k] = n[3 + k];
-    }
-
-    double e[FAST_E_STRIDE] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};   // PE KE p L contacts nonfinite
-    D3 pn = p0;   // positions the next pair pass will read
-    if (valid) {
-        const double px = p0.x, py = p0.y, pz = p0.z;
-        const double ax = F[0] / mi, ay = F[1] / mi, az = F[2] / mi;
-        const double bx = T[0] / Ii, by = T[1] / Ii, bz = T[2] / Ii;
-        const double dt = P.dt;
-        double vx, vy, vz, wx, wy, wz;
-        if (a.kick) {
-            vx = h0.x + .5 * ax * dt;
-            vy = h0.y + .5 * ay * dt;
-            vz = h0.z + .5 * az * dt;
-            wx = g0.x + .5 * bx * dt;
-            wy = g0.y + .5 * by * dt;
-            wz = g0.z + .5 * bz * dt;
-        } else {
-            vx = c.f[VX][i]; vy = c.f[VY][i]; vz = c.f[VZ][i];
-            wx = c.f[WX][i]; wy = c.f[WY][i]; wz = c.f[WZ][i];
+        // component q of force (q < 3) or torque, its acceleration, velocity and half step
+        const bool lin = q < 3;
+        const int x = lin ? q : q - 3;
+        double F = n[u];
+        if (lin) {
+            double s = sf[0][x][l], cmp = 0;
+            for (int k = 1; k < KB_C; k++) {
+                if (COMP) {
+                    const double y = sf[k][x][l] - cmp, t = s + y;
+                    cmp = (t - s) - y;
+                    s = t;
+                } else {
+                    s = s + sf[k][x][l];
+                }
+            }
+            F = (s - cmp) + F;
         }
-        const bool bad = !(isfinite(vx) && isfinite(vy) && isfinite(vz) && isfinite(wx) && isfinite(wy) &&
-                           isfinite(wz) && isfinite(px) && isfinite(py) && isfinite(pz));
-        if (bad) atomicOr(&a.flags[1], 1);
+        const int fv = (lin ? VX : WX) + x, fa = (lin ? AX : BX) + x, fh = (lin ? HX : GX) + x;
+        const double acc = F / inr[u];
+        const double v = a.kick ? h0[u] + .5 * acc * dt : c.at(fv, ic);
+        if (valid && !(isfinite(v) && isfinite(x0[u]))) atomicOr(&a.flags[1], 1);
         if (WRITE) {
-            const D3 v = d3(vx, vy, vz), wv = d3(wx, wy, wz);
-            e[1] = .5 * mi * dot(v, v) + .5 * Ii * dot(wv, wv);
-            const D3 mv = v * mi;
-            e[2] = mv.x; e[3] = mv.y; e[4] = mv.z;
-            const D3 L = cross(p0, v) * mi + wv * Ii;
-            e[5] = L.x; e[6] = L.y; e[7] = L.z;
-            e[9] = bad ? 1.0 : 0.0;
+            fin[q][l] = v;
+            if (lin) fin[6 + x][l] = x0[u];
         }
-        const State& o = a.nxt;
-        o.f[VX][i] = vx; o.f[VY][i] = vy; o.f[VZ][i] = vz;
-        o.f[WX][i] = wx; o.f[WY][i] = wy; o.f[WZ][i] = wz;
-        o.f[AX][i] = ax; o.f[AY][i] = ay; o.f[AZ][i] = az;
-        o.f[BX][i] = bx; o.f[BY][i] = by; o.f[BZ][i] = bz;
+        double xn = x0[u];              // position the next pair pass will read
+        double hn = h0[u];
         if (a.drift_next) {
-            const double hx = vx + .5 * ax * dt, hy = vy + .5 * ay * dt, hz = vz + .5 * az * dt;
-            o.f[HX][i] = hx; o.f[HY][i] = hy; o.f[HZ][i] = hz;
-            o.f[GX][i] = wx + .5 * bx * dt;
-            o.f[GY][i] = wy + .5 * by * dt;
-            o.f[GZ][i] = wz + .5 * bz * dt;
-            o.f[QX][i] = px; o.f[QY][i] = py; o.f[QZ][i] = pz;
-            pn = d3(px + hx * dt, py + hy * dt, pz + hz * dt);
-            o.f[PX][i] = pn.x;
-            o.f[PY][i] = pn.y;
-            o.f[PZ][i] = pn.z;
-        } else {
-            o.f[HX][i] = h0.x; o.f[HY][i] = h0.y; o.f[HZ][i] = h0.z;
-            o.f[GX][i] = g0.x; o.f[GY][i] = g0.y; o.f[GZ][i] = g0.z;
-            o.f[QX][i] = c.f[QX][i]; o.f[QY][i] = c.f[QY][i]; o.f[QZ][i] = c.f[QZ][i];
-            o.f[PX][i] = px; o.f[PY][i] = py; o.f[PZ][i] = pz;
+            hn = v + .5 * acc * dt;
+            xn = x0[u] + hn * dt;
         }
-    }
-    if (a.drift_next) {
-        double4 lo, hi;
-        wave_aabb(pn.x, pn.y, pn.z, Rb, valid, lo, hi);
-        if (l == 0) {
-            a.bnd[2 * blockIdx.x] = lo;
-            a.bnd[2 * blockIdx.x + 1] = hi;
+        if (valid) {
+            a.nxt[fv * np + i] = v;
+            a.nxt[fa * np + i] = acc;
+            a.nxt[fh * np + i] = hn;
+            if (lin) {
+                a.nxt[(QX + x) * np + i] = a.drift_next ? x0[u] : c.at(QX + x, i);
+                a.nxt[(PX + x) * np + i] = xn;
+            }
         }
-        a.xl[i] = local_pos(pn.x, pn.y, pn.z, Rb, valid, lo, hi, a.L0inv, l);
+        if (a.drift_next) {
+            double* bd = reinterpret_cast<double*>(a.bnd + 2 * blockIdx.x);   // lo, hi
+            float* xo = reinterpret_cast<float*>(a.xl + i);
+            if (lin) {
+                double lo, hi;
+                wave_minmax(xn, valid, lo, hi);
+                if (l == 0) {
+                    bd[x] = lo;
+                    bd[4 + x] = hi;
+                }
+                xo[x] = local_coord(xn, valid, lo, hi, a.L0inv, x == 0 ? l : 0);
+            } else if (x == 0) {
+                double lo, hi;
+                wave_minmax(Rb, valid, lo, hi);
+                if (l == 0) {
+                    bd[3] = fmax(hi, 0.0);
+                    bd[7] = 0;
+                }
+                xo[3] = valid ? (float)(Rb * a.L0inv) : 0.f;
+            }
+        }
     }
     if (WRITE) {
-        // a 64-ball block lies inside one system, so its sums are per system
-        for (int k = 1; k < FAST_E_STRIDE; k++) {
-            if (k == 8) continue;
-            const double s = wave_sum(e[k]);
-            if (l == 0) a.e_blk[blockIdx.x * FAST_E_STRIDE + k] = s;
-        }
-    }
-    // the block's near-pair energy and pair counts (each pair counted by its ball A)
-    const double bpe = WRITE ? wave_sum(npe) : 0.0;
-    const int bcc = wave_isum(ncon), bcn = wave_isum(npair);
-    if (l == 0) {
-        a.blk_ctr[2 * blockIdx.x] = ctr0 + (unsigned long long)bcc;
-        a.blk_ctr[2 * blockIdx.x + 1] = ctr1 + (unsigned long long)bcn;
-        if (WRITE) {
-            a.e_blk[blockIdx.x * FAST_E_STRIDE] = bpe;
-            a.e_blk[blockIdx.x * FAST_E_STRIDE + 8] = (double)bcc;
+        // energy, momenta and the non-finite count; a 64-ball block lies inside one system, so
+        // its sums are per system
+        __syncthreads();
+        const double mi = c.c(MASS, ic), Ii = c.c(MOI, ic);
+        const D3 v = d3(fin[0][l], fin[1][l], fin[2][l]), wv = d3(fin[3][l], fin[4][l], fin[5][l]);
+        const D3 p0 = d3(fin[6][l], fin[7][l], fin[8][l]);
+        for (int k = w; k < 8; k += KB_W) {
+            double e;
+            if (k == 0) {
+                e = .5 * mi * dot(v, v) + .5 * Ii * dot(wv, wv);
+            } else if (k < 4) {
+                const D3 mv = v * mi;
+                e = k == 1 ? mv.x : k == 2 ? mv.y : mv.z;
+            } else if (k < 7) {
+                const D3 L = cross(p0, v) * mi + wv * Ii;
+                e = k == 4 ? L.x : k == 5 ? L.y : L.z;
+            } else {
+                e = isfinite(v.x) && isfinite(v.y) && isfinite(v.z) && isfinite(wv.x) && isfinite(wv.y) &&
+                    isfinite(wv.z) && isfinite(p0.x) && isfinite(p0.y) && isfinite(p0.z) ? 0.0 : 1.0;
+            }
+            const double sum = wave_sum(valid ? e : 0.0);
+            if (l == 0) a.e_blk[blockIdx.x * FAST_E_STRIDE + (k < 7 ? k + 1 : 9)] = sum;
         }
     }
 }
@@ -1088,7 +1234,8 @@ __global__ __launch_bounds__(TB) void k_bounds(State s, const int* blk_sys, cons
         bnd[2 * blockIdx.x] = lo;
         bnd[2 * blockIdx.x + 1] = hi;
     }
-    xl[b] = local_pos(x, y, z, R, valid, lo, hi, L0inv, l);
+    xl[b] = make_float4(local_coord(x, valid, lo.x, hi.x, L0inv, l), local_coord(y, valid, lo.y, hi.y, L0inv, 0),
+                        local_coord(z, valid, lo.z, hi.z, L0inv, 0), valid ? (float)(R * L0inv) : 0.f);
 }
 
 // Start-of-call drift of the valid balls (each system with its own dt).

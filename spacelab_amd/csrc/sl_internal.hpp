@@ -91,16 +91,17 @@ struct FastBuffers {
     double L0 = 1, M0 = 1;        // length and mass units of the mixed path
     double Kf = 1;                // mixed path: force scale of the binary32 factor
     int* blk_sys = nullptr;       // device copies of the layout
+    int4* blk_info = nullptr;     // per 64-ball block: {first slot, balls, blocks of its system, system}
     int* sys_off = nullptr;
     int* sys_n = nullptr;
-    int* sys_nb = nullptr;
     int* sys_first = nullptr;     // balls of the systems before
     Phys* sysP = nullptr;
     int4* tiles = nullptr;        // {I, J, system, first block of system}, I >= J
     int n_tiles = 0, cap_tiles = 0;
     double* part = nullptr;       // far-field force partials [K][xyz][n_pad]
     unsigned long long* nbm = nullptr;   // near-partner masks [K][n_pad]
-    int part_slots = 0;           // K capacity of part and nbm
+    unsigned char* near = nullptr;       // per 64-ball block and slot K: the slot's masks have a bit set
+    int part_slots = 0;           // K capacity of part and nbm, K stride of near
     int* flags = nullptr;         // [1] non-finite state
     unsigned long long* blk_ctr = nullptr;    // per 64-ball block: touching and near pairs (running sums)
     int cap_blocks = 0;

@@ -179,6 +179,10 @@ void launch_far_any(const TileArgs& a, int choice, int precision, bool write, bo
         launch_far_split<1>(a, precision, write, grav, q, n_cu, st);
 }
 
+// Whether the tiles mark the slots that have near pairs, and write only their masks, for k_ball's
+// NEARF variant.
+bool near_flags(const FastBuffers& fb) { return fb.lay.nb_max > KB_BATCH && fast_ball_waves(fb) == 8; }
+
 TileArgs tile_args(FastBuffers& fb)
 {
     const State& c = fb.eng[fb.cur];
@@ -200,6 +204,8 @@ TileArgs tile_args(FastBuffers& fb)
     a.Kf = fb.Kf;
     a.part = fb.part;
     a.nbm = fb.nbm;
+    a.near = near_flags(fb) ? fb.near : nullptr;
+    a.near_stride = fb.part_slots;
     a.pe_tile = fb.pe_tile;
     a.queue = fb.queue;
     return a;
@@ -293,18 +299,17 @@ int launch_tiles_step(FastBuffers& fb, bool write, hipStream_t st, std::string* 
 int launch_ball_step(FastBuffers& fb, bool write, bool kick, bool drift_next, hipStream_t st, std::string* err)
 {
     BallArgs a;
-    a.cur = fb.eng[fb.cur];
-    a.nxt = fb.eng[1 - fb.cur];
+    a.cur = fb.eng[fb.cur].f[0];
+    a.nxt = fb.eng[1 - fb.cur].f[0];
+    a.konst = fb.eng[0].f[0];
     a.sysP = fb.sysP;
-    a.blk_sys = fb.blk_sys;
-    a.sys_off = fb.sys_off;
-    a.sys_n = fb.sys_n;
-    a.sys_nb = fb.sys_nb;
-    a.n_used = fb.lay.n_used;
+    a.blk_info = fb.blk_info;
     a.n_pad = fb.n_pad;
     a.part = fb.part;
     a.Kf = fb.Kf;
     a.nbm = fb.nbm;
+    a.near = near_flags(fb) ? fb.near : nullptr;
+    a.near_stride = fb.part_slots;
     a.perm = fb.perm;
     a.kick = kick;
     a.drift_next = drift_next;
@@ -317,15 +322,22 @@ int launch_ball_step(FastBuffers& fb, bool write, bool kick, bool drift_next, hi
     const int blocks = fb.lay.n_used / TB;
     if (fb.hook.before) fb.hook.before(fb.hook.user, 1);
     const bool mixed = fb.precision == SL_PREC_MIXED;
-    if (fast_ball_waves(fb) == 8) {
-        constexpr int T = kb_threads(8);
-        if (mixed) write ? k_ball<true, true, 8><<<blocks, T, 0, st>>>(a) : k_ball<true, false, 8><<<blocks, T, 0, st>>>(a);
-        else write ? k_ball<false, true, 8><<<blocks, T, 0, st>>>(a) : k_ball<false, false, 8><<<blocks, T, 0, st>>>(a);
-    } else {
-        constexpr int T = kb_threads(4);
-        if (mixed) write ? k_ball<true, true, 4><<<blocks, T, 0, st>>>(a) : k_ball<true, false, 4><<<blocks, T, 0, st>>>(a);
-        else write ? k_ball<false, true, 4><<<blocks, T, 0, st>>>(a) : k_ball<false, false, 4><<<blocks, T, 0, st>>>(a);
-    }
+    auto launch = [&](auto nwv, auto nearf) {
+        constexpr int N = decltype(nwv)::value;
+        constexpr bool F = decltype(nearf)::value;
+        if (mixed)
+            write ? k_ball<true, true, N, F><<<blocks, kb_threads(N), 0, st>>>(a)
+                  : k_ball<true, false, N, F><<<blocks, kb_threads(N), 0, st>>>(a);
+        else
+            write ? k_ball<false, true, N, F><<<blocks, kb_threads(N), 0, st>>>(a)
+                  : k_ball<false, false, N, F><<<blocks, kb_threads(N), 0, st>>>(a);
+    };
+    if (near_flags(fb))
+        launch(std::integral_constant<int, 8>{}, std::true_type{});
+    else if (fast_ball_waves(fb) == 8)
+        launch(std::integral_constant<int, 8>{}, std::false_type{});
+    else
+        launch(std::integral_constant<int, 4>{}, std::false_type{});
     if (fb.hook.after) fb.hook.after(fb.hook.user, 1);
     if (hipGetLastError() != hipSuccess) return err_hip(err, "ball kernel launch");
     fb.cur = 1 - fb.cur;
@@ -575,10 +587,10 @@ int fast_alloc(FastBuffers& fb, int n_pad, int max_sys)
     if (hipMalloc(&fb.queue, sizeof(int) * QPAD * (QSEG + 1)) != hipSuccess) return -1;
     if (hipMemset(fb.queue, 0, sizeof(int) * QPAD * (QSEG + 1)) != hipSuccess) return -1;
     if (hipMalloc(&fb.blk_sys, sizeof(int) * nblocks) != hipSuccess) return -1;
+    if (hipMalloc(&fb.blk_info, sizeof(int4) * nblocks) != hipSuccess) return -1;
     if (hipMalloc(&fb.sys_off, sizeof(int) * max_sys) != hipSuccess) return -1;
     if (hipMalloc(&fb.sys_n, sizeof(int) * max_sys) != hipSuccess) return -1;
-    if (hipMalloc(&fb.sys_nb, sizeof(int) * 2 * max_sys) != hipSuccess) return -1;
-    fb.sys_first = fb.sys_nb + max_sys;
+    if (hipMalloc(&fb.sys_first, sizeof(int) * max_sys) != hipSuccess) return -1;
     if (hipMalloc(&fb.sysP, sizeof(Phys) * max_sys) != hipSuccess) return -1;
     if (hipMalloc(&fb.flags, sizeof(int) * 4) != hipSuccess) return -1;
     const int eblocks = (n_pad + BPB - 1) / BPB;
@@ -604,8 +616,8 @@ void fast_clear_graphs(FastBuffers& fb)
 void fast_free(FastBuffers& fb)
 {
     fast_clear_graphs(fb);
-    void* ptrs[] = {fb.eng_base, fb.perm, fb.aux.q, fb.aux.g, fb.aux.q32, fb.aux.g32, fb.bnd, fb.xl, fb.gq_blk, fb.queue, fb.blk_sys,
-                    fb.sys_off, fb.sys_n, fb.sys_nb, fb.sysP, fb.tiles, fb.part, fb.nbm, fb.flags,
+    void* ptrs[] = {fb.eng_base, fb.perm, fb.aux.q, fb.aux.g, fb.aux.q32, fb.aux.g32, fb.bnd, fb.xl, fb.gq_blk, fb.queue, fb.blk_sys, fb.blk_info,
+                    fb.sys_off, fb.sys_n, fb.sys_first, fb.sysP, fb.tiles, fb.part, fb.nbm, fb.near, fb.flags,
                     fb.blk_ctr, fb.e_blk, fb.pe_tile};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
@@ -697,6 +709,8 @@ int fast_configure(FastBuffers& fb, State& canon, const FastLayout& lay, const P
                     fb.tile_sys_h.push_back(s);
                 }
             }
+        std::vector<int4> info;
+        for (int sy : fb.blk_sys_h) info.push_back(make_int4(lay.off[sy], lay.n[sy], lay.nb[sy], sy));
         const int nt = (int)tiles.size();
         if (nt > fb.cap_tiles) {
             if (fb.tiles) (void)hipFree(fb.tiles);
@@ -715,20 +729,23 @@ int fast_configure(FastBuffers& fb, State& canon, const FastLayout& lay, const P
         if (lay.nb_max > fb.part_slots) {
             if (fb.part) (void)hipFree(fb.part);
             if (fb.nbm) (void)hipFree(fb.nbm);
+            if (fb.near) (void)hipFree(fb.near);
             fb.part = nullptr;
             fb.nbm = nullptr;
+            fb.near = nullptr;
             fb.part_slots = 0;
             if (hipMalloc(&fb.part, sizeof(double) * (size_t)lay.nb_max * 3 * fb.n_pad) != hipSuccess ||
-                hipMalloc(&fb.nbm, sizeof(unsigned long long) * (size_t)lay.nb_max * fb.n_pad) != hipSuccess)
+                hipMalloc(&fb.nbm, sizeof(unsigned long long) * (size_t)lay.nb_max * fb.n_pad) != hipSuccess ||
+                hipMalloc(&fb.near, (size_t)lay.nb_max * fb.cap_blocks) != hipSuccess)
                 return err_hip(err, "partial buffer allocation");
             fb.part_slots = lay.nb_max;
         }
         if (hipMemcpyAsync(fb.tiles, tiles.data(), sizeof(int4) * nt, hipMemcpyHostToDevice, st) != hipSuccess ||
             hipMemcpyAsync(fb.blk_sys, fb.blk_sys_h.data(), sizeof(int) * fb.blk_sys_h.size(), hipMemcpyHostToDevice,
                            st) != hipSuccess ||
+            hipMemcpyAsync(fb.blk_info, info.data(), sizeof(int4) * info.size(), hipMemcpyHostToDevice, st) != hipSuccess ||
             hipMemcpyAsync(fb.sys_off, lay.off.data(), sizeof(int) * lay.n_sys, hipMemcpyHostToDevice, st) != hipSuccess ||
             hipMemcpyAsync(fb.sys_n, lay.n.data(), sizeof(int) * lay.n_sys, hipMemcpyHostToDevice, st) != hipSuccess ||
-            hipMemcpyAsync(fb.sys_nb, lay.nb.data(), sizeof(int) * lay.n_sys, hipMemcpyHostToDevice, st) != hipSuccess ||
             hipMemcpyAsync(fb.sys_first, lay.first.data(), sizeof(int) * lay.n_sys, hipMemcpyHostToDevice, st) != hipSuccess ||
             hipStreamSynchronize(st) != hipSuccess)
             return err_hip(err, "layout tables");
