@@ -366,7 +366,14 @@ int sl_mlp_gradients(sl_mlp* m, int batch, const float* x, const int* cls, const
 /* One Adam step (beta 0.9, 0.999, eps 1e-8) on a labelled batch; loss before the step. */
 int sl_mlp_train_step(sl_mlp* m, int batch, const float* x, const int* cls, const float* reg, float lr,
                       float* loss);
-const char* sl_mlp_last_error(const sl_mlp* m);
+/* The same of several nets (same n_in and n_out, each on rows of its own): net j takes the
+ * rows idx[j * batch ..] of x, cls and reg (n_rows of each).  Nets of the same widths and
+ * max_batch share their launches; the results are those of sl_mlp_train_step for each. */
+int sl_mlp_train_rows(sl_mlp* const* nets, int n, int batch, long long n_rows, const float* x, const int* cls,
+                      const float* reg, const long long* idx, float lr, float* loss);
+/* sl_mlp_forward of several nets (same n_in and n_out) on the same rows; outputs net after net. */
+int sl_mlp_forward_all(sl_mlp* const* nets, int n, int batch, const float* x, float* y, float* prob, float* ent);
+const char* sl_mlp_last_error(const sl_mlp* m);   /* calls on several nets: of the net it fails on or the first */
 void sl_mlp_destroy(sl_mlp* m);
 
 /* ---- allocation-free stepping ----------------------------------------------

@@ -215,6 +215,9 @@ def lib():
     L.sl_mlp_forward.argtypes = [vp, C.c_int, fp, fp, fp, fp]
     L.sl_mlp_gradients.argtypes = [vp, C.c_int, fp, ip, fp, fp, fp]
     L.sl_mlp_train_step.argtypes = [vp, C.c_int, fp, ip, fp, C.c_float, fp]
+    mlps, llp = C.POINTER(vp), C.POINTER(C.c_longlong)
+    L.sl_mlp_train_rows.argtypes = [mlps, C.c_int, C.c_int, C.c_longlong, fp, ip, fp, llp, C.c_float, fp]
+    L.sl_mlp_forward_all.argtypes = [mlps, C.c_int, C.c_int, fp, fp, fp, fp]
     L.sl_mlp_last_error.argtypes = [vp]
     L.sl_mlp_last_error.restype = C.c_char_p
     L.sl_mlp_destroy.argtypes = [vp]
@@ -788,6 +791,44 @@ class MLP:
         self._check(lib().sl_mlp_train_step(self._m, x.shape[0], _fp(x), _ip(cls), _fp(reg), lr, C.byref(loss)),
                     "sl_mlp_train_step")
         return float(loss.value)
+
+
+def _mlp_call(mlps: list[MLP], what: str, *args):
+    """sl_mlp_* of several nets; the message of a failure is one of theirs."""
+    rc = getattr(lib(), what)((C.c_void_p * len(mlps))(*(m._m for m in mlps)), len(mlps), *args)
+    if rc < 0:
+        msg = next((e for e in (lib().sl_mlp_last_error(m._m) for m in mlps) if e), b"")
+        raise SpacelabError(rc, f"{what}: {msg.decode()}")
+
+
+def mlp_train_rows(mlps: list[MLP], x, cls, reg, idx, lr: float) -> list[float]:
+    """One Adam step of each net on its own rows idx[j] of (x, cls, reg); the losses before it.
+    The same as train_step(x[idx[j]], cls[idx[j]], reg[idx[j]], lr) of each."""
+    x = np.ascontiguousarray(x, dtype=np.float32)
+    cls = np.ascontiguousarray(cls, dtype=np.int32)
+    reg = np.ascontiguousarray(reg, dtype=np.float32)
+    idx = np.ascontiguousarray(idx, dtype=np.int64)
+    m = mlps[0]
+    if not (idx.ndim == 2 and len(idx) == len(mlps) and x.shape[1:] == (m.n_in,) and cls.ndim == 1
+            and min(len(cls), len(reg)) >= len(x) and reg.size == len(reg) * (m.n_out - 3)):
+        raise ValueError("idx: a row of indices per net; x, cls, reg: rows of the data")
+    loss = np.zeros(len(mlps), np.float32)
+    _mlp_call(mlps, "sl_mlp_train_rows", idx.shape[1], len(x), _fp(x), _ip(cls), _fp(reg),
+              idx.ctypes.data_as(C.POINTER(C.c_longlong)), lr, _fp(loss))
+    return [float(v) for v in loss]
+
+
+def mlp_forward_all(mlps: list[MLP], x: np.ndarray):
+    """forward of each net on the same rows: (outputs, class probabilities, predictive entropy),
+    each with a leading axis over the nets."""
+    x = np.ascontiguousarray(x, dtype=np.float32)
+    n, B, m = len(mlps), x.shape[0], mlps[0]
+    if x.shape != (B, m.n_in):
+        raise ValueError("x: rows of the nets' inputs")
+    y = np.zeros((n, B, m.n_out), np.float32); p = np.zeros((n, B, 3), np.float32)
+    e = np.zeros((n, B), np.float32)
+    _mlp_call(mlps, "sl_mlp_forward_all", B, _fp(x), _fp(y), _fp(p), _fp(e))
+    return y, p, e
 
 
 def _csv_text(fn, what: str, *args, guess: int = 256) -> str:

@@ -259,7 +259,26 @@ constexpr int CHAIN_WAVES = 16;          // most wavefronts per workgroup
 constexpr int CHAIN_LD = CHAIN_MAX + 8;  // row stride of the activations in LDS: 16-byte reads of 16 rows, no conflicts
 constexpr int KF = 8;                    // weight fragments (32 of K each) a lane holds at once
 
+// Members of an ensemble that one launch carries through the same pass (grid y): nets of the
+// same widths and largest batch are laid out alike, so a member's pointer is the first
+// member's, moved by the distance between their allocations.  One net has too few workgroups
+// (16 at batch 256) and too short a pass for a launch: a training step of four nets takes the
+// device 33 us together and 27 us for one alone; driven one by one each cost 56 us with its
+// launches and its wait.  (21-256-256-256-9, batch 256, 4096 rows, one epoch of four nets:
+// 3.6 -> 1.5 ms; 10,000 rows through the four 1.03 -> 0.76 ms.)
+constexpr int MEMBERS = 16;
+struct Moved {
+    long long pool, stage, x;   // bytes: device pool, pinned buffer, input rows
+};
+template <class T>
+__device__ __forceinline__ T* moved(T* p, long long by)
+{
+    using C = std::conditional_t<std::is_const_v<T>, const char, char>;
+    return reinterpret_cast<T*>(reinterpret_cast<C*>(p) + by);
+}
+
 struct ChainArgs {
+    Moved at[MEMBERS];
     int B, n_in, n_out;
     int ld[NL + 1];                 // padded widths: input, hidden layers, output
     const float* x;                 // [B][n_in]
@@ -366,6 +385,7 @@ __global__ __launch_bounds__(CHAIN_WAVES * 64) void k_chain(ChainArgs a)
     __shared__ float yf[CHAIN_ROWS][CHAIN_MAX + 1];
     __shared__ float rg[TRAIN ? CHAIN_ROWS : 1][TRAIN ? CHAIN_MAX : 1];   // regression targets
     __shared__ float bs[NL][CHAIN_MAX];                                   // biases
+    const Moved at = a.at[blockIdx.y];
     const int t = threadIdx.x, nt = blockDim.x, nw = nt / 64;
     const int w = __builtin_amdgcn_readfirstlane(t / 64), l = t % 64;
     const int m0 = blockIdx.x * CHAIN_ROWS;
@@ -376,7 +396,7 @@ __global__ __launch_bounds__(CHAIN_WAVES * 64) void k_chain(ChainArgs a)
     auto ask = [&](auto pc) {
         constexpr int p = decltype(pc)::value;
         constexpr int k = p < NL ? p : 2 * NL - 1 - p;
-        const bf16* mat = p < NL ? a.Wf[k] : a.Wr[k];
+        const bf16* mat = p < NL ? moved(a.Wf[k], at.pool) : moved(a.Wr[k], at.pool);
         const int K = p < NL ? a.ld[k] : a.ld[k + 1], N = p < NL ? a.ld[k + 1] : a.ld[k];
         constexpr int F = p == 0 ? F0 : p == NL ? FL : KF;
         load_frags<F>(wf[p & 1], mat, min(w, N / 16 - 1), k_steps(K), 0);
@@ -385,21 +405,21 @@ __global__ __launch_bounds__(CHAIN_WAVES * 64) void k_chain(ChainArgs a)
     ask(std::integral_constant<int, 1>{});
     // the input rows, padded with zeros to a multiple of 32, the labels and the targets
     int cls = 0;
-    if (TRAIN && t < CHAIN_ROWS && m0 + t < a.B) cls = a.cls[m0 + t];
+    if (TRAIN && t < CHAIN_ROWS && m0 + t < a.B) cls = moved(a.cls, at.stage)[m0 + t];
 #pragma unroll 1
     for (int r = w; r < CHAIN_ROWS; r += nw) {
         const size_t b = m0 + r;
         const bool in = m0 + r < a.B;
 #pragma unroll 1
         for (int c = l; c < 32 * k_steps(a.ld[0]); c += 64)
-            act[0][r][c] = to_bf16(in && c < a.n_in ? a.x[b * a.n_in + c] : 0.f);
+            act[0][r][c] = to_bf16(in && c < a.n_in ? moved(a.x, at.x)[b * a.n_in + c] : 0.f);
         if (TRAIN && in)
 #pragma unroll 1
-            for (int c = l; c < a.n_out - NCLS; c += 64) rg[r][c] = a.reg[b * (a.n_out - NCLS) + c];
+            for (int c = l; c < a.n_out - NCLS; c += 64) rg[r][c] = moved(a.reg, at.stage)[b * (a.n_out - NCLS) + c];
     }
     for (int k = 0; k < NL; k++)
 #pragma unroll 1
-        for (int c = t; c < a.ld[k + 1]; c += nt) bs[k][c] = a.b[k][c];
+        for (int c = t; c < a.ld[k + 1]; c += nt) bs[k][c] = moved(a.b[k], at.pool)[c];
     lds_barrier();
     if (TRAIN)
 #pragma unroll 1
@@ -407,7 +427,7 @@ __global__ __launch_bounds__(CHAIN_WAVES * 64) void k_chain(ChainArgs a)
             const int c = e / 4, q = 4 * (e % 4);
             const unsigned lo = (unsigned)act[0][q][c] | (unsigned)act[0][q + 1][c] << 16;
             const unsigned hi = (unsigned)act[0][q + 2][c] | (unsigned)act[0][q + 3][c] << 16;
-            *reinterpret_cast<uint2*>(a.Ht[0] + (size_t)c * a.ldb + m0 + q) = make_uint2(lo, hi);
+            *reinterpret_cast<uint2*>(moved(a.Ht[0], at.pool) + (size_t)c * a.ldb + m0 + q) = make_uint2(lo, hi);
         }
     unsigned mask = 0;   // 4 bits per hidden layer and tile of this wavefront: the outputs above 0
     auto fwd = [&](auto kc) {
@@ -417,7 +437,7 @@ __global__ __launch_bounds__(CHAIN_WAVES * 64) void k_chain(ChainArgs a)
         const int N = a.ld[k + 1], ks = k_steps(a.ld[k]);
         auto tile = [&](int n0, int ti) {
             const float bias = bs[k][n0 + cl];
-            const float4_t acc = chain_tile<F>(act[k & 1], wf[k & 1], a.Wf[k], n0 / 16, ks);
+            const float4_t acc = chain_tile<F>(act[k & 1], wf[k & 1], moved(a.Wf[k], at.pool), n0 / 16, ks);
             float v[4];
 #pragma unroll
             for (int r = 0; r < 4; r++) {
@@ -436,12 +456,12 @@ __global__ __launch_bounds__(CHAIN_WAVES * 64) void k_chain(ChainArgs a)
                         if (m0 + r0 + r >= a.B) v[r] = 0.f;   // rows past the batch: nothing for k_wgrad
                     }
                 }
-                if (TRAIN) store4(a.Ht[last ? 0 : k + 1] + (size_t)(n0 + cl) * a.ldb, m0 + r0, v);
+                if (TRAIN) store4(moved(a.Ht[last ? 0 : k + 1], at.pool) + (size_t)(n0 + cl) * a.ldb, m0 + r0, v);
             }
         };
         if (16 * w < N) tile(16 * w, 0);
         if (16 * (w + nw) < N) {   // at most two tiles: CHAIN_MAX / 16 / CHAIN_WAVES
-            load_frags<F>(wf[k & 1], a.Wf[k], w + nw, ks, 0);
+            load_frags<F>(wf[k & 1], moved(a.Wf[k], at.pool), w + nw, ks, 0);
             tile(16 * (w + nw), 1);
         }
         if (!last && (N & 16) && w == nw - 1)
@@ -459,11 +479,11 @@ __global__ __launch_bounds__(CHAIN_WAVES * 64) void k_chain(ChainArgs a)
         for (int r = w; r < CHAIN_ROWS; r += nw)
             if (m0 + r < a.B)
 #pragma unroll 1
-                for (int c = l; c < a.n_out; c += 64) a.y[(size_t)(m0 + r) * a.n_out + c] = yf[r][c];
+                for (int c = l; c < a.n_out; c += 64) moved(a.y, at.stage)[(size_t)(m0 + r) * a.n_out + c] = yf[r][c];
         if (t < CHAIN_ROWS && m0 + t < a.B) {
             float p[NCLS];
-            a.ent[m0 + t] = sample_predict(yf[t], p);
-            for (int k = 0; k < NCLS; k++) a.prob[(size_t)(m0 + t) * NCLS + k] = p[k];
+            moved(a.ent, at.stage)[m0 + t] = sample_predict(yf[t], p);
+            for (int k = 0; k < NCLS; k++) moved(a.prob, at.stage)[(size_t)(m0 + t) * NCLS + k] = p[k];
         }
         return;
     }
@@ -471,7 +491,7 @@ __global__ __launch_bounds__(CHAIN_WAVES * 64) void k_chain(ChainArgs a)
     if (t < CHAIN_ROWS) {
         const int b = m0 + t;
         if (b < a.B)
-            a.loss[b] = sample_loss(yf[t], a.n_out, ldy, cls, rg[t], 1.0f / (float)a.B);
+            moved(a.loss, at.stage)[b] = sample_loss(yf[t], a.n_out, ldy, cls, rg[t], 1.0f / (float)a.B);
         else
             for (int k = 0; k < ldy; k++) yf[t][k] = 0.f;
     }
@@ -482,13 +502,13 @@ __global__ __launch_bounds__(CHAIN_WAVES * 64) void k_chain(ChainArgs a)
         for (int c = l; c < 32 * k_steps(ldy); c += 64) {
             const float g = c < ldy ? yf[r][c] : 0.f;
             act[0][r][c] = to_bf16(g);
-            if (c < ldy && m0 + r < a.B) a.dZ[NL - 1][(size_t)(m0 + r) * ldy + c] = g;
+            if (c < ldy && m0 + r < a.B) moved(a.dZ[NL - 1], at.pool)[(size_t)(m0 + r) * ldy + c] = g;
         }
 #pragma unroll 1
     for (int e = t; e < 4 * ldy; e += nt) {
         const int c = e / 4, q = 4 * (e % 4);
         const float v[4] = {yf[q][c], yf[q + 1][c], yf[q + 2][c], yf[q + 3][c]};
-        store4(a.dZt[NL - 1] + (size_t)c * a.ldb, m0 + q, v);
+        store4(moved(a.dZt[NL - 1], at.pool) + (size_t)c * a.ldb, m0 + q, v);
     }
     lds_barrier();
     auto bwd = [&](auto pc) {
@@ -498,20 +518,20 @@ __global__ __launch_bounds__(CHAIN_WAVES * 64) void k_chain(ChainArgs a)
         constexpr int cur = p & 1;                    // act[0] holds the output gradient: NL is even
         const int N = a.ld[k], ks = k_steps(a.ld[k + 1]);
         auto tile = [&](int n0, int ti) {
-            const float4_t acc = chain_tile<F>(act[cur], wf[p & 1], a.Wr[k], n0 / 16, ks);
+            const float4_t acc = chain_tile<F>(act[cur], wf[p & 1], moved(a.Wr[k], at.pool), n0 / 16, ks);
             float v[4];
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 const bool in = m0 + r0 + r < a.B;
                 v[r] = in && ((mask >> (8 * (k - 1) + 4 * ti + r)) & 1u) ? acc[r] : 0.f;
-                if (in) a.dZ[k - 1][(size_t)(m0 + r0 + r) * N + n0 + cl] = v[r];
+                if (in) moved(a.dZ[k - 1], at.pool)[(size_t)(m0 + r0 + r) * N + n0 + cl] = v[r];
                 act[cur ^ 1][r0 + r][n0 + cl] = to_bf16(v[r]);
             }
-            store4(a.dZt[k - 1] + (size_t)(n0 + cl) * a.ldb, m0 + r0, v);
+            store4(moved(a.dZt[k - 1], at.pool) + (size_t)(n0 + cl) * a.ldb, m0 + r0, v);
         };
         if (16 * w < N) tile(16 * w, 0);
         if (16 * (w + nw) < N) {
-            load_frags<F>(wf[p & 1], a.Wr[k], w + nw, ks, 0);
+            load_frags<F>(wf[p & 1], moved(a.Wr[k], at.pool), w + nw, ks, 0);
             tile(16 * (w + nw), 1);
         }
         if ((N & 16) && w == nw - 1)
@@ -544,13 +564,16 @@ struct WgradArgs {
     float *W[NL], *mW[NL], *vW[NL], *gW[NL];
     bf16 *Wf[NL], *Wr[NL];
     float *b[NL], *mb[NL], *vb[NL], *gb[NL];
-    Adam adam;
+    long long pool[MEMBERS];        // as in Moved
+    Adam adam[MEMBERS];
 };
 
 template <bool STEP>
 __global__ __launch_bounds__(256) void k_wgrad(WgradArgs a)
 {
     const int tid = threadIdx.x;
+    const long long at = a.pool[blockIdx.y];
+    const Adam adam = a.adam[blockIdx.y];
     if ((int)blockIdx.x >= a.wblocks) {
         __shared__ float part[8][32];
         const int q = blockIdx.x - a.wblocks;
@@ -561,7 +584,7 @@ __global__ __launch_bounds__(256) void k_wgrad(WgradArgs a)
         const int c = (q - a.bias0[k]) * 32 + cl;
         float sum = 0.f;
         if (c < N) {
-            const float* src = a.dZ[k] + c;
+            const float* src = moved(a.dZ[k], at) + c;
 #pragma unroll 8
             for (int r = ph; r < a.B; r += 8) sum += src[(size_t)r * N];
         }
@@ -571,9 +594,9 @@ __global__ __launch_bounds__(256) void k_wgrad(WgradArgs a)
             float g = part[0][cl];
             for (int p = 1; p < 8; p++) g += part[p][cl];
             if (STEP)
-                a.b[k][c] = adam_value(a.adam, a.b[k][c], g, a.mb[k][c], a.vb[k][c]);
+                moved(a.b[k], at)[c] = adam_value(adam, moved(a.b[k], at)[c], g, moved(a.mb[k], at)[c], moved(a.vb[k], at)[c]);
             else
-                a.gb[k][c] = g;
+                moved(a.gb[k], at)[c] = g;
         }
         return;
     }
@@ -591,13 +614,13 @@ __global__ __launch_bounds__(256) void k_wgrad(WgradArgs a)
 #pragma unroll
         for (int r = 0; r < 4; r++) {
             const size_t e = (size_t)(in0 + r) * N + out;
-            wv[r] = a.W[k][e];
-            mv[r] = a.mW[k][e];
-            vv[r] = a.vW[k][e];
+            wv[r] = moved(a.W[k], at)[e];
+            mv[r] = moved(a.mW[k], at)[e];
+            vv[r] = moved(a.vW[k], at)[e];
         }
     }
-    const bf16* ha = a.Ht[k] + (size_t)(i0 + l % 16) * a.ldb + 8 * (l / 16);
-    const bf16* zb = a.dZt[k] + (size_t)(o0 + l % 16) * a.ldb + 8 * (l / 16);
+    const bf16* ha = moved(a.Ht[k], at) + (size_t)(i0 + l % 16) * a.ldb + 8 * (l / 16);
+    const bf16* zb = moved(a.dZt[k], at) + (size_t)(o0 + l % 16) * a.ldb + 8 * (l / 16);
     // ldb covers the batch in steps of 32; rows past it in k_chain's last 16 are zeros, and
     // the 16 after those are not read
     const int Bp = (a.B + CHAIN_ROWS - 1) / CHAIN_ROWS * CHAIN_ROWS;
@@ -623,16 +646,16 @@ __global__ __launch_bounds__(256) void k_wgrad(WgradArgs a)
     for (int r = 0; r < 4; r++) {
         const size_t e = (size_t)(in0 + r) * N + out;
         if (STEP) {
-            wv[r] = adam_value(a.adam, wv[r], acc[r], mv[r], vv[r]);
-            a.W[k][e] = wv[r];
-            a.mW[k][e] = mv[r];
-            a.vW[k][e] = vv[r];
-            a.Wr[k][frag_at(out, in0 + r, k_steps(N))] = to_bf16(wv[r]);
+            wv[r] = adam_value(adam, wv[r], acc[r], mv[r], vv[r]);
+            moved(a.W[k], at)[e] = wv[r];
+            moved(a.mW[k], at)[e] = mv[r];
+            moved(a.vW[k], at)[e] = vv[r];
+            moved(a.Wr[k], at)[frag_at(out, in0 + r, k_steps(N))] = to_bf16(wv[r]);
         } else {
-            a.gW[k][e] = acc[r];
+            moved(a.gW[k], at)[e] = acc[r];
         }
     }
-    if (STEP) store4(a.Wf[k] + frag_at(in0, out, k_steps(K)), 0, wv);
+    if (STEP) store4(moved(a.Wf[k], at) + frag_at(in0, out, k_steps(K)), 0, wv);
 }
 
 // bfloat16 copies of one layer's weights: Wb in W's layout (layer form), or Wf and Wr as
@@ -829,9 +852,15 @@ int pull_flat(sl_mlp* m, const float* dev, float* out)
 
 // ---- chain form ------------------------------------------------------------------------
 
-ChainArgs chain_args(sl_mlp* m, int B)
+ChainArgs chain_args(sl_mlp* const* ms, int n, int B, bool one_input)
 {
     ChainArgs a{};
+    sl_mlp* m = ms[0];
+    for (int j = 0; j < n; j++) {
+        a.at[j].pool = ms[j]->pool - m->pool;
+        a.at[j].stage = ms[j]->stage_dev - m->stage_dev;
+        a.at[j].x = one_input ? 0 : a.at[j].stage;
+    }
     const Stage s(m->max_batch, m->n_in, m->n_out);
     auto at = [&](size_t o) { return reinterpret_cast<float*>(m->stage_dev + o); };
     a.B = B;
@@ -859,14 +888,18 @@ ChainArgs chain_args(sl_mlp* m, int B)
     return a;
 }
 
+// A batch of B of each of ms[0 .. n - 1] (alike, n <= MEMBERS), on the first one's stream;
+// inference reads the first one's input rows.
 template <bool TRAIN>
-void launch_chain(sl_mlp* m, int B)
+void launch_chain(sl_mlp* const* ms, int n, int B)
 {
+    const sl_mlp* m = ms[0];
     int widest = 0;   // column tiles of the widest layer: one wavefront each, up to CHAIN_WAVES
     for (const Layer& L : m->L) widest = std::max(widest, L.ldout / 16);
-    const int threads = 64 * std::min(widest, CHAIN_WAVES), grid = (B + CHAIN_ROWS - 1) / CHAIN_ROWS;
+    const int threads = 64 * std::min(widest, CHAIN_WAVES);
+    const dim3 grid((B + CHAIN_ROWS - 1) / CHAIN_ROWS, n);
     const bool f0 = m->L[0].ldin > 32, fl = m->L[NL - 1].ldout > 32;
-    const ChainArgs a = chain_args(m, B);
+    const ChainArgs a = chain_args(ms, n, B, !TRAIN);
     if (f0)
         fl ? k_chain<TRAIN, KF, KF><<<grid, threads, 0, m->stream>>>(a) : k_chain<TRAIN, KF, 1><<<grid, threads, 0, m->stream>>>(a);
     else
@@ -874,12 +907,16 @@ void launch_chain(sl_mlp* m, int B)
 }
 
 template <bool STEP>
-void launch_wgrad(sl_mlp* m, int B, const Adam& adam)
+void launch_wgrad(sl_mlp* const* ms, int n, int B, const Adam* adam)
 {
     WgradArgs a{};
+    sl_mlp* m = ms[0];
     a.B = B;
     a.ldb = m->ldb;
-    a.adam = adam;
+    for (int j = 0; j < n; j++) {
+        a.pool[j] = ms[j]->pool - m->pool;
+        if (adam) a.adam[j] = adam[j];
+    }
     a.ld[0] = m->L[0].ldin;
     int bias = 0;
     for (int k = 0; k < NL; k++) {
@@ -903,7 +940,7 @@ void launch_wgrad(sl_mlp* m, int B, const Adam& adam)
         a.gb[k] = L.gb;
     }
     a.wblocks = (a.tile0[NL] + 3) / 4;
-    k_wgrad<STEP><<<a.wblocks + bias, 256, 0, m->stream>>>(a);
+    k_wgrad<STEP><<<dim3(a.wblocks + bias, n), 256, 0, m->stream>>>(a);
 }
 
 // ---- layer form ------------------------------------------------------------------------
@@ -953,6 +990,32 @@ int load_batch(sl_mlp* m, int B, const float* x)
 
 // ---- both forms --------------------------------------------------------------------------
 
+float mean_loss(const float* ls, int B)
+{
+    double sum = 0;
+    for (int b = 0; b < B; b++) sum += ls[b];
+    return (float)(sum / B);
+}
+
+Adam adam_step(const sl_mlp* m, float lr)
+{
+    const float b1 = 0.9f, b2 = 0.999f;
+    const long long t = m->t + 1;
+    return Adam{lr, b1, b2, 1e-8f, 1.f - std::pow(b1, (float)t), 1.f - std::pow(b2, (float)t)};
+}
+
+// Whether one launch can carry them all: different nets in the chain form, laid out alike.
+bool alike(sl_mlp* const* ms, int n)
+{
+    for (int j = 0; j < n; j++) {
+        const sl_mlp &a = *ms[0], &b = *ms[j];
+        if (!b.chain || b.n_in != a.n_in || b.width != a.width || b.n_out != a.n_out || b.max_batch != a.max_batch) return false;
+        for (int i = 0; i < j; i++)
+            if (ms[i] == ms[j]) return false;
+    }
+    return true;
+}
+
 // Forward, loss, backward and, with adam, the update of a labelled batch; the mean loss (of
 // the parameters before the update) to *loss.
 int train_pass(sl_mlp* m, int B, const float* x, const int* cls, const float* reg, float* loss, const Adam* adam)
@@ -966,8 +1029,8 @@ int train_pass(sl_mlp* m, int B, const float* x, const int* cls, const float* re
         std::memcpy(m->stage + s.x, x, 4 * (size_t)B * m->n_in);
         std::memcpy(m->stage + s.cls, cls, 4 * (size_t)B);
         std::memcpy(m->stage + s.reg, reg, 4 * (size_t)B * nr);
-        launch_chain<true>(m, B);
-        adam ? launch_wgrad<true>(m, B, *adam) : launch_wgrad<false>(m, B, Adam{});
+        launch_chain<true>(&m, 1, B);
+        adam ? launch_wgrad<true>(&m, 1, B, adam) : launch_wgrad<false>(&m, 1, B, nullptr);
     } else {
         if (load_batch(m, B, x)) return mlp_err(m, SL_E_HIP, "input upload failed");
         if (hipMemcpyAsync(m->cls, cls, 4 * (size_t)B, hipMemcpyHostToDevice, m->stream) != hipSuccess ||
@@ -990,9 +1053,7 @@ int train_pass(sl_mlp* m, int B, const float* x, const int* cls, const float* re
     }
     if (hipGetLastError() != hipSuccess || hipStreamSynchronize(m->stream) != hipSuccess)
         return mlp_err(m, SL_E_HIP, "training pass failed");
-    double sum = 0;
-    for (int b = 0; b < B; b++) sum += ls[b];
-    if (loss) *loss = (float)(sum / B);
+    if (loss) *loss = mean_loss(ls, B);
     return SL_OK;
 }
 
@@ -1110,7 +1171,7 @@ int sl_mlp_forward(sl_mlp* m, int B, const float* x, float* y, float* prob, floa
     if (m->chain) {
         const Stage s(m->max_batch, m->n_in, m->n_out);
         std::memcpy(m->stage + s.x, x, 4 * (size_t)B * m->n_in);
-        launch_chain<false>(m, B);
+        launch_chain<false>(&m, 1, B);
         if (hipGetLastError() != hipSuccess || hipStreamSynchronize(m->stream) != hipSuccess)
             return mlp_err(m, SL_E_HIP, "forward failed");
         if (y) std::memcpy(y, m->stage + s.y, 4 * (size_t)B * m->n_out);
@@ -1152,12 +1213,107 @@ int sl_mlp_train_step(sl_mlp* m, int B, const float* x, const int* cls, const fl
     int rc = check_batch(m, B, x);
     if (rc) return rc;
     if (!cls || !reg || !(lr > 0)) return mlp_err(m, SL_E_ARG, "labels are NULL or lr <= 0");
-    const float b1 = 0.9f, b2 = 0.999f;
-    const long long t = m->t + 1;
-    const Adam adam{lr, b1, b2, 1e-8f, 1.f - std::pow(b1, (float)t), 1.f - std::pow(b2, (float)t)};
+    const Adam adam = adam_step(m, lr);
     rc = train_pass(m, B, x, cls, reg, loss, &adam);
     if (rc) return rc;
-    m->t = t;
+    m->t++;
+    return SL_OK;
+}
+
+int sl_mlp_train_rows(sl_mlp* const* ms, int n, int B, long long n_rows, const float* x, const int* cls, const float* reg,
+                      const long long* idx, float lr, float* loss)
+{
+    if (!ms || n < 1) return SL_E_ARG;
+    for (int j = 0; j < n; j++) {
+        const int rc = check_batch(ms[j], B, x);
+        if (rc) return rc;
+        if (!cls || !reg || !idx || !(lr > 0)) return mlp_err(ms[j], SL_E_ARG, "labels or rows are NULL or lr <= 0");
+        if (ms[j]->n_in != ms[0]->n_in || ms[j]->n_out != ms[0]->n_out)
+            return mlp_err(ms[j], SL_E_ARG, "nets of one ensemble have the same inputs and outputs");
+        for (int b = 0; b < B; b++) {
+            const long long row = idx[(size_t)j * B + b];
+            if (row < 0 || row >= n_rows) return mlp_err(ms[j], SL_E_ARG, "row index outside the data");
+            if (cls[row] < 0 || cls[row] >= NCLS) return mlp_err(ms[j], SL_E_ARG, "class label outside 0..2");
+        }
+    }
+    const int n_in = ms[0]->n_in, nr = ms[0]->n_out - NCLS;
+    auto rows = [&](const long long* at, float* px, int* pc, float* pr) {
+        for (int b = 0; b < B; b++) {
+            std::memcpy(px + (size_t)b * n_in, x + at[b] * n_in, 4 * (size_t)n_in);
+            pc[b] = cls[at[b]];
+            std::memcpy(pr + (size_t)b * nr, reg + at[b] * nr, 4 * (size_t)nr);
+        }
+    };
+    if (!alike(ms, n)) {
+        const size_t words = (size_t)B * (n_in + 1 + nr);
+        float* buf = new (std::nothrow) float[words];
+        if (!buf) return mlp_err(ms[0], SL_E_STATE, "out of memory");
+        float* pr = buf + (size_t)B * n_in;
+        int* pc = reinterpret_cast<int*>(pr + (size_t)B * nr);
+        int rc = SL_OK;
+        for (int j = 0; j < n && rc == SL_OK; j++) {
+            rows(idx + (size_t)j * B, buf, pc, pr);
+            rc = sl_mlp_train_step(ms[j], B, buf, pc, pr, lr, loss ? loss + j : nullptr);
+            if (rc && j) ms[0]->err = ms[j]->err;
+        }
+        delete[] buf;
+        return rc;
+    }
+    const Stage s(ms[0]->max_batch, n_in, nr + NCLS);
+    for (int j0 = 0; j0 < n; j0 += MEMBERS) {
+        const int k = std::min(n - j0, MEMBERS);
+        Adam adam[MEMBERS];
+        for (int j = 0; j < k; j++) {
+            sl_mlp* m = ms[j0 + j];
+            adam[j] = adam_step(m, lr);
+            rows(idx + (size_t)(j0 + j) * B, reinterpret_cast<float*>(m->stage + s.x), reinterpret_cast<int*>(m->stage + s.cls),
+                 reinterpret_cast<float*>(m->stage + s.reg));
+        }
+        launch_chain<true>(ms + j0, k, B);
+        launch_wgrad<true>(ms + j0, k, B, adam);
+        if (hipGetLastError() != hipSuccess || hipStreamSynchronize(ms[j0]->stream) != hipSuccess)
+            return mlp_err(ms[0], SL_E_HIP, "training pass failed");
+        for (int j = 0; j < k; j++) {
+            sl_mlp* m = ms[j0 + j];
+            if (loss) loss[j0 + j] = mean_loss(reinterpret_cast<const float*>(m->stage + s.loss), B);
+            m->t++;
+        }
+    }
+    return SL_OK;
+}
+
+int sl_mlp_forward_all(sl_mlp* const* ms, int n, int B, const float* x, float* y, float* prob, float* ent)
+{
+    if (!ms || n < 1) return SL_E_ARG;
+    for (int j = 0; j < n; j++) {
+        const int rc = check_batch(ms[j], B, x);
+        if (rc) return rc;
+        if (ms[j]->n_in != ms[0]->n_in || ms[j]->n_out != ms[0]->n_out)
+            return mlp_err(ms[j], SL_E_ARG, "nets of one ensemble have the same inputs and outputs");
+    }
+    const size_t ny = (size_t)B * ms[0]->n_out, np = (size_t)B * NCLS;
+    const bool together = alike(ms, n);
+    const Stage s(ms[0]->max_batch, ms[0]->n_in, ms[0]->n_out);
+    for (int j0 = 0; j0 < n; j0 += MEMBERS) {
+        const int k = std::min(n - j0, MEMBERS);
+        if (together) {
+            std::memcpy(ms[j0]->stage + s.x, x, 4 * (size_t)B * ms[0]->n_in);
+            launch_chain<false>(ms + j0, k, B);
+            if (hipGetLastError() != hipSuccess || hipStreamSynchronize(ms[j0]->stream) != hipSuccess)
+                return mlp_err(ms[0], SL_E_HIP, "forward failed");
+        }
+        for (int j = j0; j < j0 + k; j++) {
+            float *yj = y ? y + j * ny : nullptr, *pj = prob ? prob + j * np : nullptr, *ej = ent ? ent + (size_t)j * B : nullptr;
+            if (together) {
+                if (yj) std::memcpy(yj, ms[j]->stage + s.y, 4 * ny);
+                if (pj) std::memcpy(pj, ms[j]->stage + s.prob, 4 * np);
+                if (ej) std::memcpy(ej, ms[j]->stage + s.ent, 4 * (size_t)B);
+            } else if (const int rc = sl_mlp_forward(ms[j], B, x, yj, pj, ej)) {
+                if (j) ms[0]->err = ms[j]->err;
+                return rc;
+            }
+        }
+    }
     return SL_OK;
 }
 

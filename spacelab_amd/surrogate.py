@@ -33,7 +33,8 @@ import numpy as np
 
 from . import (N_DESCRIPTORS, OUTCOME_BOUNCE, OUTCOME_FRAGMENT, OUTCOME_STICK, ORDER_FAST,
                PREC_FP64, Batch, CollisionSetup, MLP, calibrate, collision_approach,
-               collision_descriptors_batch, collision_outcome, generate_collision, preset)
+               collision_descriptors_batch, collision_outcome, generate_collision, mlp_forward_all,
+               mlp_train_rows, preset)
 
 CLASS_NAMES = ("stick", "bounce", "fragment")
 # regression targets: mass fraction of the largest body, share of the projectile's mass
@@ -211,17 +212,17 @@ class Surrogate:
         reg = np.ascontiguousarray(reg, dtype=np.float32)
         n = len(Xn)
         hist = np.zeros(epochs)
-        for k, m in enumerate(self.mlps):
-            rng = np.random.default_rng(seed * 1000 + k)
-            for ep in range(epochs):
-                perm = rng.permutation(n)
-                tot, cnt = 0.0, 0
-                lr_ep = lr * 0.5 * (1 + math.cos(math.pi * ep / epochs))
-                for b0 in range(0, n - batch + 1, batch):
-                    idx = perm[b0:b0 + batch]
-                    tot += m.train_step(Xn[idx], cls[idx], reg[idx], lr_ep) * len(idx)
-                    cnt += len(idx)
-                hist[ep] += tot / max(cnt, 1) / len(self.mlps)
+        rngs = [np.random.default_rng(seed * 1000 + k) for k in range(len(self.mlps))]
+        for ep in range(epochs if rngs else 0):
+            perm = np.stack([rng.permutation(n) for rng in rngs])
+            tot, cnt = np.zeros(len(self.mlps)), 0
+            lr_ep = lr * 0.5 * (1 + math.cos(math.pi * ep / epochs))
+            for b0 in range(0, n - batch + 1, batch):
+                loss = mlp_train_rows(self.mlps, Xn, cls, reg, perm[:, b0:b0 + batch], lr_ep)
+                tot += np.multiply(loss, batch)
+                cnt += batch
+            for t in tot.tolist():
+                hist[ep] += t / max(cnt, 1) / len(self.mlps)
         if log:
             log(f"loss by epoch: {np.round(hist, 4).tolist()}")
         return hist.tolist()
@@ -232,9 +233,9 @@ class Surrogate:
         Xn = self.norm(X)
         P = np.zeros((len(Xn), 3))
         Y = np.zeros((len(Xn), N_REG))
-        for m in self.mlps:
-            for k in range(0, len(Xn), self.max_batch):
-                y, p, _ = m.forward(Xn[k:k + self.max_batch])
+        for k in range(0, len(Xn) if self.mlps else 0, self.max_batch):
+            ys, ps, _ = mlp_forward_all(self.mlps, Xn[k:k + self.max_batch])
+            for y, p in zip(ys, ps):
                 P[k:k + len(p)] += p
                 Y[k:k + len(y)] += y[:, 3:]
         P /= len(self.mlps)
