@@ -230,36 +230,55 @@ __device__ __forceinline__ double grav_share(const TileArgs& a, int I, int J)
     return (double)a.gq_blk[I] * (double)a.gq_blk[J] * d2m * d2m * dmax;
 }
 
-// vdW energy of a far pair from s = d^2 - S^2, t = d^2 - (Ri-Rj)^2 (use: the lane's pair
-// counts).  With y = 4 Ri Rj / t the reference's sum 2RiRj/s + 2RiRj/t + ln(s/t) is
+// Largest y = 4 Ri Rj / (d^2 - (Ri - Rj)^2) of the pairs of tile (I, J), from the gap between the
+// blocks' boxes and their largest radii; +inf where the boxes are not apart, NaN where a
+// position is.
+__device__ __forceinline__ double energy_reach(const TileArgs& a, int I, int J)
+{
+    const double4 li = a.bnd[2 * I], ui = a.bnd[2 * I + 1], lj = a.bnd[2 * J], uj = a.bnd[2 * J + 1];
+    const double gx = fmax(0.0, fmax(lj.x - ui.x, li.x - uj.x));
+    const double gy = fmax(0.0, fmax(lj.y - ui.y, li.y - uj.y));
+    const double gz = fmax(0.0, fmax(lj.z - ui.z, li.z - uj.z));
+    const double rm = fmax(li.w, lj.w), t = gx * gx + gy * gy + gz * gz - rm * rm;
+    return t > 0 ? 4 * li.w * lj.w / t : __builtin_huge_val();
+}
+
+// vdW energy of a far pair over -Ha/6, from s = d^2 - S^2, t = d^2 - (Ri-Rj)^2 (use: the lane's
+// pair counts).  With y = 4 Ri Rj / t the reference's sum 2RiRj/s + 2RiRj/t + ln(s/t) is
 // y/2/(1-y) + y/2 + ln(1-y) = sum over k >= 3 of (1/2 - 1/k) y^k: its first two orders
 // cancel, so for y <= 1/8 (about three diameters apart and more: nearly every pair) 18 terms
 // of the series give it to 2^-52, for 23 instructions, where the three divisions and the
 // logarithm took about 75 and lost 6 / y^2 ulps.  (With the line at y = 1/16, 13 terms, the
-// closed form's loss just above it was 2e-13 of a pair, and the sweep was no faster.)  The write step's sweep at 40,000 spheres
-// went from 4557 to 2155 us (without energies: 1130), at 5000 from 87 to 55.  The choice is made pair by pair, so a pair's energy does not
-// depend on which pairs share its wavefront.
-__device__ __forceinline__ double far_energy(double Ha, double Ri, double Rj, double s, double t, bool use)
+// closed form's loss just above it was 2e-13 of a pair, and the sweep was no faster.)
+// FAR: y <= 2^-5 for every pair of the tile (eleven radii apart), so 11 terms do (the first left
+// out is 2.6 y^11 of the sum, 2^-53.6) and no lane needs the closed form.
+// The write step's sweep at 40,000 spheres took 4557 us in the closed form, 2205 by 18 terms
+// and 1890 with the short series (without energies: 1020); at 5,000 87, 55 and 54.
+template <bool FAR>
+__device__ __forceinline__ double far_energy(double Ri, double Rj, double s, double t, bool use)
 {
     const double two = 2 * Ri * Rj;
     double rt = __builtin_amdgcn_rcp(t);
     rt = __builtin_fma(rt, __builtin_fma(-t, rt, 1.0), rt);
     rt = __builtin_fma(rt, __builtin_fma(-t, rt, 1.0), rt);
     const double y = 2 * two * rt;
-    double p = 0.5 - 1.0 / 20;
+    constexpr int LAST = FAR ? 13 : 20;
+    double p = 0.5 - 1.0 / LAST;
 #pragma unroll
-    for (int k = 19; k >= 3; k--) p = __builtin_fma(p, y, 0.5 - 1.0 / k);
+    for (int k = LAST - 1; k >= 3; k--) p = __builtin_fma(p, y, 0.5 - 1.0 / k);
     double u = p * (y * y * y);
-    const bool close = use && !(y <= 0.125);
-    if (__any(close)) {
-        const double q = s * rt;   // 1 - y, from s
-        double rq = __builtin_amdgcn_rcp(q);
-        rq = __builtin_fma(rq, __builtin_fma(-q, rq, 1.0), rq);
-        rq = __builtin_fma(rq, __builtin_fma(-q, rq, 1.0), rq);
-        const double v = __builtin_fma(0.5 * y, rq, 0.5 * y) + ::log(q);
-        u = close ? v : u;
+    if constexpr (!FAR) {
+        const bool close = use && !(y <= 0.125);
+        if (__any(close)) {
+            const double q = s * rt;   // 1 - y, from s
+            double rq = __builtin_amdgcn_rcp(q);
+            rq = __builtin_fma(rq, __builtin_fma(-q, rq, 1.0), rq);
+            rq = __builtin_fma(rq, __builtin_fma(-q, rq, 1.0), rq);
+            const double v = __builtin_fma(0.5 * y, rq, 0.5 * y) + ::log(q);
+            u = close ? v : u;
+        }
     }
-    return -Ha / 6 * u;
+    return u;
 }
 
 // Sweep range of part h of SPLIT: off-diagonal tiles sweep s = 0..63; diagonal
@@ -399,13 +418,14 @@ __device__ __forceinline__ void tile_pass(const TileArgs& a, int tbase)
     }
     __syncthreads();
 
-    double ax = 0, ay = 0, az = 0, bx = 0, by = 0, bz = 0, pe = 0;
+    double ax = 0, ay = 0, az = 0, bx = 0, by = 0, bz = 0, pe = 0, pg = 0;
     unsigned long long any = 0;         // bit s: some lane met a near pair at step s
     if (live) {
         const JRec64* rec = &sj[tl][l];
         const double Ri4 = 4 * Ri;
         const double h_min = P.h_min;
         const double hmin2 = h_min * h_min, two_hmin = 2 * h_min;
+        const bool efar = WRITE && !test && energy_reach(a, I, J) <= 0x1p-5;
         int s0, s1;
         sweep_range<SPLIT>(diag, h, s0, s1);
         if (PREC == SL_PREC_MIXED && f32) {
@@ -468,7 +488,7 @@ __device__ __forceinline__ void tile_pass(const TileArgs& a, int tbase)
             const float r4i = 4.0f * (float)Ri * L0inv;
             float fax = 0.f, fay = 0.f, faz = 0.f, fbx = 0.f, fby = 0.f, fbz = 0.f;
             const JRecMix* recm = reinterpret_cast<const JRecMix*>(sj[tl]) + l;
-            auto pair = [&](int s, bool act, auto ntest) {
+            auto pair = [&](int s, bool act, auto ntest, auto efar) {
                 const JRecMix& r = recm[s];
                 const double dx = r.x - xi, dy = r.y - yi, dz = r.z - zi;
                 const double d2 = __builtin_fma(dz, dz, __builtin_fma(dy, dy, dx * dx));
@@ -504,29 +524,34 @@ __device__ __forceinline__ void tile_pass(const TileArgs& a, int tbase)
                 fbz = rot1(__builtin_fmaf(-f, dzf, fbz));
                 if (WRITE) {
                     const double tv = __builtin_fma(Ri4, r.R, sv);
-                    double u = far_energy(P.Ha, Ri, r.R, sv, tv, use);
-                    if (GRAV) u = u - (a.aux.g[i] * a.aux.g[J * TB + ((l + s) & (TB - 1))]) * rsq_f64(d2);
+                    const double u = far_energy<decltype(efar)::value>(Ri, r.R, sv, tv, use);
                     pe = use ? pe + u : pe;
+                    if (GRAV) {
+                        const double gg = a.aux.g[i] * a.aux.g[J * TB + ((l + s) & (TB - 1))];
+                        pg = use ? __builtin_fma(gg, rsq_f64(d2), pg) : pg;
+                    }
                 }
             };
-            auto sweep = [&](auto ntest) {
+            auto sweep = [&](auto ntest, auto efar) {
                 if (!diag) {
                     constexpr int NS = TB / SPLIT;
                     if constexpr (WRITE) {
-                        for (int k = 0; k < NS; k++) pair(s0 + k, true, ntest);
+                        for (int k = 0; k < NS; k++) pair(s0 + k, true, ntest, efar);
                     } else {
 #pragma unroll SL_TILE_UNROLL
-                        for (int k = 0; k < NS; k++) pair(s0 + k, true, ntest);
+                        for (int k = 0; k < NS; k++) pair(s0 + k, true, ntest, efar);
                     }
                 } else {
-                    for (int s = s0; s < s1 - 1; s++) pair(s, true, ntest);
-                    pair(s1 - 1, s1 - 1 < TB / 2 || l < TB / 2, ntest);
+                    for (int s = s0; s < s1 - 1; s++) pair(s, true, ntest, efar);
+                    pair(s1 - 1, s1 - 1 < TB / 2 || l < TB / 2, ntest, efar);
                 }
             };
             if (test)
-                sweep(std::true_type{});
-            else
-                sweep(std::false_type{});
+                sweep(std::true_type{}, std::false_type{});
+            else if (!efar)
+                sweep(std::false_type{}, std::false_type{});
+            else if constexpr (WRITE)
+                sweep(std::false_type{}, std::true_type{});
             const int back = (TB - (s1 & (TB - 1))) & (TB - 1);
             if (back) {
                 fbx = rotk(fbx, back);
@@ -544,7 +569,7 @@ __device__ __forceinline__ void tile_pass(const TileArgs& a, int tbase)
             // spheres of 1e-5 cm the largest share is 2^-33, at 40,000 2^-29).  The sweep at
             // 40,000 went from 1141 to 1020 us, at 5,000 from 28.6 to 27.5, of 96 uneven
             // systems of up to 4,500 from 225 to 207.
-            auto pair = [&](int s, bool act, auto ntest, auto raw) {
+            auto pair = [&](int s, bool act, auto ntest, auto raw, auto efar) {
                 const JRec64& r = rec[s];
                 const double dx = r.x - xi, dy = r.y - yi, dz = r.z - zi;
                 const double Rj = r.R;
@@ -577,34 +602,39 @@ __device__ __forceinline__ void tile_pass(const TileArgs& a, int tbase)
                 by = rot1(__builtin_fma(-f, dy, by));
                 bz = rot1(__builtin_fma(-f, dz, bz));
                 if (WRITE) {
-                    double u = far_energy(P.Ha, Ri, Rj, sv, tv, use);
-                    if (GRAV) u = u - (gi * r.g) * (decltype(raw)::value ? rsq_f64(d2) : rinv);
+                    const double u = far_energy<decltype(efar)::value>(Ri, Rj, sv, tv, use);
                     pe = use ? pe + u : pe;
+                    // (gravity's share of the energy is at most 6 times that of the force)
+                    if (GRAV) pg = use ? __builtin_fma(gi * r.g, rinv, pg) : pg;
                 }
             };
-            auto sweep = [&](auto ntest, auto raw) {
+            auto sweep = [&](auto ntest, auto raw, auto efar) {
                 if (!diag) {
                     constexpr int NS = TB / SPLIT;
                     if constexpr (WRITE) {
-                        for (int k = 0; k < NS; k++) pair(s0 + k, true, ntest, raw);
+                        for (int k = 0; k < NS; k++) pair(s0 + k, true, ntest, raw, efar);
                     } else {
 #pragma unroll SL_TILE_UNROLL
-                        for (int k = 0; k < NS; k++) pair(s0 + k, true, ntest, raw);
+                        for (int k = 0; k < NS; k++) pair(s0 + k, true, ntest, raw, efar);
                     }
                 } else {
-                    for (int s = s0; s < s1 - 1; s++) pair(s, true, ntest, raw);
-                    pair(s1 - 1, s1 - 1 < TB / 2 || l < TB / 2, ntest, raw);
+                    for (int s = s0; s < s1 - 1; s++) pair(s, true, ntest, raw, efar);
+                    pair(s1 - 1, s1 - 1 < TB / 2 || l < TB / 2, ntest, raw, efar);
                 }
             };
             const bool raw = GRAV && grav_share(a, I, J) < 0x1p-31;
-            if (raw && test)
-                sweep(std::true_type{}, std::true_type{});
-            else if (raw)
-                sweep(std::false_type{}, std::true_type{});
-            else if (test)
-                sweep(std::true_type{}, std::false_type{});
+            auto go = [&](auto rw) {
+                if (test)
+                    sweep(std::true_type{}, rw, std::false_type{});
+                else if (!efar)
+                    sweep(std::false_type{}, rw, std::false_type{});
+                else if constexpr (WRITE)
+                    sweep(std::false_type{}, rw, std::true_type{});
+            };
+            if (raw)
+                go(std::true_type{});
             else
-                sweep(std::false_type{}, std::false_type{});
+                go(std::false_type{});
             const int back = (TB - (s1 & (TB - 1))) & (TB - 1);
             if (back) {
                 bx = rotk(bx, back);
@@ -628,7 +658,7 @@ __device__ __forceinline__ void tile_pass(const TileArgs& a, int tbase)
             }
         }
         if (WRITE) {
-            const double ws = wave_sum(pe);
+            const double ws = wave_sum(-P.Ha / 6 * pe - pg);
             if (l == 0) pe_w[w] = ws;
         }
     }

@@ -1,0 +1,44 @@
+"""Potential energy across tiles whose pairs are all eleven radii apart or more, where the fast
+engine takes 11 terms of the series instead of 18 or the closed form: lattices of several blocks
+with spacings on both sides of that line, with and without gravity, against the sum in extended
+precision.
+
+Tolerance 1e-13: a term carries a few ulps of 1.1e-16, the terms left out are below 2^-52 of a
+pair, gravity's unrefined root (2^-24.4 of a share of at most 6 x 2^-31) below 2^-52, and the
+sum of at most 19,900 equal-signed terms in a tree of 64 adds fewer than 300 ulps (3.4e-14)."""
+import numpy as np
+import pytest
+
+import spacelab_amd as sl
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("precision", [sl.PREC_FP64, sl.PREC_MIXED])
+@pytest.mark.parametrize("spacing", [8.0, 11.0, 11.6, 12.4, 24.0, 60.0, 3000.0])
+@pytest.mark.parametrize("n,preset", [(65, "config"), (128, "reference"), (200, "config")])
+def test_far_tiles(n, preset, spacing, precision):
+    rng = np.random.default_rng(int(spacing * 10) + n)
+    side = 4     # 4 x 4 x n / 16: a block is a slab of 64
+    grid = np.stack([np.arange(n) % side, np.arange(n) // side % side, np.arange(n) // side ** 2], 1)
+    R = 1e-5 * rng.uniform(0.95, 1.05, n)
+    pos = spacing * 1e-5 * grid.astype(np.float64)
+    m = 2.25 * 4 / 3 * np.pi * R ** 3
+    zero = np.zeros((n, 3))
+    p = sl.calibrate(sl.preset(preset), R, m, velocity=0.36, cor=0.64).replace(order=sl.ORDER_FAST, precision=precision)
+    with sl.Collider(n, p) as c:
+        c.upload(sl.BallGroup(pos, zero, zero.copy(), R, m, 0.4 * m * R * R))
+        e = c.init_conditions()
+        split = c.get_option("tile_split")
+    L = np.longdouble
+    x, r, mm = pos.astype(L), R.astype(L), m.astype(L)
+    i, j = np.tril_indices(n, -1)
+    d2 = ((x[i] - x[j]) ** 2).sum(1)
+    y = 4 * r[i] * r[j] / (d2 - (r[i] - r[j]) ** 2)
+    u = sum((L(0.5) - L(1) / k) * y ** k for k in range(3, 90))
+    want = -L(p.Ha) / 6 * u
+    if p.far_gravity:
+        want = want - L(p.G) * mm[i] * mm[j] / np.sqrt(d2)
+    want = float(want.sum())
+    assert e.contacts == 0 and split >= 0
+    assert abs(e.PE - want) <= 1e-13 * abs(want)
