@@ -148,7 +148,7 @@ void sl_destroy(sl_ctx* ctx);
 #define SL_OPT_TILE_SPLIT 2
 #define SL_OPT_BALL_WAVES 3
 /*   SL_OPT_ORDERED_SHAPE launch shape of the SL_ORDER_ORDERED pair pass (balls per
- *                      workgroup, evaluating wavefronts, partners per chunk): 0 (default)
+ *                      workgroup, wavefronts, evaluation steps per batch): 0 (default)
  *                      = chosen by timing each shape on the first step and stored with
  *                      the tile splits, or 1..n to force one.  Every shape gives the same
  *                      results bit for bit.  sl_get_option reports the shape in use (0

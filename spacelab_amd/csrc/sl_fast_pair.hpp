@@ -44,4 +44,42 @@ __device__ __forceinline__ double rsq_f64(double x)
     return __builtin_fma(y, e, y);
 }
 
+// vdW energy of a far pair over -Ha/6, from s = d^2 - S^2, t = d^2 - (Ri-Rj)^2 (use: the lane's
+// pair counts).  With y = 4 Ri Rj / t the reference's sum 2RiRj/s + 2RiRj/t + ln(s/t) is
+// y/2/(1-y) + y/2 + ln(1-y) = sum over k >= 3 of (1/2 - 1/k) y^k: its first two orders
+// cancel, so for y <= 1/8 (about three diameters apart and more: nearly every pair) 18 terms
+// of the series give it to 2^-52, for 23 instructions, where the three divisions and the
+// logarithm took about 75 and lost 6 / y^2 ulps.  (With the line at y = 1/16, 13 terms, the
+// closed form's loss just above it was 2e-13 of a pair, and the sweep was no faster.)
+// FAR: y <= 2^-5 for every pair of the tile (eleven radii apart), so 11 terms do (the first left
+// out is 2.6 y^11 of the sum, 2^-53.6) and no lane needs the closed form.
+// The write step's sweep at 40,000 spheres took 4557 us in the closed form, 2205 by 18 terms
+// and 1890 with the short series (without energies: 1020); at 5,000 87, 55 and 54.
+template <bool FAR>
+__device__ __forceinline__ double far_energy(double Ri, double Rj, double s, double t, bool use)
+{
+    const double two = 2 * Ri * Rj;
+    double rt = __builtin_amdgcn_rcp(t);
+    rt = __builtin_fma(rt, __builtin_fma(-t, rt, 1.0), rt);
+    rt = __builtin_fma(rt, __builtin_fma(-t, rt, 1.0), rt);
+    const double y = 2 * two * rt;
+    constexpr int LAST = FAR ? 13 : 20;
+    double p = 0.5 - 1.0 / LAST;
+#pragma unroll
+    for (int k = LAST - 1; k >= 3; k--) p = __builtin_fma(p, y, 0.5 - 1.0 / k);
+    double u = p * (y * y * y);
+    if constexpr (!FAR) {
+        const bool close = use && !(y <= 0.125);
+        if (__any(close)) {
+            const double q = s * rt;   // 1 - y, from s
+            double rq = __builtin_amdgcn_rcp(q);
+            rq = __builtin_fma(rq, __builtin_fma(-q, rq, 1.0), rq);
+            rq = __builtin_fma(rq, __builtin_fma(-q, rq, 1.0), rq);
+            const double v = __builtin_fma(0.5 * y, rq, 0.5 * y) + ::log(q);
+            u = close ? v : u;
+        }
+    }
+    return u;
+}
+
 }  // namespace sl

@@ -15,6 +15,7 @@
 // over A in ascending order by the caller: the same for every launch shape, but grouped
 // per ball rather than the reference's single running sum, so it agrees to rounding only.
 #include "sl_common.hpp"
+#include "sl_fast_pair.hpp"
 #include "sl_pair_ref.hpp"
 
 #include <type_traits>
@@ -177,6 +178,10 @@ struct PartnerRec {
 // sums by a wavefront of its own, the kick in a launch of its own) and now: 129 balls 16.5 ->
 // 9 us, 1,000 29 -> 19, 2,200 87 -> 57, 5,000 259 -> 161, 15,039 1,750 -> 1,095.
 //
+// Write steps take a far pair's energy from far_energy's series (the logarithm and two
+// divisions cost two thirds of a step more, and spilled up to 72 registers) and two wavefronts
+// per SIMD: 15,039 balls 1,894 -> 1,584-1,720 us, 5,000 269 -> 238.
+//
 // With a second set of arrays (os.nxt) the owner of the last batch also kicks its balls and,
 // with os.drift, drifts them into the next step (the operations of k_kick and k_drift): one
 // launch a step instead of two.  The other workgroups may still be reading this step's positions and
@@ -191,7 +196,7 @@ struct OrdState {
 };
 
 template <int NB, int CH, int W, int AD, int WPE, int UNR, bool SCAN, bool WRITE>
-__global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(WPE)))
+__global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(WRITE && WPE > 2 ? 2 : WPE)))
 void k_pairs_ordered(OrdState os, Phys P, int n, double* __restrict__ pe_ball,
                      unsigned long long* __restrict__ contacts)
 {
@@ -389,8 +394,8 @@ void k_pairs_ordered(OrdState os, Phys P, int n, double* __restrict__ pe_ball,
             double c0 = div_rcp(F.x, mi, ymi), c1 = div_rcp(F.y, mi, ymi), c2 = div_rcp(F.z, mi, ymi);
             double u = 0;
             if (WRITE && IA) {                                 // :228-240
-                u = vdw_energy(P.Ha, Ri, Rj, S, h);
-                if (P.far_gravity) u = u + -P.G * mi * mj / dist;
+                u = -P.Ha / 6 * far_energy<false>(Ri, Rj, sv, tv, pair && !(overlap > 0));
+                if (P.far_gravity) u = u + div_rcp(-P.G * mi * mj, dist, yd);
             }
             if (CHK && !pair) c0 = c1 = c2 = u = 0;            // no partner, or the ball itself
             const int o_ = il * RS + jl;

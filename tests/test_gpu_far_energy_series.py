@@ -42,3 +42,32 @@ def test_far_tiles(n, preset, spacing, precision):
     want = float(want.sum())
     assert e.contacts == 0 and split >= 0
     assert abs(e.PE - want) <= 1e-13 * abs(want)
+
+
+@pytest.mark.parametrize("shape", [0, 2, 4, 8])
+@pytest.mark.parametrize("spacing", [2.3, 5.4, 5.9, 12.0, 400.0])
+def test_ordered_far_pairs(spacing, shape):
+    """The ordered pass takes the same series for its far pairs (per-ball sums of at most 130
+    terms, then over 130 balls: fewer than 300 ulps again; below y = 0.4 the series above)."""
+    n = 130
+    rng = np.random.default_rng(int(spacing * 10))
+    grid = np.stack([np.arange(n) % 5, np.arange(n) // 5 % 5, np.arange(n) // 25], 1)
+    R = 1e-5 * rng.uniform(0.95, 1.05, n)
+    pos = spacing * 1e-5 * grid.astype(np.float64)
+    m = 2.25 * 4 / 3 * np.pi * R ** 3
+    zero = np.zeros((n, 3))
+    p = sl.calibrate(sl.preset("config"), R, m, velocity=0.36, cor=0.64)
+    with sl.Collider(n, p) as c:
+        c.set_option("ordered_shape", shape)
+        c.upload(sl.BallGroup(pos, zero, zero.copy(), R, m, 0.4 * m * R * R))
+        e = c.init_conditions()
+    L = np.longdouble
+    x, r, mm = pos.astype(L), R.astype(L), m.astype(L)
+    i, j = np.tril_indices(n, -1)
+    d2 = ((x[i] - x[j]) ** 2).sum(1)
+    y = 4 * r[i] * r[j] / (d2 - (r[i] - r[j]) ** 2)
+    small = np.minimum(y, L(0.4))
+    u = np.where(y < 0.4, sum((L(0.5) - L(1) / k) * small ** k for k in range(3, 90)), y / 2 / (1 - y) + y / 2 + np.log1p(-y))
+    want = float((-L(p.Ha) / 6 * u - p.far_gravity * L(p.G) * mm[i] * mm[j] / np.sqrt(d2)).sum())
+    assert e.contacts == 0
+    assert abs(e.PE - want) <= 1e-13 * abs(want)
