@@ -55,29 +55,34 @@ __device__ __forceinline__ double rsq_f64(double x)
 // out is 2.6 y^11 of the sum, 2^-53.6) and no lane needs the closed form.
 // The write step's sweep at 40,000 spheres took 4557 us in the closed form, 2205 by 18 terms
 // and 1890 with the short series (without energies: 1020); at 5,000 87, 55 and 54.
-template <bool FAR>
-__device__ __forceinline__ double far_energy(double Ri, double Rj, double s, double t, bool use)
+// energy_series: the sum to the term LAST, y and 1/t.
+template <int LAST>
+__device__ __forceinline__ double energy_series(double Ri, double Rj, double t, double& y, double& rt)
 {
-    const double two = 2 * Ri * Rj;
-    double rt = __builtin_amdgcn_rcp(t);
+    rt = __builtin_amdgcn_rcp(t);
     rt = __builtin_fma(rt, __builtin_fma(-t, rt, 1.0), rt);
     rt = __builtin_fma(rt, __builtin_fma(-t, rt, 1.0), rt);
-    const double y = 2 * two * rt;
-    constexpr int LAST = FAR ? 13 : 20;
+    y = 4 * Ri * Rj * rt;
     double p = 0.5 - 1.0 / LAST;
 #pragma unroll
     for (int k = LAST - 1; k >= 3; k--) p = __builtin_fma(p, y, 0.5 - 1.0 / k);
-    double u = p * (y * y * y);
-    if constexpr (!FAR) {
-        const bool close = use && !(y <= 0.125);
-        if (__any(close)) {
-            const double q = s * rt;   // 1 - y, from s
-            double rq = __builtin_amdgcn_rcp(q);
-            rq = __builtin_fma(rq, __builtin_fma(-q, rq, 1.0), rq);
-            rq = __builtin_fma(rq, __builtin_fma(-q, rq, 1.0), rq);
-            const double v = __builtin_fma(0.5 * y, rq, 0.5 * y) + ::log(q);
-            u = close ? v : u;
-        }
+    return p * (y * y * y);
+}
+
+template <bool FAR>
+__device__ __forceinline__ double far_energy(double Ri, double Rj, double s, double t, bool use)
+{
+    double y, rt;
+    if constexpr (FAR) return energy_series<13>(Ri, Rj, t, y, rt);
+    double u = energy_series<20>(Ri, Rj, t, y, rt);
+    const bool close = use && !(y <= 0.125);
+    if (__any(close)) {
+        const double q = s * rt;   // 1 - y, from s
+        double rq = __builtin_amdgcn_rcp(q);
+        rq = __builtin_fma(rq, __builtin_fma(-q, rq, 1.0), rq);
+        rq = __builtin_fma(rq, __builtin_fma(-q, rq, 1.0), rq);
+        const double v = __builtin_fma(0.5 * y, rq, 0.5 * y) + ::log(q);
+        u = close ? v : u;
     }
     return u;
 }

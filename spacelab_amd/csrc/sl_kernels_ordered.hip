@@ -178,7 +178,7 @@ struct PartnerRec {
 // sums by a wavefront of its own, the kick in a launch of its own) and now: 129 balls 16.5 ->
 // 9 us, 1,000 29 -> 19, 2,200 87 -> 57, 5,000 259 -> 161, 15,039 1,750 -> 1,095.
 //
-// Write steps take a far pair's energy from far_energy's series (the logarithm and two
+// Write steps take a far pair's energy from the series (y <= 1/8; the logarithm and three
 // divisions cost two thirds of a step more, and spilled up to 72 registers) and two wavefronts
 // per SIMD: 15,039 balls 1,894 -> 1,584-1,720 us, 5,000 269 -> 238.
 //
@@ -394,7 +394,13 @@ void k_pairs_ordered(OrdState os, Phys P, int n, double* __restrict__ pe_ball,
             double c0 = div_rcp(F.x, mi, ymi), c1 = div_rcp(F.y, mi, ymi), c2 = div_rcp(F.z, mi, ymi);
             double u = 0;
             if (WRITE && IA) {                                 // :228-240
-                u = -P.Ha / 6 * far_energy<false>(Ri, Rj, sv, tv, pair && !(overlap > 0));
+                double y, rt;
+                u = -P.Ha / 6 * energy_series<20>(Ri, Rj, tv, y, rt);
+                const bool close = pair && !(y <= 0.125);
+                if (__any(close)) {
+                    const double v = vdw_energy(P.Ha, Ri, Rj, S, h);
+                    u = close ? v : u;
+                }
                 if (P.far_gravity) u = u + div_rcp(-P.G * mi * mj, dist, yd);
             }
             if (CHK && !pair) c0 = c1 = c2 = u = 0;            // no partner, or the ball itself
