@@ -121,7 +121,8 @@ struct TileArgs {
     unsigned char* near;    // per 64-ball block and slot (near_stride apart): the slot's masks have a bit
                             // set (NULL: every mask is written)
     int near_stride;
-    double* pe_tile;        // per tile: far-field pair energy (write steps)
+    double* pe_row;         // write steps: far-field energy of tile (I, J) at 64-ball block I's row
+    int pe_stride;          // (pe_stride apart), slot J
     int* queue;             // k_tiles_q: next group per segment, workgroups done (all 0 between launches)
 };
 
@@ -677,7 +678,7 @@ __device__ __forceinline__ void tile_pass(const TileArgs& a, int tbase)
     if (WRITE && l == 0) {
         double pt = pe_w[w0];
         for (int q = 1; q < SPLIT; q++) pt = pt + pe_w[w0 + q];
-        a.pe_tile[t] = pt;
+        a.pe_row[(size_t)I * a.pe_stride + si] = pt;
     }
 }
 
@@ -809,6 +810,8 @@ struct BallArgs {
     double4* bnd;       // per 64-ball block: bounding box of the drifted positions (lo, hi)
     float4* xl;         // per ball: drifted position relative to its block's box centre, R (units of L0)
     double L0inv;
+    const double* pe_row;   // write steps: far-field energies of the block's tiles, as in TileArgs
+    int pe_stride;
     double* e_blk;      // FAST_E_STRIDE doubles per 64-ball block (write steps)
     unsigned long long* blk_ctr;   // per 64-ball block: running sums of touching and near pairs
     int* flags;         // [1]: a non-finite state appeared
@@ -857,6 +860,10 @@ constexpr int kb_threads(int nwv) { return nwv * TB; }
 // behind the pairs took it from 12.6 to 9.4 us at 1,000 spheres, from 13.2 to 11.2 at 5,000
 // (mixed 12.6 to 10.8), from 40 to 32 for 512 systems of 33 to 550 and from 56 to 49 for 96 of
 // 200 to 4,500.
+//
+// Write steps: the far-field energies of the block's tiles are added here, lane l those of slots
+// l, l + 64, ... and then the lanes as a tree, so that a step brings ten values per block to
+// the host (at 40,000 spheres, 195,625 tiles' energies copied and added there took 1 ms).
 //
 // NEARF, for systems of more than KB_BATCH slots: the masks of slots without near pairs, nine
 // in ten of a large system's, are neither written nor read (200 of 800 bytes a ball and slot
@@ -908,6 +915,7 @@ __global__ __launch_bounds__(kb_threads(NWV)) void k_ball(BallArgs a)
     // what this wavefront's components need of the balls' own state goes out first
     double x0[QW], h0[QW], inr[QW], Rb = 0;
     unsigned long long ctr0 = 0, ctr1 = 0;
+    double far_pe = 0;   // lane l: slots l, l + 64, ... of the block's row of far-field energies
 #pragma unroll
     for (int u = 0; u < QW; u++) {
         const int q = w + u * NWV;
@@ -921,9 +929,13 @@ __global__ __launch_bounds__(kb_threads(NWV)) void k_ball(BallArgs a)
             h0[u] = c.at(GX + q - 3, ic);
             inr[u] = c.c(MOI, ic);
             if (q == 3) Rb = c.c(RAD, ic);
-        } else if (q == 6 && l == 0) {
-            ctr0 = a.blk_ctr[2 * blockIdx.x];
-            ctr1 = a.blk_ctr[2 * blockIdx.x + 1];
+        } else if (q == 6) {
+            if (l == 0) {
+                ctr0 = a.blk_ctr[2 * blockIdx.x];
+                ctr1 = a.blk_ctr[2 * blockIdx.x + 1];
+            }
+            if (WRITE)
+                for (int J = l; J <= (int)blockIdx.x - off / TB; J += TB) far_pe = far_pe + a.pe_row[(size_t)blockIdx.x * a.pe_stride + J];
         }
     }
 
@@ -1106,8 +1118,8 @@ __global__ __launch_bounds__(kb_threads(NWV)) void k_ball(BallArgs a)
         const int q = w + u * NWV;
         if (q >= 6) {
             if (q == 6) {
-                // the block's near-pair energy and pair counts (each pair counted by its ball A)
-                const double bpe = WRITE ? wave_sum(npe) : 0.0;
+                // the block's pair energy and pair counts (each pair counted by its ball A)
+                const double bpe = WRITE ? wave_sum(far_pe) + wave_sum(npe) : 0.0;
                 const int bcc = wave_isum(ncon), bcn = wave_isum(npair);
                 if (l == 0) {
                     a.blk_ctr[2 * blockIdx.x] = ctr0 + (unsigned long long)bcc;
@@ -1210,17 +1222,41 @@ __global__ __launch_bounds__(kb_threads(NWV)) void k_ball(BallArgs a)
 }
 
 // Bounding boxes of the 64-ball blocks (one wavefront per block), for positions that
-// did not come from k_ball's drift.
-__global__ __launch_bounds__(TB) void k_bounds(State s, const int* blk_sys, const int* sys_off, const int* sys_n,
-                                               double4* bnd, float4* xl, double L0inv)
+// did not come from k_ball's drift; DRIFT: after drifting the valid balls (each system with
+// its own dt), the start of a call.
+template <bool DRIFT>
+__global__ __launch_bounds__(TB) void k_bounds(State s, const int4* blk_info, const Phys* sysP, double4* bnd, float4* xl,
+                                               double L0inv)
 {
     const int l = threadIdx.x;
     const int b = blockIdx.x * TB + l;
-    const int sy = blk_sys[blockIdx.x];
-    const bool valid = b - sys_off[sy] < sys_n[sy];
-    const int bc = valid ? b : sys_off[sy];
+    const int4 bi = blk_info[blockIdx.x];
+    const bool valid = b - bi.x < bi.y;
+    const int bc = valid ? b : bi.x;
+    double x = s.f[PX][bc], y = s.f[PY][bc], z = s.f[PZ][bc];
+    const double R = s.f[RAD][bc];
+    if (DRIFT && valid) {
+        const double dt = sysP[bi.w].dt;
+        s.f[QX][b] = x;
+        s.f[QY][b] = y;
+        s.f[QZ][b] = z;
+        const double hx = s.f[VX][b] + .5 * s.f[AX][b] * dt;
+        const double hy = s.f[VY][b] + .5 * s.f[AY][b] * dt;
+        const double hz = s.f[VZ][b] + .5 * s.f[AZ][b] * dt;
+        s.f[HX][b] = hx;
+        s.f[HY][b] = hy;
+        s.f[HZ][b] = hz;
+        s.f[GX][b] = s.f[WX][b] + .5 * s.f[BX][b] * dt;
+        s.f[GY][b] = s.f[WY][b] + .5 * s.f[BY][b] * dt;
+        s.f[GZ][b] = s.f[WZ][b] + .5 * s.f[BZ][b] * dt;
+        x = x + hx * dt;
+        y = y + hy * dt;
+        z = z + hz * dt;
+        s.f[PX][b] = x;
+        s.f[PY][b] = y;
+        s.f[PZ][b] = z;
+    }
     double4 lo, hi;
-    const double x = s.f[PX][bc], y = s.f[PY][bc], z = s.f[PZ][bc], R = s.f[RAD][bc];
     wave_aabb(x, y, z, R, valid, lo, hi);
     if (l == 0) {
         bnd[2 * blockIdx.x] = lo;
@@ -1228,33 +1264,6 @@ __global__ __launch_bounds__(TB) void k_bounds(State s, const int* blk_sys, cons
     }
     xl[b] = make_float4(local_coord(x, valid, lo.x, hi.x, L0inv, l), local_coord(y, valid, lo.y, hi.y, L0inv, 0),
                         local_coord(z, valid, lo.z, hi.z, L0inv, 0), valid ? (float)(R * L0inv) : 0.f);
-}
-
-// Start-of-call drift of the valid balls (each system with its own dt).
-__global__ void k_drift_sys(State s, const int* blk_sys, const int* sys_off, const int* sys_n,
-                            const Phys* sysP, int n_used)
-{
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= n_used) return;
-    const int sy = blk_sys[b / TB];
-    if (b - sys_off[sy] >= sys_n[sy]) return;
-    const double dt = sysP[sy].dt;
-    const double px = s.f[PX][b], py = s.f[PY][b], pz = s.f[PZ][b];
-    s.f[QX][b] = px;
-    s.f[QY][b] = py;
-    s.f[QZ][b] = pz;
-    const double hx = s.f[VX][b] + .5 * s.f[AX][b] * dt;
-    const double hy = s.f[VY][b] + .5 * s.f[AY][b] * dt;
-    const double hz = s.f[VZ][b] + .5 * s.f[AZ][b] * dt;
-    s.f[HX][b] = hx;
-    s.f[HY][b] = hy;
-    s.f[HZ][b] = hz;
-    s.f[GX][b] = s.f[WX][b] + .5 * s.f[BX][b] * dt;
-    s.f[GY][b] = s.f[WY][b] + .5 * s.f[BY][b] * dt;
-    s.f[GZ][b] = s.f[WZ][b] + .5 * s.f[BZ][b] * dt;
-    s.f[PX][b] = px + hx * dt;
-    s.f[PY][b] = py + hy * dt;
-    s.f[PZ][b] = pz + hz * dt;
 }
 
 }  // namespace fastk

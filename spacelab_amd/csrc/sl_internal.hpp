@@ -71,7 +71,6 @@ struct FastBuffers {
     FastLayout lay;
     std::vector<Phys> P;          // per system
     std::vector<int> blk_sys_h;   // per 64-ball block: system (host copy)
-    std::vector<int> tile_sys_h;  // per tile: system (host copy)
     // The engine keeps its own two state sets (ping-pong), with each system's balls
     // in Morton order of their positions at configuration, so that the 64-ball blocks
     // are compact in space: most tiles then have no near pair.  perm maps engine slot
@@ -105,10 +104,9 @@ struct FastBuffers {
     int* flags = nullptr;         // [1] non-finite state
     unsigned long long* blk_ctr = nullptr;    // per 64-ball block: touching and near pairs (running sums)
     int cap_blocks = 0;
-    double* e_blk = nullptr;      // per 64-ball block: near-pair PE, KE, p, L, contacts, nonfinite
-    double* pe_tile = nullptr;    // per tile: pair energy (write steps)
-    double* h_e_blk = nullptr;    // pinned host copies
-    double* h_pe_tile = nullptr;
+    double* pe_row = nullptr;     // per 64-ball block and slot J (part_slots apart): tile's far-field energy (write steps)
+    double* e_blk = nullptr;      // per 64-ball block: PE, KE, p, L, contacts, nonfinite
+    double* h_e_blk = nullptr;    // pinned host copy
     int precision = 0;
     int split = 0;                // wavefronts per 64x64 tile (0: not tuned yet)
     bool queue_launch = false;    // tiles from the work queue (k_tiles_q) rather than one per workgroup

@@ -206,7 +206,8 @@ TileArgs tile_args(FastBuffers& fb)
     a.nbm = fb.nbm;
     a.near = near_flags(fb) ? fb.near : nullptr;
     a.near_stride = fb.part_slots;
-    a.pe_tile = fb.pe_tile;
+    a.pe_row = fb.pe_row;
+    a.pe_stride = fb.part_slots;
     a.queue = fb.queue;
     return a;
 }
@@ -316,6 +317,8 @@ int launch_ball_step(FastBuffers& fb, bool write, bool kick, bool drift_next, hi
     a.bnd = fb.bnd;
     a.xl = fb.xl;
     a.L0inv = 1.0 / fb.L0;
+    a.pe_row = fb.pe_row;
+    a.pe_stride = fb.part_slots;
     a.e_blk = fb.e_blk;
     a.blk_ctr = fb.blk_ctr;
     a.flags = fb.flags;
@@ -345,37 +348,26 @@ int launch_ball_step(FastBuffers& fb, bool write, bool kick, bool drift_next, hi
     return 0;
 }
 
-int launch_bounds(FastBuffers& fb, hipStream_t st, std::string* err)
+int launch_bounds(FastBuffers& fb, bool drift, hipStream_t st, std::string* err)
 {
-    k_bounds<<<fb.lay.n_used / TB, TB, 0, st>>>(fb.eng[fb.cur], fb.blk_sys, fb.sys_off, fb.sys_n, fb.bnd, fb.xl,
-                                                1.0 / fb.L0);
-    if (hipGetLastError() != hipSuccess) return err_hip(err, "block bounds");
+    const auto k = drift ? &k_bounds<true> : &k_bounds<false>;
+    k<<<fb.lay.n_used / TB, TB, 0, st>>>(fb.eng[fb.cur], fb.blk_info, fb.sysP, fb.bnd, fb.xl, 1.0 / fb.L0);
+    if (hipGetLastError() != hipSuccess) return err_hip(err, drift ? "drift" : "block bounds");
     return 0;
 }
 
-int launch_drift_sys(FastBuffers& fb, hipStream_t st, std::string* err)
-{
-    k_drift_sys<<<(fb.lay.n_used + 255) / 256, 256, 0, st>>>(fb.eng[fb.cur], fb.blk_sys, fb.sys_off, fb.sys_n,
-                                                             fb.sysP, fb.lay.n_used);
-    if (hipGetLastError() != hipSuccess) return err_hip(err, "drift");
-    return launch_bounds(fb, st, err);
-}
-
-// Read back the partials of a write step and sum them per system, in a fixed order:
-// the far-field energy of the tiles in table order, then the near-pair energy,
-// kinetic energy, momenta and contacts of the 64-ball blocks in ascending order.
+// Read back the partials of a write step and sum them per system, in a fixed order: the pair
+// energy, kinetic energy, momenta and contacts of the 64-ball blocks in ascending order.
 int read_energies(FastBuffers& fb, sl_energy* out, hipStream_t st, std::string* err)
 {
     const int nblk = fb.lay.n_used / BPB;
-    if (hipMemcpyAsync(fb.h_pe_tile, fb.pe_tile, sizeof(double) * fb.n_tiles, hipMemcpyDeviceToHost, st) != hipSuccess ||
-        hipMemcpyAsync(fb.h_e_blk, fb.e_blk, sizeof(double) * FAST_E_STRIDE * nblk, hipMemcpyDeviceToHost, st) !=
+    if (hipMemcpyAsync(fb.h_e_blk, fb.e_blk, sizeof(double) * FAST_E_STRIDE * nblk, hipMemcpyDeviceToHost, st) !=
             hipSuccess ||
         hipStreamSynchronize(st) != hipSuccess)
         return err_hip(err, "energy read-back");
     const int ns = fb.lay.n_sys;
     std::vector<sl_energy> e(ns);
     for (auto& x : e) x = sl_energy{};
-    for (int t = 0; t < fb.n_tiles; t++) e[fb.tile_sys_h[t]].PE += fb.h_pe_tile[t];
     for (int b = 0; b < nblk; b++) {
         const int s = fb.blk_sys_h[(b * BPB) / TB];
         const double* v = fb.h_e_blk + (size_t)b * FAST_E_STRIDE;
@@ -400,7 +392,7 @@ int read_energies(FastBuffers& fb, sl_energy* out, hipStream_t st, std::string* 
 int direct_step(FastBuffers& fb, bool write, bool drift_next, hipStream_t st, std::string* err)
 {
     int rc;
-    if (!fb.drifted && (rc = launch_drift_sys(fb, st, err))) return rc;
+    if (!fb.drifted && (rc = launch_bounds(fb, true, st, err))) return rc;
     fb.drifted = false;
     if ((rc = launch_tiles_step(fb, write, st, err))) return rc;
     return launch_ball_step(fb, write, true, drift_next, st, err);
@@ -618,11 +610,10 @@ void fast_free(FastBuffers& fb)
     fast_clear_graphs(fb);
     void* ptrs[] = {fb.eng_base, fb.perm, fb.aux.q, fb.aux.g, fb.aux.q32, fb.aux.g32, fb.bnd, fb.xl, fb.gq_blk, fb.queue, fb.blk_sys, fb.blk_info,
                     fb.sys_off, fb.sys_n, fb.sys_first, fb.sysP, fb.tiles, fb.part, fb.nbm, fb.near, fb.flags,
-                    fb.blk_ctr, fb.e_blk, fb.pe_tile};
+                    fb.blk_ctr, fb.e_blk, fb.pe_row};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     if (fb.h_e_blk) (void)hipHostFree(fb.h_e_blk);
-    if (fb.h_pe_tile) (void)hipHostFree(fb.h_pe_tile);
     fb = FastBuffers{};
 }
 
@@ -687,7 +678,6 @@ int fast_configure(FastBuffers& fb, State& canon, const FastLayout& lay, const P
         const int nblocks = lay.n_used / TB;
         fb.blk_sys_h.assign(std::max(nblocks, 1), 0);
         std::vector<int4> tiles;
-        fb.tile_sys_h.clear();
         // The diagonal tiles of every system first (half a sweep each, and most of the
         // per-pair near tests), then the others by band, I - J = 1, 2, ...: blocks close in
         // the space-filling-curve order are close in space, so the tiles that need the
@@ -706,7 +696,6 @@ int fast_configure(FastBuffers& fb, State& canon, const FastLayout& lay, const P
                 const int b0 = lay.off[s] / TB;
                 for (int I = d; I < lay.nb[s]; I++) {
                     tiles.push_back(make_int4(b0 + I, b0 + I - d, s, b0));
-                    fb.tile_sys_h.push_back(s);
                 }
             }
         std::vector<int4> info;
@@ -714,15 +703,9 @@ int fast_configure(FastBuffers& fb, State& canon, const FastLayout& lay, const P
         const int nt = (int)tiles.size();
         if (nt > fb.cap_tiles) {
             if (fb.tiles) (void)hipFree(fb.tiles);
-            if (fb.pe_tile) (void)hipFree(fb.pe_tile);
-            if (fb.h_pe_tile) (void)hipHostFree(fb.h_pe_tile);
             fb.tiles = nullptr;
-            fb.pe_tile = nullptr;
-            fb.h_pe_tile = nullptr;
             fb.cap_tiles = 0;
-            if (hipMalloc(&fb.tiles, sizeof(int4) * nt) != hipSuccess ||
-                hipMalloc(&fb.pe_tile, sizeof(double) * nt) != hipSuccess ||
-                hipHostMalloc(&fb.h_pe_tile, sizeof(double) * nt, 0) != hipSuccess)
+            if (hipMalloc(&fb.tiles, sizeof(int4) * nt) != hipSuccess)
                 return err_hip(err, "tile table allocation");
             fb.cap_tiles = nt;
         }
@@ -730,13 +713,16 @@ int fast_configure(FastBuffers& fb, State& canon, const FastLayout& lay, const P
             if (fb.part) (void)hipFree(fb.part);
             if (fb.nbm) (void)hipFree(fb.nbm);
             if (fb.near) (void)hipFree(fb.near);
+            if (fb.pe_row) (void)hipFree(fb.pe_row);
             fb.part = nullptr;
             fb.nbm = nullptr;
             fb.near = nullptr;
+            fb.pe_row = nullptr;
             fb.part_slots = 0;
             if (hipMalloc(&fb.part, sizeof(double) * (size_t)lay.nb_max * 3 * fb.n_pad) != hipSuccess ||
                 hipMalloc(&fb.nbm, sizeof(unsigned long long) * (size_t)lay.nb_max * fb.n_pad) != hipSuccess ||
-                hipMalloc(&fb.near, (size_t)lay.nb_max * fb.cap_blocks) != hipSuccess)
+                hipMalloc(&fb.near, (size_t)lay.nb_max * fb.cap_blocks) != hipSuccess ||
+                hipMalloc(&fb.pe_row, sizeof(double) * (size_t)lay.nb_max * fb.cap_blocks) != hipSuccess)
                 return err_hip(err, "partial buffer allocation");
             fb.part_slots = lay.nb_max;
         }
@@ -810,7 +796,7 @@ int fast_init(FastBuffers& fb, State& canon, sl_energy* e_sys, hipStream_t st, s
     if (launch_copy_prev(fb.eng[fb.cur], fb.lay.n_used, st) != hipSuccess) return err_hip(err, "copy positions");
     fb.drifted = false;
     fb.canon_valid = false;
-    rc = launch_bounds(fb, st, err);
+    rc = launch_bounds(fb, false, st, err);
     if (!rc) rc = launch_tiles_step(fb, true, st, err);
     if (!rc) rc = launch_ball_step(fb, true, false, false, st, err);
     if (!rc) rc = read_energies(fb, e_sys, st, err);
