@@ -373,6 +373,13 @@ int sl_mlp_train_rows(sl_mlp* const* nets, int n, int batch, long long n_rows, c
                       const float* reg, const long long* idx, float lr, float* loss);
 /* sl_mlp_forward of several nets (same n_in and n_out) on the same rows; outputs net after net. */
 int sl_mlp_forward_all(sl_mlp* const* nets, int n, int batch, const float* x, float* y, float* prob, float* ent);
+/* What the nets say together of any number of rows of binary64 inputs, each first brought to
+ * (x - mean) / std in binary32: prob, the mean of their class probabilities, and reg, of their
+ * regression outputs (sums in binary64, net after net); cls, the most probable class; ent, the
+ * entropy (nats) of prob.  SL_E_STATE where the nets cannot share launches (more than 16, or
+ * of different widths or max_batch, or wider than 512). */
+int sl_mlp_ensemble(sl_mlp* const* nets, int n, long long rows, const double* x, const double* mean, const double* std,
+                    int* cls, float* reg, double* prob, double* ent);
 const char* sl_mlp_last_error(const sl_mlp* m);   /* calls on several nets: of the net it fails on or the first */
 void sl_mlp_destroy(sl_mlp* m);
 

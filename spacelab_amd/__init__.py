@@ -218,6 +218,7 @@ def lib():
     mlps, llp = C.POINTER(vp), C.POINTER(C.c_longlong)
     L.sl_mlp_train_rows.argtypes = [mlps, C.c_int, C.c_int, C.c_longlong, fp, ip, fp, llp, C.c_float, fp]
     L.sl_mlp_forward_all.argtypes = [mlps, C.c_int, C.c_int, fp, fp, fp, fp]
+    L.sl_mlp_ensemble.argtypes = [mlps, C.c_int, C.c_longlong, dp, dp, dp, ip, fp, dp, dp]
     L.sl_mlp_last_error.argtypes = [vp]
     L.sl_mlp_last_error.restype = C.c_char_p
     L.sl_mlp_destroy.argtypes = [vp]
@@ -801,9 +802,35 @@ def _mlp_call(mlps: list[MLP], what: str, *args):
         raise SpacelabError(rc, f"{what}: {msg.decode()}")
 
 
+def mlp_alike(mlps: list[MLP]) -> bool:
+    """Whether the nets share launches: up to 16 different ones, of the same widths and largest
+    batch, no layer wider than 512."""
+    if any(type(m) is not MLP for m in mlps):
+        return False
+    sizes = {(m.n_in, m.width, m.n_out, m.max_batch) for m in mlps}
+    return 1 <= len({id(m) for m in mlps}) == len(mlps) <= 16 and len(sizes) == 1 and max(next(iter(sizes))[:3]) <= 512
+
+
+def mlp_ensemble(mlps: list[MLP], x, mean, std):
+    """(class, regression outputs, class probabilities, predictive entropy) of nets that are
+    mlp_alike, together, on rows of x brought to (x - mean) / std."""
+    m = mlps[0]
+    x = np.ascontiguousarray(x, dtype=np.float64)
+    mean, std = (np.ascontiguousarray(np.broadcast_to(np.asarray(a, np.float64), (m.n_in,))) for a in (mean, std))
+    n = len(x)
+    if x.shape != (n, m.n_in):
+        raise ValueError("x: rows of the nets' inputs")
+    cls = np.empty(n, np.int32); reg = np.empty((n, m.n_out - 3), np.float32)
+    prob = np.empty((n, 3)); ent = np.empty(n)
+    _mlp_call(mlps, "sl_mlp_ensemble", n, _dp(x), _dp(mean), _dp(std), _ip(cls), _fp(reg), _dp(prob), _dp(ent))
+    return cls, reg, prob, ent
+
+
 def mlp_train_rows(mlps: list[MLP], x, cls, reg, idx, lr: float) -> list[float]:
     """One Adam step of each net on its own rows idx[j] of (x, cls, reg); the losses before it.
     The same as train_step(x[idx[j]], cls[idx[j]], reg[idx[j]], lr) of each."""
+    if any(type(m) is not MLP for m in mlps):
+        return [m.train_step(x[i], cls[i], reg[i], lr) for m, i in zip(mlps, idx)]
     x = np.ascontiguousarray(x, dtype=np.float32)
     cls = np.ascontiguousarray(cls, dtype=np.int32)
     reg = np.ascontiguousarray(reg, dtype=np.float32)
@@ -821,6 +848,8 @@ def mlp_train_rows(mlps: list[MLP], x, cls, reg, idx, lr: float) -> list[float]:
 def mlp_forward_all(mlps: list[MLP], x: np.ndarray):
     """forward of each net on the same rows: (outputs, class probabilities, predictive entropy),
     each with a leading axis over the nets."""
+    if any(type(m) is not MLP for m in mlps):
+        return tuple(np.stack(a) for a in zip(*(m.forward(x) for m in mlps)))
     x = np.ascontiguousarray(x, dtype=np.float32)
     n, B, m = len(mlps), x.shape[0], mlps[0]
     if x.shape != (B, m.n_in):

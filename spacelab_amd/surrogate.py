@@ -33,8 +33,8 @@ import numpy as np
 
 from . import (N_DESCRIPTORS, OUTCOME_BOUNCE, OUTCOME_FRAGMENT, OUTCOME_STICK, ORDER_FAST,
                PREC_FP64, Batch, CollisionSetup, MLP, calibrate, collision_approach,
-               collision_descriptors_batch, collision_outcome, generate_collision, mlp_forward_all,
-               mlp_train_rows, preset)
+               collision_descriptors_batch, collision_outcome, generate_collision, mlp_alike,
+               mlp_ensemble, mlp_forward_all, mlp_train_rows, preset)
 
 CLASS_NAMES = ("stick", "bounce", "fragment")
 # regression targets: mass fraction of the largest body, share of the projectile's mass
@@ -230,6 +230,8 @@ class Surrogate:
     def predict(self, X):
         """(class, regression outputs, class probabilities, predictive entropy) of
         descriptor rows."""
+        if type(self.norm) is Normaliser and mlp_alike(self.mlps):
+            return mlp_ensemble(self.mlps, X, self.norm.mean, self.norm.std)
         Xn = self.norm(X)
         P = np.zeros((len(Xn), 3))
         Y = np.zeros((len(Xn), N_REG))

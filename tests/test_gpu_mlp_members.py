@@ -54,3 +54,35 @@ def test_the_same_net_twice_and_errors():
             with pytest.raises(sl.SpacelabError):
                 sl.mlp_train_rows([m, q], **{**dict(x=x, cls=cls, reg=reg, idx=idx, lr=1e-3), **bad})
         assert bits_equal(m.get_params(), w)
+
+
+@pytest.mark.parametrize("members,max_batch,rows", [(4, 64, 0), (4, 64, 1), (4, 64, 32), (4, 64, 33), (4, 64, 97), (1, 1, 3), (16, 2, 5),
+                                                    (2, 3, 7), (3, 4096, 5000)])
+def test_ensemble_is_the_members_mean(members, max_batch, rows):
+    """Normalising, the sums over the members and the choice are the same operations as in
+    numpy, so the same bits; the entropy's logarithm may differ by an ulp or two."""
+    rng = np.random.default_rng(members + rows)
+    X = rng.standard_normal((rows, 21)) * 3 + 1
+    if rows > 4:
+        X[2, 5] = np.nan
+        X[3, 0] = 1e300
+    mean, std = rng.standard_normal(21), rng.uniform(0.5, 2, 21)
+    nets = [sl.MLP(21, 9, 80, max_batch, seed=k) for k in range(members)]
+    assert sl.mlp_alike(nets) and not sl.mlp_alike(nets + nets[:1])
+    cls, reg, prob, ent = sl.mlp_ensemble(nets, X, mean, std)
+    P, Y = np.zeros((rows, 3)), np.zeros((rows, 6))
+    with np.errstate(over="ignore", invalid="ignore"):
+        Xn = np.ascontiguousarray((X - mean) / std, dtype=np.float32)
+        for m in nets:
+            for k in range(0, rows, max_batch):
+                y, p, _ = m.forward(Xn[k:k + max_batch])
+                P[k:k + len(p)] += p
+                Y[k:k + len(y)] += y[:, 3:]
+        P /= members
+        Y /= members
+        want = -(P * np.log(np.where(P > 0, P, 1.0))).sum(1)
+    assert bits_equal(cls, P.argmax(1).astype(np.int32))
+    assert np.array_equal(reg, Y.astype(np.float32), equal_nan=True) and np.array_equal(prob, P, equal_nan=True)
+    assert np.allclose(ent, want, rtol=0, atol=1e-15 * 8, equal_nan=True)
+    for m in nets:
+        m.close()
