@@ -52,6 +52,9 @@ constexpr int NW = 4;                 // wavefronts per block
 #define SL_TILE_UNROLL 2              // pairs of the tile sweep unrolled per wavefront
 #endif
 constexpr int NT = TB * NW;
+constexpr int KB_C = 8;              // k_ball's slot classes K = c, c + KB_C, ...: they fix the order of every sum
+constexpr int SLOTS_IN_FLIGHT = 10;  // slots per lane k_ball loads together: 40 loads
+constexpr int KB_BATCH = SLOTS_IN_FLIGHT * KB_C;   // one batch for systems of up to 80 blocks
 
 // Lane l receives the value held by lane (l + 1) mod 64 (DPP wave_rol:1).
 __device__ __forceinline__ float rot1(float v)
@@ -100,6 +103,16 @@ __device__ __forceinline__ double block_sum(double v, double* red)
     return r;
 }
 
+// Systems of more than KB_BATCH blocks list their tiles in groups of NW of one row I, J = 4 g ..
+// 4 g + 3 (the last group of a row is filled up with I = -1), and the binary64 sweep, where a
+// workgroup takes several tiles, adds the i sides of a group's tiles before they go to memory:
+// one partial instead of four (two, with two wavefronts a tile), in the slot of the group's
+// first tile.  Per ball that leaves 5 of 8 partials to write and to read (the mixed sweep keeps
+// them apart: binary32 sums depend on their order).  At 40,000 spheres the per-ball kernel went
+// from 171 to 113 us (600 to 375 MB of partials) and the sweep from 1020 to 1005.  Smaller
+// systems' partials are one batch of loads per ball and not what bounds them.
+constexpr int ROW_GROUP = 1 << 30;
+
 struct TileArgs {
     const double* px;
     const double* py;
@@ -112,7 +125,7 @@ struct TileArgs {
     const float* gq_blk;    // mixed: per 64-ball block, the largest g/q of its balls (scaled weights)
     int n_pad;
     int n_tiles;
-    const int4* tiles;      // {I, J, system, first block of the system}
+    const int4* tiles;      // {I, J, system, first block of the system | ROW_GROUP}; I < 0: no tile
     float L0inv, L0inv2;    // mixed: 1 / L0 and 1 / L0^2 (scaled units)
     double Kf;              // mixed: force = Kf * (scaled binary32 factor) * (r / L0)
     double* part;           // [slot][xyz][n_pad]; the mixed mode stores binary32 sums, Kf left out,
@@ -322,9 +335,11 @@ __device__ __forceinline__ void tile_pass(const TileArgs& a, int tbase)
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / TB), l = threadIdx.x % TB;
     const int tl = w / SPLIT, h = w % SPLIT;
     const int t = tbase + tl;
-    const bool live = t < a.n_tiles;
-    const int4 tt = fetch_tile(a, t, live);
-    const int I = tt.x, J = tt.y, sys = tt.z, blk0 = tt.w;
+    int4 tt = fetch_tile(a, t, t < a.n_tiles);
+    const bool live = t < a.n_tiles && tt.x >= 0;
+    if (!live) tt = make_int4(0, 0, 0, 0);
+    const int I = tt.x, J = tt.y, sys = tt.z, blk0 = tt.w & (ROW_GROUP - 1);
+    const bool grouped = PREC == SL_PREC_FP64 && TPB > 1 && (tt.w & ROW_GROUP) != 0;
     const Phys& P = a.sysP[sys];
     const bool diag = I == J;
     const bool test = live && !tile_is_far(a, I, J, P.h_min);
@@ -635,6 +650,19 @@ __device__ __forceinline__ void tile_pass(const TileArgs& a, int tbase)
         comb[w][5][l] = bz;
     }
     __syncthreads();
+    if (grouped && h == 0 && live && tl == 0) {
+        // the i sides of the group's tiles, J to the diagonal (whose j side is on the same balls)
+        const int in_group = min(TPB, I - J + 1);
+        for (int k = 0; k < 3; k++) {
+            double acc = 0;
+            for (int g = 0; g < in_group; g++) {
+                for (int q = 0; q < SPLIT; q++) acc = acc + comb[g * SPLIT + q][k][l];
+                if (J + g == I)
+                    for (int q = 0; q < SPLIT; q++) acc = acc + comb[g * SPLIT + q][k + 3][l];
+            }
+            a.part[((size_t)(J - blk0) * 3 + k) * a.n_pad + i] = acc;
+        }
+    }
     if (!(live && h == 0)) return;
     const int w0 = tl * SPLIT;
     const size_t np = (size_t)a.n_pad;
@@ -652,16 +680,20 @@ __device__ __forceinline__ void tile_pass(const TileArgs& a, int tbase)
     PT* part = reinterpret_cast<PT*>(a.part);
     if (diag) {
         // the i side and the j side of the diagonal tile land on the same balls
-        part[(si * 3 + 0) * np + i] = v[0] + v[3];
-        part[(si * 3 + 1) * np + i] = v[1] + v[4];
-        part[(si * 3 + 2) * np + i] = v[2] + v[5];
+        if (!grouped) {
+            part[(si * 3 + 0) * np + i] = v[0] + v[3];
+            part[(si * 3 + 1) * np + i] = v[1] + v[4];
+            part[(si * 3 + 2) * np + i] = v[2] + v[5];
+        }
         const bool near = !a.near || __any((mi | mj) != 0);
         if (near) a.nbm[si * np + i] = mi | mj;
         if (a.near && l == 0) a.near[(size_t)I * a.near_stride + si] = near;
     } else {
-        part[(si * 3 + 0) * np + i] = v[0];
-        part[(si * 3 + 1) * np + i] = v[1];
-        part[(si * 3 + 2) * np + i] = v[2];
+        if (!grouped) {
+            part[(si * 3 + 0) * np + i] = v[0];
+            part[(si * 3 + 1) * np + i] = v[1];
+            part[(si * 3 + 2) * np + i] = v[2];
+        }
         part[(sj_ * 3 + 0) * np + j0] = v[3];
         part[(sj_ * 3 + 1) * np + j0] = v[4];
         part[(sj_ * 3 + 2) * np + j0] = v[5];
@@ -801,6 +833,7 @@ struct BallArgs {
     const int4* blk_info;   // per 64-ball block: {first slot, balls, blocks of its system, system}
     int n_pad;
     const double* part;     // [slot][xyz][n_pad]; mixed: binary32, to be scaled by Kf
+    int group;              // binary64, systems of more than KB_BATCH blocks: tiles to an i-side partial
     double Kf;
     const unsigned long long* nbm;   // near-partner masks; NEARF: of the slots that near marks
     const unsigned char* near;
@@ -826,9 +859,6 @@ __device__ __forceinline__ float local_coord(double x, bool valid, double lo, do
 }
 
 constexpr int BPB = TB;              // balls per k_ball block
-constexpr int KB_C = 8;              // slot classes K = c, c + KB_C, ...: they fix the order of every sum
-constexpr int SLOTS_IN_FLIGHT = 10;  // slots per lane loaded together: 40 loads
-constexpr int KB_BATCH = SLOTS_IN_FLIGHT * KB_C;   // one batch for systems of up to 80 blocks
 // k_ball workgroups have 8 wavefronts (one slot class each: the fewest dependent loads
 // per wavefront, for a lone system of few blocks) or 4 (two classes each, at most 170 VGPRs
 // and 53 KB of LDS: three workgroups share a CU, for launches of more blocks than CUs).
@@ -866,8 +896,8 @@ constexpr int kb_threads(int nwv) { return nwv * TB; }
 // the host (at 40,000 spheres, 195,625 tiles' energies copied and added there took 1 ms).
 //
 // NEARF, for systems of more than KB_BATCH slots: the masks of slots without near pairs, nine
-// in ten of a large system's, are neither written nor read (200 of 800 bytes a ball and slot
-// at 40,000 spheres: 201 -> 170 us).  Smaller systems load one batch of masks unseen: finding
+// in ten of a large system's, are neither written nor read (a quarter of what there was to
+// read at 40,000 spheres: 201 -> 170 us).  Smaller systems load one batch of masks unseen: finding
 // out which first cost 0.4 us of 11 at 79 slots and 5 of 49 in the four-wavefront shape.
 template <bool COMP, bool WRITE, int NWV, bool NEARF>
 __global__ __launch_bounds__(kb_threads(NWV)) void k_ball(BallArgs a)
@@ -942,6 +972,9 @@ __global__ __launch_bounds__(kb_threads(NWV)) void k_ball(BallArgs a)
     // slots K0, K0 + KB_C, ... of a class: SLOTS_IN_FLIGHT loaded together (4 for small systems)
     const bool wide = nb > 4 * KB_C;
     auto slot = [&](int K0, int u) { return K0 + u * KB_C < nb ? K0 + u * KB_C : nb - 1; };
+    // the block's sums, one after another: those of the groups up to the diagonal, then of the rows below
+    const int grp = !COMP && nb > KB_BATCH ? a.group : 1;
+    const int row = blockIdx.x - off / TB, ng = row / grp + 1, nsum = ng + nb - 1 - row;
     auto each_slot = [&](auto f) {
 #pragma unroll
         for (int u = 0; u < 4; u++) f(u);
@@ -964,7 +997,8 @@ __global__ __launch_bounds__(kb_threads(NWV)) void k_ball(BallArgs a)
     auto near_slots = [&](int K0, int byte) { return __ballot(byte != 0 && K0 + KB_C * l < nb); };
     auto load_sums = [&](int K0, PT (*q)[3]) {
         each_slot([&](int u) {
-            const PT* pp = reinterpret_cast<const PT*>(a.part) + (size_t)slot(K0, u) * 3 * np + ic;
+            const int e = min(K0 + u * KB_C, nsum - 1), K = e < ng ? e * grp : row + 1 + e - ng;
+            const PT* pp = reinterpret_cast<const PT*>(a.part) + (size_t)K * 3 * np + ic;
             q[u][0] = pp[0];
             q[u][1] = pp[np];
             q[u][2] = pp[2 * np];
@@ -991,7 +1025,7 @@ __global__ __launch_bounds__(kb_threads(NWV)) void k_ball(BallArgs a)
     };
     auto add = [&](int K0, PT (*q)[3], Sum& t) {
         each_slot([&](int u) {
-            if (K0 + u * KB_C >= nb) return;
+            if (K0 + u * KB_C >= nsum) return;
 #pragma unroll
             for (int x = 0; x < 3; x++) {
                 if (COMP) {
@@ -1008,7 +1042,7 @@ __global__ __launch_bounds__(kb_threads(NWV)) void k_ball(BallArgs a)
     auto class_sums = [&](int cl) {   // q0: the class's first slots, loaded
         Sum t{};
         add(cl, q0, t);
-        for (int K0 = cl + KB_BATCH; K0 < nb; K0 += KB_BATCH) {
+        for (int K0 = cl + KB_BATCH; K0 < nsum; K0 += KB_BATCH) {
             load_sums(K0, q0);
             add(K0, q0, t);
         }

@@ -307,6 +307,7 @@ int launch_ball_step(FastBuffers& fb, bool write, bool kick, bool drift_next, hi
     a.blk_info = fb.blk_info;
     a.n_pad = fb.n_pad;
     a.part = fb.part;
+    a.group = NW / std::max(fb.split, 1);
     a.Kf = fb.Kf;
     a.nbm = fb.nbm;
     a.near = near_flags(fb) ? fb.near : nullptr;
@@ -684,18 +685,27 @@ int fast_configure(FastBuffers& fb, State& canon, const FastLayout& lay, const P
         // per-pair near test come early and the launch ends on far tiles.  (Diagonal first
         // was measured 0.7% faster than row order.)  The order only schedules the tiles;
         // each tile's sums and the slots they land in do not depend on it.  Each system's
-        // tiles keep the same relative order whether it runs alone or in a batch.
+        // tiles keep the same relative order whether it runs alone or in a batch.  Systems of
+        // more than KB_BATCH blocks: the same bands of groups (ROW_GROUP).
         for (int s = 0; s < lay.n_sys; s++) {
             const int b0 = lay.off[s] / TB;
             for (int k = 0; k < lay.nb[s]; k++) fb.blk_sys_h[b0 + k] = s;
         }
         int nb_top = 0;
         for (int s = 0; s < lay.n_sys; s++) nb_top = std::max(nb_top, lay.nb[s]);
+        const int4 none = make_int4(-1, 0, 0, 0);
         for (int d = 0; d < nb_top; d++)
             for (int s = 0; s < lay.n_sys; s++) {
                 const int b0 = lay.off[s] / TB;
-                for (int I = d; I < lay.nb[s]; I++) {
-                    tiles.push_back(make_int4(b0 + I, b0 + I - d, s, b0));
+                if (lay.nb[s] <= KB_BATCH) {
+                    for (int I = d; I < lay.nb[s]; I++) tiles.push_back(make_int4(b0 + I, b0 + I - d, s, b0));
+                } else if (d % NW == 0) {   // groups by band: of row I the one that starts at J = 4 (I / 4) - d
+                    while (tiles.size() % NW) tiles.push_back(none);
+                    for (int I = d; I < lay.nb[s]; I++) {
+                        const int J0 = I / NW * NW - d;
+                        for (int J = J0; J < J0 + NW; J++)
+                            tiles.push_back(J <= I ? make_int4(b0 + I, b0 + J, s, b0 | ROW_GROUP) : none);
+                    }
                 }
             }
         std::vector<int4> info;

@@ -81,3 +81,33 @@ def test_marked_slots_same_bits(n, precision):
         assert bits_equal(getattr(a, f), getattr(b, f)), f
     assert [x.as_array().tobytes() for x in ea] == [x.as_array().tobytes() for x in eb]
     assert [x.contacts for x in ea] == [x.contacts for x in eb]
+
+
+@pytest.mark.parametrize("n", [5121, 5185, 5249, 5313])
+@pytest.mark.parametrize("queue", [1, 2])
+def test_grouped_rows(n, queue):
+    """81 to 84 blocks: rows whose last group of four tiles has every length.  One and two
+    wavefronts a tile add the i sides of four and two tiles before they are stored, four
+    wavefronts keep every tile's: sums of at most 84 x 64 terms in another order, each rounded
+    once (1.1e-16) on at most the sum of the terms' sizes, which for these lattices is below 50
+    times the largest acceleration: 84 x 64 x 1.1e-16 x 50 = 3e-11 at the very worst, and
+    sqrt of the count in practice: 1e-12 of the largest."""
+    rng = np.random.default_rng(n)
+    k = int(np.ceil(n ** (1 / 3)))
+    cell = rng.permutation(k ** 3)[:n]
+    pos = (np.stack([cell % k, cell // k % k, cell // k ** 2], 1) + rng.uniform(-.05, .05, (n, 3))) * 2.5e-5
+    R = np.full(n, 1e-5)
+    m = 2.25 * 4 / 3 * np.pi * R ** 3
+    zero = np.zeros((n, 3))
+    g = sl.BallGroup(pos, zero, zero.copy(), R, m, 0.4 * m * R * R)
+    p = sl.calibrate(sl.preset("config"), R, m, velocity=0.36301555459799423, cor=0.64).replace(order=sl.ORDER_FAST)
+    acc = []
+    for split in (4, 2, 1):
+        with sl.Collider(n, p) as c:
+            c.set_option("tile_split", split)
+            c.set_option("tile_queue", queue)
+            c.upload(g)
+            c.init_conditions()
+            acc.append(c.download().acc)
+    top = np.abs(acc[0]).max()
+    assert np.abs(acc[1] - acc[0]).max() <= 1e-12 * top and np.abs(acc[2] - acc[0]).max() <= 1e-12 * top
