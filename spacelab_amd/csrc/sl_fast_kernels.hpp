@@ -18,17 +18,18 @@
 //              sweep, so the sweep itself spends no vector instructions on them.  Each
 //              tile writes its i-side and j-side force sums and partner masks once,
 //              to slot J of the balls of block I and slot I of the balls of block J
-//              (system-local block numbers), so every (ball, slot) is written by
-//              exactly one tile per step and nothing needs clearing.
+//              (system-local block numbers), so every (ball, slot) that is read is written by
+//              exactly one tile per step and nothing needs clearing (large systems: see
+//              ROW_GROUP and the near marks).
 //   k_ball     one workgroup per 64-ball block, eight or four wavefronts with lane
 //              l working for ball l: the far-field partials of every eighth slot
 //              (one slot class) are summed by one wavefront (Kahan-compensated in
 //              the mixed mode), which counts the ball's partner-mask bits; the block
 //              numbers its near pairs ball by ball and evaluates them with the
 //              reference arithmetic, one per thread, in rounds of one entry per
-//              thread; then wavefront 0 adds the near results of
-//              each ball in entry order, forms acc and aacc, applies the closing
-//              kick, the write-step energies and the next step's drift (writing the
+//              thread; then each component of force and torque is finished by a
+//              wavefront: the near results of each ball in entry order, acc and aacc, the
+//              closing kick and the next step's drift (writing the
 //              other state set).  A near pair is evaluated once for each of its two
 //              balls, by the blocks that hold them.
 // Every sum has a fixed order at a given tile split, so results are reproducible run

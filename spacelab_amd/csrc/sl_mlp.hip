@@ -11,6 +11,8 @@
 //           sample), k_wgrad forms the weight and bias gradients of all layers and applies
 //           Adam.  Two launches a training step, one an inference; the batch is read from
 //           and the results written to pinned host memory by the kernels themselves.
+//           Several nets laid out alike share these launches (one grid row per net), and an
+//           ensemble's prediction normalises its rows and averages its nets on the device.
 //   layers  one launch per product (k_gemm), for wide networks, where a 16-sample
 //           workgroup would read each layer's whole weight matrix alone.
 //
