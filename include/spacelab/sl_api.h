@@ -366,11 +366,12 @@ int sl_mlp_gradients(sl_mlp* m, int batch, const float* x, const int* cls, const
 /* One Adam step (beta 0.9, 0.999, eps 1e-8) on a labelled batch; loss before the step. */
 int sl_mlp_train_step(sl_mlp* m, int batch, const float* x, const int* cls, const float* reg, float lr,
                       float* loss);
-/* The same of several nets (same n_in and n_out, each on rows of its own): net j takes the
- * rows idx[j * batch ..] of x, cls and reg (n_rows of each).  Nets of the same widths and
- * max_batch share their launches; the results are those of sl_mlp_train_step for each. */
-int sl_mlp_train_rows(sl_mlp* const* nets, int n, int batch, long long n_rows, const float* x, const int* cls,
-                      const float* reg, const long long* idx, float lr, float* loss);
+/* The same of several nets (same n_in and n_out, each on rows of its own), `batches` steps in a
+ * row: step k of net j takes the rows idx[(k n + j) batch ..] of x, cls and reg (n_rows of each);
+ * its loss goes to loss[k n + j].  Nets of the same widths and max_batch share their launches;
+ * the results are those of sl_mlp_train_step for each. */
+int sl_mlp_train_rows(sl_mlp* const* nets, int n, int batch, int batches, long long n_rows, const float* x,
+                      const int* cls, const float* reg, const long long* idx, float lr, float* loss);
 /* sl_mlp_forward of several nets (same n_in and n_out) on the same rows; outputs net after net. */
 int sl_mlp_forward_all(sl_mlp* const* nets, int n, int batch, const float* x, float* y, float* prob, float* ent);
 /* What the nets say together of any number of rows of binary64 inputs, each first brought to

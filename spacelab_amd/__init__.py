@@ -216,7 +216,7 @@ def lib():
     L.sl_mlp_gradients.argtypes = [vp, C.c_int, fp, ip, fp, fp, fp]
     L.sl_mlp_train_step.argtypes = [vp, C.c_int, fp, ip, fp, C.c_float, fp]
     mlps, llp = C.POINTER(vp), C.POINTER(C.c_longlong)
-    L.sl_mlp_train_rows.argtypes = [mlps, C.c_int, C.c_int, C.c_longlong, fp, ip, fp, llp, C.c_float, fp]
+    L.sl_mlp_train_rows.argtypes = [mlps, C.c_int, C.c_int, C.c_int, C.c_longlong, fp, ip, fp, llp, C.c_float, fp]
     L.sl_mlp_forward_all.argtypes = [mlps, C.c_int, C.c_int, fp, fp, fp, fp]
     L.sl_mlp_ensemble.argtypes = [mlps, C.c_int, C.c_longlong, dp, dp, dp, ip, fp, dp, dp]
     L.sl_mlp_last_error.argtypes = [vp]
@@ -826,23 +826,25 @@ def mlp_ensemble(mlps: list[MLP], x, mean, std):
     return cls, reg, prob, ent
 
 
-def mlp_train_rows(mlps: list[MLP], x, cls, reg, idx, lr: float) -> list[float]:
-    """One Adam step of each net on its own rows idx[j] of (x, cls, reg); the losses before it.
-    The same as train_step(x[idx[j]], cls[idx[j]], reg[idx[j]], lr) of each."""
+def mlp_train_rows(mlps: list[MLP], x, cls, reg, idx, lr: float) -> np.ndarray:
+    """len(idx) Adam steps of each net, step k of net j on the rows idx[k][j] of (x, cls, reg); the
+    losses before each step, [step][net].  The same as train_step(x[i], cls[i], reg[i], lr) with
+    i = idx[k][j], for k in order."""
     if any(type(m) is not MLP for m in mlps):
-        return [m.train_step(x[i], cls[i], reg[i], lr) for m, i in zip(mlps, idx)]
+        return np.array([[m.train_step(x[i], cls[i], reg[i], lr) for m, i in zip(mlps, step)] for step in idx])
     x = np.ascontiguousarray(x, dtype=np.float32)
     cls = np.ascontiguousarray(cls, dtype=np.int32)
     reg = np.ascontiguousarray(reg, dtype=np.float32)
     idx = np.ascontiguousarray(idx, dtype=np.int64)
     m = mlps[0]
-    if not (idx.ndim == 2 and len(idx) == len(mlps) and x.shape[1:] == (m.n_in,) and cls.ndim == 1
+    if not (idx.ndim == 3 and idx.shape[1] == len(mlps) and x.shape[1:] == (m.n_in,) and cls.ndim == 1
             and min(len(cls), len(reg)) >= len(x) and reg.size == len(reg) * (m.n_out - 3)):
-        raise ValueError("idx: a row of indices per net; x, cls, reg: rows of the data")
-    loss = np.zeros(len(mlps), np.float32)
-    _mlp_call(mlps, "sl_mlp_train_rows", idx.shape[1], len(x), _fp(x), _ip(cls), _fp(reg),
-              idx.ctypes.data_as(C.POINTER(C.c_longlong)), lr, _fp(loss))
-    return [float(v) for v in loss]
+        raise ValueError("idx: a row of indices per step and net; x, cls, reg: rows of the data")
+    loss = np.zeros(idx.shape[:2], np.float32)
+    if len(idx):
+        _mlp_call(mlps, "sl_mlp_train_rows", idx.shape[2], len(idx), len(x), _fp(x), _ip(cls), _fp(reg),
+                  idx.ctypes.data_as(C.POINTER(C.c_longlong)), lr, _fp(loss))
+    return loss.astype(np.float64)
 
 
 def mlp_forward_all(mlps: list[MLP], x: np.ndarray):

@@ -267,7 +267,8 @@ constexpr int KF = 8;                    // weight fragments (32 of K each) a la
 // (16 at batch 256) and too short a pass for a launch: a training step of four nets takes the
 // device 33 us together and 27 us for one alone; driven one by one each cost 56 us with its
 // launches and its wait.  (21-256-256-256-9, batch 256, 4096 rows, one epoch of four nets:
-// 3.6 -> 1.5 ms; 10,000 rows through the four 1.03 -> 0.76 ms.)
+// 3.6 -> 1.5 ms, 1.2 with the next batch gathered meanwhile; 10,000 rows through the four 1.03
+// -> 0.76 ms.)
 constexpr int MEMBERS = 16;
 struct Moved {
     long long pool, stage, x;   // bytes: device pool, pinned buffer, input rows
@@ -1358,28 +1359,29 @@ int sl_mlp_train_step(sl_mlp* m, int B, const float* x, const int* cls, const fl
     return SL_OK;
 }
 
-int sl_mlp_train_rows(sl_mlp* const* ms, int n, int B, long long n_rows, const float* x, const int* cls, const float* reg,
-                      const long long* idx, float lr, float* loss)
+int sl_mlp_train_rows(sl_mlp* const* ms, int n, int B, int batches, long long n_rows, const float* x, const int* cls,
+                      const float* reg, const long long* idx, float lr, float* loss)
 {
-    if (!ms || n < 1) return SL_E_ARG;
+    if (!ms || n < 1 || batches < 0) return SL_E_ARG;
     for (int j = 0; j < n; j++) {
         const int rc = check_batch(ms[j], B, x);
         if (rc) return rc;
         if (!cls || !reg || !idx || !(lr > 0)) return mlp_err(ms[j], SL_E_ARG, "labels or rows are NULL or lr <= 0");
         if (ms[j]->n_in != ms[0]->n_in || ms[j]->n_out != ms[0]->n_out)
             return mlp_err(ms[j], SL_E_ARG, "nets of one ensemble have the same inputs and outputs");
-        for (int b = 0; b < B; b++) {
-            const long long row = idx[(size_t)j * B + b];
-            if (row < 0 || row >= n_rows) return mlp_err(ms[j], SL_E_ARG, "row index outside the data");
-            if (cls[row] < 0 || cls[row] >= NCLS) return mlp_err(ms[j], SL_E_ARG, "class label outside 0..2");
-        }
+    }
+    auto at = [&](int k, int j) { return idx + ((size_t)k * n + j) * B; };   // rows of batch k of net j
+    for (size_t e = 0; e < (size_t)batches * n * B; e++) {
+        sl_mlp* m = ms[e / B % n];
+        if (idx[e] < 0 || idx[e] >= n_rows) return mlp_err(m, SL_E_ARG, "row index outside the data");
+        if (cls[idx[e]] < 0 || cls[idx[e]] >= NCLS) return mlp_err(m, SL_E_ARG, "class label outside 0..2");
     }
     const int n_in = ms[0]->n_in, nr = ms[0]->n_out - NCLS;
-    auto rows = [&](const long long* at, float* px, int* pc, float* pr) {
+    auto rows = [&](const long long* r, float* px, int* pc, float* pr) {
         for (int b = 0; b < B; b++) {
-            std::memcpy(px + (size_t)b * n_in, x + at[b] * n_in, 4 * (size_t)n_in);
-            pc[b] = cls[at[b]];
-            std::memcpy(pr + (size_t)b * nr, reg + at[b] * nr, 4 * (size_t)nr);
+            std::memcpy(px + (size_t)b * n_in, x + r[b] * n_in, 4 * (size_t)n_in);
+            pc[b] = cls[r[b]];
+            std::memcpy(pr + (size_t)b * nr, reg + r[b] * nr, 4 * (size_t)nr);
         }
     };
     if (!alike(ms, n)) {
@@ -1389,33 +1391,55 @@ int sl_mlp_train_rows(sl_mlp* const* ms, int n, int B, long long n_rows, const f
         float* pr = buf + (size_t)B * n_in;
         int* pc = reinterpret_cast<int*>(pr + (size_t)B * nr);
         int rc = SL_OK;
-        for (int j = 0; j < n && rc == SL_OK; j++) {
-            rows(idx + (size_t)j * B, buf, pc, pr);
-            rc = sl_mlp_train_step(ms[j], B, buf, pc, pr, lr, loss ? loss + j : nullptr);
-            if (rc && j) ms[0]->err = ms[j]->err;
-        }
+        for (int k = 0; k < batches && rc == SL_OK; k++)
+            for (int j = 0; j < n && rc == SL_OK; j++) {
+                rows(at(k, j), buf, pc, pr);
+                rc = sl_mlp_train_step(ms[j], B, buf, pc, pr, lr, loss ? loss + (size_t)k * n + j : nullptr);
+                if (rc && j) ms[0]->err = ms[j]->err;
+            }
         delete[] buf;
         return rc;
     }
+    // Batches that take up to half of the pinned buffer are gathered into its halves in turn,
+    // one while the device trains on the other.
     const Stage s(ms[0]->max_batch, n_in, nr + NCLS);
+    const int ahead = 2 * B <= ms[0]->max_batch ? 2 : 1;
+    const size_t half = ahead == 2 ? (size_t)(ms[0]->max_batch / 2) : 0;   // rows
     for (int j0 = 0; j0 < n; j0 += MEMBERS) {
-        const int k = std::min(n - j0, MEMBERS);
-        Adam adam[MEMBERS];
-        for (int j = 0; j < k; j++) {
-            sl_mlp* m = ms[j0 + j];
-            adam[j] = adam_step(m, lr);
-            rows(idx + (size_t)(j0 + j) * B, reinterpret_cast<float*>(m->stage + s.x), reinterpret_cast<int*>(m->stage + s.cls),
-                 reinterpret_cast<float*>(m->stage + s.reg));
+        const int g = std::min(n - j0, MEMBERS);
+        sl_mlp* const* mg = ms + j0;
+        auto part = [&](sl_mlp* m, size_t p, size_t bytes, int k) { return m->stage + p + k % ahead * half * bytes; };
+        auto collect = [&](int k) -> int {
+            if (hipEventSynchronize(mg[0]->half[k % 2]) != hipSuccess) return mlp_err(ms[0], SL_E_HIP, "training pass failed");
+            for (int j = 0; loss && j < g; j++)
+                loss[(size_t)k * n + j0 + j] = mean_loss(reinterpret_cast<const float*>(part(mg[j], s.loss, 4, k)), B);
+            return SL_OK;
+        };
+        ChainArgs c = chain_args(mg, g, B, false);
+        const ChainArgs c0 = c;
+        for (int k = 0; k < batches; k++) {
+            if (k >= ahead)
+                if (const int rc = collect(k - ahead)) return rc;
+            Adam adam[MEMBERS];
+            for (int j = 0; j < g; j++) {
+                sl_mlp* m = mg[j];
+                adam[j] = adam_step(m, lr);
+                m->t++;
+                rows(at(k, j0 + j), reinterpret_cast<float*>(part(m, s.x, 4 * (size_t)n_in, k)),
+                     reinterpret_cast<int*>(part(m, s.cls, 4, k)), reinterpret_cast<float*>(part(m, s.reg, 4 * (size_t)nr, k)));
+            }
+            const size_t r0 = k % ahead * half;
+            c.x = c0.x + r0 * n_in;
+            c.cls = c0.cls + r0;
+            c.reg = c0.reg + r0 * nr;
+            c.loss = c0.loss + r0;
+            launch_chain<true>(mg, g, B, c);
+            launch_wgrad<true>(mg, g, B, adam);
+            if (hipGetLastError() != hipSuccess || hipEventRecord(mg[0]->half[k % 2], mg[0]->stream) != hipSuccess)
+                return mlp_err(ms[0], SL_E_HIP, "training pass failed");
         }
-        launch_chain<true>(ms + j0, k, B);
-        launch_wgrad<true>(ms + j0, k, B, adam);
-        if (hipGetLastError() != hipSuccess || hipStreamSynchronize(ms[j0]->stream) != hipSuccess)
-            return mlp_err(ms[0], SL_E_HIP, "training pass failed");
-        for (int j = 0; j < k; j++) {
-            sl_mlp* m = ms[j0 + j];
-            if (loss) loss[j0 + j] = mean_loss(reinterpret_cast<const float*>(m->stage + s.loss), B);
-            m->t++;
-        }
+        for (int k = std::max(0, batches - ahead); k < batches; k++)
+            if (const int rc = collect(k)) return rc;
     }
     return SL_OK;
 }

@@ -217,9 +217,9 @@ class Surrogate:
             perm = np.stack([rng.permutation(n) for rng in rngs])
             tot, cnt = np.zeros(len(self.mlps)), 0
             lr_ep = lr * 0.5 * (1 + math.cos(math.pi * ep / epochs))
-            for b0 in range(0, n - batch + 1, batch):
-                loss = mlp_train_rows(self.mlps, Xn, cls, reg, perm[:, b0:b0 + batch], lr_ep)
-                tot += np.multiply(loss, batch)
+            steps = [perm[:, b0:b0 + batch] for b0 in range(0, n - batch + 1, batch)]
+            for loss in mlp_train_rows(self.mlps, Xn, cls, reg, np.stack(steps), lr_ep) if steps else ():
+                tot += loss * batch
                 cnt += batch
             for t in tot.tolist():
                 hist[ep] += t / max(cnt, 1) / len(self.mlps)
