@@ -1,8 +1,8 @@
 """Potential energy of far pairs in the fast engine, on lattices of separate spheres.
 
 The engine takes the van der Waals energy of a pair from a series in y = 4 Ri Rj / (d^2 - (Ri -
-Rj)^2) for y <= 1/16 and from the closed form above; spacings of 7.6 to 8.4 radii put pairs on
-both sides of the line, 3 and 40 radii nearly all on one.  The expected sum is the same series
+Rj)^2) for y <= 1/8 and from the closed form above; spacings of 5.4 to 5.9 radii put pairs on
+both sides of the line, 3, 8 and 40 radii nearly all on one.  The expected sum is the same series
 (to 80 terms) or the closed form in extended precision, added exactly.
 
 Tolerance 1e-13: a series term carries a few ulps of 1.1e-16, the closed form at y > 1/8 loses
