@@ -241,8 +241,10 @@ constexpr int ORD_GRAPH_MAX_STEPS = 128;
 // len ordered steps without energies, as one replay of a graph captured on first use: the
 // drift, then one launch per step (pair pass, closing kick, next step's drift), between the
 // context's arrays and the fast engine's first set, which this order leaves idle (its owner
-// reloads it before its next step).  An even number of steps ends in the context's arrays.
-// One sphere, or a single step, takes the direct launches' kernels.
+// reloads it before its next step).  The last step ends in the context's arrays: an odd
+// number of steps starts in the other set, where the drift puts them.  (63 steps of 1,000 balls
+// as 62 and a step of three launches took 10 us more.)  One sphere takes the direct launches'
+// kernels.
 int ordered_run(sl_ctx* c, int len)
 {
     hipGraphExec_t ex = nullptr;
@@ -253,15 +255,18 @@ int ordered_run(sl_ctx* c, int len)
         const Phys P = phys_of(c->p);
         if (hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal) != hipSuccess)
             return set_err(c, SL_E_HIP, "ordered step capture");
-        bool ok = launch_drift(c->st, c->n, c->p.dt, c->stream) == hipSuccess;
-        if (c->n > 1 && len % 2 == 0) {
+        bool ok = true;
+        if (c->n > 1) {
             double* set[2] = {c->base, c->fb.eng[0].f[0]};
-            for (int k = 0; k < len && ok; k++)
-                ok = launch_step_ordered(c->base, set[k & 1], set[1 - (k & 1)], c->n_pad, P, c->n, k + 1 < len, c->cnt,
+            const int odd = len & 1;
+            ok = (odd ? launch_drift_to(c->st, c->fb.eng[0], c->n, c->p.dt, c->stream)
+                      : launch_drift(c->st, c->n, c->p.dt, c->stream)) == hipSuccess;
+            for (int k = odd; k < len + odd && ok; k++)
+                ok = launch_step_ordered(c->base, set[k & 1], set[1 - (k & 1)], c->n_pad, P, c->n, k + 1 < len + odd, c->cnt,
                                          c->nonfinite, c->stream, c->ord_shape) == hipSuccess;
         } else {
             for (int k = 0; k < len && ok; k++)
-                ok = (k == 0 || launch_drift(c->st, c->n, c->p.dt, c->stream) == hipSuccess) &&
+                ok = launch_drift(c->st, c->n, c->p.dt, c->stream) == hipSuccess &&
                      launch_pairs_ordered(c->st, P, c->n, 0, c->pe_part, c->cnt, c->stream, c->ord_shape) == hipSuccess &&
                      launch_kick(c->st, c->n, c->p.dt, 0, 1, c->e_part, c->nonfinite, c->stream) == hipSuccess;
         }
@@ -628,7 +633,6 @@ int sl_step(sl_ctx* c, int n_steps, int write_every, sl_energy* e_out, int e_cap
                 if (write_every > 0 && s % write_every == 0) break;
                 len++;
             }
-            if (len > 1 && c->n > 1) len -= len % 2;
             if (len > 0) {
                 const int rc = ordered_run(c, len);
                 if (rc) return rc;

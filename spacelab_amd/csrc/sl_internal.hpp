@@ -12,6 +12,7 @@ namespace sl {
 
 // ---- ordered (bitwise) path: sl_kernels_ordered.hip
 hipError_t launch_drift(const State& s, int n, double dt, hipStream_t st);
+hipError_t launch_drift_to(const State& s, const State& d, int n, double dt, hipStream_t st);   // into the set d
 hipError_t launch_copy_prev(const State& s, int n, hipStream_t st);
 // Launch shapes of the pair pass (all give the same bits); shape = index below ordered_shapes().
 int ordered_shapes();

@@ -64,27 +64,31 @@ __device__ __forceinline__ double block_sum(double v, double* red)
 }  // namespace
 
 // First pass (ColliderSingleCore.cpp:82-97) plus the hysteresis state: the
-// positions before the drift are the ones the previous pair pass used.
-__global__ void k_drift(State s, int n, double dt)
+// positions before the drift are the ones the previous pair pass used.  To d: the state
+// itself, or (COPY) another set, with the velocities and spins the step will read.
+template <bool COPY>
+__global__ void k_drift(State s, State d, int n, double dt)
 {
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
     if (b >= n) return;
     const double px = s.f[PX][b], py = s.f[PY][b], pz = s.f[PZ][b];
-    s.f[QX][b] = px;
-    s.f[QY][b] = py;
-    s.f[QZ][b] = pz;
+    if (COPY)
+        for (int f = VX; f < VX + 6; f++) d.f[f][b] = s.f[f][b];
+    d.f[QX][b] = px;
+    d.f[QY][b] = py;
+    d.f[QZ][b] = pz;
     const double hx = s.f[VX][b] + .5 * s.f[AX][b] * dt;
     const double hy = s.f[VY][b] + .5 * s.f[AY][b] * dt;
     const double hz = s.f[VZ][b] + .5 * s.f[AZ][b] * dt;
-    s.f[HX][b] = hx;
-    s.f[HY][b] = hy;
-    s.f[HZ][b] = hz;
-    s.f[GX][b] = s.f[WX][b] + .5 * s.f[BX][b] * dt;
-    s.f[GY][b] = s.f[WY][b] + .5 * s.f[BY][b] * dt;
-    s.f[GZ][b] = s.f[WZ][b] + .5 * s.f[BZ][b] * dt;
-    s.f[PX][b] = px + hx * dt;
-    s.f[PY][b] = py + hy * dt;
-    s.f[PZ][b] = pz + hz * dt;
+    d.f[HX][b] = hx;
+    d.f[HY][b] = hy;
+    d.f[HZ][b] = hz;
+    d.f[GX][b] = s.f[WX][b] + .5 * s.f[BX][b] * dt;
+    d.f[GY][b] = s.f[WY][b] + .5 * s.f[BY][b] * dt;
+    d.f[GZ][b] = s.f[WZ][b] + .5 * s.f[BZ][b] * dt;
+    d.f[PX][b] = px + hx * dt;
+    d.f[PY][b] = py + hy * dt;
+    d.f[PZ][b] = pz + hz * dt;
 }
 
 // Positions the step-0 pass uses are also its hysteresis reference (k = kout
@@ -656,7 +660,13 @@ __global__ __launch_bounds__(256) void k_kick(State s, int n, double dt, int wri
 hipError_t launch_drift(const State& s, int n, double dt, hipStream_t st)
 {
     if (n <= 0) return hipSuccess;
-    k_drift<<<(n + 255) / 256, 256, 0, st>>>(s, n, dt);
+    k_drift<false><<<(n + 255) / 256, 256, 0, st>>>(s, s, n, dt);
+    return hipGetLastError();
+}
+
+hipError_t launch_drift_to(const State& s, const State& d, int n, double dt, hipStream_t st)
+{
+    k_drift<true><<<(n + 255) / 256, 256, 0, st>>>(s, d, n, dt);
     return hipGetLastError();
 }
 
