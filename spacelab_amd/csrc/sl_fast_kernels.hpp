@@ -1056,9 +1056,11 @@ __global__ __launch_bounds__(kb_threads(NWV)) void k_ball(BallArgs a)
         Near t{};
         unsigned long long near = 0;
         if constexpr (NEARF) near = near_slots(cl, near0);
-        load_masks(cl, near, mk);
-        load_sums(cl, q0);
-        count(cl, cl, mk, t);
+        if (cl < nb) {   // a system of few blocks has no slots in the higher classes
+            load_masks(cl, near, mk);
+            load_sums(cl, q0);
+            count(cl, cl, mk, t);
+        }
         int batch = 1;
         for (int K0 = cl + KB_BATCH; K0 < nb; K0 += KB_BATCH, batch++) {
             if constexpr (NEARF) near = batch % 6 ? near >> SLOTS_IN_FLIGHT : near_slots(K0, near_bytes(K0));
