@@ -123,7 +123,7 @@ struct TileArgs {
     const Phys* sysP;       // per system
     const double4* bnd;     // per 64-ball block: bounding box of the centres (lo with max R, hi)
     const float4* xl;       // mixed: per ball, position relative to its block's box centre and R, in units of L0
-    const float* gq_blk;    // mixed: per 64-ball block, the largest g/q of its balls (scaled weights)
+    const double* gq_blk;   // per 64-ball block, the largest g/q of its balls (aux.g, aux.q): grav_share, both precisions
     int n_pad;
     int n_tiles;
     const int4* tiles;      // {I, J, system, first block of the system | ROW_GROUP}; I < 0: no tile
@@ -234,15 +234,15 @@ __device__ __forceinline__ bool tile_is_far(const TileArgs& a, int I, int J, dou
 
 // Largest share of gravity in the force of any pair of tile (I, J): g_i g_j / d^3 over
 // q_i q_j / (s t)^2 is at most (g/q)_I (g/q)_J dmax^5, because s, t <= d^2 <= dmax^2 (dmax: the
-// largest distance between the blocks' boxes).  NaN where a position is.
+// largest distance between the blocks' boxes).  NaN where a position is.  From the binary64
+// weights: the mixed path's overflow at radii of 7e12 median ones, which made the share 0.
 __device__ __forceinline__ double grav_share(const TileArgs& a, int I, int J)
 {
     const double4 li = a.bnd[2 * I], ui = a.bnd[2 * I + 1], lj = a.bnd[2 * J], uj = a.bnd[2 * J + 1];
     const double ex = fmax(uj.x - li.x, ui.x - lj.x), ey = fmax(uj.y - li.y, ui.y - lj.y);
     const double ez = fmax(uj.z - li.z, ui.z - lj.z);
-    const double dmax = __builtin_sqrt(ex * ex + ey * ey + ez * ez) * (double)a.L0inv;
-    const double d2m = dmax * dmax;
-    return (double)a.gq_blk[I] * (double)a.gq_blk[J] * d2m * d2m * dmax;
+    const double d2m = ex * ex + ey * ey + ez * ez;
+    return a.gq_blk[I] * a.gq_blk[J] * d2m * d2m * __builtin_sqrt(d2m);
 }
 
 // Largest y = 4 Ri Rj / (d^2 - (Ri - Rj)^2) of the pairs of tile (I, J), from the gap between the

@@ -87,7 +87,7 @@ struct FastBuffers {
     FastAux aux{};
     double4* bnd = nullptr;       // per 64-ball block: bounding box of the positions (lo, hi)
     float4* xl = nullptr;         // per ball: position relative to its block's box centre, R (units of L0)
-    float* gq_blk = nullptr;      // per 64-ball block: largest g/q of the mixed path's scaled weights
+    double* gq_blk = nullptr;     // per 64-ball block: largest g/q of its balls (both precisions' bound on gravity)
     double L0 = 1, M0 = 1;        // length and mass units of the mixed path
     double Kf = 1;                // mixed path: force scale of the binary32 factor
     int* blk_sys = nullptr;       // device copies of the layout

@@ -68,17 +68,17 @@ __global__ void k_aux(State s, FastAux aux, int n, double sqrtC, double sqrtG, d
 }
 
 // Per 64-ball block (one wavefront each): the largest gravity-to-cohesion weight ratio
-// g/q of its balls, the mixed path's bound on where gravity can matter in a far tile.
-__global__ void k_gq_blk(FastAux aux, const int* blk_sys, const int* sys_off, const int* sys_n, float* gq)
+// g/q of its balls.  Both precisions bound gravity's share of a tile by it (grav_share).
+__global__ void k_gq_blk(FastAux aux, const int* blk_sys, const int* sys_off, const int* sys_n, double* gq)
 {
     const int l = threadIdx.x;
     const int b = blockIdx.x * TB + l;
     const int sy = blk_sys[blockIdx.x];
     const bool valid = b - sys_off[sy] < sys_n[sy];
-    const float q = aux.q32[b], g = aux.g32[b];
+    const double q = aux.q[b], g = aux.g[b];
     // a ball without cohesion (q = 0) but with gravity has no bound: +inf keeps gravity on
-    float r = !valid ? 0.f : (q > 0.f ? g / q : (g > 0.f ? __builtin_huge_valf() : 0.f));
-    for (int m = 1; m < TB; m <<= 1) r = fmaxf(r, __shfl_xor(r, m, TB));
+    double r = !valid ? 0.0 : (q > 0 ? g / q : (g > 0 ? __builtin_huge_val() : 0.0));
+    for (int m = 1; m < TB; m <<= 1) r = fmax(r, __shfl_xor(r, m, TB));
     if (l == 0) gq[blockIdx.x] = r;
 }
 
@@ -576,7 +576,7 @@ int fast_alloc(FastBuffers& fb, int n_pad, int max_sys)
     if (hipMalloc(&fb.aux.g32, sizeof(float) * n_pad) != hipSuccess) return -1;
     if (hipMalloc(&fb.bnd, sizeof(double4) * 2 * nblocks) != hipSuccess) return -1;
     if (hipMalloc(&fb.xl, sizeof(float4) * n_pad) != hipSuccess) return -1;
-    if (hipMalloc(&fb.gq_blk, sizeof(float) * nblocks) != hipSuccess) return -1;
+    if (hipMalloc(&fb.gq_blk, sizeof(double) * nblocks) != hipSuccess) return -1;
     if (hipMalloc(&fb.queue, sizeof(int) * QPAD * (QSEG + 1)) != hipSuccess) return -1;
     if (hipMemset(fb.queue, 0, sizeof(int) * QPAD * (QSEG + 1)) != hipSuccess) return -1;
     if (hipMalloc(&fb.blk_sys, sizeof(int) * nblocks) != hipSuccess) return -1;

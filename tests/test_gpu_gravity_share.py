@@ -45,3 +45,30 @@ def test_gravity_share(n, share):
     ref = terms.sum(1) / m[:, None]
     size = np.abs(terms).sum(1) / m[:, None]
     assert (np.abs(acc - ref) <= 3e-14 * size).all(), float((np.abs(acc - ref) / size).max())
+
+
+@pytest.mark.parametrize("ratio", [1e12, 1e13, 1e16])
+def test_gravity_share_of_bodies_far_larger_than_the_median(ratio):
+    """64 bodies (a block of their own) of `ratio` median radii, held by gravity alone: the
+    median of 128 grains sets the scaled binary32 weights, which overflow at 7e12.  Same
+    tolerance; the bodies lie 10 to 70 radii apart, inside the padding slots' distance."""
+    big = 64
+    R = np.concatenate([np.full(128, 1e8 / ratio), np.full(big, 1e8)])
+    m = 2.25 * 4 / 3 * np.pi * R ** 3
+    rng = np.random.default_rng(7)
+    cell = np.stack(np.meshgrid(*[np.arange(4)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    grain = np.stack(np.meshgrid(np.arange(8), np.arange(4), np.arange(4), indexing="ij"), -1).reshape(-1, 3)
+    x = np.concatenate([grain * 10 * R[0], 2e10 + (cell + rng.uniform(-.1, .1, (big, 3))) * 1.5e9])
+    n = len(R)
+    p = sl.preset("config").replace(order=sl.ORDER_FAST, kin=1.0, kout=0.64, dt=1e-9)
+    with sl.Collider(n, p) as c:
+        c.upload(sl.BallGroup(x, np.zeros((n, 3)), np.zeros((n, 3)), R, m, 0.4 * m * R ** 2))
+        c.init_conditions()
+        acc = c.download().acc[128:]
+    L = np.longdouble
+    d = x.astype(L)[None] - x.astype(L)[128:, None]
+    d2 = (d ** 2).sum(-1)
+    d2[np.arange(big), 128 + np.arange(big)] = 1
+    terms = (L(p.G) * m.astype(L)[None] / d2 ** L(1.5))[..., None] * d
+    ref, size = terms.sum(1), np.abs(terms).sum(1)
+    assert (np.abs(acc - ref) <= 3e-14 * size).all(), float((np.abs(acc - ref) / size).max())
