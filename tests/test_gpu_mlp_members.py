@@ -87,3 +87,49 @@ def test_ensemble_is_the_members_mean(members, max_batch, rows):
     assert np.allclose(ent, want, rtol=0, atol=1e-15 * 8, equal_nan=True)
     for m in nets:
         m.close()
+
+
+def _forms():
+    X = np.random.default_rng(3).standard_normal((37, 21)) * 2 + 0.3
+    f32 = lambda a: a.astype(np.float32)
+    return {"rows": (X, None), "fortran": (np.asfortranarray(X), None), "every other": (np.repeat(X, 2, 0)[::2], None),
+            "reversed": (X[::-1, ::-1], None), "integers": ((10 * X).astype(np.int64), None), "list": (X.tolist(), None),
+            "binary32 rows": (f32(X), None), "binary32 throughout": (f32(X), f32), "binary32 statistics": (X, f32),
+            "extended": (X.astype(np.longdouble), None), "one column": (X[:, :1], None), "one row's statistics": (X, lambda a: a[None]),
+            "scalar statistics": (X, lambda a: a[0]), "scalar for binary32 rows": (f32(X), lambda a: float(a[0])), "none": (X[:0], None)}
+
+
+@pytest.mark.parametrize("form", list(_forms()))
+def test_predict_takes_every_form_of_rows(form):
+    """Rows and statistics of any shape, order and type that numpy normalises: the same bits as
+    normalising them there and averaging the nets one by one."""
+    from spacelab_amd import surrogate as S
+    X, change = _forms()[form]
+    rng = np.random.default_rng(4)
+    mean, std = rng.standard_normal(21), rng.uniform(0.5, 2, 21)
+    s = S.Surrogate(width=64, n_models=3, max_batch=16)
+    s.norm = S.Normaliser(mean, std) if change is None else S.Normaliser(change(mean), change(std))
+    Xn = np.ascontiguousarray((X - s.norm.mean) / s.norm.std, dtype=np.float32)
+    P, Y = np.zeros((len(Xn), 3)), np.zeros((len(Xn), S.N_REG))
+    for m in s.mlps:
+        for k in range(0, len(Xn), 16):
+            y, p, _ = m.forward(Xn[k:k + 16])
+            P[k:k + len(p)] += p
+            Y[k:k + len(y)] += y[:, 3:]
+    P, Y = P / 3, Y / 3
+    cls, reg, prob, ent = s.predict(X)
+    assert bits_equal(cls, P.argmax(1)) and bits_equal(reg, Y.astype(np.float32)) and bits_equal(prob, P)
+    assert np.allclose(ent, -(P * np.log(np.where(P > 0, P, 1.0))).sum(1), rtol=0, atol=1e-15 * 8)
+    s.close()
+
+
+def test_predict_refuses_nets_of_other_outputs_or_smaller_batches():
+    from spacelab_amd import surrogate as S
+    X = np.zeros((40, 21))
+    for nets, error in (([sl.MLP(21, 8, 64, 64, k) for k in range(2)], ValueError),
+                        ([sl.MLP(21, 9, 64, 32, k) for k in range(2)], sl.SpacelabError)):
+        s = S.Surrogate(max_batch=64, mlps=nets)
+        s.norm = S.Normaliser(np.zeros(21), np.ones(21))
+        with pytest.raises(error):
+            s.predict(X)
+        s.close()
