@@ -837,9 +837,11 @@ def mlp_train_rows(mlps: list[MLP], x, cls, reg, idx, lr: float) -> np.ndarray:
     reg = np.ascontiguousarray(reg, dtype=np.float32)
     idx = np.ascontiguousarray(idx, dtype=np.int64)
     m = mlps[0]
-    if not (idx.ndim == 3 and idx.shape[1] == len(mlps) and x.shape[1:] == (m.n_in,) and cls.ndim == 1
-            and min(len(cls), len(reg)) >= len(x) and reg.size == len(reg) * (m.n_out - 3)):
+    if not (idx.ndim == 3 and idx.shape[1] == len(mlps) and x.shape[1:] == (m.n_in,) and cls.ndim and cls.size == len(cls)
+            and reg.size == len(reg) * (m.n_out - 3)):
         raise ValueError("idx: a row of indices per step and net; x, cls, reg: rows of the data")
+    if min(len(cls), len(reg)) < len(x):
+        raise IndexError(f"x has {len(x)} rows, cls {len(cls)}, reg {len(reg)}")
     loss = np.zeros(idx.shape[:2], np.float32)
     if len(idx):
         _mlp_call(mlps, "sl_mlp_train_rows", idx.shape[2], len(idx), len(x), _fp(x), _ip(cls), _fp(reg),

@@ -133,3 +133,18 @@ def test_predict_refuses_nets_of_other_outputs_or_smaller_batches():
         with pytest.raises(error):
             s.predict(X)
         s.close()
+
+
+def test_fit_takes_labels_in_a_column():
+    from spacelab_amd import surrogate as S
+    rng = np.random.default_rng(5)
+    X, cls, reg = rng.standard_normal((64, 21)), rng.integers(0, 3, 64), rng.standard_normal((64, 6))
+    a, b = (S.Surrogate(width=64, n_models=2, max_batch=32) for _ in range(2))
+    assert a.fit(X, cls, reg, epochs=2, batch=32) == b.fit(X, cls[:, None], reg.reshape(64, 2, 3), epochs=2, batch=32)
+    for p, q in zip(a.mlps, b.mlps):
+        assert bits_equal(p.get_params(), q.get_params())
+    for short in (dict(cls=cls[:40]), dict(reg=reg[:40])):
+        with pytest.raises(IndexError):
+            a.fit(X, **{**dict(cls=cls, reg=reg), **short}, epochs=1, batch=32)
+    a.close()
+    b.close()
