@@ -354,6 +354,7 @@ int sl_collision_descriptors_batch(int count, const int* n_t, const int* n_p, co
 typedef struct sl_mlp sl_mlp;
 int sl_mlp_create(sl_mlp** out, int n_in, int width, int n_out, int max_batch, unsigned long long seed);
 int sl_mlp_n_params(const sl_mlp* m);
+int sl_mlp_device(const sl_mlp* m);                      /* the device it was created on */
 int sl_mlp_get_params(sl_mlp* m, float* params);
 int sl_mlp_set_params(sl_mlp* m, const float* params);   /* also resets the Adam state */
 /* y: batch x n_out outputs; prob: batch x 3 class probabilities; ent: predictive
@@ -368,7 +369,7 @@ int sl_mlp_train_step(sl_mlp* m, int batch, const float* x, const int* cls, cons
                       float* loss);
 /* The same of several nets (same n_in and n_out, each on rows of its own), `batches` steps in a
  * row: step k of net j takes the rows idx[(k n + j) batch ..] of x, cls and reg (n_rows of each);
- * its loss goes to loss[k n + j].  Nets of the same widths and max_batch share their launches;
+ * its loss goes to loss[k n + j].  Nets of the same widths and max_batch on one device share their launches;
  * the results are those of sl_mlp_train_step for each. */
 int sl_mlp_train_rows(sl_mlp* const* nets, int n, int batch, int batches, long long n_rows, const float* x,
                       const int* cls, const float* reg, const long long* idx, float lr, float* loss);
@@ -378,7 +379,7 @@ int sl_mlp_forward_all(sl_mlp* const* nets, int n, int batch, const float* x, fl
  * (x - mean) / std in binary32: prob, the mean of their class probabilities, and reg, of their
  * regression outputs (sums in binary64, net after net); cls, the most probable class; ent, the
  * entropy (nats) of prob.  SL_E_STATE where the nets cannot share launches (more than 16, or
- * of different widths or max_batch, or wider than 512). */
+ * of different widths, max_batch or devices, or wider than 512). */
 int sl_mlp_ensemble(sl_mlp* const* nets, int n, long long rows, const double* x, const double* mean, const double* std,
                     int* cls, float* reg, double* prob, double* ent);
 const char* sl_mlp_last_error(const sl_mlp* m);   /* calls on several nets: of the net it fails on or the first */

@@ -212,6 +212,7 @@ def lib():
     L.sl_mlp_n_params.argtypes = [vp]
     L.sl_mlp_get_params.argtypes = [vp, fp]
     L.sl_mlp_set_params.argtypes = [vp, fp]
+    L.sl_mlp_device.argtypes = [vp]
     L.sl_mlp_forward.argtypes = [vp, C.c_int, fp, fp, fp, fp]
     L.sl_mlp_gradients.argtypes = [vp, C.c_int, fp, ip, fp, fp, fp]
     L.sl_mlp_train_step.argtypes = [vp, C.c_int, fp, ip, fp, C.c_float, fp]
@@ -727,6 +728,7 @@ class MLP:
         if rc:
             raise SpacelabError(rc, "sl_mlp_create")
         self.n_in, self.n_out, self.width, self.max_batch = n_in, n_out, width, max_batch
+        self.device = int(lib().sl_mlp_device(self._m))
 
     def _check(self, rc: int, what: str) -> int:
         if rc < 0:
@@ -803,11 +805,11 @@ def _mlp_call(mlps: list[MLP], what: str, *args):
 
 
 def mlp_alike(mlps: list[MLP]) -> bool:
-    """Whether the nets share launches: up to 16 different ones, of the same widths and largest
-    batch, no layer wider than 512."""
+    """Whether the nets share launches: up to 16 different ones on one device, of the same widths
+    and largest batch, no layer wider than 512."""
     if any(type(m) is not MLP for m in mlps):
         return False
-    sizes = {(m.n_in, m.width, m.n_out, m.max_batch) for m in mlps}
+    sizes = {(m.n_in, m.width, m.n_out, m.max_batch, m.device) for m in mlps}
     return 1 <= len({id(m) for m in mlps}) == len(mlps) <= 16 and len(sizes) == 1 and max(next(iter(sizes))[:3]) <= 512
 
 

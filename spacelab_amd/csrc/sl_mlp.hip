@@ -19,6 +19,7 @@
 // Output layout: y[0..2] are the class logits (stick, bounce, fragment), y[3..] are
 // regression targets.  Loss per sample: softmax cross-entropy of the logits plus the
 // mean squared error of the regression outputs; the batch loss is their mean.
+#include "sl_mlp_host.hpp"
 #include "spacelab/sl_api.h"
 
 #include <hip/hip_runtime.h>
@@ -737,6 +738,7 @@ struct Layer {
 }  // namespace
 
 struct sl_mlp {
+    int device = 0;
     int n_in = 0, width = 0, n_out = 0, max_batch = 0;
     bool chain = false;              // the chain form (layer widths up to CHAIN_MAX)
     hipStream_t stream = nullptr;
@@ -1076,12 +1078,13 @@ Adam adam_step(const sl_mlp* m, float lr)
     return Adam{lr, b1, b2, 1e-8f, 1.f - std::pow(b1, (float)t), 1.f - std::pow(b2, (float)t)};
 }
 
-// Whether one launch can carry them all: different nets in the chain form, laid out alike.
+// Whether one launch can carry them all: different nets in the chain form, laid out alike on
+// one device.
 bool alike(sl_mlp* const* ms, int n)
 {
+    auto kind = [](const sl_mlp& m) { return sl::NetKind{m.device, m.chain, m.n_in, m.width, m.n_out, m.max_batch}; };
     for (int j = 0; j < n; j++) {
-        const sl_mlp &a = *ms[0], &b = *ms[j];
-        if (!b.chain || b.n_in != a.n_in || b.width != a.width || b.n_out != a.n_out || b.max_batch != a.max_batch) return false;
+        if (!sl::shares_launch(kind(*ms[0]), kind(*ms[j]))) return false;
         for (int i = 0; i < j; i++)
             if (ms[i] == ms[j]) return false;
     }
@@ -1170,7 +1173,9 @@ int sl_mlp_create(sl_mlp** out, int n_in, int width, int n_out, int max_batch, u
         delete m;
         return code;
     };
-    if (hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking) != hipSuccess) return fail(SL_E_HIP);
+    if (hipGetDevice(&m->device) != hipSuccess ||
+        hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking) != hipSuccess)
+        return fail(SL_E_HIP);
     for (hipEvent_t& e : m->half)
         if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return fail(SL_E_HIP);
     if (hipMalloc(&m->pool, place(m, nullptr)) != hipSuccess) return fail(SL_E_HIP);
@@ -1206,6 +1211,8 @@ int sl_mlp_create(sl_mlp** out, int n_in, int width, int n_out, int max_batch, u
     *out = m;
     return SL_OK;
 }
+
+int sl_mlp_device(const sl_mlp* m) { return m ? m->device : SL_E_ARG; }
 
 int sl_mlp_n_params(const sl_mlp* m)
 {
