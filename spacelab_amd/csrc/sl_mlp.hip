@@ -1091,6 +1091,13 @@ bool alike(sl_mlp* const* ms, int n)
     return true;
 }
 
+// Waits for the net's stream; whether that and the launches before it went well.
+bool finished(const sl_mlp* m)
+{
+    const bool launched = hipGetLastError() == hipSuccess;
+    return hipStreamSynchronize(m->stream) == hipSuccess && launched;
+}
+
 // Forward, loss, backward and, with adam, the update of a labelled batch; the mean loss (of
 // the parameters before the update) to *loss.
 int train_pass(sl_mlp* m, int B, const float* x, const int* cls, const float* reg, float* loss, const Adam* adam)
@@ -1126,8 +1133,7 @@ int train_pass(sl_mlp* m, int B, const float* x, const int* cls, const float* re
                                                                       *adam);
             }
     }
-    if (hipGetLastError() != hipSuccess || hipStreamSynchronize(m->stream) != hipSuccess)
-        return mlp_err(m, SL_E_HIP, "training pass failed");
+    if (!finished(m)) return mlp_err(m, SL_E_HIP, "training pass failed");
     if (loss) *loss = mean_loss(ls, B);
     return SL_OK;
 }
@@ -1253,8 +1259,7 @@ int sl_mlp_forward(sl_mlp* m, int B, const float* x, float* y, float* prob, floa
         const Stage s(m->max_batch, m->n_in, m->n_out);
         std::memcpy(m->stage + s.x, x, 4 * (size_t)B * m->n_in);
         launch_chain<false>(&m, 1, B);
-        if (hipGetLastError() != hipSuccess || hipStreamSynchronize(m->stream) != hipSuccess)
-            return mlp_err(m, SL_E_HIP, "forward failed");
+        if (!finished(m)) return mlp_err(m, SL_E_HIP, "forward failed");
         if (y) std::memcpy(y, m->stage + s.y, 4 * (size_t)B * m->n_out);
         if (prob) std::memcpy(prob, m->stage + s.prob, 4 * (size_t)B * NCLS);
         if (ent) std::memcpy(ent, m->stage + s.ent, 4 * (size_t)B);
@@ -1306,11 +1311,7 @@ int sl_mlp_ensemble(sl_mlp* const* ms, int n, long long rows, const double* x, c
         std::memcpy(reg + nr * b0, at(m->stage, s.er, 4 * (size_t)nr, k), 4 * nr * B);
         return SL_OK;
     };
-    const long long batches = (rows + per - 1) / per;
-    const int ahead = halves ? 2 : 1;
-    for (long long k = 0; k < batches; k++) {
-        if (k >= ahead)
-            if (const int rc = collect(k - ahead)) return rc;
+    auto issue = [&](long long k) -> int {
         const int B = size(k);
         std::memcpy(at(m->stage, s.ex, 8 * (size_t)n_in, k), x + (size_t)k * per * n_in, 8 * (size_t)B * n_in);
         auto dev = [&](size_t part, size_t bytes) { return at(m->stage_dev, part, bytes, k); };
@@ -1337,10 +1338,9 @@ int sl_mlp_ensemble(sl_mlp* const* ms, int n, long long rows, const double* x, c
         k_ensemble<<<(B + 63) / 64, 64, 0, m->stream>>>(e);
         if (hipGetLastError() != hipSuccess || hipEventRecord(m->half[k % 2], m->stream) != hipSuccess)
             return mlp_err(m, SL_E_HIP, "ensemble pass failed");
-    }
-    for (long long k = std::max(0ll, batches - ahead); k < batches; k++)
-        if (const int rc = collect(k)) return rc;
-    return SL_OK;
+        return SL_OK;
+    };
+    return sl::run_ahead((rows + per - 1) / per, halves ? 2 : 1, issue, collect, [&] { (void)hipStreamSynchronize(m->stream); });
 }
 
 int sl_mlp_gradients(sl_mlp* m, int B, const float* x, const int* cls, const float* reg, float* loss, float* grads)
@@ -1377,7 +1377,7 @@ int sl_mlp_train_rows(sl_mlp* const* ms, int n, int B, int batches, long long n_
         if (ms[j]->n_in != ms[0]->n_in || ms[j]->n_out != ms[0]->n_out)
             return mlp_err(ms[j], SL_E_ARG, "nets of one ensemble have the same inputs and outputs");
     }
-    auto at = [&](int k, int j) { return idx + ((size_t)k * n + j) * B; };   // rows of batch k of net j
+    auto at = [&](long long k, int j) { return idx + ((size_t)k * n + j) * B; };   // rows of batch k of net j
     for (size_t e = 0; e < (size_t)batches * n * B; e++) {
         sl_mlp* m = ms[e / B % n];
         if (idx[e] < 0 || idx[e] >= n_rows) return mlp_err(m, SL_E_ARG, "row index outside the data");
@@ -1415,8 +1415,8 @@ int sl_mlp_train_rows(sl_mlp* const* ms, int n, int B, int batches, long long n_
     for (int j0 = 0; j0 < n; j0 += MEMBERS) {
         const int g = std::min(n - j0, MEMBERS);
         sl_mlp* const* mg = ms + j0;
-        auto part = [&](sl_mlp* m, size_t p, size_t bytes, int k) { return m->stage + p + k % ahead * half * bytes; };
-        auto collect = [&](int k) -> int {
+        auto part = [&](sl_mlp* m, size_t p, size_t bytes, long long k) { return m->stage + p + k % ahead * half * bytes; };
+        auto collect = [&](long long k) -> int {
             if (hipEventSynchronize(mg[0]->half[k % 2]) != hipSuccess) return mlp_err(ms[0], SL_E_HIP, "training pass failed");
             for (int j = 0; loss && j < g; j++)
                 loss[(size_t)k * n + j0 + j] = mean_loss(reinterpret_cast<const float*>(part(mg[j], s.loss, 4, k)), B);
@@ -1424,14 +1424,11 @@ int sl_mlp_train_rows(sl_mlp* const* ms, int n, int B, int batches, long long n_
         };
         ChainArgs c = chain_args(mg, g, B, false);
         const ChainArgs c0 = c;
-        for (int k = 0; k < batches; k++) {
-            if (k >= ahead)
-                if (const int rc = collect(k - ahead)) return rc;
+        auto issue = [&](long long k) -> int {
             Adam adam[MEMBERS];
             for (int j = 0; j < g; j++) {
                 sl_mlp* m = mg[j];
                 adam[j] = adam_step(m, lr);
-                m->t++;
                 rows(at(k, j0 + j), reinterpret_cast<float*>(part(m, s.x, 4 * (size_t)n_in, k)),
                      reinterpret_cast<int*>(part(m, s.cls, 4, k)), reinterpret_cast<float*>(part(m, s.reg, 4 * (size_t)nr, k)));
             }
@@ -1444,9 +1441,10 @@ int sl_mlp_train_rows(sl_mlp* const* ms, int n, int B, int batches, long long n_
             launch_wgrad<true>(mg, g, B, adam);
             if (hipGetLastError() != hipSuccess || hipEventRecord(mg[0]->half[k % 2], mg[0]->stream) != hipSuccess)
                 return mlp_err(ms[0], SL_E_HIP, "training pass failed");
-        }
-        for (int k = std::max(0, batches - ahead); k < batches; k++)
-            if (const int rc = collect(k)) return rc;
+            for (int j = 0; j < g; j++) mg[j]->t++;   // a step that was sent
+            return SL_OK;
+        };
+        if (const int rc = sl::run_ahead(batches, ahead, issue, collect, [&] { (void)hipStreamSynchronize(mg[0]->stream); })) return rc;
     }
     return SL_OK;
 }
@@ -1468,8 +1466,7 @@ int sl_mlp_forward_all(sl_mlp* const* ms, int n, int B, const float* x, float* y
         if (together) {
             std::memcpy(ms[j0]->stage + s.x, x, 4 * (size_t)B * ms[0]->n_in);
             launch_chain<false>(ms + j0, k, B);
-            if (hipGetLastError() != hipSuccess || hipStreamSynchronize(ms[j0]->stream) != hipSuccess)
-                return mlp_err(ms[0], SL_E_HIP, "forward failed");
+            if (!finished(ms[j0])) return mlp_err(ms[0], SL_E_HIP, "forward failed");
         }
         for (int j = j0; j < j0 + k; j++) {
             float *yj = y ? y + j * ny : nullptr, *pj = prob ? prob + j * np : nullptr, *ej = ent ? ent + (size_t)j * B : nullptr;

@@ -17,4 +17,21 @@ inline bool shares_launch(const NetKind& a, const NetKind& b)
            a.max_batch == b.max_batch;
 }
 
+// n passes with `ahead` of them in flight: issue(k) sends pass k, collect(k) waits for it and
+// takes its results, in order.  After a failure nothing more is sent and wait() is called, so
+// that no launch outlives the call, whose buffers the next call writes.  Returns the first
+// nonzero code.
+template <class Issue, class Collect, class Wait>
+int run_ahead(long long n, int ahead, Issue issue, Collect collect, Wait wait)
+{
+    int rc = 0;
+    for (long long k = 0; k < n && !rc; k++) {
+        if (k >= ahead) rc = collect(k - ahead);
+        if (!rc) rc = issue(k);
+    }
+    for (long long k = n > ahead ? n - ahead : 0; k < n && !rc; k++) rc = collect(k);
+    if (rc) wait();
+    return rc;
+}
+
 }  // namespace sl

@@ -25,8 +25,46 @@ static void sharing()
     for (const NetKind& x : b) check(!shares_launch(a, x) && !shares_launch(x, a), "nets of another device, form or size do not");
 }
 
+// Passes 0 .. n - 1 with issue or collect of pass `bad` failing (-1: none).
+static void ahead(long long n, int in_flight, long long bad, bool in_issue)
+{
+    long long issued = 0, collected = 0, waits = 0;
+    bool order = true;
+    const int rc = run_ahead(
+        n, in_flight,
+        [&](long long k) {
+            order = order && k == issued && issued - collected < in_flight && waits == 0;
+            if (in_issue && k == bad) return -2;
+            issued++;
+            return 0;
+        },
+        [&](long long k) {
+            order = order && k == collected && k < issued && waits == 0;
+            if (!in_issue && k == bad) return -3;
+            collected++;
+            return 0;
+        },
+        [&] { waits++; });
+    check(order, "passes in order, no more in flight than asked");
+    if (bad < 0) {
+        check(rc == 0 && issued == n && collected == n && waits == 0, "every pass sent and collected");
+    } else {
+        check(rc == (in_issue ? -2 : -3), "the first failure is returned");
+        check(waits == 1, "after a failure the work in flight is waited for");
+        check(in_issue ? issued == bad : collected == bad, "nothing after the failure");
+    }
+}
+
 int main()
 {
     sharing();
+    for (long long n = 0; n < 6; n++)
+        for (int a = 1; a < 3; a++) {
+            ahead(n, a, -1, true);
+            for (long long bad = 0; bad < n; bad++) {
+                ahead(n, a, bad, true);
+                ahead(n, a, bad, false);
+            }
+        }
     return 0;
 }

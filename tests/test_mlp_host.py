@@ -1,5 +1,5 @@
 """Host rules of the surrogate network that a machine without a GPU can check: which nets one
-launch may carry."""
+launch may carry, and that passes sent ahead are waited for when one of them fails."""
 import os
 import subprocess
 
