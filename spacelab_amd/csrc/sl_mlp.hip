@@ -749,9 +749,11 @@ struct sl_mlp {
     char* pool = nullptr;
     size_t n_flat = 0;
     float *params = nullptr, *grads = nullptr, *moments = nullptr;
-    // One pinned host allocation: a batch and its results in the chain form (the kernels
-    // read and write it), the padded parameters during exchanges.
+    // One pinned host allocation (sl::pinned_bytes): a batch and its results in the chain form
+    // (the kernels read and write it), the losses in the layer form, the padded parameters, or a
+    // piece of them, during exchanges.
     char* stage = nullptr;
+    size_t stage_bytes = 0;
     char* stage_dev = nullptr;       // its device address
     hipEvent_t half[2] = {};         // an ensemble's batches in flight
     // chain form: activations and output gradients, feature-major, and the gradients in binary32
@@ -886,19 +888,52 @@ size_t place(sl_mlp* m, char* base)
     return o;
 }
 
-// Parameters already padded in the pinned buffer: to the device, with their bfloat16 copies.
-int push_params(sl_mlp* m)
+// Waits for the net's stream; whether that and the launches before it went well.
+bool finished(const sl_mlp* m)
 {
-    if (hipMemcpyAsync(m->params, m->stage, sizeof(float) * m->n_flat, hipMemcpyHostToDevice, m->stream) != hipSuccess)
-        return SL_E_HIP;
+    const bool launched = hipGetLastError() == hipSuccess;
+    return hipStreamSynchronize(m->stream) == hipSuccess && launched;
+}
+
+// The padded floats [f0, f1) of the parameters' layout that the caller's unpadded one has too:
+// f(padded offset, unpadded offset, count) for each run of them.
+template <class F>
+void each_run(const sl_mlp* m, size_t f0, size_t f1, F f)
+{
+    size_t user = 0;
+    for (const Layer& L : m->L) {
+        auto rows = [&](const float* start, size_t count) {
+            const size_t at = start - m->params, ld = L.ldout, len = L.out;
+            for (size_t i = f0 > at ? (f0 - at) / ld : 0; i < count && at + i * ld < f1; i++) {
+                const size_t lo = std::max(at + i * ld, f0), hi = std::min(at + i * ld + len, f1);
+                if (lo < hi) f(lo, user + lo - at - i * (ld - len), hi - lo);
+            }
+            user += count * len;
+        };
+        rows(L.W, L.in);
+        rows(L.b, 1);
+    }
+}
+
+// The caller's parameters to the device, padded, with their bfloat16 copies.
+int push_params(sl_mlp* m, const float* w)
+{
+    float* host = reinterpret_cast<float*>(m->stage);
+    const size_t per = m->stage_bytes / sizeof(float);
+    for (size_t f0 = 0; f0 < m->n_flat; f0 += per) {
+        const size_t n = std::min(per, m->n_flat - f0);
+        std::memset(host, 0, sizeof(float) * n);
+        each_run(m, f0, f0 + n, [&](size_t at, size_t user, size_t c) { std::memcpy(host + (at - f0), w + user, sizeof(float) * c); });
+        if (hipMemcpyAsync(m->params + f0, host, sizeof(float) * n, hipMemcpyHostToDevice, m->stream) != hipSuccess ||
+            (f0 + n < m->n_flat && hipStreamSynchronize(m->stream) != hipSuccess))
+            return SL_E_HIP;
+    }
     for (Layer& L : m->L) {
         const int nw = L.ldin * L.ldout;
         k_weights_bf16<<<(nw + 255) / 256, 256, 0, m->stream>>>(L.ldin, L.ldout, L.W, L.Wb, L.Wf, L.Wr);
     }
-    if (hipGetLastError() != hipSuccess ||
-        hipMemsetAsync(m->moments, 0, 2 * sizeof(float) * m->n_flat, m->stream) != hipSuccess ||
-        hipStreamSynchronize(m->stream) != hipSuccess)
-        return SL_E_HIP;
+    const bool ok = hipMemsetAsync(m->moments, 0, 2 * sizeof(float) * m->n_flat, m->stream) == hipSuccess;
+    if (!finished(m) || !ok) return SL_E_HIP;
     m->t = 0;
     return SL_OK;
 }
@@ -906,15 +941,14 @@ int push_params(sl_mlp* m)
 // A flat device block (parameters or gradients) into the caller's unpadded layout.
 int pull_flat(sl_mlp* m, const float* dev, float* out)
 {
-    if (hipMemcpyAsync(m->stage, dev, sizeof(float) * m->n_flat, hipMemcpyDeviceToHost, m->stream) != hipSuccess ||
-        hipStreamSynchronize(m->stream) != hipSuccess)
-        return SL_E_HIP;
     const float* host = reinterpret_cast<const float*>(m->stage);
-    for (Layer& L : m->L) {
-        const float *W = host + (L.W - m->params), *b = host + (L.b - m->params);
-        for (int i = 0; i < L.in; i++, out += L.out) std::memcpy(out, W + (size_t)i * L.ldout, sizeof(float) * L.out);
-        std::memcpy(out, b, sizeof(float) * L.out);
-        out += L.out;
+    const size_t per = m->stage_bytes / sizeof(float);
+    for (size_t f0 = 0; f0 < m->n_flat; f0 += per) {
+        const size_t n = std::min(per, m->n_flat - f0);
+        if (hipMemcpyAsync(m->stage, dev + f0, sizeof(float) * n, hipMemcpyDeviceToHost, m->stream) != hipSuccess ||
+            hipStreamSynchronize(m->stream) != hipSuccess)
+            return SL_E_HIP;
+        each_run(m, f0, f0 + n, [&](size_t at, size_t user, size_t c) { std::memcpy(out + user, host + (at - f0), sizeof(float) * c); });
     }
     return SL_OK;
 }
@@ -1091,13 +1125,6 @@ bool alike(sl_mlp* const* ms, int n)
     return true;
 }
 
-// Waits for the net's stream; whether that and the launches before it went well.
-bool finished(const sl_mlp* m)
-{
-    const bool launched = hipGetLastError() == hipSuccess;
-    return hipStreamSynchronize(m->stream) == hipSuccess && launched;
-}
-
 // Forward, loss, backward and, with adam, the update of a labelled batch; the mean loss (of
 // the parameters before the update) to *loss.
 int train_pass(sl_mlp* m, int B, const float* x, const int* cls, const float* reg, float* loss, const Adam* adam)
@@ -1106,7 +1133,7 @@ int train_pass(sl_mlp* m, int B, const float* x, const int* cls, const float* re
         if (cls[b] < 0 || cls[b] >= NCLS) return mlp_err(m, SL_E_ARG, "class label outside 0..2");
     const int nr = m->n_out - NCLS;
     const Stage s(m->max_batch, m->n_in, m->n_out);
-    const float* ls = reinterpret_cast<const float*>(m->stage + s.loss);
+    const float* ls = reinterpret_cast<const float*>(m->stage + (m->chain ? s.loss : 0));
     if (m->chain) {
         std::memcpy(m->stage + s.x, x, 4 * (size_t)B * m->n_in);
         std::memcpy(m->stage + s.cls, cls, 4 * (size_t)B);
@@ -1122,7 +1149,7 @@ int train_pass(sl_mlp* m, int B, const float* x, const int* cls, const float* re
         const Layer& L = m->L[NL - 1];
         k_loss<<<(B + 255) / 256, 256, 0, m->stream>>>(B, m->n_out, L.ldout, m->Z[NL - 1], m->cls, m->reg,
                                                        m->dZ[NL - 1], m->dZb[NL - 1], m->loss_s);
-        if (hipMemcpyAsync(m->stage + s.loss, m->loss_s, 4 * (size_t)B, hipMemcpyDeviceToHost, m->stream) != hipSuccess)
+        if (hipMemcpyAsync(m->stage, m->loss_s, 4 * (size_t)B, hipMemcpyDeviceToHost, m->stream) != hipSuccess)
             return mlp_err(m, SL_E_HIP, "loss read-back failed");
         backward(m, B);
         if (adam)
@@ -1192,11 +1219,11 @@ int sl_mlp_create(sl_mlp** out, int n_in, int width, int n_out, int max_batch, u
             if (hipMemsetAsync(L.Wf, 0, 2 * (size_t)32 * k_steps(L.ldin) * L.ldout, m->stream) != hipSuccess ||
                 hipMemsetAsync(L.Wr, 0, 2 * (size_t)32 * k_steps(L.ldout) * L.ldin, m->stream) != hipSuccess)
                 return fail(SL_E_HIP);
-    const size_t stage = std::max(Stage(max_batch, n_in, n_out).end, sizeof(float) * m->n_flat);
-    if (hipHostMalloc(&m->stage, stage, 0) != hipSuccess ||
+    m->stage_bytes = sl::pinned_bytes(m->chain, Stage(max_batch, n_in, n_out).end, sizeof(float) * m->n_flat, max_batch);
+    if (hipHostMalloc(&m->stage, m->stage_bytes, 0) != hipSuccess ||
         hipHostGetDevicePointer(reinterpret_cast<void**>(&m->stage_dev), m->stage, 0) != hipSuccess)
         return fail(SL_E_HIP);
-    // He-uniform initialisation from a SplitMix64 stream; padded entries are zero
+    // He-uniform initialisation from a SplitMix64 stream
     uint64_t s = seed;
     auto rnd = [&]() {
         uint64_t z = (s += 0x9E3779B97F4A7C15ull);
@@ -1205,15 +1232,16 @@ int sl_mlp_create(sl_mlp** out, int n_in, int width, int n_out, int max_batch, u
         z ^= z >> 31;
         return ((z >> 11) + 0.5) * (1.0 / 9007199254740992.0);
     };
-    float* host = reinterpret_cast<float*>(m->stage);
-    std::memset(host, 0, sizeof(float) * m->n_flat);
-    for (Layer& L : m->L) {
-        float* W = host + (L.W - m->params);
+    float* w = new (std::nothrow) float[sl_mlp_n_params(m)], *next = w;
+    if (!w) return fail(SL_E_STATE);
+    for (const Layer& L : m->L) {
         const double lim = std::sqrt(6.0 / L.in);
-        for (int i = 0; i < L.in; i++)
-            for (int j = 0; j < L.out; j++) W[(size_t)i * L.ldout + j] = (float)((2 * rnd() - 1) * lim);
+        for (int e = 0; e < L.in * L.out; e++) *next++ = (float)((2 * rnd() - 1) * lim);
+        for (int e = 0; e < L.out; e++) *next++ = 0.f;
     }
-    if (push_params(m)) return fail(SL_E_HIP);
+    const int rc = push_params(m, w);
+    delete[] w;
+    if (rc) return fail(SL_E_HIP);
     *out = m;
     return SL_OK;
 }
@@ -1239,15 +1267,7 @@ int sl_mlp_get_params(sl_mlp* m, float* w)
 int sl_mlp_set_params(sl_mlp* m, const float* w)
 {
     if (!m || !w) return SL_E_ARG;
-    float* host = reinterpret_cast<float*>(m->stage);
-    std::memset(host, 0, sizeof(float) * m->n_flat);
-    for (Layer& L : m->L) {
-        float *W = host + (L.W - m->params), *b = host + (L.b - m->params);
-        for (int i = 0; i < L.in; i++, w += L.out) std::memcpy(W + (size_t)i * L.ldout, w, sizeof(float) * L.out);
-        std::memcpy(b, w, sizeof(float) * L.out);
-        w += L.out;
-    }
-    if (push_params(m)) return mlp_err(m, SL_E_HIP, "parameter upload failed");
+    if (push_params(m, w)) return mlp_err(m, SL_E_HIP, "parameter upload failed");
     return SL_OK;
 }
 

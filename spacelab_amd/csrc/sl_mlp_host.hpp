@@ -1,7 +1,22 @@
 // Host-side rules of the surrogate network (sl_mlp.hip) that need no GPU to be checked.
 #pragma once
 
+#include <algorithm>
+#include <cstddef>
+
 namespace sl {
+
+// Pinned host memory a net holds for life.  In the chain form: a batch and its results, which the
+// kernels read and write there, or the padded parameters during exchanges (at most 4.3 MB,
+// CHAIN_MAX wide).  In the layer form a batch's losses or a piece of the parameters: all of
+// them are 136 MB at width 4096, more than many nets can pin.  (Through unpinned memory of
+// the exchange's own: width 1024 read in 770 us instead of 430, 4096 in 41 ms instead of 11.)
+inline size_t pinned_bytes(bool chain, size_t batch_bytes, size_t params_bytes, int max_batch)
+{
+    const size_t piece = (size_t)4 << 20;
+    return chain ? std::max(batch_bytes, params_bytes)
+                 : std::max(sizeof(float) * (size_t)max_batch, std::min(params_bytes, piece));
+}
 
 // What decides whether nets are laid out alike, so that one launch can carry them: a member's
 // memory is then the first member's, moved by a distance, on the same device.

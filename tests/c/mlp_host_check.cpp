@@ -55,9 +55,20 @@ static void ahead(long long n, int in_flight, long long bad, bool in_issue)
     }
 }
 
+static void pinned()
+{
+    const size_t wide = (size_t)136 << 20, batch = 1 << 20, narrow = 600 << 10;
+    check(pinned_bytes(false, batch, wide, 4096) == 4 << 20, "a wide net in the layer form pins a piece of its parameters");
+    check(pinned_bytes(false, wide, narrow, 64) == narrow && pinned_bytes(false, wide, narrow, 1 << 20) == 4 << 20,
+          "a net in the layer form pins its losses and no batch");
+    check(pinned_bytes(true, batch, narrow, 4096) == batch && pinned_bytes(true, narrow, batch, 4096) == batch,
+          "a net in the chain form pins what a batch and an exchange need");
+}
+
 int main()
 {
     sharing();
+    pinned();
     for (long long n = 0; n < 6; n++)
         for (int a = 1; a < 3; a++) {
             ahead(n, a, -1, true);

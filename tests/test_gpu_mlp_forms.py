@@ -49,3 +49,26 @@ def test_gradients_and_step(n_in, width, n_out, B):
     yo1 = M.forward(new, x, emulate=True)[0][-1]
     assert np.abs(y1 - yo1).max() <= 2e-3 * np.abs(yo1).max()
     assert loss1 == pytest.approx(M.loss_and_grads(new, x, cls, reg, emulate=True)[0], rel=1e-5)
+
+
+@pytest.mark.parametrize("n_in,width,n_out", [(21, 256, 9), (37, 1000, 10), (1500, 720, 9), (3, 1024, 2000)])
+def test_parameters_exchanged_in_pieces(n_in, width, n_out):
+    """Wide nets' parameters pass through pinned memory of 4 MB at a time, cut anywhere in a row:
+    read back as set, and each where it belongs."""
+    rng = np.random.default_rng(width)
+    dims, B = [n_in, width, width, width, n_out], 3
+    x = rng.standard_normal((B, n_in)).astype(np.float32)
+    cls, reg = np.zeros(B, np.int32), rng.standard_normal((B, n_out - 3)).astype(np.float32)
+    with sl.MLP(n_in, n_out, width, max_batch=B, seed=5) as m:
+        w = m.get_params() + np.float32(0.02) * rng.standard_normal(m.n_params).astype(np.float32)
+        m.set_params(w)
+        assert np.array_equal(m.get_params(), w)
+        y = m.forward(x)[0]
+        _, g = m.gradients(x, cls, reg)
+    layers = M.unflatten(w.astype(np.float64), dims)
+    yo = M.forward(layers, x, emulate=True)[0][-1]
+    assert np.abs(y - yo).max() <= 2e-3 * np.abs(yo).max()
+    go = M.loss_and_grads(layers, x, cls, reg, emulate=True)[1]
+    for k, (got, want) in enumerate(zip(M.unflatten(g.astype(np.float64), dims), go)):
+        for a, o in zip(got, want):
+            assert np.linalg.norm(a - o) <= 2e-3 * np.linalg.norm(o), k
