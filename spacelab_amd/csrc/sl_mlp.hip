@@ -31,7 +31,6 @@
 #include <new>
 #include <string>
 #include <type_traits>
-#include <vector>
 
 namespace {
 
@@ -1289,17 +1288,22 @@ int sl_mlp_forward(sl_mlp* m, int B, const float* x, float* y, float* prob, floa
     forward(m, B);
     const Layer& L = m->L[NL - 1];
     k_predict<<<(B + 255) / 256, 256, 0, m->stream>>>(B, L.ldout, m->Z[NL - 1], m->prob, m->ent);
-    std::vector<float> z((size_t)B * L.ldout);
-    if (hipMemcpyAsync(z.data(), m->Z[NL - 1], 4 * z.size(), hipMemcpyDeviceToHost, m->stream) != hipSuccess)
-        return mlp_err(m, SL_E_HIP, "output read-back failed");
     if (prob && hipMemcpyAsync(prob, m->prob, 4 * (size_t)B * NCLS, hipMemcpyDeviceToHost, m->stream) != hipSuccess)
         return mlp_err(m, SL_E_HIP, "probability read-back failed");
     if (ent && hipMemcpyAsync(ent, m->ent, 4 * (size_t)B, hipMemcpyDeviceToHost, m->stream) != hipSuccess)
         return mlp_err(m, SL_E_HIP, "entropy read-back failed");
-    if (hipStreamSynchronize(m->stream) != hipSuccess) return mlp_err(m, SL_E_HIP, "forward failed");
-    if (y)
-        for (int b = 0; b < B; b++)
-            for (int k = 0; k < m->n_out; k++) y[(size_t)b * m->n_out + k] = z[(size_t)b * L.ldout + k];
+    if (!finished(m)) return mlp_err(m, SL_E_HIP, "forward failed");
+    // the outputs through the pinned buffer, whole padded rows at a time
+    const int per = (int)std::min<size_t>(B, m->stage_bytes / (4 * (size_t)L.ldout));
+    for (int b0 = 0; y && b0 < B; b0 += per) {
+        const int n = std::min(per, B - b0);
+        if (hipMemcpyAsync(m->stage, m->Z[NL - 1] + (size_t)b0 * L.ldout, 4 * (size_t)n * L.ldout, hipMemcpyDeviceToHost, m->stream) !=
+                hipSuccess ||
+            hipStreamSynchronize(m->stream) != hipSuccess)
+            return mlp_err(m, SL_E_HIP, "output read-back failed");
+        for (int b = 0; b < n; b++)
+            std::memcpy(y + (size_t)(b0 + b) * m->n_out, m->stage + 4 * (size_t)b * L.ldout, 4 * (size_t)m->n_out);
+    }
     return SL_OK;
 }
 

@@ -72,3 +72,14 @@ def test_parameters_exchanged_in_pieces(n_in, width, n_out):
     for k, (got, want) in enumerate(zip(M.unflatten(g.astype(np.float64), dims), go)):
         for a, o in zip(got, want):
             assert np.linalg.norm(a - o) <= 2e-3 * np.linalg.norm(o), k
+
+
+@pytest.mark.parametrize("B", [1, 17, 18, 40])
+def test_wide_outputs_read_in_pieces(B):
+    """The layer form's outputs pass through the pinned buffer, here 17 rows of 608 at a time."""
+    x = np.random.default_rng(B).standard_normal((B, 21)).astype(np.float32)
+    with sl.MLP(21, 600, 16, max_batch=64, seed=2) as m:
+        y, p, e = m.forward(x)
+        for b in range(B):
+            for all_rows, one in zip((y, p, e), m.forward(x[b:b + 1])):
+                assert np.array_equal(all_rows[b], one[0]), b
