@@ -45,6 +45,12 @@ struct GlobalContact {
 
 __device__ __forceinline__ D3 load3(const State& s, int f, int b) { return d3(s.f[f][b], s.f[f + 1][b], s.f[f + 2][b]); }
 
+// Lanes of the mask below this one.
+__device__ __forceinline__ int lanes_below(unsigned long long mask)
+{
+    return __builtin_popcountll(mask & ((1ull << (threadIdx.x % 64)) - 1));
+}
+
 template <int N>
 __device__ __forceinline__ double block_sum(double v, double* red)
 {
@@ -144,6 +150,12 @@ struct PartnerRec {
     double x, y, z, R, m, pref;
 };
 
+// A ball of the workgroup: position, radius, mass, 1/m (divisions by m through div_rcp) and its
+// factors of the reference's products when it is A (Ha/6*64 Ra^3, G mA).
+struct BallRec {
+    double x, y, z, R, m, ym, pref, Gm;
+};
+
 // The pair pass as a ring of wavefronts.  A workgroup owns NB balls and its W wavefronts take
 // the partners in batches of BP = CH * 64/NB, batch m by wavefront m mod W:
 //   evaluate  lane (ball l % NB, slot l / NB) evaluates CH pairs of its ball, one per step q,
@@ -165,14 +177,21 @@ struct PartnerRec {
 // needs: sums, then turn; turn, then sums.
 //
 // Touching pairs.  The contact arm is five times the far arm's instructions, for one or two
-// lanes of a wavefront.  With SCAN the workgroup first tests its balls against every partner
+// lanes of a wavefront, so a batch's touching pairs are numbered and evaluated side by side, up
+// to 64 at a time, before the turn (64 AD of them: beyond, ab is used again and the turn has to
+// come first).  Evaluated step by step, by the lanes that met them, and after the first AD steps
+// within the turn, a ball with a thousand contacts took 180 us a step at 1,000 balls and 836 at
+// 5,000; now 44 and 157, and 129 ordinary balls 8.4 instead of 9.6, 1,000 18.7 instead of 19.3.
+// With SCAN the workgroup first tests its balls against every partner
 // (16 instructions a step), and one wavefront evaluates the touching pairs found, up to
 // 64, side by side while the others start on their batches; a pair met in the sweep is then
 // copied from that table.  Pairs that did not fit in it, and all touching pairs without SCAN,
-// are evaluated where they are met, those of the first AD steps before the turn.  The scan
+// are evaluated in their batch.  The scan
 // pays up to about 2,500 balls (4 balls, 4 wavefronts, us per step with / without: 2,000 balls
 // 43.7 / 45.4, 3,000 77 / 73.5, 5,000 175 / 161): its cost grows with the partners, what it
 // saves only with the contacts.
+// While contacts are evaluated a lane's own ball waits in LDS (BallRec): in registers it took
+// 26 spills more, the next batch's partners among them, which then had to arrive first.
 //
 // Bound by the binary64 pipe: 131 VALU instructions a step of 64 evaluations (105 of them the
 // reference's arithmetic), 150-170 with the staging, the adding and the contacts; at 15,039
@@ -214,10 +233,13 @@ void k_pairs_ordered(OrdState os, Phys P, int n, double* __restrict__ pe_ball,
     // the adding lanes' 16-byte reads each cover every LDS bank once.
     constexpr int RS = (BP + 31) / 32 * 32 + 32 / NB, CS = NB * RS + 2;
     constexpr int AH = BP < 16 ? BP : 16;   // contributions a lane adds from registers at once
-    static_assert(64 % NB == 0 && BP <= 64 && NQ * NB <= 64 && BP % AH == 0 && CH <= 32, "batch shape");
+    static_assert(64 % NB == 0 && BP <= 64 && NQ * NB <= 64 && BP % AH == 0 && CH <= 4, "batch shape");
     __shared__ __attribute__((aligned(16))) double cb[W][NQ][CS];   // acc contributions (and energies)
-    __shared__ double ab[W][AD][3][64];     // aacc contributions of AD steps' touching pairs, by lane
+    constexpr int AE = 64 * AD;             // touching pairs of a batch evaluated before its turn
+    __shared__ double ab[W][3][AE];         // their aacc contributions, by number
+    __shared__ unsigned char numbered[W][AE];   // their step << 6 | lane
     __shared__ PartnerRec sp[W][BP];
+    __shared__ BallRec ball[NB];
     __shared__ double run[7][NB];           // the sums: acc xyz, aacc xyz, energy
     __shared__ double own[3][3][NB];        // half-step velocities and spins, positions: for the kick and the drift
     __shared__ int turn, ready, found;
@@ -244,16 +266,12 @@ void k_pairs_ordered(OrdState os, Phys P, int n, double* __restrict__ pe_ball,
     const int il = l % NB, jq = l / NB;
     const int i0 = blockIdx.x * NB, i = i0 + il;
     const bool iv = i < n;
-    const int ic = iv ? i : 0;
-    const D3 pi = d3(s.f[PX][ic], s.f[PY][ic], s.f[PZ][ic]);
-    const double Ri = s.f[RAD][ic], mi = s.f[MASS][ic];
-    const double ymi = 1.0 / mi;             // divisions by m_i through div_rcp
-    // ball i's factors of the reference's products when it is A (2 Ra, 4 Ra, Ha/6*64 Ra^3, G mA)
-    const double two_Ri = 2 * Ri, four_Ri = 4 * Ri;
     const double Hc = P.Ha / 6 * 64;
-    const double prefA = Hc * Ri * Ri * Ri;
-    const double Gmi = P.G * mi;
-    const bool gen_i = !FarRange::params(P) || !FarRange::ball(Ri, mi);
+    if (t < NB) {
+        const int b = i0 + t < n ? i0 + t : 0;
+        const double R = s.f[RAD][b], mass = s.f[MASS][b];
+        ball[t] = BallRec{s.f[PX][b], s.f[PY][b], s.f[PZ][b], R, mass, 1.0 / mass, Hc * R * R * R, P.G * mass};
+    }
     unsigned cnt = 0;
 
     const int nm = (n + BP - 1) / BP;        // batches
@@ -265,10 +283,12 @@ void k_pairs_ordered(OrdState os, Phys P, int n, double* __restrict__ pe_ball,
     };
     load_batch(w);
     __syncthreads();
-    // Pair (ball bi, partner j) in full, by the touching arm where it holds: acc and aacc
-    // contributions to c3[0], c3[cs], .. and a3[0], a3[as], ..; returns 1 if it touches.
-    auto contact = [&](int bi, int j, const D3& pb, double Rb, double mb, double ymb, double* c3, int cs, double* a3,
-                       int as, double* pe) -> int {
+    // Pair (ball bl of the workgroup, partner j) in full, by the touching arm where it holds: acc
+    // and aacc contributions to c3[0], c3[cs], .. and a3[0], a3[as], ..; returns 1 if it touches.
+    auto contact = [&](int bl, int j, double* c3, int cs, double* a3, int as, double* pe) -> int {
+        const int bi = i0 + bl;
+        const D3 pb = d3(ball[bl].x, ball[bl].y, ball[bl].z);
+        const double Rb = ball[bl].R, mb = ball[bl].m, ymb = ball[bl].ym;
         const bool iA = bi > j;
         const D3 pj = d3(s.f[PX][j], s.f[PY][j], s.f[PZ][j]);
         const double Rj = s.f[RAD][j], mj = s.f[MASS][j];
@@ -304,6 +324,8 @@ void k_pairs_ordered(OrdState os, Phys P, int n, double* __restrict__ pe_ball,
         // every wavefront scans every W-th group of JS partners; a superset of the touching
         // pairs (d^2 against S^2, a little enlarged)
         constexpr int SU = 4;   // groups whose loads are in flight together
+        const D3 pi = d3(ball[il].x, ball[il].y, ball[il].z);
+        const double Ri = ball[il].R;
         for (int j1 = w * JS + jq; j1 - jq < n; j1 += SU * W * JS) {
             D3 pj[SU];
             double Rj[SU];
@@ -330,11 +352,8 @@ void k_pairs_ordered(OrdState os, Phys P, int n, double* __restrict__ pe_ball,
             __builtin_amdgcn_s_setprio(3);
             if (l < nt) {
                 const unsigned key = tkey[l];
-                const int bi = i0 + (int)(key >> 24), j = (int)(key & 0xffffffu);
-                const D3 pb = d3(s.f[PX][bi], s.f[PY][bi], s.f[PZ][bi]);
-                const double mb = s.f[MASS][bi];
                 double pe = 0;
-                const int touch = contact(bi, j, pb, s.f[RAD][bi], mb, 1.0 / mb, &tres[l][0], 1, &tres[l][3], 1, &pe);
+                const int touch = contact((int)(key >> 24), (int)(key & 0xffffffu), &tres[l][0], 1, &tres[l][3], 1, &pe);
                 if (WRITE) tres[l][6] = pe;
                 if (!touch) tkey[l] = ~0u;
             }
@@ -344,6 +363,22 @@ void k_pairs_ordered(OrdState os, Phys P, int n, double* __restrict__ pe_ball,
         }
     }
     bool have_table = false;
+    const bool gen_i = !FarRange::params(P) || !FarRange::ball(ball[il].R, ball[il].m);
+    // this lane's ball, read again after contacts, which have its registers meanwhile
+    D3 pi;
+    double Ri, mi, ymi, prefA, Gmi, two_Ri, four_Ri;
+    auto load_ball = [&]() {
+        const BallRec& b = ball[il];
+        pi = d3(b.x, b.y, b.z);
+        Ri = b.R;
+        mi = b.m;
+        ymi = b.ym;
+        prefA = b.pref;
+        Gmi = b.Gm;
+        two_Ri = 2 * Ri;
+        four_Ri = 4 * Ri;
+    };
+    load_ball();
 
 #pragma unroll 1
     for (int m = w; m < nm; m += W) {
@@ -434,44 +469,14 @@ void k_pairs_ordered(OrdState os, Phys P, int n, double* __restrict__ pe_ball,
         asm volatile("" ::: "memory");
 
         __builtin_amdgcn_s_setprio(3);
-        // the lanes of step q with a touching pair, and their contributions into cb and ab
-        auto touching = [&](int q, int d) -> unsigned long long {
-            bool mine = (pend >> q) & 1u;
-            unsigned long long lanes = __ballot(mine);
-            unsigned long long out = 0;
-            if constexpr (SCAN) {
-                if (!have_table) {
-                    while (!__builtin_amdgcn_readfirstlane(__hip_atomic_load(&ready, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP))) {
-                    }
-                    asm volatile("" ::: "memory");
-                    if (l < min(found, 64)) mykey = tkey[l];
-                    have_table = true;
+        auto get_table = [&]() {
+            if (!have_table) {
+                while (!__builtin_amdgcn_readfirstlane(__hip_atomic_load(&ready, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP))) {
                 }
-                for (unsigned long long z = lanes; z; z &= z - 1) {
-                    const int ln = __ffsll((long long)z) - 1;
-                    const unsigned key = (unsigned)(ln % NB) << 24 | (unsigned)(j0 + JS * q + ln / NB);
-                    const unsigned long long hit = __ballot(mykey == key);
-                    if (!hit) continue;
-                    const int e = __ffsll((long long)hit) - 1;
-                    const int o_ = ln % NB * RS + JS * q + ln / NB;
-                    if (l < 3) cb[w][l][o_] = tres[e][l];
-                    else if (l < 6) ab[w][d][l - 3][ln] = tres[e][l];
-                    else if (WRITE && l == 6) cb[w][NQ - 1][o_] = tres[e][6];
-                    out |= 1ull << ln;
-                    if (l == ln) mine = false;
-                }
-                if (((out >> l) & 1ull) && i > j0 + JS * q + jq) cnt++;
+                asm volatile("" ::: "memory");
+                if (l < min(found, 64)) mykey = tkey[l];
+                have_table = true;
             }
-            if (mine) {
-                const int j = j0 + JS * q + jq;
-                const int o_ = il * RS + JS * q + jq;
-                double pe = 0;
-                const int touch = contact(i, j, pi, Ri, mi, ymi, &cb[w][0][o_], CS, &ab[w][d][0][l], 64, &pe);
-                if (WRITE) cb[w][NQ - 1][o_] = pe;
-                if (touch && i > j) cnt++;
-            }
-            asm volatile("" ::: "memory");
-            return out | __ballot(mine);
         };
         const bool adds = l < NQ * NB;
         const int comp = adds ? jq : 0;
@@ -486,43 +491,91 @@ void k_pairs_ordered(OrdState os, Phys P, int n, double* __restrict__ pe_ball,
             }
             asm volatile("" ::: "memory");
         };
-        // aacc: the touching lanes of a step in ascending order (their slots ascend with j)
-        auto add_aacc = [&](unsigned long long lanes, int d) {
+        // The batch's touching pairs, numbered ball by ball, j ascending.
+        int first = 0, own_pairs = 0, pairs = 0;   // this lane's ball's first number, its pairs; all pairs
+        auto number_pairs = [&]() {
+            constexpr unsigned long long ball0 = ~0ull / ((1ull << NB) - 1);   // lanes of ball 0
+#pragma unroll 1
+            for (int b = 0; b < NB; b++) {
+                int c = 0;
+#pragma unroll
+                for (int q = 0; q < CH; q++) c += __popcll(__ballot((pend >> q) & 1u) & (ball0 << b));
+                if (b == il) {
+                    first = pairs;
+                    own_pairs = c;
+                }
+                pairs += c;
+            }
+        };
+        // Contributions of pairs e0 .. e0 + AE - 1 to cb and ab, from the contact table or evaluated.
+        auto fill_pairs = [&](int e0) {
+            constexpr unsigned long long ball0 = ~0ull / ((1ull << NB) - 1);
+            int e = first - e0;
+#pragma unroll 1
+            for (int q = 0; q < CH; q++) {
+                const bool mine = (pend >> q) & 1u;
+                const unsigned long long lanes = __ballot(mine) & (ball0 << il);
+                const int at = e + lanes_below(lanes);
+                if (mine && at >= 0 && at < AE) numbered[w][at] = (unsigned char)(q << 6 | l);
+                e += __popcll(lanes);
+            }
+            asm volatile("" ::: "memory");
+            const int m1 = min(pairs - e0, AE);
+#pragma unroll 1
+            for (int r0 = 0; r0 < m1; r0 += 64) {
+                const int at = min(r0 + l, m1 - 1);
+                const int z = numbered[w][at];
+                const int bl = (z & 63) % NB, jl = JS * (z >> 6) + (z & 63) / NB, bi = i0 + bl, j = j0 + jl;
+                double* const c3 = &cb[w][0][bl * RS + jl];
+                double* const a3 = &ab[w][0][0] + at;
+                bool mine = r0 + l < m1;
+                if constexpr (SCAN) {
+                    get_table();
+                    const unsigned key = (unsigned)bl << 24 | (unsigned)j;
+                    int te = -1;
+                    for (int k = 0; k < min(found, 64); k++) te = (unsigned)__builtin_amdgcn_readlane(mykey, k) == key ? k : te;
+                    if (mine && te >= 0) {
+                        for (int k = 0; k < 3; k++) {
+                            c3[k * CS] = tres[te][k];
+                            a3[k * AE] = tres[te][3 + k];
+                        }
+                        if (WRITE) cb[w][NQ - 1][bl * RS + jl] = tres[te][6];
+                        if (bi > j) cnt++;
+                        mine = false;
+                    }
+                }
+                if (mine) {
+                    double pe = 0;
+                    const int touch = contact(bl, j, c3, CS, a3, AE, &pe);
+                    if (WRITE) cb[w][NQ - 1][bl * RS + jl] = pe;
+                    if (touch && bi > j) cnt++;
+                }
+            }
+            asm volatile("" ::: "memory");
+        };
+        // Theirs to aacc: the lane's ball's, in order.
+        auto add_aacc = [&](int e0) {
             if (comp < 3 && adds) {
                 double ra = run[3 + comp][il];
-                for (unsigned long long z = lanes; z; z &= z - 1) {
-                    const int ln = __ffsll((long long)z) - 1;
-                    const double c = ab[w][d][comp][ln];
-                    if (ln % NB == il) ra = ra + c;
-                }
+                const double* src = &ab[w][0][0] + comp * AE;
+                const int e1 = min(first + own_pairs - e0, AE);
+#pragma unroll 4
+                for (int e = max(first - e0, 0); e < e1; e++) ra = ra + src[e];
                 run[3 + comp][il] = ra;
             }
             asm volatile("" ::: "memory");
         };
-        unsigned long long lanes[AD];       // touching lanes of up to AD steps, evaluated before the turn
-        unsigned steps = 0;                 // steps with touching lanes, those not yet evaluated
-        bool any = false;
+        int last = 0;                       // those in ab: AE from here
         if (__any(pend != 0)) {
-            unsigned o = pend;
-            for (int k = 1; k < 64; k <<= 1) o |= __shfl_xor(o, k, 64);
-            steps = __builtin_amdgcn_readfirstlane(o);
-            any = true;
-        }
-#pragma unroll
-        for (int d = 0; d < AD; d++) {
-            lanes[d] = 0;
-            if (steps) {
-                lanes[d] = touching(__ffs(steps) - 1, d);
-                steps &= steps - 1;
+            number_pairs();
+#pragma unroll 1
+            for (; ; last += AE) {
+                fill_pairs(last);
+                if (last + AE >= pairs) break;
+                wait_turn();                // ab is used again: these sums' turn has to come first
+                add_aacc(last);
             }
-        }
-        // ab holds AD steps' pairs: with more steps the sums' turn has to come first
-        if (steps) {
-            wait_turn();
-#pragma unroll
-            for (int d = 0; d < AD; d++) add_aacc(lanes[d], d);
-            any = false;
-            for (; steps; steps &= steps - 1) add_aacc(touching(__ffs(steps) - 1, 0), 0);
+            load_ball();
         }
         // add: lane (ball l % NB, component l / NB)
         if (adds) {
@@ -548,11 +601,7 @@ void k_pairs_ordered(OrdState os, Phys P, int n, double* __restrict__ pe_ball,
             }
             *pr = r;
         }
-        if (any) {
-#pragma unroll
-            for (int d = 0; d < AD; d++)
-                if (lanes[d]) add_aacc(lanes[d], d);
-        }
+        if (pairs) add_aacc(last);
         asm volatile("" ::: "memory");
         if (l == 0) __hip_atomic_store(&turn, m + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         if (m == nm - 1 && adds && iv) {

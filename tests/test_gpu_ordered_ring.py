@@ -93,3 +93,35 @@ def test_contacts_counted_on_every_path():
             assert c.init_conditions().contacts == want
             after.append(c.step(1, 1)[0].contacts)
     assert len(set(after)) == 1 and abs(after[0] - want) < 0.01 * want, after
+
+
+@pytest.mark.parametrize("n,at", [(66, 0), (150, 75), (150, 149), (270, 131)])
+def test_a_ball_with_contacts_all_over_bitwise(oracle_mod, n, at):
+    """One large sphere that all others touch, first, last or between: every batch of its
+    workgroup has touching pairs at every step, more than the contact table holds."""
+    k = np.arange(n - 1) + 0.5
+    polar, turn = np.arccos(1 - 2 * k / (n - 1)), np.pi * (1 + 5 ** 0.5) * k
+    u = np.stack([np.cos(turn) * np.sin(polar), np.sin(turn) * np.sin(polar), np.cos(polar)], 1)
+    R = np.concatenate([[1e-5 * np.sqrt(0.4 * n)], np.full(n - 1, 1e-5)])
+    pos = np.concatenate([[[0, 0, 0]], u * (R[0] + 0.999e-5)])
+    order = np.roll(np.arange(n), at)
+    rng = np.random.default_rng(n + at)
+    pos, R = np.ascontiguousarray(pos[order]), R[order]
+    m = 2.25 * 4 / 3 * np.pi * R ** 3
+    g = sl.BallGroup(pos, 1e-3 * rng.standard_normal((n, 3)), 10 * rng.standard_normal((n, 3)), R, m, 0.4 * m * R * R)
+    p = sl.calibrate(sl.preset("config"), R, m, velocity=0.36301555459799423, cor=0.64)
+    P = oracle_mod.Params(G=p.G, Ha=p.Ha, h_min=p.h_min, u_s=p.u_s, u_r=p.u_r, kin=p.kin, kout=p.kout, dt=p.dt,
+                          far_gravity=p.far_gravity)
+    s, _, _ = oracle_mod.run(oracle_mod.State(g.pos, g.vel, g.w, g.R, g.m, g.moi), P, 6, 0, mode="gather")
+    touching = int(np.triu(np.linalg.norm(pos[:, None] - pos[None], axis=2) < R[:, None] + R[None], 1).sum())
+    assert touching >= n - 1
+    for shape in range(1, 10):
+        with sl.Collider(n, p) as c:
+            c.set_option("ordered_shape", shape)
+            c.upload(g)
+            assert c.init_conditions().contacts == touching
+            c.step(1)
+            c.step(4)
+            out = c.download()
+        for f in ("pos", "vel", "velh", "w", "wh", "acc", "aacc"):
+            assert bits_equal(getattr(out, f), getattr(s, f)), (shape, f)
