@@ -27,7 +27,7 @@ HOSTDIR = os.path.join(PKG, "host")
 # host programs over the C ABI: (source, executable in lib/)
 PROGRAMS = [("collider_main.cpp", "spacelab_collider")]
 HEADERS = ["sl_common.hpp", "sl_pair_ref.hpp", "sl_internal.hpp", "sl_fast_pair.hpp",
-           "sl_fast_kernels.hpp", "sl_mlp_host.hpp"]
+           "sl_fast_kernels.hpp", "sl_mlp_host.hpp", "sl_ordered_rule.hpp"]
 
 ARCH = "gfx950"
 COMMON = ["-O3", "-std=c++17", "-fPIC", "-ffp-contract=off", "-fno-fast-math",

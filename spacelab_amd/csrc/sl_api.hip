@@ -315,8 +315,8 @@ int tune_ordered(sl_ctx* c)
         c->ord_shape = c->forced_ord_shape - 1;
         return SL_OK;
     }
-    // (entries of older caches, "ordered:n...", number other shapes)
-    const std::string key = "ordered:ring:n" + std::to_string(c->n) + ":grav" + std::to_string(c->p.far_gravity);
+    // (entries of older caches, "ordered:n..." and "ordered:ring:...", are of other kernels)
+    const std::string key = "ordered:ring2:n" + std::to_string(c->n) + ":grav" + std::to_string(c->p.far_gravity);
     if (const int cached = tune_cache_get(key); cached >= 1 && cached <= ordered_shapes()) {
         c->ord_shape = cached - 1;
         return SL_OK;

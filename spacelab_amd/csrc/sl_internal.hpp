@@ -3,6 +3,7 @@
 
 #include "spacelab/sl_api.h"
 #include "sl_common.hpp"
+#include "sl_ordered_rule.hpp"
 
 #include <map>
 #include <string>
@@ -16,7 +17,6 @@ hipError_t launch_drift_to(const State& s, const State& d, int n, double dt, hip
 hipError_t launch_copy_prev(const State& s, int n, hipStream_t st);
 // Launch shapes of the pair pass (all give the same bits); shape = index below ordered_shapes().
 int ordered_shapes();
-int ordered_default_shape(int n);
 int ordered_blocks(int n, int shape);
 // pe_ball: on write steps, per ball i the energy of its pairs (i, j < i) in ascending j.
 hipError_t launch_pairs_ordered(const State& s, const Phys& P, int n, int write, double* pe_ball,

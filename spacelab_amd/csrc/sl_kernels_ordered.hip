@@ -187,9 +187,9 @@ struct BallRec {
 // 64, side by side while the others start on their batches; a pair met in the sweep is then
 // copied from that table.  Pairs that did not fit in it, and all touching pairs without SCAN,
 // are evaluated in their batch.  The scan
-// pays up to about 2,500 balls (4 balls, 4 wavefronts, us per step with / without: 2,000 balls
-// 43.7 / 45.4, 3,000 77 / 73.5, 5,000 175 / 161): its cost grows with the partners, what it
-// saves only with the contacts.
+// pays up to about 1,700 balls (4 balls, 4 wavefronts, us per step with / without: 1,500 balls
+// 35.1 / 37.1, 1,800 42.9 / 42.6, 2,200 58.9 / 54.9, 5,000 181 / 161): its cost grows with the
+// partners, what it saves only with the contacts.
 // While contacts are evaluated a lane's own ball waits in LDS (BallRec): in registers it took
 // 26 spills more, the next batch's partners among them, which then had to arrive first.
 //
@@ -727,8 +727,11 @@ hipError_t launch_copy_prev(const State& s, int n, hipStream_t st)
 }
 
 // Launch shapes of the ordered pair pass: balls per workgroup, pairs per lane and batch,
-// wavefronts, steps of touching pairs kept, wavefronts per SIMD the registers are held to, pairs unrolled.  All give
-// the same results bit for bit.
+// wavefronts, rounds of 64 touching pairs before the turn, wavefronts per SIMD the registers are
+// held to, pairs unrolled, scan.  All give the same results bit for bit.  The sizes at which each
+// is the fastest are at ordered_default_shape; 8 has a few of the smallest (16 balls 6.74 us,
+// shape 7 6.79); 2 and 6 have none of those measured (2 comes next after 5 at 1,100 to 1,500 balls
+// and 3 at 1,800, 6 after 1 at 1,000) and stay because callers force shapes by these numbers.
 #define SL_ORD_SHAPES(X) \
     X(0, 2, 2, 8, 2, 2, 2, true) \
     X(1, 4, 4, 8, 2, 2, 2, true) \
@@ -748,18 +751,6 @@ constexpr int N_ORD_SHAPES = (int)(sizeof(ORD_BALLS) / sizeof(ORD_BALLS[0]));
 }  // namespace
 
 int ordered_shapes() { return N_ORD_SHAPES; }
-
-// The shape used when none is chosen (the allocation-free entry point, and until the tuner has
-// run).  Shapes 0 and 1 put 8 wavefronts on a CU, one workgroup of 2 or 4 balls: they are the
-// fastest while every workgroup has a CU of its own (512 and 1,024 balls on 256 CUs: 450
-// balls 11.8 and 14.8 us per step, 600 19.2 and 16.8, 1,000 26 and 18.9, 1,200 41 and 33.6).
-// Then 4 wavefronts and three workgroups a CU, with the scan up to 2,500 balls; from about
-// 20,000 on 8 balls a workgroup (fewer adds per pair: 15,039 balls 1,099 and 1,132 us with 4
-// and 8, 40,000 7,485 and 7,266).
-int ordered_default_shape(int n)
-{
-    return n <= 512 ? 0 : n <= 1024 ? 1 : n <= 2500 ? 2 : n <= 20000 ? 3 : 4;
-}
 
 int ordered_blocks(int n, int shape)
 {
