@@ -188,6 +188,9 @@ int sl_batch_init_forces(sl_batch* b, sl_energy* e_sys);
 int sl_batch_step(sl_batch* b, int n_steps, int write_every, sl_energy* e, int e_cap);
 int sl_batch_download(sl_batch* b, double* pos3, double* vel3, double* w3, double* acc3,
                       double* aacc3);
+/* The same into n_parts places: the next systems[k] systems' five vectors, one after another, to
+ * out[k].  The parts hold all systems. */
+int sl_batch_download_parts(sl_batch* b, int n_parts, const int* systems, double* const* out);
 int sl_batch_set_option(sl_batch* b, int option, int value);
 int sl_batch_get_option(sl_batch* b, int option, int* value);
 long long sl_batch_step_count(const sl_batch* b);

@@ -115,10 +115,11 @@ class Energy:
 
     @staticmethod
     def _from_buffer(buf, n: int) -> list["Energy"]:
-        """The first n of a ctypes array of _Energy; p and L are rows of arrays of this call."""
+        """The first n of a ctypes array of _Energy; p and L are rows of arrays of 1024 energies."""
         a = np.frombuffer(buf, dtype=_ENERGY, count=n)
+        rows = lambda f: (r for k in range(0, n, 1024) for r in a[f][k:k + 1024].copy())
         return [Energy(pe, ke, p, L, bool(bad), contacts) for pe, ke, p, L, bad, contacts in
-                zip(a["PE"].tolist(), a["KE"].tolist(), a["p"].copy(), a["L"].copy(),
+                zip(a["PE"].tolist(), a["KE"].tolist(), rows("p"), rows("L"),
                     a["nonfinite"].tolist(), a["contacts"].tolist())]
 
 
@@ -165,6 +166,7 @@ def lib():
     L.sl_batch_set_system_params.argtypes = [vp, dp, dp, dp]
     L.sl_batch_init_forces.argtypes = [vp, C.POINTER(_Energy)]
     L.sl_batch_step.argtypes = [vp, C.c_int, C.c_int, C.POINTER(_Energy), C.c_int]
+    L.sl_batch_download_parts.argtypes = [vp, C.c_int, ip, C.POINTER(vp)]
     L.sl_batch_download.argtypes = [vp] + [dp] * 5
     L.sl_batch_set_option.argtypes = [vp, C.c_int, C.c_int]
     L.sl_batch_get_option.argtypes = [vp, C.c_int, C.POINTER(C.c_int)]
@@ -680,18 +682,25 @@ class Batch:
         return int(lib().sl_batch_step_count(self._b))
 
     def download(self) -> list[BallGroup]:
-        n = sum(self.sizes)
-        pos = np.empty((n, 3)); vel = np.empty((n, 3)); w = np.empty((n, 3))
-        acc = np.empty((n, 3)); aacc = np.empty((n, 3))
-        self._check(lib().sl_batch_download(self._b, _dp(pos), _dp(vel), _dp(w), _dp(acc),
-                                            _dp(aacc)), "sl_batch_download")
-        # each group's arrays are its parts of this call's arrays
-        R, m, moi = (a.copy() for a in self._static)
-        out, o = [], 0
+        """Every group's state.  A group's arrays are parts of arrays of up to 16384 balls (2.4 MB
+        with all eight) that it shares with its neighbours; arrays for the whole batch would all
+        be kept while one group is."""
+        parts, end = [], 16384        # the groups' places in each part; balls in the last one
         for k in self.sizes:
-            e = o + k
-            out.append(BallGroup(pos[o:e], vel[o:e], w[o:e], R[o:e], m[o:e], moi[o:e], acc[o:e], aacc[o:e]))
-            o = e
+            if end + k > 16384:
+                parts.append([])
+                end = 0
+            parts[-1].append(slice(end, end + k))
+            end += k
+        bufs = [np.empty((5, p[-1].stop, 3)) for p in parts]
+        self._check(lib().sl_batch_download_parts(
+            self._b, len(parts), (C.c_int * len(parts))(*map(len, parts)),
+            (C.c_void_p * len(parts))(*(b.ctypes.data for b in bufs))), "sl_batch_download_parts")
+        out, at = [], 0
+        for p, (pos, vel, w, acc, aacc) in zip(parts, bufs):
+            R, m, moi = (a[at:at + len(pos)].copy() for a in self._static)
+            at += len(pos)
+            out += [BallGroup(pos[s], vel[s], w[s], R[s], m[s], moi[s], acc[s], aacc[s]) for s in p]
         return out
 
     def set_option(self, name: str, value: int):

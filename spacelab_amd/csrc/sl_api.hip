@@ -674,13 +674,13 @@ int sl_download_state(sl_ctx* c, double* pos3, double* vel3, double* w3, double*
     const int fields[MAX_READ] = {PX, VX, WX, AX, BX, HX, GX};
     double* const outs[MAX_READ] = {pos3, vel3, w3, acc3, aacc3, velh3, wh3};
     int field[MAX_READ], nv = 0;
-    double* out[MAX_READ];
+    ReadPart all{c->n, {}};
     for (int v = 0; v < MAX_READ; v++)
         if (outs[v]) {
             field[nv] = fields[v];
-            out[nv++] = outs[v];
+            all.out[nv++] = outs[v];
         }
-    return fast_read(c->fb, c->st, c->stage, field, out, nv, c->stream, &c->err);
+    return fast_read(c->fb, c->st, c->stage, field, &all, nv, c->stream, &c->err);
 }
 
 int sl_download(sl_ctx* c, double* pos3, double* vel3, double* w3, double* acc3, double* aacc3)

@@ -51,6 +51,8 @@ int berr(sl_batch* b, int code, const char* fmt, ...)
 
 bool positive(double x) { return x > 0 && std::isfinite(x); }
 
+constexpr int READ_FIELDS[5] = {PX, VX, WX, AX, BX};   // first fields of the vectors that are read back
+
 void release(sl_batch* b)
 {
     fast_free(b->fb);
@@ -229,16 +231,36 @@ int sl_batch_download(sl_batch* b, double* pos3, double* vel3, double* w3, doubl
 {
     if (!b) return SL_E_ARG;
     if (!b->uploaded) return berr(b, SL_E_STATE, "download before upload");
-    const int fields[5] = {PX, VX, WX, AX, BX};
     double* const outs[5] = {pos3, vel3, w3, acc3, aacc3};
     int field[5], nv = 0;
-    double* out[5];
+    ReadPart all{b->lay.first.back() + b->lay.n.back(), {}};
     for (int v = 0; v < 5; v++)
         if (outs[v]) {
-            field[nv] = fields[v];
-            out[nv++] = outs[v];
+            field[nv] = READ_FIELDS[v];
+            all.out[nv++] = outs[v];
         }
-    return fast_read(b->fb, b->st, b->stage, field, out, nv, b->stream, &b->err);
+    return fast_read(b->fb, b->st, b->stage, field, &all, nv, b->stream, &b->err);
+}
+
+int sl_batch_download_parts(sl_batch* b, int n_parts, const int* systems, double* const* out)
+{
+    if (!b) return SL_E_ARG;
+    if (!b->uploaded) return berr(b, SL_E_STATE, "download before upload");
+    if (n_parts < 1 || !systems || !out) return berr(b, SL_E_ARG, "no parts");
+    std::vector<ReadPart> parts;
+    int sys = 0;
+    for (int k = 0; k < n_parts; k++) {
+        if (systems[k] < 1 || systems[k] > b->lay.n_sys - sys || !out[k])
+            return berr(b, SL_E_ARG, "parts: each of at least one system, all systems in all, none NULL");
+        const int last = sys + systems[k] - 1;
+        const long long balls = b->lay.first[last] + b->lay.n[last] - b->lay.first[sys];
+        ReadPart p{balls, {}};
+        for (int v = 0; v < 5; v++) p.out[v] = out[k] + 3 * balls * v;
+        parts.push_back(p);
+        sys = last + 1;
+    }
+    if (sys != b->lay.n_sys) return berr(b, SL_E_ARG, "parts: each of at least one system, all systems in all, none NULL");
+    return fast_read(b->fb, b->st, b->stage, READ_FIELDS, parts.data(), 5, b->stream, &b->err);
 }
 
 int sl_batch_set_option(sl_batch* b, int option, int value)

@@ -147,13 +147,19 @@ inline size_t stage_size(long long n_max)
     const long long want = 2LL * MAX_READ * 24 * ((n_max + FAST_TILE - 1) / FAST_TILE) * FAST_TILE;
     return (size_t)(want < (2 << 20) ? want : (2 << 20));
 }
+// A run of balls, in the caller's order, and where their vectors go.
+struct ReadPart {
+    long long balls;
+    double* out[MAX_READ];
+};
 // nv vectors (fields field[v] .. + 2) of the state s, whose slot for the caller's slot c is
-// slot_of[c] (NULL: c), to out[v] (x, y, z per ball, systems one after another).  Waits for
-// the stream's work.  fb: the device's layout tables (more than one system).
+// slot_of[c] (NULL: c), to the parts' out[v] (x, y, z per ball, systems one after another); the
+// parts hold all balls.  Waits for the stream's work.  fb: the device's layout tables (more than
+// one system).
 int read_state(HostStage& hs, const State& s, const int* slot_of, const FastLayout& lay, const FastBuffers* fb,
-               const int* field, double* const* out, int nv, hipStream_t st);
+               const int* field, const ReadPart* parts, int nv, hipStream_t st);
 // The engine's (or, when it is the one up to date, the canonical) state read like that.
-int fast_read(FastBuffers& fb, State& canon, HostStage& hs, const int* field, double* const* out, int nv, hipStream_t st,
+int fast_read(FastBuffers& fb, State& canon, HostStage& hs, const int* field, const ReadPart* parts, int nv, hipStream_t st,
               std::string* err);
 
 int fast_alloc(FastBuffers& fb, int n_pad, int max_sys);

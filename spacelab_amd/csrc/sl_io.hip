@@ -64,7 +64,7 @@ void stage_free(HostStage& hs)
 }
 
 int read_state(HostStage& hs, const State& s, const int* slot_of, const FastLayout& lay, const FastBuffers* fb,
-               const int* field, double* const* out, int nv, hipStream_t st)
+               const int* field, const ReadPart* parts, int nv, hipStream_t st)
 {
     PackArgs a{};
     a.s = s;
@@ -104,14 +104,24 @@ int read_state(HostStage& hs, const State& s, const int* slot_of, const FastLayo
         return hipGetLastError() == hipSuccess && hipEventRecord(hs.ev[k & 1], st) == hipSuccess ? SL_OK : SL_E_HIP;
     };
     const int pieces = (lay.n_used + per - 1) / per;
+    long long done = 0;             // balls of *parts that are out
     if (pack(0)) return SL_E_HIP;
     for (int k = 0; k < pieces; k++) {
         if (k + 1 < pieces && pack(k + 1)) return SL_E_HIP;
         if (hipEventSynchronize(hs.ev[k & 1]) != hipSuccess) return SL_E_HIP;
         const Piece p = piece[k & 1];
         const double* src = reinterpret_cast<const double*>(hs.h + (k & 1) * half);
-        for (int v = 0; v < nv; v++)
-            std::memcpy(out[v] + 3 * (size_t)p.ball0, src + (size_t)v * p.balls * 3, sizeof(double) * 3 * p.balls);
+        for (long long b = 0; b < p.balls;) {
+            if (done == parts->balls) {
+                parts++;
+                done = 0;
+            }
+            const long long n = std::min<long long>(p.balls - b, parts->balls - done);
+            for (int v = 0; v < nv; v++)
+                std::memcpy(parts->out[v] + 3 * done, src + 3 * ((size_t)v * p.balls + b), sizeof(double) * 3 * n);
+            b += n;
+            done += n;
+        }
     }
     return SL_OK;
 }

@@ -784,11 +784,11 @@ int fast_sync_to(FastBuffers& fb, State& canon, hipStream_t st, std::string* err
     return 0;
 }
 
-int fast_read(FastBuffers& fb, State& canon, HostStage& hs, const int* field, double* const* out, int nv, hipStream_t st,
+int fast_read(FastBuffers& fb, State& canon, HostStage& hs, const int* field, const ReadPart* parts, int nv, hipStream_t st,
               std::string* err)
 {
     const bool here = fb.canon_valid;
-    if (read_state(hs, here ? canon : fb.eng[fb.cur], here ? nullptr : fb.slot_of, fb.lay, &fb, field, out, nv, st) != SL_OK)
+    if (read_state(hs, here ? canon : fb.eng[fb.cur], here ? nullptr : fb.slot_of, fb.lay, &fb, field, parts, nv, st) != SL_OK)
         return err_hip(err, "state read-back");
     return 0;
 }

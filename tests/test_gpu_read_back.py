@@ -71,3 +71,45 @@ def test_batch_read_back(sizes):
             for f in FIELDS:
                 assert bits_equal(getattr(e, f), getattr(o, f)), f
             assert not bits_equal(e.pos, g.pos)
+
+
+def _root(a):
+    while a.base is not None:
+        a = a.base
+    return a
+
+
+def test_a_kept_group_does_not_keep_the_batch():
+    """What one group of a batch, or one energy of many, holds in memory is its own or bounded."""
+    sizes = [250] * 40 + [17000] + [3] * 30 + [8192, 8192, 1, 64]
+    groups = [_grid(n, k) for k, n in enumerate(sizes)]
+    with sl.Batch(len(sizes), sum(sizes), _params(groups[0], order=sl.ORDER_FAST)) as b:
+        b.upload(groups)
+        energies = b.init_conditions()
+        for g, o in zip(groups, b.download()):
+            assert o.num_particles == g.num_particles
+            for f in ("pos", "vel", "w", "R", "m", "moi"):
+                assert bits_equal(getattr(o, f), getattr(g, f)), f
+            held = {id(r): r.nbytes for r in (_root(getattr(o, f)) for f in ("pos", "vel", "w", "R", "m", "moi", "acc", "aacc"))}
+            assert sum(held.values()) <= 18 * 8 * max(16384, g.num_particles)
+    assert all(_root(e.p).nbytes <= 24 * 1024 for e in energies)
+    with sl.Collider(2, _params(_grid(2, 0), order=sl.ORDER_FAST)) as c:
+        c.upload(_grid(2, 0))
+        c.init_conditions()
+        e = c.step(3000, 1)
+    assert len(e) == 3000 and all(_root(x.p).nbytes <= 24 * 1024 and _root(x.L).nbytes <= 24 * 1024 for x in e)
+
+
+def test_parts_that_do_not_hold_every_system_are_refused():
+    import ctypes as C
+    groups = [_grid(n, n) for n in (5, 70, 3)]
+    with sl.Batch(3, 78, _params(groups[0], order=sl.ORDER_FAST)) as b:
+        with pytest.raises(sl.SpacelabError):
+            b.download()                      # nothing uploaded
+        b.upload(groups)
+        bufs = [np.empty((5, 78, 3)) for _ in range(3)]
+        call = lambda *ns: sl.lib().sl_batch_download_parts(b._b, len(ns), (C.c_int * len(ns))(*ns),
+                                                            (C.c_void_p * 3)(*(x.ctypes.data for x in bufs)))
+        assert call(1, 2) == 0 and call(3) == 0 and call(1, 1, 1) == 0
+        for bad in ((1, 1), (2, 2), (0, 3), (4,), (-1, 4), ()):
+            assert call(*bad) < 0, bad
