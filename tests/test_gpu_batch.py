@@ -152,6 +152,33 @@ def test_batch_reupload_and_system_params():
             assert bits_equal(getattr(out[k], f), getattr(s, f)), (k, f)
 
 
+@pytest.mark.parametrize("split,queue", [(1, 1), (2, 1), (4, 1), (2, 2)])
+def test_large_systems_among_small_ones(split, queue):
+    """Systems of more than 80 blocks, whose tiles are listed in groups of a row with fillers and
+    whose masks are marked, between small ones in one batch: forces, states and energies of each
+    are those of the system alone."""
+    groups, params = _ensemble([100, 5400, 64, 5130, 300, 7], 0x5EED0600)
+    with sl.Batch(6, sum(g.num_particles for g in groups), params[0]) as b:
+        b.set_option("tile_split", split)
+        b.set_option("tile_queue", queue)
+        b.upload(groups, kin=[p.kin for p in params], kout=[p.kout for p in params], dt=[p.dt for p in params])
+        e0 = b.init_conditions()
+        first = b.download()
+        ew = b.step(5, 5)
+        last = b.download()
+    for k, (g, p) in enumerate(zip(groups, params)):
+        with sl.Collider(g.num_particles, p) as c:
+            c.set_option("tile_split", split)
+            c.set_option("tile_queue", queue)
+            c.upload(g)
+            assert _ebytes(c.init_conditions()) == _ebytes(e0[k]), k
+            for f in FIELDS:
+                assert bits_equal(getattr(first[k], f), getattr(c.download(), f)), (k, f)
+            assert _ebytes(c.step(5, 5)[0]) == _ebytes(ew[0][k]), k
+            for f in FIELDS:
+                assert bits_equal(getattr(last[k], f), getattr(c.download(), f)), (k, f)
+
+
 def test_batch_mixed_energy_close_to_fp64():
     groups, params = _ensemble([800, 200, 50], 0x5EED0400)
     kin = [p.kin for p in params]
