@@ -32,7 +32,4 @@ struct Phys {
     int far_gravity;
 };
 
-// Energy partials per block: PE, KE, p.xyz, L.xyz
-constexpr int NE = 8;
-
 }  // namespace sl

@@ -89,21 +89,6 @@ __device__ __forceinline__ unsigned long long rotl64(unsigned long long x, int k
     return k ? (x << k) | (x >> (64 - k)) : x;
 }
 
-template <int N>
-__device__ __forceinline__ double block_sum(double v, double* red)
-{
-    const int t = threadIdx.x;
-    red[t] = v;
-    __syncthreads();
-    for (int s = N / 2; s > 0; s >>= 1) {
-        if (t < s) red[t] = red[t] + red[t + s];
-        __syncthreads();
-    }
-    const double r = red[0];
-    __syncthreads();
-    return r;
-}
-
 // Systems of more than KB_BATCH blocks list their tiles in groups of NW of one row I, J = 4 g ..
 // 4 g + 3 (the last group of a row is filled up with I = -1), and the binary64 sweep, where a
 // workgroup takes several tiles, adds the i sides of a group's tiles before they go to memory:
@@ -144,12 +129,6 @@ struct TileArgs {
 __device__ __forceinline__ double wave_sum(double v)
 {
     for (int m = 1; m < TB; m <<= 1) v = v + __shfl_xor(v, m, TB);
-    return v;
-}
-
-__device__ __forceinline__ unsigned long long wave_or(unsigned long long v)
-{
-    for (int m = 1; m < TB; m <<= 1) v |= __shfl_xor(v, m, TB);
     return v;
 }
 

@@ -180,7 +180,6 @@ int fast_init(FastBuffers& fb, State& canon, sl_energy* e_sys, hipStream_t st, s
 // cap writes.  Returns the number of write steps or a negative error.
 int fast_steps(FastBuffers& fb, State& canon, int n_steps, long long* step_count, int write_every,
                sl_energy* e_writes, int cap, hipStream_t st, std::string* err);
-int fast_max_tile_blocks(int n_pad);
 void fast_clear_graphs(FastBuffers& fb);
 // wavefronts per k_ball workgroup for the current layout (forced, or by block count)
 int fast_ball_waves(const FastBuffers& fb);

@@ -556,12 +556,6 @@ FastLayout fast_layout(int n_sys, const int* n_per_sys)
     return L;
 }
 
-int fast_max_tile_blocks(int n_pad)
-{
-    const long long nb = (n_pad + TB - 1) / TB;
-    return (int)std::min<long long>(nb * (nb + 1) / 2, 1 << 30);
-}
-
 int fast_alloc(FastBuffers& fb, int n_pad, int max_sys)
 {
     fb.n_pad = n_pad;
