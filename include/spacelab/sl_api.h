@@ -385,6 +385,9 @@ int sl_mlp_forward_all(sl_mlp* const* nets, int n, int batch, const float* x, fl
  * of different widths, max_batch or devices, or wider than 512). */
 int sl_mlp_ensemble(sl_mlp* const* nets, int n, long long rows, const double* x, const double* mean, const double* std,
                     int* cls, float* reg, double* prob, double* ent);
+/* The same of binary32 rows, normalised in binary32 throughout. */
+int sl_mlp_ensemble32(sl_mlp* const* nets, int n, long long rows, const float* x, const float* mean, const float* std,
+                      int* cls, float* reg, double* prob, double* ent);
 const char* sl_mlp_last_error(const sl_mlp* m);   /* calls on several nets: of the net it fails on or the first */
 void sl_mlp_destroy(sl_mlp* m);
 

@@ -222,6 +222,7 @@ def lib():
     L.sl_mlp_train_rows.argtypes = [mlps, C.c_int, C.c_int, C.c_int, C.c_longlong, fp, ip, fp, llp, C.c_float, fp]
     L.sl_mlp_forward_all.argtypes = [mlps, C.c_int, C.c_int, fp, fp, fp, fp]
     L.sl_mlp_ensemble.argtypes = [mlps, C.c_int, C.c_longlong, dp, dp, dp, ip, fp, dp, dp]
+    L.sl_mlp_ensemble32.argtypes = [mlps, C.c_int, C.c_longlong, fp, fp, fp, ip, fp, dp, dp]
     L.sl_mlp_last_error.argtypes = [vp]
     L.sl_mlp_last_error.restype = C.c_char_p
     L.sl_mlp_destroy.argtypes = [vp]
@@ -822,18 +823,23 @@ def mlp_alike(mlps: list[MLP]) -> bool:
     return 1 <= len({id(m) for m in mlps}) == len(mlps) <= 16 and len(sizes) == 1 and max(next(iter(sizes))[:3]) <= 512
 
 
-def mlp_ensemble(mlps: list[MLP], x, mean, std):
+def mlp_ensemble(mlps: list[MLP], x, mean, std, dtype=np.float64):
     """(class, regression outputs, class probabilities, predictive entropy) of nets that are
-    mlp_alike, together, on rows of x brought to (x - mean) / std."""
+    mlp_alike, together, on rows of x brought to (x - mean) / std in dtype (binary64 or 32)."""
     m = mlps[0]
-    x = np.ascontiguousarray(x, dtype=np.float64)
-    mean, std = (np.ascontiguousarray(np.broadcast_to(np.asarray(a, np.float64), (m.n_in,))) for a in (mean, std))
+    wide = np.dtype(dtype) == np.float64
+    if not wide and np.dtype(dtype) != np.float32:
+        raise ValueError("dtype: float64 or float32")
+    x = np.ascontiguousarray(x, dtype=dtype)
+    mean, std = (np.ascontiguousarray(np.broadcast_to(np.asarray(a, dtype), (m.n_in,))) for a in (mean, std))
     n = len(x)
     if x.shape != (n, m.n_in):
         raise ValueError("x: rows of the nets' inputs")
     cls = np.empty(n, np.int32); reg = np.empty((n, m.n_out - 3), np.float32)
     prob = np.empty((n, 3)); ent = np.empty(n)
-    _mlp_call(mlps, "sl_mlp_ensemble", n, _dp(x), _dp(mean), _dp(std), _ip(cls), _fp(reg), _dp(prob), _dp(ent))
+    ptr = _dp if wide else _fp
+    _mlp_call(mlps, "sl_mlp_ensemble" if wide else "sl_mlp_ensemble32", n, ptr(x), ptr(mean), ptr(std), _ip(cls), _fp(reg),
+              _dp(prob), _dp(ent))
     return cls, reg, prob, ent
 
 

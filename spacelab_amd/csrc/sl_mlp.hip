@@ -661,9 +661,9 @@ __global__ __launch_bounds__(256) void k_wgrad(WgradArgs a)
     if (STEP) store4(moved(a.Wf[k], at) + frag_at(in0, out, k_steps(K)), 0, wv);
 }
 
-// Rows of binary64 descriptors to the nets' inputs, (x - mean) / std rounded to binary32.
-__global__ __launch_bounds__(256) void k_normalise(int n, int n_in, const double* x, const double* mean, const double* std,
-                                                   float* out)
+// Rows of descriptors to the nets' inputs, (x - mean) / std in T, rounded to binary32.
+template <class T>
+__global__ __launch_bounds__(256) void k_normalise(int n, int n_in, const T* x, const T* mean, const T* std, float* out)
 {
     const int e = blockIdx.x * 256 + threadIdx.x;
     if (e < n * n_in) out[e] = (float)((x[e] - mean[e % n_in]) / std[e % n_in]);
@@ -1171,6 +1171,68 @@ int check_batch(sl_mlp* m, int B, const void* x)
     return SL_OK;
 }
 
+// sl_mlp_ensemble, the rows and their normalising in T.
+template <class T>
+int ensemble(sl_mlp* const* ms, int n, long long rows, const T* x, const T* mean, const T* std, int* cls, float* reg,
+             double* prob, double* ent)
+{
+    if (!ms || n < 1 || rows < 0) return SL_E_ARG;
+    for (int j = 0; j < n; j++)
+        if (!ms[j]) return SL_E_ARG;
+    sl_mlp* m = ms[0];
+    if (!mean || !std || (rows > 0 && !(x && cls && reg && prob && ent))) return mlp_err(m, SL_E_ARG, "an array is NULL");
+    if (n > MEMBERS || !alike(ms, n)) return mlp_err(m, SL_E_STATE, "the nets cannot share launches");
+    const int n_in = m->n_in, nr = m->n_out - NCLS;
+    // two batches in flight, each in its half of the buffers: one is copied in and the other's
+    // answers out while the device works
+    const int per = std::max(1, m->max_batch / 2);
+    const Stage s(m->max_batch, n_in, m->n_out);
+    std::memcpy(m->stage + s.em, mean, sizeof(T) * n_in);
+    std::memcpy(m->stage + s.em + sizeof(T) * n_in, std, sizeof(T) * n_in);
+    const bool halves = m->max_batch > 1;
+    auto at = [&](char* base, size_t part, size_t bytes, long long k) { return base + part + (halves && k % 2 ? bytes * per : 0); };
+    auto size = [&](long long k) { return (int)std::min<long long>(per, rows - k * per); };
+    auto collect = [&](long long k) -> int {
+        if (hipEventSynchronize(m->half[k % 2]) != hipSuccess) return mlp_err(m, SL_E_HIP, "ensemble pass failed");
+        const size_t b0 = (size_t)k * per, B = size(k);
+        std::memcpy(prob + NCLS * b0, at(m->stage, s.ep, 8 * NCLS, k), 8 * NCLS * B);
+        std::memcpy(ent + b0, at(m->stage, s.eh, 8, k), 8 * B);
+        std::memcpy(cls + b0, at(m->stage, s.ec, 4, k), 4 * B);
+        std::memcpy(reg + nr * b0, at(m->stage, s.er, 4 * (size_t)nr, k), 4 * nr * B);
+        return SL_OK;
+    };
+    auto issue = [&](long long k) -> int {
+        const int B = size(k);
+        std::memcpy(at(m->stage, s.ex, sizeof(T) * n_in, k), x + (size_t)k * per * n_in, sizeof(T) * B * n_in);
+        auto dev = [&](size_t part, size_t bytes) { return at(m->stage_dev, part, bytes, k); };
+        const T* em = reinterpret_cast<const T*>(m->stage_dev + s.em);
+        k_normalise<<<(B * n_in + 255) / 256, 256, 0, m->stream>>>(
+            B, n_in, reinterpret_cast<const T*>(dev(s.ex, sizeof(T) * n_in)), em, em + n_in, m->xin);
+        ChainArgs c = chain_args(ms, n, B, true);
+        EnsembleArgs e{};
+        for (int j = 0; j < n; j++) c.at[j].stage = e.at[j] = c.at[j].pool;
+        c.x = m->xin;
+        c.y = m->yout;
+        c.prob = m->prob;
+        c.ent = m->ent;
+        launch_chain<false>(ms, n, B, c);
+        e.n = n;
+        e.B = B;
+        e.n_out = m->n_out;
+        e.y = m->yout;
+        e.prob = m->prob;
+        e.cls = reinterpret_cast<int*>(dev(s.ec, 4));
+        e.reg = reinterpret_cast<float*>(dev(s.er, 4 * (size_t)nr));
+        e.p = reinterpret_cast<double*>(dev(s.ep, 8 * NCLS));
+        e.ent = reinterpret_cast<double*>(dev(s.eh, 8));
+        k_ensemble<<<(B + 63) / 64, 64, 0, m->stream>>>(e);
+        if (hipGetLastError() != hipSuccess || hipEventRecord(m->half[k % 2], m->stream) != hipSuccess)
+            return mlp_err(m, SL_E_HIP, "ensemble pass failed");
+        return SL_OK;
+    };
+    return sl::run_ahead((rows + per - 1) / per, halves ? 2 : 1, issue, collect, [&] { (void)hipStreamSynchronize(m->stream); });
+}
+
 }  // namespace
 
 extern "C" {
@@ -1310,61 +1372,13 @@ int sl_mlp_forward(sl_mlp* m, int B, const float* x, float* y, float* prob, floa
 int sl_mlp_ensemble(sl_mlp* const* ms, int n, long long rows, const double* x, const double* mean, const double* std, int* cls,
                     float* reg, double* prob, double* ent)
 {
-    if (!ms || n < 1 || rows < 0) return SL_E_ARG;
-    for (int j = 0; j < n; j++)
-        if (!ms[j]) return SL_E_ARG;
-    sl_mlp* m = ms[0];
-    if (!mean || !std || (rows > 0 && !(x && cls && reg && prob && ent))) return mlp_err(m, SL_E_ARG, "an array is NULL");
-    if (n > MEMBERS || !alike(ms, n)) return mlp_err(m, SL_E_STATE, "the nets cannot share launches");
-    const int n_in = m->n_in, nr = m->n_out - NCLS;
-    // two batches in flight, each in its half of the buffers: one is copied in and the other's
-    // answers out while the device works
-    const int per = std::max(1, m->max_batch / 2);
-    const Stage s(m->max_batch, n_in, m->n_out);
-    std::memcpy(m->stage + s.em, mean, sizeof(double) * n_in);
-    std::memcpy(m->stage + s.em + sizeof(double) * n_in, std, sizeof(double) * n_in);
-    const bool halves = m->max_batch > 1;
-    auto at = [&](char* base, size_t part, size_t bytes, long long k) { return base + part + (halves && k % 2 ? bytes * per : 0); };
-    auto size = [&](long long k) { return (int)std::min<long long>(per, rows - k * per); };
-    auto collect = [&](long long k) -> int {
-        if (hipEventSynchronize(m->half[k % 2]) != hipSuccess) return mlp_err(m, SL_E_HIP, "ensemble pass failed");
-        const size_t b0 = (size_t)k * per, B = size(k);
-        std::memcpy(prob + NCLS * b0, at(m->stage, s.ep, 8 * NCLS, k), 8 * NCLS * B);
-        std::memcpy(ent + b0, at(m->stage, s.eh, 8, k), 8 * B);
-        std::memcpy(cls + b0, at(m->stage, s.ec, 4, k), 4 * B);
-        std::memcpy(reg + nr * b0, at(m->stage, s.er, 4 * (size_t)nr, k), 4 * nr * B);
-        return SL_OK;
-    };
-    auto issue = [&](long long k) -> int {
-        const int B = size(k);
-        std::memcpy(at(m->stage, s.ex, 8 * (size_t)n_in, k), x + (size_t)k * per * n_in, 8 * (size_t)B * n_in);
-        auto dev = [&](size_t part, size_t bytes) { return at(m->stage_dev, part, bytes, k); };
-        const double* em = reinterpret_cast<const double*>(m->stage_dev + s.em);
-        k_normalise<<<(B * n_in + 255) / 256, 256, 0, m->stream>>>(
-            B, n_in, reinterpret_cast<const double*>(dev(s.ex, 8 * (size_t)n_in)), em, em + n_in, m->xin);
-        ChainArgs c = chain_args(ms, n, B, true);
-        EnsembleArgs e{};
-        for (int j = 0; j < n; j++) c.at[j].stage = e.at[j] = c.at[j].pool;
-        c.x = m->xin;
-        c.y = m->yout;
-        c.prob = m->prob;
-        c.ent = m->ent;
-        launch_chain<false>(ms, n, B, c);
-        e.n = n;
-        e.B = B;
-        e.n_out = m->n_out;
-        e.y = m->yout;
-        e.prob = m->prob;
-        e.cls = reinterpret_cast<int*>(dev(s.ec, 4));
-        e.reg = reinterpret_cast<float*>(dev(s.er, 4 * (size_t)nr));
-        e.p = reinterpret_cast<double*>(dev(s.ep, 8 * NCLS));
-        e.ent = reinterpret_cast<double*>(dev(s.eh, 8));
-        k_ensemble<<<(B + 63) / 64, 64, 0, m->stream>>>(e);
-        if (hipGetLastError() != hipSuccess || hipEventRecord(m->half[k % 2], m->stream) != hipSuccess)
-            return mlp_err(m, SL_E_HIP, "ensemble pass failed");
-        return SL_OK;
-    };
-    return sl::run_ahead((rows + per - 1) / per, halves ? 2 : 1, issue, collect, [&] { (void)hipStreamSynchronize(m->stream); });
+    return ensemble(ms, n, rows, x, mean, std, cls, reg, prob, ent);
+}
+
+int sl_mlp_ensemble32(sl_mlp* const* ms, int n, long long rows, const float* x, const float* mean, const float* std, int* cls,
+                      float* reg, double* prob, double* ent)
+{
+    return ensemble(ms, n, rows, x, mean, std, cls, reg, prob, ent);
 }
 
 int sl_mlp_gradients(sl_mlp* m, int B, const float* x, const int* cls, const float* reg, float* loss, float* grads)

@@ -230,8 +230,9 @@ class Surrogate:
     def predict(self, X):
         """(class, regression outputs, class probabilities, predictive entropy) of
         descriptor rows."""
-        if self._on_device(X):
-            return mlp_ensemble(self.mlps, X, self.norm.mean, self.norm.std)
+        dtype = self._device_dtype(X)
+        if dtype:
+            return mlp_ensemble(self.mlps, X, self.norm.mean, self.norm.std, dtype)
         Xn = self.norm(X)
         P = np.zeros((len(Xn), 3))
         Y = np.zeros((len(Xn), N_REG))
@@ -245,16 +246,18 @@ class Surrogate:
         ent = -(P * np.log(np.where(P > 0, P, 1.0))).sum(1)
         return P.argmax(1).astype(np.int32), Y.astype(np.float32), P, ent
 
-    def _on_device(self, X) -> bool:
-        """Whether mlp_ensemble says of X what the rest of predict would: its normalising is
-        numpy's where that is all in binary64, row by row; its outputs are the nets'."""
+    def _device_dtype(self, X):
+        """The type in which mlp_ensemble says of X what the rest of predict would: numpy's for
+        (X - mean) / std, row by row, of nets with the surrogate's outputs.  None if there is none."""
         if not (type(self.norm) is Normaliser and mlp_alike(self.mlps)):
-            return False
+            return None
         m, arrays = self.mlps[0], (X, self.norm.mean, self.norm.std)
-        return (all(type(a) is np.ndarray for a in arrays) and X.ndim == 2
+        if not (all(type(a) is np.ndarray for a in arrays) and X.ndim == 2
                 and {X.shape[1:], arrays[1].shape, arrays[2].shape} == {(m.n_in,)}
-                and np.result_type(*arrays[:2]) == np.result_type(*arrays) == np.float64
-                and m.n_out == 3 + N_REG and 1 <= self.max_batch <= m.max_batch)
+                and m.n_out == 3 + N_REG and 1 <= self.max_batch <= m.max_batch):
+            return None
+        dtype = np.result_type(*arrays[:2])
+        return dtype if dtype in (np.float32, np.float64) and np.result_type(*arrays) == dtype else None
 
     def calibrate_gate(self, X, cls, target: float) -> dict:
         """Smallest fallback share whose gated agreement on (X, cls) reaches ``target``:

@@ -2,12 +2,15 @@
 same, so every comparison is of bits.  Nets laid out alike share launches, up to 16 of them;
 nets of different widths or largest batch, in the layer form, or the same net twice go one by
 one."""
+import functools
+
 import numpy as np
 import pytest
 
 from conftest import bits_equal
 
 import spacelab_amd as sl
+from oracle.mlp import bf16
 
 pytestmark = pytest.mark.gpu
 
@@ -89,10 +92,19 @@ def test_ensemble_is_the_members_mean(members, max_batch, rows):
         m.close()
 
 
+@functools.lru_cache
 def _forms():
     X = np.random.default_rng(3).standard_normal((37, 21)) * 2 + 0.3
     f32 = lambda a: a.astype(np.float32)
-    return {"rows": (X, None), "fortran": (np.asfortranarray(X), None), "every other": (np.repeat(X, 2, 0)[::2], None),
+    # rows whose normalising rounds to other bfloat16 inputs in binary32 than in binary64
+    rng = np.random.default_rng(4)
+    mean, std = rng.standard_normal(21), rng.uniform(0.5, 2, 21)
+    Z = f32(rng.standard_normal((300000, 21)))
+    edge = Z[(bf16((Z - f32(mean)) / f32(std)) != bf16(f32((Z.astype(float) - f32(mean)) / f32(std)))).any(1)]
+    assert len(edge) > 5
+    return {"binary32 where it differs": (edge, f32), "halves": (X.astype(np.float16), f32),
+            "binary32 rows and mean": (edge, (f32, lambda a: a)),
+            "rows": (X, None), "fortran": (np.asfortranarray(X), None), "every other": (np.repeat(X, 2, 0)[::2], None),
             "reversed": (X[::-1, ::-1], None), "integers": ((10 * X).astype(np.int64), None), "list": (X.tolist(), None),
             "binary32 rows": (f32(X), None), "binary32 throughout": (f32(X), f32), "binary32 statistics": (X, f32),
             "extended": (X.astype(np.longdouble), None), "one column": (X[:, :1], None), "one row's statistics": (X, lambda a: a[None]),
@@ -108,7 +120,8 @@ def test_predict_takes_every_form_of_rows(form):
     rng = np.random.default_rng(4)
     mean, std = rng.standard_normal(21), rng.uniform(0.5, 2, 21)
     s = S.Surrogate(width=64, n_models=3, max_batch=16)
-    s.norm = S.Normaliser(mean, std) if change is None else S.Normaliser(change(mean), change(std))
+    change = change if isinstance(change, tuple) else (change, change)
+    s.norm = S.Normaliser(*(a if c is None else c(a) for c, a in zip(change, (mean, std))))
     Xn = np.ascontiguousarray((X - s.norm.mean) / s.norm.std, dtype=np.float32)
     P, Y = np.zeros((len(Xn), 3)), np.zeros((len(Xn), S.N_REG))
     for m in s.mlps:
