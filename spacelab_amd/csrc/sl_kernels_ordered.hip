@@ -181,7 +181,7 @@ struct BallRec {
 // to 64 at a time, before the turn (64 AD of them: beyond, ab is used again and the turn has to
 // come first).  Evaluated step by step, by the lanes that met them, and after the first AD steps
 // within the turn, a ball with a thousand contacts took 180 us a step at 1,000 balls and 836 at
-// 5,000; now 44 and 157, and 129 ordinary balls 8.4 instead of 9.6, 1,000 18.7 instead of 19.3.
+// 5,000; now 43 and 157, and 129 ordinary balls 8.3 instead of 9.7, 1,000 18.2 instead of 19.3.
 // With SCAN the workgroup first tests its balls against every partner
 // (16 instructions a step), and one wavefront evaluates the touching pairs found, up to
 // 64, side by side while the others start on their batches; a pair met in the sweep is then
@@ -493,28 +493,24 @@ void k_pairs_ordered(OrdState os, Phys P, int n, double* __restrict__ pe_ball,
         };
         // The batch's touching pairs, numbered ball by ball, j ascending.
         int first = 0, own_pairs = 0, pairs = 0;   // this lane's ball's first number, its pairs; all pairs
+        const unsigned long long own_lanes = (~0ull / ((1ull << NB) - 1)) << il;   // lanes of this lane's ball
         auto number_pairs = [&]() {
-            constexpr unsigned long long ball0 = ~0ull / ((1ull << NB) - 1);   // lanes of ball 0
-#pragma unroll 1
-            for (int b = 0; b < NB; b++) {
-                int c = 0;
 #pragma unroll
-                for (int q = 0; q < CH; q++) c += __popcll(__ballot((pend >> q) & 1u) & (ball0 << b));
-                if (b == il) {
-                    first = pairs;
-                    own_pairs = c;
-                }
+            for (int q = 0; q < CH; q++) own_pairs += __builtin_popcountll(__ballot((pend >> q) & 1u) & own_lanes);
+#pragma unroll
+            for (int b = 0; b < NB; b++) {
+                const int c = __builtin_amdgcn_readlane(own_pairs, b);   // lane b's ball is b
+                if (b < il) first += c;
                 pairs += c;
             }
         };
         // Contributions of pairs e0 .. e0 + AE - 1 to cb and ab, from the contact table or evaluated.
         auto fill_pairs = [&](int e0) {
-            constexpr unsigned long long ball0 = ~0ull / ((1ull << NB) - 1);
             int e = first - e0;
 #pragma unroll 1
             for (int q = 0; q < CH; q++) {
                 const bool mine = (pend >> q) & 1u;
-                const unsigned long long lanes = __ballot(mine) & (ball0 << il);
+                const unsigned long long lanes = __ballot(mine) & own_lanes;
                 const int at = e + lanes_below(lanes);
                 if (mine && at >= 0 && at < AE) numbered[w][at] = (unsigned char)(q << 6 | l);
                 e += __popcll(lanes);
