@@ -229,9 +229,10 @@ void k_pairs_ordered(OrdState os, Phys P, int n, double* __restrict__ pe_ball,
     constexpr int BP = CH * JS;             // partners per batch
     constexpr int NQ = WRITE ? 4 : 3;       // acc xyz, pair energy
     // A ball's contributions lie in a row, so that an adding lane reads two at once.  Row and
-    // component strides: the 32 lanes of half a wavefront's store (32/NB slots of NB balls) and
-    // the adding lanes' 16-byte reads each cover every LDS bank once.
-    constexpr int RS = (BP + 31) / 32 * 32 + 32 / NB, CS = NB * RS + 2;
+    // component strides: 16 lanes' stores (16/NB slots of NB balls) and 8 adding lanes' 16-byte
+    // reads each cover the 32 banks once (65 thousand conflict cycles a launch at 5,000 balls;
+    // 4.8 million when the stores were spread for 32 lanes and 64 banks, in the same time).
+    constexpr int RS = (BP + 31) / 32 * 32 + 16 / NB, CS = NB * RS + 2;
     constexpr int AH = BP < 16 ? BP : 16;   // contributions a lane adds from registers at once
     static_assert(64 % NB == 0 && BP <= 64 && NQ * NB <= 64 && BP % AH == 0 && CH <= 4, "batch shape");
     __shared__ __attribute__((aligned(16))) double cb[W][NQ][CS];   // acc contributions (and energies)
