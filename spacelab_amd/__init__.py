@@ -683,12 +683,12 @@ class Batch:
         return int(lib().sl_batch_step_count(self._b))
 
     def download(self) -> list[BallGroup]:
-        """Every group's state.  A group's arrays are parts of arrays of up to 16384 balls (2.4 MB
+        """Every group's state.  A group's arrays are parts of arrays of up to 32768 balls (4.7 MB
         with all eight) that it shares with its neighbours; arrays for the whole batch would all
         be kept while one group is."""
-        parts, end = [], 16384        # the groups' places in each part; balls in the last one
+        parts, end = [], 32768        # the groups' places in each part; balls in the last one
         for k in self.sizes:
-            if end + k > 16384:
+            if end + k > 32768:
                 parts.append([])
                 end = 0
             parts[-1].append(slice(end, end + k))

@@ -91,7 +91,7 @@ def test_a_kept_group_does_not_keep_the_batch():
             for f in ("pos", "vel", "w", "R", "m", "moi"):
                 assert bits_equal(getattr(o, f), getattr(g, f)), f
             held = {id(r): r.nbytes for r in (_root(getattr(o, f)) for f in ("pos", "vel", "w", "R", "m", "moi", "acc", "aacc"))}
-            assert sum(held.values()) <= 18 * 8 * max(16384, g.num_particles)
+            assert sum(held.values()) <= 18 * 8 * max(32768, g.num_particles)
     assert all(_root(e.p).nbytes <= 24 * 1024 for e in energies)
     with sl.Collider(2, _params(_grid(2, 0), order=sl.ORDER_FAST)) as c:
         c.upload(_grid(2, 0))
