@@ -167,7 +167,7 @@ struct BallRec {
 //             lane per (ball, component) adds its BP contributions in ascending j and hands
 //             the sums on.  aacc gets only the touching pairs' contributions: the others are
 //             +0.0, a no-op on a sum that starts at +0.0.
-// Only the adding is serial (about 20 cycles a partner), and only the wavefront whose turn
+// Only the adding is serial (6.5 cycles a partner), and only the wavefront whose turn
 // it is takes part in it: the others go on evaluating, with no barrier anywhere.  Every
 // sum has the same order whatever the shape, so all launch shapes give the same bits (the
 // energies included: per-ball sums, added over the balls in ascending order by the caller).
@@ -194,12 +194,12 @@ struct BallRec {
 // 26 spills more, the next batch's partners among them, which then had to arrive first.
 //
 // Bound by the binary64 pipe: 131 VALU instructions a step of 64 evaluations (105 of them the
-// reference's arithmetic), 150-170 with the staging, the adding and the contacts; at 15,039
-// balls that is 75% of the time, at 5,000 57% (1,250 workgroups, 3 to a CU).  Small systems are
-// bound by the chain of adds (6.5 cycles each and about 400 a batch) and by the first
+// reference's arithmetic), 165 with the staging, the adding and the contacts; at 15,039
+// balls that is 75% of the time, at 5,000 63% (1,250 workgroups, 3 to a CU).  Small systems are
+// bound by the chain of adds (about 400 cycles a batch of 64) and by the first
 // contacts' 5,000 cycles.  Measured per step, before (chunks of partners, a barrier each,
 // sums by a wavefront of its own, the kick in a launch of its own) and now: 129 balls 16.5 ->
-// 9 us, 1,000 29 -> 19, 2,200 87 -> 57, 5,000 259 -> 161, 15,039 1,750 -> 1,095.
+// 8.3 us, 1,000 29 -> 18.2, 2,200 87 -> 54.5, 5,000 259 -> 161, 15,039 1,750 -> 1,095.
 //
 // Write steps take a far pair's energy from the series (y <= 1/8; the logarithm and three
 // divisions cost two thirds of a step more, and spilled up to 72 registers) and two wavefronts

@@ -673,7 +673,8 @@ __global__ __launch_bounds__(256) void k_normalise(int n, int n_in, const T* x, 
 // regression outputs added in binary64 in their order and divided by their number, the most
 // probable class (the first of equals; the first NaN, if any) and the entropy.
 // With k_normalise in front and the nets' outputs kept on the device: 10,000 rows through four
-// nets 763 -> 246 us (the host's normalising, adding and entropy were three quarters of it).
+// nets 763 -> 246 us (the host's normalising, adding and entropy were three quarters of it);
+// binary32 rows 205 us.
 struct EnsembleArgs {
     long long at[MEMBERS];   // members' outputs, as in Moved
     int n, B, n_out;

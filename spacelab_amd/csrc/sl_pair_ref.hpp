@@ -97,8 +97,8 @@ __device__ __forceinline__ void sqrt_rcp(double x, double& s, double& y)
     y = __builtin_fma(__builtin_fma(-s, y2, 1.0), y2, y2);
 }
 
-// RN(n / d): two Newton steps on the hardware reciprocal, one residual correction (the
-// sequence of the compiler's division).
+// RN(n / d): two Newton steps on the hardware reciprocal, then Markstein's correction of the
+// quotient by its FMA-exact residual.
 __device__ __forceinline__ double div_plain(double n, double d)
 {
     double y = __builtin_amdgcn_rcp(d);
